@@ -168,10 +168,14 @@ def _tensor(array):
 _FUNCTORS = {"add": capi.OP_ADD, "max": capi.OP_MAX, "min": capi.OP_MIN}
 
 
+def _input_seed(seed):
+    """The generators' seed of one set of inputs."""
+    return datagen.DEFAULT_SEED ^ (seed * 0x9E3779B97F4A7C15 & 0xFFFFFFFFFFFFFFFF)
+
+
 def prepare(case, seed):
     n, kind, op = case["n"], case["type"], case["op"]
-    seed = datagen.DEFAULT_SEED ^ (seed * 0x9E3779B97F4A7C15 & 0xFFFFFFFFFFFFFFFF)
-    state = {"case": case, "source": _device_array(_values(case, seed), kind)}
+    state = {"case": case, "source": _device_array(_values(case, _input_seed(seed)), kind)}
     if op in ("sort", "pairs"):
         value_bytes = 0
         state["keys"] = capi.DeviceArray(n, kind)
@@ -263,3 +267,16 @@ def tolerance(case):
         if case["type"] == "float64":
             return {"rel": 5e-15}
     return "exact"
+
+
+def exact(case, seed):
+    """Sums in 64 bits by torch, where the result is rounded; orders, counts and
+    extrema have no rounding to compare."""
+    if case["op"] not in ("scan", "reduce") or case["functor"] != "add" \
+            or not case["type"].startswith("float"):
+        return None
+    column = _values(case, _input_seed(seed)).to(torch.float64)
+    if case["op"] == "reduce":
+        return column.sum().reshape(1)
+    total = torch.cumsum(column, 0)
+    return total if case["inclusive"] else torch.cat([total.new_zeros(1), total[:-1]])
