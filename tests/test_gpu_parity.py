@@ -262,6 +262,18 @@ def test_histogram_4096_bins_gaussian_mixture(n):
     assert_hist_equal(v, np.zeros(4096, dtype=np.uint64), capi.LOCATOR_IDENTITY)
 
 
+@pytest.mark.parametrize("bins", [1000, 4096, 12288])
+def test_histogram_lengths_where_the_number_of_blocks_changes(bins):
+    """A block per 16 elements of every bin, at least half a block per compute unit
+    (128), at most three (768)."""
+    for n in [1, 16 * bins * 127 + 5, 16 * bins * 130 + 3]:
+        note("histogram blocks", bins, n)
+        v = random_ints(np.int32, n, seed=n)
+        got, overflow = gpu_histogram(v, np.zeros(bins, dtype=np.int32), capi.LOCATOR_MODULO)
+        assert np.array_equal(got, np.bincount(np.abs(v.astype(np.int64)) % bins, minlength=bins))
+        assert not overflow
+
+
 def test_histogram_many_bins_uses_global_atomics():
     n, bins = 200000, 100000
     v = random_ints(np.int32, n, seed=4, lo=0, hi=bins - 1)
