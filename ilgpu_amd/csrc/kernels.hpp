@@ -95,8 +95,9 @@ struct TransformArgs {
 };
 int32_t launch_transform(hipStream_t stream, const TransformArgs& args);
 
-// fill kernel shared by scan and sort: words[0..count) = 0, as a kernel so
-// that callers may capture the stream into a graph.
-int32_t launch_zero_words(hipStream_t stream, uint32_t* words, int64_t count);
+// fill kernel shared by scan and sort: words[0..count) = 0, and more[0..more_count)
+// in the same launch, as a kernel so that callers may capture the stream into a graph.
+int32_t launch_zero_words(hipStream_t stream, uint32_t* words, int64_t count,
+                          uint32_t* more = nullptr, int64_t more_count = 0);
 
 }  // namespace ilgpu_hip

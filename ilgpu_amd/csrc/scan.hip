@@ -24,6 +24,7 @@
 // Each tile's words sit in a 128-byte line of their own.
 //
 // Algorithmic HBM traffic: 2 * n * sizeof(T) bytes (status: 128 B/tile).
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -84,6 +85,24 @@ constexpr int64_t kHeaderBytes = 256;  // ticket counter, padded
 template <typename T> constexpr int tile_elems() {
   return kBlock * scan_vecs<T>() * Vec16<T>::N;
 }
+// Short tiles, a quarter as long: an input of a few dozen full tiles leaves most
+// compute units idle, and the scan lasts as long as one tile takes from its
+// loads to its stores.  Inputs of two to kShortMaxTiles full tiles take them.
+// Their status words stand a quarter of a line apart, so that they fit the
+// temp view of the full tiles; that few words are not what such an input waits for.
+// (Kernel time in us, full / short tiles: 130 000 int32 18.0 / 6.8, 500 000 12.2 / 5.4, 10^6
+// 13.2 / 6.4, 1.9 * 10^6 float 18.2 / 9.9; 130 000 int64 9.8 / 5.5, 500 000 10.0 / 7.0, 10^6 the same.
+// From 128 full tiles on the longer chain costs more than the shorter tiles
+// save: a call on 2^21 int64 takes 14.3 / 17.5, on 2^22 18.0 / 30.0.)
+#ifndef ILGPU_HIP_SCAN_SHORT_DIVISOR
+#define ILGPU_HIP_SCAN_SHORT_DIVISOR 4
+#endif
+#ifndef ILGPU_HIP_SCAN_SHORT_MAX_TILES
+#define ILGPU_HIP_SCAN_SHORT_MAX_TILES 64
+#endif
+constexpr int kShortDivisor = ILGPU_HIP_SCAN_SHORT_DIVISOR;
+constexpr int64_t kShortMaxTiles = ILGPU_HIP_SCAN_SHORT_MAX_TILES;
+static_assert(kStatusStride / kShortDivisor >= 2, "two status words per tile of 8-byte elements");
 
 template <typename T> struct Bits;
 template <> struct Bits<int32_t> { using type = uint32_t; };
@@ -111,16 +130,17 @@ template <typename T, int SIZE = sizeof(T)> struct TileState;
 
 template <typename T> struct TileState<T, 4> {
   uint64_t* words;
+  int stride;  // words from one tile's to the next one's
   __device__ __forceinline__ void publish(int tile, uint32_t flag, T v) const {
     const uint64_t w = ((uint64_t)flag << 32) | to_bits(v);
-    __hip_atomic_store(&words[(int64_t)tile * kStatusStride], w, __ATOMIC_RELAXED,
+    __hip_atomic_store(&words[(int64_t)tile * stride], w, __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
   }
   // Spins until the tile has published something; returns its flag.
   __device__ __forceinline__ uint32_t wait(int tile, T* v) const {
     uint64_t w;
     while (true) {
-      w = __hip_atomic_load(&words[(int64_t)tile * kStatusStride], __ATOMIC_RELAXED,
+      w = __hip_atomic_load(&words[(int64_t)tile * stride], __ATOMIC_RELAXED,
                             __HIP_MEMORY_SCOPE_AGENT);
       if ((uint32_t)(w >> 32) != kFlagInvalid) break;
       __builtin_amdgcn_s_sleep(1);
@@ -138,9 +158,10 @@ template <typename T> struct TileState<T, 4> {
 // whole L2 of the XCD for every tile.
 template <typename T> struct TileState<T, 8> {
   uint64_t* words;
+  int stride;  // words from one tile's to the next one's
   __device__ __forceinline__ void publish(int tile, uint32_t flag, T v) const {
     const uint64_t bits = to_bits(v);
-    uint64_t* w = &words[(int64_t)tile * kStatusStride];
+    uint64_t* w = &words[(int64_t)tile * stride];
     __hip_atomic_store(&w[0], ((uint64_t)flag << 32) | (uint32_t)bits,
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(&w[1], ((uint64_t)flag << 32) | (bits >> 32),
@@ -148,7 +169,7 @@ template <typename T> struct TileState<T, 8> {
   }
   __device__ __forceinline__ uint32_t wait(int tile, T* v) const {
     uint64_t lo, hi;
-    const uint64_t* w = &words[(int64_t)tile * kStatusStride];
+    const uint64_t* w = &words[(int64_t)tile * stride];
     while (true) {
       lo = __hip_atomic_load(&w[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       hi = __hip_atomic_load(&w[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -282,7 +303,7 @@ __device__ __forceinline__ T resolve_prefix(const TileState<T>& st, int tile,
 // Four waves per SIMD, i.e. 128 registers and two blocks per CU: left to itself
 // the compiler takes 180 to 256 registers for the floating-point Max and Min
 // kernels, which halves their residency (measured 0.56 -> 0.44 ms at 2^28 float).
-template <typename T, int OP, bool VECTOR>
+template <typename T, int OP, bool VECTOR, int VECS>
 __global__ __launch_bounds__(kBlock, ILGPU_HIP_SCAN_WAVES_PER_EU) void scan_kernel(
     const T* __restrict__ in, T* __restrict__ out, int64_t n,
     int64_t in_stride, int64_t out_stride, int inclusive,
@@ -290,8 +311,8 @@ __global__ __launch_bounds__(kBlock, ILGPU_HIP_SCAN_WAVES_PER_EU) void scan_kern
   using F = Functor<T, OP>;
   using V = typename Vec16<T>::type;
   constexpr int VN = Vec16<T>::N;
-  constexpr int kTileVecs = scan_vecs<T>();
-  constexpr int kTile = tile_elems<T>();
+  constexpr int kTileVecs = VECS;
+  constexpr int kTile = kBlock * VECS * VN;
   constexpr int kWaveElems = kTile / kWaves;
 
   __shared__ int s_tile;
@@ -643,28 +664,30 @@ __global__ __launch_bounds__(kBlock) void unique_kernel(
     out_length[0] = (int64_t)s_prefix + (int64_t)block_total;
 }
 
-__global__ void zero_words_kernel(uint32_t* words, int64_t count) {
+__global__ void zero_words_kernel(uint32_t* words, int64_t count, uint32_t* more,
+                                  int64_t more_count) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count;
-       i += stride)
-    words[i] = 0u;
+  const int64_t first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  for (int64_t i = first; i < count; i += stride) words[i] = 0u;
+  for (int64_t i = first; i < more_count; i += stride) more[i] = 0u;
 }
 
 template <typename T> int64_t num_tiles(int64_t n) {
   return div_up(n, tile_elems<T>());
 }
 
-template <typename T, int OP>
-int32_t launch_typed(hipStream_t stream, const void* in, int64_t in_stride,
+template <typename T, int OP, int VECS>
+int32_t launch_tiles(hipStream_t stream, const void* in, int64_t in_stride,
                      void* out, int64_t out_stride, int64_t n, int32_t kind,
-                     void* temp) {
-  const int64_t tiles = num_tiles<T>(n);
+                     void* temp, int status_stride) {
+  const int64_t tiles = div_up(n, (int64_t)kBlock * VECS * Vec16<T>::N);
   char* base = reinterpret_cast<char*>(align_up((int64_t)(uintptr_t)temp, 256));
   uint32_t* ticket = reinterpret_cast<uint32_t*>(base);
   TileState<T> st;
   st.words = reinterpret_cast<uint64_t*>(base + kHeaderBytes);
+  st.stride = status_stride;
   if (tiles > 1) {
-    const int64_t zero_words = (kHeaderBytes + tiles * kStatusBytes) / 4;
+    const int64_t zero_words = (kHeaderBytes + tiles * status_stride * 8) / 4;
     const int32_t rc = launch_zero_words(stream, reinterpret_cast<uint32_t*>(base), zero_words);
     if (rc != ILGPU_HIP_SUCCESS) return rc;
   } else {
@@ -677,18 +700,30 @@ int32_t launch_typed(hipStream_t stream, const void* in, int64_t in_stride,
   const int inclusive = kind == ILGPU_HIP_SCAN_INCLUSIVE ? 1 : 0;
   ProfileScope scope(stream, "scan");
   if (vector) {
-    hipLaunchKernelGGL((scan_kernel<T, OP, true>), dim3((unsigned)tiles),
+    hipLaunchKernelGGL((scan_kernel<T, OP, true, VECS>), dim3((unsigned)tiles),
                        dim3(kBlock), 0, stream, static_cast<const T*>(in),
                        static_cast<T*>(out), n, in_stride, out_stride,
                        inclusive, ticket, st);
   } else {
-    hipLaunchKernelGGL((scan_kernel<T, OP, false>), dim3((unsigned)tiles),
+    hipLaunchKernelGGL((scan_kernel<T, OP, false, VECS>), dim3((unsigned)tiles),
                        dim3(kBlock), 0, stream, static_cast<const T*>(in),
                        static_cast<T*>(out), n, in_stride, out_stride,
                        inclusive, ticket, st);
   }
   ILGPU_HIP_CHECK(hipGetLastError());
   return ILGPU_HIP_SUCCESS;
+}
+
+template <typename T, int OP>
+int32_t launch_typed(hipStream_t stream, const void* in, int64_t in_stride,
+                     void* out, int64_t out_stride, int64_t n, int32_t kind,
+                     void* temp) {
+  const int64_t tiles = num_tiles<T>(n);
+  if (tiles > 1 && tiles <= kShortMaxTiles)
+    return launch_tiles<T, OP, scan_vecs<T>() / kShortDivisor>(
+        stream, in, in_stride, out, out_stride, n, kind, temp, kStatusStride / kShortDivisor);
+  return launch_tiles<T, OP, scan_vecs<T>()>(stream, in, in_stride, out, out_stride, n, kind,
+                                             temp, kStatusStride);
 }
 
 template <typename T>
@@ -712,13 +747,14 @@ int32_t launch_op(hipStream_t stream, const void* in, int64_t in_stride,
 
 }  // namespace
 
-int32_t launch_zero_words(hipStream_t stream, uint32_t* words, int64_t count) {
-  if (count <= 0) return ILGPU_HIP_SUCCESS;
-  int64_t blocks = div_up(count, 256 * 4);
+int32_t launch_zero_words(hipStream_t stream, uint32_t* words, int64_t count, uint32_t* more,
+                          int64_t more_count) {
+  if (count <= 0 && more_count <= 0) return ILGPU_HIP_SUCCESS;
+  int64_t blocks = div_up(std::max(count, more_count), 256 * 4);
   if (blocks > 2048) blocks = 2048;
   ProfileScope scope(stream, "zero_words");
   hipLaunchKernelGGL(zero_words_kernel, dim3((unsigned)blocks), dim3(256), 0,
-                     stream, words, count);
+                     stream, words, count, more, more_count);
   ILGPU_HIP_CHECK(hipGetLastError());
   return ILGPU_HIP_SUCCESS;
 }
@@ -804,6 +840,7 @@ int32_t launch_unique_typed(hipStream_t stream, void* data, int64_t n,
   uint32_t* ticket = reinterpret_cast<uint32_t*>(base);
   TileState<uint32_t> st;
   st.words = reinterpret_cast<uint64_t*>(base + kHeaderBytes);
+  st.stride = kStatusStride;
   if (tiles > 1) {
     const int32_t rc = launch_zero_words(stream, reinterpret_cast<uint32_t*>(base),
                                          (kHeaderBytes + tiles * kStatusBytes) / 4);

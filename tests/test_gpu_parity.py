@@ -1594,6 +1594,20 @@ def test_scan_tile_edges(dtype):
                 assert np.array_equal(got[:n], O.scan(vals, op=op, inclusive=inclusive)), (n, op, inclusive)
 
 
+@pytest.mark.parametrize("dtype", [np.int32, np.int64, np.float32])
+def test_scan_edges_of_the_short_tiles(dtype):
+    # a quarter of a full tile, for inputs of two to 64 full tiles
+    full = 512 * 16 * 16 // np.dtype(dtype).itemsize
+    short = full // 4
+    for n in [full + 1, full + short - 1, full + short, full + short + 1, 7 * short + 3,
+              64 * full - 1, 64 * full, 64 * full + 1]:
+        vals = random_ints(np.int32, n, seed=n, lo=-3, hi=4).astype(dtype)
+        for inclusive in (True, False):
+            note("short scan tile", np.dtype(dtype).name, n, inclusive)
+            got = gpu_scan(vals, capi.OP_ADD, inclusive)
+            assert np.array_equal(got[:n], O.scan(vals, op=capi.OP_ADD, inclusive=inclusive)), n
+
+
 # ------------------------------------------------------------- dominant digits
 # A digit that holds an eighth of the keys or more is ranked by ballots instead
 # of LDS slots (up to four such digits per pass).
