@@ -306,6 +306,40 @@ struct SortPlan {
   uint32_t last_executed;           // index of the last pass that runs
   uint32_t executed;                // number of passes that run
   uint32_t final_in_alt;            // result sits in the alternate buffer
+  uint32_t ties_left;               // the lower digits are left to ties_kernel
+};
+static_assert(sizeof(SortPlan) <= 256, "the temp view holds 256 bytes for the plan");
+
+// 8-byte keys whose upper halves rarely meet are sorted by that half alone, four
+// passes instead of eight; what is left is to order the few neighbours whose
+// upper halves are the same (ties_kernel), which reads the keys once.  Whether
+// they rarely meet no digit histogram tells, so the histogram kernel
+// also draws up to kTieSamples keys from positions that are independent of each
+// other and counts the draws whose upper half it has met before at another position,
+// in a hash table of kTieSlots entries, upper half and position (in the alternate key
+// buffer, which no pass has written yet).  m draws of which c meet an earlier one: about 2 n c / m^2 ties per
+// key.  The short way is taken up to half a tie per key: uniform keys have n / 2^32
+// of them.
+// From kTieMinKeys keys on: below that a pass takes so little time that the
+// sampling, the ties kernel and four passes that return at once cost the same.
+// (Whole sorts with the copy of the keys in front of them, all digits / upper half, us: 2^27
+// pairs of uniform u64 keys and generated u32 values 5964 / 3642, 2^22 pairs 289 / 188; keys
+// alone 2^27 4187 / 2760, 2^24 628 / 400, 2^21 177 / 122.  Where the draws say no the sampling
+// is lost: values below 10^6 as int64, three passes, 2^24 340 / 351, 2^22 126 / 132.)
+constexpr int kTiePasses = 4;                // passes over the upper half
+constexpr uint32_t kTieSamples = 1u << 17;
+constexpr uint32_t kTieSlotBits = 19;
+constexpr uint32_t kTieSlots = 1u << kTieSlotBits;
+#ifndef ILGPU_HIP_SORT_TIE_MIN_LOG2
+#define ILGPU_HIP_SORT_TIE_MIN_LOG2 21
+#endif
+constexpr int64_t kTieMinKeys = 1ll << ILGPU_HIP_SORT_TIE_MIN_LOG2;
+static_assert(kTieMinKeys >= (int64_t)kTieSlots, "the table lies in the alternate keys");
+struct TieSampling {
+  unsigned long long* table;  // nullptr: no sampling
+  uint32_t* collisions;       // eight counts, kTicketStride words apart
+  uint32_t samples;       // at most one per thread of the histogram's grid
+  uint32_t max_collisions;
 };
 
 // The first active lane's key, as a wave-uniform value.
@@ -328,11 +362,44 @@ __device__ __forceinline__ uint32_t readfirstlane_key(uint8_t k) {
 template <typename K, bool FLOAT_KEYS>
 __global__ __launch_bounds__(kHistBlock) void sort_histogram_kernel(
     const K* __restrict__ keys, int64_t n, KeyXform xf, int passes,
-    int replica_shift, uint32_t* __restrict__ global_hist) {
+    int replica_shift, uint32_t* __restrict__ global_hist, TieSampling ties) {
   using V = typename Vec16<K>::type;
   constexpr int VN = Vec16<K>::N;
   extern __shared__ uint32_t s_hist[];  // [passes][256][replicas]
   const int words = (passes * kRadix) << replica_shift;
+  // This thread's draw of the tie sampling.  Draws meet within their block first, in LDS: where
+  // many keys share an upper half, all draws of the grid would queue at one slot of the
+  // table (2^17 of them: 1.5 ms).  An empty slot holds 0, a draw its complement, so
+  // that small keys do not look like empty slots.  Of two draws that share a slot the
+  // later one stays, and a third that meets the first goes uncounted: rare at four
+  // slots per draw.
+  unsigned long long draw = 0, met = 0;  // upper half, position
+  bool collided = false, drawn = false;
+  if constexpr (sizeof(K) == 8) {
+    if (ties.table != nullptr) {
+      constexpr uint32_t kBlockSlots = 4 * kHistBlock;
+      static_assert(kBlockSlots <= (uint32_t)kRadix * 8, "a slot is a counter of the histogram");
+      const uint32_t s = blockIdx.x * (uint32_t)kHistBlock + threadIdx.x;
+      drawn = s < ties.samples;
+      if (drawn) {
+        uint64_t z = ((uint64_t)s + 1ull) * 0x9E3779B97F4A7C15ull;  // splitmix64
+        z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+        z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+        z ^= z >> 31;
+        const uint64_t at = __umul64hi(z, (uint64_t)n);
+        draw = (keys[at] & ~0xFFFFFFFFull) | at;
+      }
+      for (uint32_t i = threadIdx.x; i < kBlockSlots; i += kHistBlock) s_hist[i] = 0u;
+      __syncthreads();
+      const uint32_t upper = (uint32_t)(draw >> 32);
+      const uint32_t hash = upper * 0x9E3779B1u;
+      if (drawn)
+        collided = atomicExch(&s_hist[hash % kBlockSlots], ~upper) == ~upper;
+      if (drawn && !collided)
+        met = ~atomicExch(&ties.table[hash >> (32 - kTieSlotBits)], ~draw);
+      __syncthreads();
+    }
+  }
   for (int i = threadIdx.x; i < words; i += kHistBlock) s_hist[i] = 0u;
   __syncthreads();
 
@@ -483,7 +550,15 @@ __global__ __launch_bounds__(kHistBlock) void sort_histogram_kernel(
   }
   flush_key_run();
   flush_half_run();
-  __syncthreads();
+  if constexpr (sizeof(K) == 8) {
+    if (drawn && !collided) collided = (met >> 32) == (draw >> 32) && met != draw;
+    // One add per block, to one of eight lines: 2^11 adds to one word, a wave each, took 20 us.
+    const int collisions = __syncthreads_count(collided);
+    if (threadIdx.x == 0 && collisions != 0)
+      atomicAdd(ties.collisions + (blockIdx.x % kTicketGroups) * kTicketStride, (uint32_t)collisions);
+  } else {
+    __syncthreads();
+  }
 
   const int replicas = 1 << replica_shift;
   for (int b = threadIdx.x; b < passes * kRadix; b += kHistBlock) {
@@ -497,7 +572,7 @@ __global__ __launch_bounds__(kHistBlock) void sort_histogram_kernel(
 // ---- plan: exclusive digit offsets, skipped passes, buffer parity ---------
 __global__ __launch_bounds__(kRadix) void plan_kernel(
     const uint32_t* __restrict__ global_hist, uint32_t* __restrict__ excl,
-    SortPlan* __restrict__ plan, int passes, uint32_t n) {
+    SortPlan* __restrict__ plan, int passes, uint32_t n, TieSampling ties) {
   __shared__ uint32_t s_wave[kRadix / kWaveSize];
   __shared__ int s_trivial;
   __shared__ unsigned long long s_hot[kMaxHot];  // count << 8 | digit, most frequent first
@@ -510,6 +585,25 @@ __global__ __launch_bounds__(kRadix) void plan_kernel(
   uint32_t counts[kMaxPasses];
 #pragma unroll
   for (int p = 0; p < kMaxPasses; ++p) counts[p] = p < passes ? global_hist[p * kRadix + d] : 0u;
+  // The lower digits [0, left) are left to the ties if the draws rarely met and
+  // that saves at least two passes (a digit that all keys share needs none).
+  // An even number of passes ends in the caller's buffer, where the ties are ordered: an
+  // odd one takes a lower digit along.
+  int left = 0;
+  if (ties.table != nullptr) {
+    uint32_t collisions = 0;
+    for (int g = 0; g < kTicketGroups; ++g) collisions += ties.collisions[g * kTicketStride];
+    if (collisions <= ties.max_collisions) {
+      uint32_t varies = 0;
+#pragma unroll
+      for (int p = 0; p < kMaxPasses; ++p)
+        varies |= __syncthreads_or(counts[p] == n) ? 0u : 1u << p;
+      left = kMaxPasses - kTiePasses;
+      if (__popc(varies >> left) & 1)
+        while (left > 0 && !(varies >> --left & 1u)) {}
+      if (__popc(varies & ((1u << left) - 1u)) < 2) left = 0;
+    }
+  }
 #pragma unroll
   for (int p = 0; p < kMaxPasses; ++p) {
     if (p >= passes) break;
@@ -538,7 +632,7 @@ __global__ __launch_bounds__(kRadix) void plan_kernel(
     uint32_t off = 0;
     for (int w = 0; w < wave; ++w) off += s_wave[w];
     excl[p * kRadix + d] = off + inc - c;
-    const bool trivial = s_trivial != 0;
+    const bool trivial = s_trivial != 0 || p < left;
     if (d == 0) {
       plan->skip[p] = trivial ? 1u : 0u;
       plan->src_is_alt[p] = parity;
@@ -558,6 +652,7 @@ __global__ __launch_bounds__(kRadix) void plan_kernel(
     plan->last_executed = last;
     plan->executed = executed;
     plan->final_in_alt = parity;
+    plan->ties_left = left > 0 ? 1u : 0u;
   }
 }
 
@@ -1961,7 +2056,7 @@ void small_sort_kernel(typename KeyOf<KEY_BYTES>::type* keys,
 
 // ---- finish ----------------------------------------------------------------
 template <int KEY_BYTES, int VALUE_BYTES>
-__global__ __launch_bounds__(256) void finish_kernel(
+__device__ __forceinline__ void finish(
     typename KeyOf<KEY_BYTES>::type* keys_a,
     const typename KeyOf<KEY_BYTES>::type* keys_b,
     typename ValueOf<VALUE_BYTES>::type* vals_a,
@@ -1979,6 +2074,177 @@ __global__ __launch_bounds__(256) void finish_kernel(
       if constexpr (VALUE_BYTES > 0) vals_a[i] = vals_b[i];
     } else {
       if constexpr (VALUE_BYTES > 0) vals_a[i] = index_value<VALUE_BYTES>(i, values_from_index);
+    }
+  }
+}
+
+template <int KEY_BYTES, int VALUE_BYTES>
+__global__ __launch_bounds__(256) void finish_kernel(
+    typename KeyOf<KEY_BYTES>::type* keys_a,
+    const typename KeyOf<KEY_BYTES>::type* keys_b,
+    typename ValueOf<VALUE_BYTES>::type* vals_a,
+    const typename ValueOf<VALUE_BYTES>::type* vals_b, int64_t n,
+    const SortPlan* __restrict__ plan, int values_from_index) {
+  finish<KEY_BYTES, VALUE_BYTES>(keys_a, keys_b, vals_a, vals_b, n, plan, values_from_index);
+}
+
+// ---- ties of the upper half --------------------------------------------------
+// After the passes over the upper half (plan->ties_left): keys whose upper halves
+// are the same stand next to each other in their original order.  Every run of such
+// keys is put into the order of the whole key, equal keys left in their order,
+// by the lane that sees its first key (runs of up to kTieRun keys, nearly always
+// two), or by that lane's wave.  Nobody else writes the run, and whoever looks
+// at its neighbours compares upper halves, which do not change.
+//
+// A read of the keys, then: a lane takes kTieRows keys, a row of a wave 64
+// neighbouring ones, and the runs of all rows are ordered together, since each
+// costs a chain of two or three memory round trips. 
+constexpr int kTieRows = 8;
+constexpr int kTieRun = 16;
+
+// A run of more than kTieRun keys, by a whole wave: a look at its order first (many
+// copies of one key need nothing), then a stable merge sort, every key finding its
+// place in the other half by bisection; the other buffer's same range is scratch.
+// The sampling lets runs of some 2^-13 of the input pass at most.
+template <typename Val, int VALUE_BYTES>
+__device__ void order_long_run(uint64_t* keys, uint64_t* other_keys, Val* vals, Val* other_vals,
+                               int64_t start, int64_t n, const KeyXform& xf, int lane) {
+  const uint32_t upper = (uint32_t)(keys[start] >> 32);
+  int64_t len = 0;
+  bool inverted = false;
+  for (;;) {
+    const int64_t i = start + len + lane;
+    const bool same = i < n && (uint32_t)(keys[i] >> 32) == upper;
+    if (same && i + 1 < n) {
+      const uint64_t next = keys[i + 1];
+      if ((uint32_t)(next >> 32) == upper && ordered_bits(next, xf) < ordered_bits(keys[i], xf))
+        inverted = true;
+    }
+    const uint64_t lanes = __ballot(same);
+    len += __popcll(lanes);
+    if (lanes != ~0ull) break;
+  }
+  if (__ballot(inverted) == 0ull) return;
+  uint64_t* src = keys + start;
+  uint64_t* dst = other_keys + start;
+  Val* src_vals = VALUE_BYTES > 0 ? vals + start : nullptr;
+  Val* dst_vals = VALUE_BYTES > 0 ? other_vals + start : nullptr;
+  for (int64_t width = 1; width < len; width <<= 1) {
+    for (int64_t i = lane; i < len; i += kWaveSize) {
+      const uint64_t k = src[i];
+      const uint64_t o = ordered_bits(k, xf);
+      const int64_t pair = i & ~(2 * width - 1);
+      const int64_t middle = pair + width < len ? pair + width : len;
+      const int64_t end = pair + 2 * width < len ? pair + 2 * width : len;
+      const bool left = i < middle;
+      int64_t lo = left ? middle : pair, hi = left ? end : middle;
+      const int64_t first = lo;
+      while (lo < hi) {  // keys of the other half that go in front of this one
+        const int64_t m = lo + (hi - lo) / 2;
+        const uint64_t q = ordered_bits(src[m], xf);
+        if (left ? q < o : q <= o) lo = m + 1;
+        else hi = m;
+      }
+      const int64_t at = pair + (left ? i - pair : i - middle) + (lo - first);
+      dst[at] = k;
+      if constexpr (VALUE_BYTES > 0) dst_vals[at] = src_vals[i];
+    }
+    __threadfence();  // the next step reads what other lanes wrote
+    uint64_t* k = src; src = dst; dst = k;
+    Val* v = src_vals; src_vals = dst_vals; dst_vals = v;
+  }
+  if (src != keys + start) {
+    for (int64_t i = lane; i < len; i += kWaveSize) {
+      dst[i] = src[i];
+      if constexpr (VALUE_BYTES > 0) dst_vals[i] = src_vals[i];
+    }
+  }
+}
+
+template <int VALUE_BYTES>
+__global__ __launch_bounds__(256) void ties_kernel(
+    uint64_t* keys_a, uint64_t* keys_b, typename ValueOf<VALUE_BYTES>::type* vals_a,
+    typename ValueOf<VALUE_BYTES>::type* vals_b, int64_t n, KeyXform xf,
+    const SortPlan* __restrict__ plan, int values_from_index) {
+  using Val = typename ValueOf<VALUE_BYTES>::type;
+  if (plan->ties_left == 0) {  // every digit was sorted
+    finish<8, VALUE_BYTES>(keys_a, keys_b, vals_a, vals_b, n, plan, values_from_index);
+    return;
+  }
+  uint64_t* keys = keys_a;  // an even number of passes ran
+  Val* vals = vals_a;
+  const int lane = threadIdx.x & (kWaveSize - 1);
+  const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWaveSize;
+  const int64_t waves = (int64_t)gridDim.x * blockDim.x / kWaveSize;
+  constexpr int64_t kChunk = kTieRows * kWaveSize;
+  for (int64_t base = wave * kChunk; base < n; base += waves * kChunk) {
+    // Upper halves of the rows; what lies outside of the input repeats the
+    // nearest key and is masked below.
+    uint32_t upper[kTieRows];
+#pragma unroll
+    for (int r = 0; r < kTieRows; ++r) {
+      const int64_t i = base + r * kWaveSize + lane;
+      upper[r] = (uint32_t)(keys[i < n ? i : n - 1] >> 32);
+    }
+    uint32_t before = (uint32_t)(keys[base > 0 ? base - 1 : 0] >> 32);
+    const uint32_t after = (uint32_t)(keys[base + kChunk < n ? base + kChunk : n - 1] >> 32);
+    uint32_t leads = 0;  // rows in which this lane holds a run's first key
+#pragma unroll
+    for (int r = 0; r < kTieRows; ++r) {
+      const int64_t i = base + r * kWaveSize + lane;
+      const uint32_t last = (uint32_t)__builtin_amdgcn_readlane((int)upper[r], kWaveSize - 1);
+      const uint32_t following =
+          r + 1 < kTieRows ? (uint32_t)__builtin_amdgcn_readfirstlane((int)upper[r + 1 < kTieRows ? r + 1 : r])
+                           : after;
+      uint32_t prev = shfl_up(upper[r], 1);
+      uint32_t next = __shfl_down(upper[r], 1);
+      if (lane == 0) prev = before;
+      if (lane == kWaveSize - 1) next = following;
+      if (i + 1 < n && next == upper[r] && (i == 0 || prev != upper[r])) leads |= 1u << r;
+      before = last;
+    }
+    while (__ballot(leads != 0) != 0ull) {
+      int64_t start = 0;
+      bool is_long = false;
+      if (leads != 0) {
+        start = base + (int64_t)(__builtin_ctz(leads) * kWaveSize + lane);
+        leads &= leads - 1;
+        const uint64_t k0 = keys[start];
+        int len = 2;
+        while (start + len < n && (keys[start + len] >> 32) == (k0 >> 32)) {
+          if (++len > kTieRun) break;
+        }
+        is_long = len > kTieRun;
+        if (!is_long) {
+          for (int j = 1; j < len; ++j) {
+            const uint64_t k = keys[start + j];
+            const uint64_t o = ordered_bits(k, xf);
+            int at = j;
+            Val v{};
+            for (; at > 0; --at) {
+              const uint64_t q = keys[start + at - 1];
+              if (ordered_bits(q, xf) <= o) break;
+              if constexpr (VALUE_BYTES > 0) {
+                if (at == j) v = vals[start + j];
+                vals[start + at] = vals[start + at - 1];
+              }
+              keys[start + at] = q;
+            }
+            if (at < j) {
+              keys[start + at] = k;
+              if constexpr (VALUE_BYTES > 0) vals[start + at] = v;
+            }
+          }
+        }
+      }
+      for (uint64_t longs = __ballot(is_long); longs != 0ull; longs &= longs - 1) {
+        const int owner = __builtin_ctzll(longs);
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)start, owner);
+        const uint32_t hi =
+            (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)start >> 32), owner);
+        order_long_run<Val, VALUE_BYTES>(keys, keys_b, vals, vals_b,
+                                         (int64_t)(((uint64_t)hi << 32) | lo), n, xf, lane);
+      }
     }
   }
 }
@@ -2252,7 +2518,15 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
                              ? 1
                              : (a.value_source == ILGPU_HIP_VALUES_FROM_INDEX_AS_FLOAT ? 2 : 0);
 
-  int32_t rc = launch_zero_words(stream, hist, (L.total - L.zero_begin) / 4);
+  TieSampling ties{};
+  if (KEY_BYTES == 8 && a.n >= kTieMinKeys) {
+    ties.table = reinterpret_cast<unsigned long long*>(keys_b);
+    // A word of the first ticket's line that no group uses, cleared with it.
+    ties.collisions = reinterpret_cast<uint32_t*>(base + L.tickets) + 1;
+  }
+  int32_t rc = launch_zero_words(stream, hist, (L.total - L.zero_begin) / 4,
+                                 reinterpret_cast<uint32_t*>(ties.table),
+                                 ties.table != nullptr ? 2 * (int64_t)kTieSlots : 0);
   if (rc != ILGPU_HIP_SUCCESS) return rc;
 
   {
@@ -2273,6 +2547,11 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
     if (blocks > (int64_t)cus * ILGPU_HIP_SORT_HIST_BLOCKS_PER_CU)
       blocks = (int64_t)cus * ILGPU_HIP_SORT_HIST_BLOCKS_PER_CU;
     if (blocks < 1) blocks = 1;
+    if (ties.table != nullptr) {
+      ties.samples = (uint32_t)std::min<int64_t>(kTieSamples, blocks * kHistBlock);
+      ties.max_collisions =
+          (uint32_t)((uint64_t)ties.samples * ties.samples / (4ull * (uint64_t)a.n));
+    }
     ProfileScope scope(stream, "sort_histogram");
     auto* histogram_kernel = sort_histogram_kernel<K, false>;
     if constexpr (KEY_BYTES >= 2) {  // there is no 1-byte floating-point key
@@ -2280,13 +2559,13 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
     }
     hipLaunchKernelGGL(histogram_kernel, dim3((unsigned)blocks),
                        dim3(kHistBlock), lds, stream, keys_a, a.n, xf, passes,
-                       shift, hist);
+                       shift, hist, ties);
     ILGPU_HIP_CHECK(hipGetLastError());
   }
   {
     ProfileScope scope(stream, "sort_plan");
     hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(kRadix), 0, stream, hist, excl,
-                       plan, passes, (uint32_t)a.n);
+                       plan, passes, (uint32_t)a.n, ties);
   }
   ILGPU_HIP_CHECK(hipGetLastError());
 
@@ -2310,6 +2589,17 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
   } else
     rc = launch_passes<KEY_BYTES, VALUE_BYTES, kSortBlock>(stream, a, L, base, xf, cus);
   if (rc != ILGPU_HIP_SUCCESS) return rc;
+  if constexpr (KEY_BYTES == 8) {
+    if (ties.table != nullptr) {
+      int64_t blocks = div_up(a.n, 256 * kTieRows);
+      if (blocks > (int64_t)cus * 8) blocks = (int64_t)cus * 8;
+      ProfileScope scope(stream, "sort_finish");
+      hipLaunchKernelGGL((ties_kernel<VALUE_BYTES>), dim3((unsigned)blocks), dim3(256), 0, stream,
+                         keys_a, keys_b, vals_a, vals_b, a.n, xf, plan, from_index);
+      ILGPU_HIP_CHECK(hipGetLastError());
+      return ILGPU_HIP_SUCCESS;
+    }
+  }
   {
     // Mostly there is nothing to copy and every block returns at once; 16
     // keys per thread are few enough blocks for that and enough for the copy.

@@ -1856,3 +1856,90 @@ def test_calls_can_be_captured_into_a_graph_and_replayed():
         assert junk > 0
         graph.replay()
         check(k, v, ("replay", r))
+
+
+def upper_half_keys(n, seed, run_lengths=()):
+    """64-bit patterns whose upper halves are random, but for runs of keys, at
+    random places, that share one and whose lower halves take a few values."""
+    rng = np.random.default_rng(seed)
+    keys = rng.integers(0, 1 << 64, n, dtype=np.uint64)
+    places = rng.permutation(n)
+    at = 0
+    for length in run_lengths:
+        upper = rng.integers(0, 1 << 32, dtype=np.uint64) << np.uint64(32)
+        lower = rng.integers(0, max(length // 2, 2), length, dtype=np.uint64)
+        keys[places[at:at + length]] = upper | lower
+        at += length
+    return keys
+
+
+# Lengths around one row of a wave and the longest run that one lane orders.
+TIE_RUNS = [2, 2, 3, 15, 16, 17, 18, 63, 64, 65, 66, 127, 1000, 2500]
+TIE_LENGTH = (1 << 21) + 3  # the shortest inputs sorted by the upper half are 2^21 keys
+
+
+@pytest.mark.parametrize("dtype,descending,total_order", [
+    (np.uint64, False, False), (np.int64, True, False), (np.float64, False, False),
+    (np.float64, True, True)])
+@pytest.mark.parametrize("value_dtype", [None, np.uint32, np.uint64])
+def test_sort_by_the_upper_half_orders_the_ties(dtype, descending, total_order, value_dtype):
+    n = TIE_LENGTH
+    note("upper half", np.dtype(dtype).name, descending, total_order, value_dtype)
+    bits = upper_half_keys(n, 77, TIE_RUNS)
+    bits[1000:3000] = bits[5]  # many copies of one key
+    sign = np.uint64(1 << 63)
+    top = bits >> np.uint64(63)
+    if dtype is np.uint64:
+        order_bits = bits
+    elif dtype is np.int64:
+        order_bits = bits ^ sign
+    elif total_order:
+        order_bits = np.where(top == 1, ~bits, bits ^ sign)
+    else:  # the order as written: the last bit of positive values is flipped
+        order_bits = bits ^ sign ^ (np.uint64(1) - top)
+    order = np.argsort(~order_bits if descending else order_bits, kind="stable")
+    keys = D.from_numpy(bits.view(dtype))
+    value_bytes = 0 if value_dtype is None else np.dtype(value_dtype).itemsize
+    temp = capi.temp_buffer(capi.radix_sort_temp_bytes(n, dtype, value_bytes))
+    if value_dtype is None:
+        capi.radix_sort_keys(keys, temp, descending=descending, float_total_order=total_order)
+    else:
+        from_index = value_dtype is np.uint32
+        values = D.zeros(n, value_dtype) if from_index else D.from_numpy(
+            np.arange(n, dtype=value_dtype))
+        capi.radix_sort_pairs(keys, values, temp, descending=descending,
+                              float_total_order=total_order, values_from_index=from_index)
+    sync()
+    assert capi.radix_sort_passes(temp, n, dtype, value_bytes) == (4, 4)
+    assert np.array_equal(keys.numpy().view(np.uint64), bits[order])
+    if value_dtype is not None:
+        assert np.array_equal(values.numpy(), order.astype(value_dtype))
+
+
+@pytest.mark.parametrize("kind,passes", [
+    ("grouped", 8), ("few lower digits", 5), ("one upper digit", 3), ("constant", 0),
+    ("three upper digits", 4)])
+def test_sort_of_long_inputs_chooses_its_digits(kind, passes):
+    """Few upper halves, or no two passes to save: every digit is sorted (a digit
+    that all keys share needs no pass either way)."""
+    n = TIE_LENGTH
+    note("upper halves that meet", kind)
+    rng = np.random.default_rng(5)
+    keys = upper_half_keys(n, 78)
+    if kind == "grouped":
+        keys = (rng.choice(keys[:1000], n) & ~np.uint64(0xFFFFFFFF)) | (keys >> np.uint64(32))
+    elif kind == "few lower digits":
+        keys &= ~np.uint64(0xFFFFFF)
+    elif kind == "three upper digits":  # and one of the lower half
+        keys >>= np.uint64(8)
+    elif kind == "one upper digit":
+        keys = rng.integers(0, 1 << 24, n, dtype=np.uint64)
+    else:
+        keys[:] = keys[0]
+    d, v = D.from_numpy(keys), D.zeros(n, np.uint32)
+    temp = capi.temp_buffer(capi.radix_sort_temp_bytes(n, np.uint64, 4))
+    capi.radix_sort_pairs(d, v, temp, values_from_index=True)
+    sync()
+    assert capi.radix_sort_passes(temp, n, np.uint64, 4)[0] == passes
+    order = np.argsort(keys, kind="stable")
+    assert np.array_equal(d.numpy(), keys[order]) and np.array_equal(v.numpy(), order)
