@@ -323,12 +323,14 @@ static_assert(sizeof(SortPlan) <= 256, "the temp view holds 256 bytes for the pl
 // From kTieMinKeys keys on: below that a pass takes so little time that the
 // sampling, the ties kernel and four passes that return at once cost the same.
 // (Whole sorts with the copy of the keys in front of them, all digits / upper half, us: 2^27
-// pairs of uniform u64 keys and generated u32 values 5964 / 3642, 2^22 pairs 289 / 188; keys
-// alone 2^27 4187 / 2760, 2^24 628 / 400, 2^21 177 / 122.  Where the draws say no the sampling
-// is lost: values below 10^6 as int64, three passes, 2^24 340 / 351, 2^22 126 / 132.)
+// pairs of uniform u64 keys and generated u32 values 5964 / 3642, 2^22 pairs 289 / 183; keys
+// alone 2^27 4187 / 2760, 2^24 616 / 388, 2^21 177 / 122.  Where the draws say no the sampling
+// is lost: values below 10^6 as int64, three passes, 2^24 336 / 337, 2^22 126 / 127; with
+// 2^17 draws, a table of 2^19 entries and fewer waves in the last kernel 340 / 351 and
+// 126 / 132.)
 constexpr int kTiePasses = 4;                // passes over the upper half
-constexpr uint32_t kTieSamples = 1u << 17;
-constexpr uint32_t kTieSlotBits = 19;
+constexpr uint32_t kTieSamples = 1u << 16;
+constexpr uint32_t kTieSlotBits = 18;
 constexpr uint32_t kTieSlots = 1u << kTieSlotBits;
 #ifndef ILGPU_HIP_SORT_TIE_MIN_LOG2
 #define ILGPU_HIP_SORT_TIE_MIN_LOG2 21
@@ -369,7 +371,7 @@ __global__ __launch_bounds__(kHistBlock) void sort_histogram_kernel(
   const int words = (passes * kRadix) << replica_shift;
   // This thread's draw of the tie sampling.  Draws meet within their block first, in LDS: where
   // many keys share an upper half, all draws of the grid would queue at one slot of the
-  // table (2^17 of them: 1.5 ms).  An empty slot holds 0, a draw its complement, so
+  // table (2^17 draws: 1.5 ms).  An empty slot holds 0, a draw its complement, so
   // that small keys do not look like empty slots.  Of two draws that share a slot the
   // later one stays, and a third that meets the first goes uncounted: rare at four
   // slots per draw.
@@ -2161,8 +2163,9 @@ __device__ void order_long_run(uint64_t* keys, uint64_t* other_keys, Val* vals, 
   }
 }
 
+// (Compiled for 32 waves per CU, as the copy of finish() wants them too.)
 template <int VALUE_BYTES>
-__global__ __launch_bounds__(256) void ties_kernel(
+__global__ __launch_bounds__(256, 8) void ties_kernel(
     uint64_t* keys_a, uint64_t* keys_b, typename ValueOf<VALUE_BYTES>::type* vals_a,
     typename ValueOf<VALUE_BYTES>::type* vals_b, int64_t n, KeyXform xf,
     const SortPlan* __restrict__ plan, int values_from_index) {
