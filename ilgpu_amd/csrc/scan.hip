@@ -9,7 +9,8 @@
 //
 // Tile layout (kBlock = 512 threads, 8 waves, kVecs = 16 16-byte vectors per
 // lane, i.e. 128 KiB per tile: time per launch falls with the number of tiles
-// until about this size, then register pressure takes over):
+// until about this size, then register pressure takes over; inputs of two to 64 such
+// tiles take short ones of 32 KiB):
 //   wave w owns a contiguous chunk of kVecs*64 vectors; vector j of lane l is
 //   chunk[j*64 + l], so every load/store instruction of a wave covers 1 KiB of
 //   consecutive addresses (dwordx4 per lane).  Scan order inside a wave is
@@ -21,9 +22,10 @@
 // eight XCDs of the device have separate L2s.
 //   4-byte T: one 64-bit word {flag, value} per tile;
 //   8-byte T: two such words per tile, one per half of the value.
-// Each tile's words sit in a 128-byte line of their own.
+// Each tile's words sit in a 128-byte line of their own, or in a quarter of one
+// where the tiles are short (kShortDivisor).
 //
-// Algorithmic HBM traffic: 2 * n * sizeof(T) bytes (status: 128 B/tile).
+// Algorithmic HBM traffic: 2 * n * sizeof(T) bytes (status: 128 B/tile, 32 B/short tile).
 #include <algorithm>
 #include <atomic>
 #include <mutex>
@@ -103,6 +105,10 @@ template <typename T> constexpr int tile_elems() {
 constexpr int kShortDivisor = ILGPU_HIP_SCAN_SHORT_DIVISOR;
 constexpr int64_t kShortMaxTiles = ILGPU_HIP_SCAN_SHORT_MAX_TILES;
 static_assert(kStatusStride / kShortDivisor >= 2, "two status words per tile of 8-byte elements");
+// Status words per tile of VECS vectors per thread.
+template <typename T, int VECS> constexpr int status_stride() {
+  return VECS == scan_vecs<T>() ? kStatusStride : kStatusStride / kShortDivisor;
+}
 
 template <typename T> struct Bits;
 template <> struct Bits<int32_t> { using type = uint32_t; };
@@ -125,22 +131,23 @@ __device__ __forceinline__ T from_bits(typename Bits<T>::type b) {
   return v;
 }
 
-// Look-back state in temp memory.
-template <typename T, int SIZE = sizeof(T)> struct TileState;
+// Look-back state in temp memory; STRIDE words from one tile's to the next one's.
+// (A constant: as a member of the structure it cost unique_kernel<uint32_t> two
+// vector registers and four more spilled scalar ones, 1 % of a call on 2^26 keys.)
+template <typename T, int STRIDE = kStatusStride, int SIZE = sizeof(T)> struct TileState;
 
-template <typename T> struct TileState<T, 4> {
+template <typename T, int STRIDE> struct TileState<T, STRIDE, 4> {
   uint64_t* words;
-  int stride;  // words from one tile's to the next one's
   __device__ __forceinline__ void publish(int tile, uint32_t flag, T v) const {
     const uint64_t w = ((uint64_t)flag << 32) | to_bits(v);
-    __hip_atomic_store(&words[(int64_t)tile * stride], w, __ATOMIC_RELAXED,
+    __hip_atomic_store(&words[(int64_t)tile * STRIDE], w, __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
   }
   // Spins until the tile has published something; returns its flag.
   __device__ __forceinline__ uint32_t wait(int tile, T* v) const {
     uint64_t w;
     while (true) {
-      w = __hip_atomic_load(&words[(int64_t)tile * stride], __ATOMIC_RELAXED,
+      w = __hip_atomic_load(&words[(int64_t)tile * STRIDE], __ATOMIC_RELAXED,
                             __HIP_MEMORY_SCOPE_AGENT);
       if ((uint32_t)(w >> 32) != kFlagInvalid) break;
       __builtin_amdgcn_s_sleep(1);
@@ -156,12 +163,11 @@ template <typename T> struct TileState<T, 4> {
 // the halves of the same value; a reader that catches the words in different
 // states reads again.  No fences: an agent-scope release would write back the
 // whole L2 of the XCD for every tile.
-template <typename T> struct TileState<T, 8> {
+template <typename T, int STRIDE> struct TileState<T, STRIDE, 8> {
   uint64_t* words;
-  int stride;  // words from one tile's to the next one's
   __device__ __forceinline__ void publish(int tile, uint32_t flag, T v) const {
     const uint64_t bits = to_bits(v);
-    uint64_t* w = &words[(int64_t)tile * stride];
+    uint64_t* w = &words[(int64_t)tile * STRIDE];
     __hip_atomic_store(&w[0], ((uint64_t)flag << 32) | (uint32_t)bits,
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(&w[1], ((uint64_t)flag << 32) | (bits >> 32),
@@ -169,7 +175,7 @@ template <typename T> struct TileState<T, 8> {
   }
   __device__ __forceinline__ uint32_t wait(int tile, T* v) const {
     uint64_t lo, hi;
-    const uint64_t* w = &words[(int64_t)tile * stride];
+    const uint64_t* w = &words[(int64_t)tile * STRIDE];
     while (true) {
       lo = __hip_atomic_load(&w[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       hi = __hip_atomic_load(&w[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -269,8 +275,8 @@ __device__ __forceinline__ T wave_reduce(T v) {
 
 // Executed by the first wave of the block.  Publishes the tile's aggregate,
 // resolves the exclusive prefix of the tile and publishes the inclusive one.
-template <typename T, int OP>
-__device__ __forceinline__ T resolve_prefix(const TileState<T>& st, int tile,
+template <typename T, int OP, int STRIDE>
+__device__ __forceinline__ T resolve_prefix(const TileState<T, STRIDE>& st, int tile,
                                             T aggregate, int lane) {
   using F = Functor<T, OP>;
   if (tile == 0) {
@@ -307,7 +313,7 @@ template <typename T, int OP, bool VECTOR, int VECS>
 __global__ __launch_bounds__(kBlock, ILGPU_HIP_SCAN_WAVES_PER_EU) void scan_kernel(
     const T* __restrict__ in, T* __restrict__ out, int64_t n,
     int64_t in_stride, int64_t out_stride, int inclusive,
-    uint32_t* __restrict__ ticket, TileState<T> st) {
+    uint32_t* __restrict__ ticket, TileState<T, status_stride<T, VECS>()> st) {
   using F = Functor<T, OP>;
   using V = typename Vec16<T>::type;
   constexpr int VN = Vec16<T>::N;
@@ -679,15 +685,14 @@ template <typename T> int64_t num_tiles(int64_t n) {
 template <typename T, int OP, int VECS>
 int32_t launch_tiles(hipStream_t stream, const void* in, int64_t in_stride,
                      void* out, int64_t out_stride, int64_t n, int32_t kind,
-                     void* temp, int status_stride) {
+                     void* temp) {
   const int64_t tiles = div_up(n, (int64_t)kBlock * VECS * Vec16<T>::N);
   char* base = reinterpret_cast<char*>(align_up((int64_t)(uintptr_t)temp, 256));
   uint32_t* ticket = reinterpret_cast<uint32_t*>(base);
-  TileState<T> st;
+  TileState<T, status_stride<T, VECS>()> st;
   st.words = reinterpret_cast<uint64_t*>(base + kHeaderBytes);
-  st.stride = status_stride;
   if (tiles > 1) {
-    const int64_t zero_words = (kHeaderBytes + tiles * status_stride * 8) / 4;
+    const int64_t zero_words = (kHeaderBytes + tiles * status_stride<T, VECS>() * 8) / 4;
     const int32_t rc = launch_zero_words(stream, reinterpret_cast<uint32_t*>(base), zero_words);
     if (rc != ILGPU_HIP_SUCCESS) return rc;
   } else {
@@ -721,9 +726,8 @@ int32_t launch_typed(hipStream_t stream, const void* in, int64_t in_stride,
   const int64_t tiles = num_tiles<T>(n);
   if (tiles > 1 && tiles <= kShortMaxTiles)
     return launch_tiles<T, OP, scan_vecs<T>() / kShortDivisor>(
-        stream, in, in_stride, out, out_stride, n, kind, temp, kStatusStride / kShortDivisor);
-  return launch_tiles<T, OP, scan_vecs<T>()>(stream, in, in_stride, out, out_stride, n, kind,
-                                             temp, kStatusStride);
+        stream, in, in_stride, out, out_stride, n, kind, temp);
+  return launch_tiles<T, OP, scan_vecs<T>()>(stream, in, in_stride, out, out_stride, n, kind, temp);
 }
 
 template <typename T>
@@ -840,7 +844,6 @@ int32_t launch_unique_typed(hipStream_t stream, void* data, int64_t n,
   uint32_t* ticket = reinterpret_cast<uint32_t*>(base);
   TileState<uint32_t> st;
   st.words = reinterpret_cast<uint64_t*>(base + kHeaderBytes);
-  st.stride = kStatusStride;
   if (tiles > 1) {
     const int32_t rc = launch_zero_words(stream, reinterpret_cast<uint32_t*>(base),
                                          (kHeaderBytes + tiles * kStatusBytes) / 4);
