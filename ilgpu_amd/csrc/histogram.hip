@@ -19,6 +19,7 @@
 //
 // Algorithmic HBM traffic: n * sizeof(T) bytes read; bins are negligible.
 #include <algorithm>
+#include <type_traits>
 
 #include "kernels.hpp"
 
@@ -28,16 +29,22 @@ namespace {
 
 constexpr int kBlock = 512;
 constexpr int kUnroll = 2;
+#ifndef ILGPU_HIP_HISTOGRAM_FEW_UNROLL
+#define ILGPU_HIP_HISTOGRAM_FEW_UNROLL 4
+#endif
+constexpr int kFewUnroll = ILGPU_HIP_HISTOGRAM_FEW_UNROLL;  // at most one block per CU
+constexpr int kCrowdedMaxReplicaShift = 2;  // fewer than eight replicas of a bin
 constexpr int kLdsBudgetWords = 12288;  // 48 KiB of counters per block
 constexpr int kMaxReplicas = 32;
 // A block's fixed cost is its flush, one returning global atomic per bin that it
 // has counted into; with three blocks per CU whatever the input, 8 M ints into 4096
 // bins spent 40 of 50 us on 3.1 M of them.  A block is worth its flush from
 // kMinElementsPerBin elements per bin on; half a block per CU is taken anyway, to
-// read short inputs.  (4096 bins, initialize and histogram, us before / now: 10^6 ints
-// 28.9 / 21.0, 8 * 10^6 49.7 / 20.9, 2^24 53.0 / 23.7, 2^26 70.7 / 55.1, the last by the
-// order of the flush alone; with 4, 8 and 32 elements per bin 2^24 takes 31.0, 25.0
-// and 32.2.)
+// read short inputs.  (4096 bins, initialize and histogram, us with three blocks per
+// CU / now: 10^6 ints 30.3 / 16.7, 8 * 10^6 49.5 / 18.8, 2^24 50.1 / 19.9, 2^26
+// 71.9 / 54.6, the last by the order of the flush alone.  With 4, 8 and 32 elements
+// per bin 2^24 took 31.0, 25.0 and 32.2 where 16 took 23.7, before the loads of
+// kFormCrowdedFew.)
 #ifndef ILGPU_HIP_HISTOGRAM_ELEMENTS_PER_BIN
 #define ILGPU_HIP_HISTOGRAM_ELEMENTS_PER_BIN 16
 #endif
@@ -226,8 +233,15 @@ __device__ __forceinline__ bool add_to_bin_dyn(int bin_type, void* bins,
 }
 
 // RANGE_CHECK = false when every value of T is a valid bin (e.g. u8 into
-// >= 256 bins with the identity locator).
-template <typename T, int LOC, bool RANGE_CHECK>
+// >= 256 bins with the identity locator).  FORM: the plain loop stands by itself, so that
+// what the others need costs it no registers (2^30 bytes into 256 bins: 3 %).
+enum {
+  kFormPlain,       // many replicas
+  kFormCrowded,     // looks for waves that meet in one bin
+  kFormCrowdedFew,  // the same with at most one block per CU: more loads per thread
+  kFormStrided,
+};
+template <typename T, int LOC, bool RANGE_CHECK, int FORM>
 __global__ __launch_bounds__(kBlock) void histogram_lds_kernel(
     const T* __restrict__ in, int64_t n, int64_t in_stride, void* bins,
     int num_bins, int bin_type, int32_t* overflow, int replica_shift) {
@@ -247,6 +261,28 @@ __global__ __launch_bounds__(kBlock) void histogram_lds_kernel(
     if (!RANGE_CHECK || (uint64_t)b < (uint64_t)num_bins)
       atomicAdd(&s_counts[((uint32_t)b << replica_shift) + replica], 1u);
   };
+  // Where most lanes of a wave meet in one bin (a constant column, a sorted one)
+  // and fewer than eight replicas part them, the LDS would serve them one after
+  // the other: the lanes that agree with the first one are added by one of them
+  // instead.  Looked for once per round of vectors.  (A constant column of ints, us
+  // with three blocks per CU / with the block limit / with the limit and these
+  // sums: 8 M into 4096 bins 22.2 / 33.1 / 17.7, 2^26 into 12 000 229 / 331 / 51.)
+  auto crowded = [&](T v) -> bool {
+    const int64_t b = locate<T, LOC>(v, num_bins);
+    const int first = __builtin_amdgcn_readfirstlane((int)b);
+    return __popcll(__ballot((int)b == first)) >= kWaveSize / 2;
+  };
+  auto count_crowded = [&](T v) {
+    const int64_t b = locate<T, LOC>(v, num_bins);
+    const bool inside = !RANGE_CHECK || (uint64_t)b < (uint64_t)num_bins;
+    const int bin = inside ? (int)b : -1;
+    const int first = __builtin_amdgcn_readfirstlane(bin);
+    const uint64_t same = __ballot(bin == first);
+    uint32_t c = 1u;
+    if (bin == first)
+      c = (threadIdx.x & (kWaveSize - 1)) == (uint32_t)__builtin_ctzll(same) ? (uint32_t)__popcll(same) : 0u;
+    if (inside && c != 0u) atomicAdd(&s_counts[((uint32_t)b << replica_shift) + replica], c);
+  };
 
   const uintptr_t addr = reinterpret_cast<uintptr_t>(in);
   int64_t head = (int64_t)(((16 - (addr & 15)) & 15) / sizeof(T));
@@ -257,7 +293,7 @@ __global__ __launch_bounds__(kBlock) void histogram_lds_kernel(
 
   const int64_t stride = (int64_t)gridDim.x * kBlock;
   int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (in_stride != 1) {
+  if constexpr (FORM == kFormStrided) {
     // Stride1D.General with an element stride above one: sample i lives at
     // in[i * in_stride]; one scalar load per sample, no vector body.
     for (int64_t e = i; e < n; e += stride) count(in[e * in_stride]);
@@ -265,13 +301,23 @@ __global__ __launch_bounds__(kBlock) void histogram_lds_kernel(
     head = 0;
     tail_start = n;
   }
-  for (; i + (kUnroll - 1) * stride < nvec; i += kUnroll * stride) {
-    V v[kUnroll];
+  constexpr int kRound = FORM == kFormCrowdedFew ? kFewUnroll : kUnroll;
+  for (; i + (kRound - 1) * stride < nvec; i += kRound * stride) {
+    V v[kRound];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u)
+    for (int u = 0; u < kRound; ++u)
       v[u] = __builtin_nontemporal_load(&body[i + u * stride]);
+    if constexpr (FORM != kFormPlain) {
+      if (crowded(v[0][0])) {
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u)
+        for (int u = 0; u < kRound; ++u)
+#pragma unroll
+          for (int k = 0; k < VN; ++k) count_crowded(v[u][k]);
+        continue;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kRound; ++u)
 #pragma unroll
       for (int k = 0; k < VN; ++k) count(v[u][k]);
   }
@@ -294,10 +340,14 @@ __global__ __launch_bounds__(kBlock) void histogram_lds_kernel(
   const bool checked = overflow != nullptr;
   bool passed = false;
   const int replicas = 1 << replica_shift;
-  // Blocks start their flush at different bins: all of them reach it at about the
-  // same time, and in one order every bin would take the adds of all blocks at
-  // once.
-  const int first_bin = (int)((uint64_t)blockIdx.x * (uint32_t)num_bins / gridDim.x);
+  // Blocks start their flush at different bins, in steps of a wave's adds: all of
+  // them reach it at about the same time, and in one order every bin would take the
+  // adds of all blocks at once.  Not where there are few bins: in two or three
+  // steps of the block a rotation gains nothing (2^30 bytes into 256 bins lose 0.8 %
+  // by it, 2^26 ints into 1000 2 %).
+  const int first_bin =
+      FORM == kFormPlain ? 0
+                         : (int)((uint64_t)blockIdx.x * (uint32_t)num_bins / gridDim.x) & ~(kWaveSize - 1);
   for (int i = threadIdx.x; i < num_bins; i += kBlock) {
     const int b = i + first_bin < num_bins ? i + first_bin : i + first_bin - num_bins;
     uint32_t c = 0;
@@ -378,7 +428,7 @@ int32_t launch_typed(hipStream_t stream, const void* in, int64_t n,
   if (per_cu < 1) per_cu = 1;
   if (blocks > cus * per_cu) blocks = cus * per_cu;
   // Blocks that are worth their flush (kMinElementsPerBin).
-  const int64_t worth = std::max<int64_t>(n / (num_bins * kMinElementsPerBin), cus / kMinBlocksDivisor);
+  const int64_t worth = std::max<int64_t>(n / (num_bins * kMinElementsPerBin), std::max(cus / kMinBlocksDivisor, 1));
   if (blocks > worth) blocks = worth;
   // Values of T that cannot leave [0, num_bins) need no range check.
   const bool unsigned_small =
@@ -386,17 +436,27 @@ int32_t launch_typed(hipStream_t stream, const void* in, int64_t n,
       !is_fp<T>::value && type_max_as_double<T>() < (double)num_bins;
   const bool no_check = LOC == ILGPU_HIP_LOCATOR_MODULO ? !is_fp<T>::value
                                                         : unsigned_small;
-  if (no_check) {
-    hipLaunchKernelGGL((histogram_lds_kernel<T, LOC, false>),
-                       dim3((unsigned)blocks), dim3(kBlock), lds_bytes, stream,
-                       src, n, in_stride, bins, (int)num_bins, bin_type, overflow,
-                       shift);
-  } else {
-    hipLaunchKernelGGL((histogram_lds_kernel<T, LOC, true>),
-                       dim3((unsigned)blocks), dim3(kBlock), lds_bytes, stream,
-                       src, n, in_stride, bins, (int)num_bins, bin_type, overflow,
-                       shift);
-  }
+  // One block per CU, or fewer, is bound by the latency of its loads: four vectors per
+  // round and thread (8 M ints into 4096 bins 21.0 -> 19.4 us), but two with more
+  // blocks (2^26: 53.9 against 59.5).
+  const int form = in_stride != 1                      ? kFormStrided
+                   : shift > kCrowdedMaxReplicaShift   ? kFormPlain
+                   : blocks <= cus                     ? kFormCrowdedFew
+                                                       : kFormCrowded;
+  auto launch = [&](auto range_check, auto f) {
+    hipLaunchKernelGGL(
+        (histogram_lds_kernel<T, LOC, decltype(range_check)::value, decltype(f)::value>),
+        dim3((unsigned)blocks), dim3(kBlock), lds_bytes, stream, src, n, in_stride, bins,
+        (int)num_bins, bin_type, overflow, shift);
+  };
+  auto launch_form = [&](auto range_check) {
+    if (form == kFormPlain) launch(range_check, std::integral_constant<int, kFormPlain>{});
+    else if (form == kFormCrowded) launch(range_check, std::integral_constant<int, kFormCrowded>{});
+    else if (form == kFormCrowdedFew) launch(range_check, std::integral_constant<int, kFormCrowdedFew>{});
+    else launch(range_check, std::integral_constant<int, kFormStrided>{});
+  };
+  if (no_check) launch_form(std::false_type{});
+  else launch_form(std::true_type{});
   ILGPU_HIP_CHECK(hipGetLastError());
   return ILGPU_HIP_SUCCESS;
 }

@@ -274,6 +274,31 @@ def test_histogram_lengths_where_the_number_of_blocks_changes(bins):
         assert not overflow
 
 
+@pytest.mark.parametrize("stride", [1, 3])
+@pytest.mark.parametrize("bins", [1536, 1537, 4096, 12288])
+def test_histogram_of_columns_that_crowd_one_bin(bins, stride):
+    """Waves that meet in one bin are added by one lane, where a bin has fewer than
+    eight replicas (1537 bins and more); lengths around the rounds of the vector
+    loops, and enough for more than one block per compute unit."""
+    rng = np.random.default_rng(bins)
+    for n in [1, 63, 65, 8193, 200_003] + ([bins * 16 * 257 + 9] if bins < 4096 else []):
+        column = rng.integers(-3, bins + 3, n).astype(np.int32)  # some outside of the bins
+        sorted_column = np.sort(column)
+        mostly = np.where(rng.random(n) < 0.7, np.int32(bins - 1), column)
+        outside = np.where(rng.random(n) < 0.7, np.int32(-1), column)
+        half = np.concatenate([np.full(n // 2, bins // 3, dtype=np.int32), column[n // 2:]])
+        for kind, v in [("constant", np.full(n, 7, dtype=np.int32)), ("sorted", sorted_column),
+                        ("mostly one", mostly), ("mostly outside", outside), ("half", half)]:
+            note("histogram crowded", bins, stride, n, kind)
+            view = D.from_numpy(v) if stride == 1 else strided_buffer(v, stride)[1]
+            d_bins, overflow = D.zeros(bins, np.int32), D.zeros(1, np.int32)
+            capi.histogram(view, d_bins, overflow)
+            sync()
+            inside = v[(v >= 0) & (v < bins)]
+            assert np.array_equal(d_bins.numpy(), np.bincount(inside, minlength=bins))
+            assert overflow.numpy()[0] == 0
+
+
 def test_histogram_many_bins_uses_global_atomics():
     n, bins = 200000, 100000
     v = random_ints(np.int32, n, seed=4, lo=0, hi=bins - 1)
