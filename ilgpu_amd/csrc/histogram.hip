@@ -33,6 +33,10 @@ constexpr int kUnroll = 2;
 #define ILGPU_HIP_HISTOGRAM_FEW_UNROLL 4
 #endif
 constexpr int kFewUnroll = ILGPU_HIP_HISTOGRAM_FEW_UNROLL;  // at most one block per CU
+#ifndef ILGPU_HIP_HISTOGRAM_STRIDED_UNROLL
+#define ILGPU_HIP_HISTOGRAM_STRIDED_UNROLL 4
+#endif
+constexpr int kStridedUnroll = ILGPU_HIP_HISTOGRAM_STRIDED_UNROLL;
 constexpr int kCrowdedMaxReplicaShift = 2;  // fewer than eight replicas of a bin
 constexpr int kLdsBudgetWords = 12288;  // 48 KiB of counters per block
 constexpr int kMaxReplicas = 32;
@@ -295,8 +299,25 @@ __global__ __launch_bounds__(kBlock) void histogram_lds_kernel(
   int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if constexpr (FORM == kFormStrided) {
     // Stride1D.General with an element stride above one: sample i lives at
-    // in[i * in_stride]; one scalar load per sample, no vector body.
-    for (int64_t e = i; e < n; e += stride) count(in[e * in_stride]);
+    // in[i * in_stride]; one scalar load per sample, no vector body.  Several in
+    // flight per thread, since the block limit leaves few waves to hide them (8 M
+    // ints into 4096 bins, us with three blocks per CU / one load at a time under
+    // the limit / four: every second element 52.1 / 46.7 / 25.2, and of 16 values
+    // only 22.9 / 43.7 / 22.1; every fourth 55.0 / 48.2 / 27.5, 29.8 / 45.8 / 25.3).
+    int64_t e = i;
+    for (; e + (kStridedUnroll - 1) * stride < n; e += kStridedUnroll * stride) {
+      T v[kStridedUnroll];
+#pragma unroll
+      for (int u = 0; u < kStridedUnroll; ++u) v[u] = in[(e + u * stride) * in_stride];
+      if (replica_shift <= kCrowdedMaxReplicaShift && crowded(v[0])) {
+#pragma unroll
+        for (int u = 0; u < kStridedUnroll; ++u) count_crowded(v[u]);
+      } else {
+#pragma unroll
+        for (int u = 0; u < kStridedUnroll; ++u) count(v[u]);
+      }
+    }
+    for (; e < n; e += stride) count(in[e * in_stride]);
     nvec = 0;
     head = 0;
     tail_start = n;
