@@ -448,8 +448,11 @@ int32_t launch_typed(hipStream_t stream, const void* in, int64_t n,
   if (per_cu > 3) per_cu = 3;
   if (per_cu < 1) per_cu = 1;
   if (blocks > cus * per_cu) blocks = cus * per_cu;
-  // Blocks that are worth their flush (kMinElementsPerBin).
-  const int64_t worth = std::max<int64_t>(n / (num_bins * kMinElementsPerBin), std::max(cus / kMinBlocksDivisor, 1));
+  // Blocks that are worth their flush (kMinElementsPerBin), in whole rounds of the
+  // CUs: 349 blocks over 256 of them took as long as 512 (2^26 ints of 16 values into
+  // 12 000 bins 64 us, now 51; 50 with three blocks per CU).
+  int64_t worth = std::max<int64_t>(n / (num_bins * kMinElementsPerBin), std::max(cus / kMinBlocksDivisor, 1));
+  if (worth > cus) worth = div_up(worth, cus) * cus;
   if (blocks > worth) blocks = worth;
   // Values of T that cannot leave [0, num_bins) need no range check.
   const bool unsigned_small =
