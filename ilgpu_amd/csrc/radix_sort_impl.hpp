@@ -2093,83 +2093,352 @@ __global__ __launch_bounds__(256) void finish_kernel(
 // ---- ties of the upper half --------------------------------------------------
 // After the passes over the upper half (plan->ties_left): keys whose upper halves
 // are the same stand next to each other in their original order.  Every run of such
-// keys is put into the order of the whole key, equal keys left in their order,
-// by the lane that sees its first key (runs of up to kTieRun keys, nearly always
-// two), or by that lane's wave.  Nobody else writes the run, and whoever looks
-// at its neighbours compares upper halves, which do not change.
+// keys is put into the order of the whole key, equal keys left in their order.
+// Nobody else writes the run, and whoever looks at its neighbours compares upper
+// halves, which do not change.
 //
 // A read of the keys, then: a lane takes kTieRows keys, a row of a wave 64
 // neighbouring ones, and the runs of all rows are ordered together, since each
-// costs a chain of two or three memory round trips. 
+// costs a chain of two or three memory round trips.  Runs of two or three keys, which nearly
+// all of them are, are ordered by the lane that sees the first one, longer ones by 16, 32 or
+// 64 lanes with a key per lane, or a wave with two.  Runs of 128 keys and more wait until
+// the block's waves have seen all of their keys, and are then ordered by the block.
 constexpr int kTieRows = 8;
-constexpr int kTieRun = 16;
+constexpr int kTieChunk = kTieRows * kWaveSize;
+constexpr int kTieBlock = 256;
+constexpr int kTieWaves = kTieBlock / kWaveSize;
+constexpr int kTieItems = 8;        // keys per thread that are ordered in LDS at a time
+constexpr int kTieMerges = 4;       // memory reads of a thread in flight where runs are merged
+// Runs of 128 keys and more that can start in one chunk.
+constexpr int kTieLongsPerChunk = kTieChunk / 128;
 
-// A run of more than kTieRun keys, by a whole wave: a look at its order first (many
-// copies of one key need nothing), then a stable merge sort, every key finding its
-// place in the other half by bisection; the other buffer's same range is scratch.
-// The sampling lets runs of some 2^-13 of the input pass at most.
-template <typename Val, int VALUE_BYTES>
-__device__ void order_long_run(uint64_t* keys, uint64_t* other_keys, Val* vals, Val* other_vals,
-                               int64_t start, int64_t n, const KeyXform& xf, int lane) {
-  const uint32_t upper = (uint32_t)(keys[start] >> 32);
-  int64_t len = 0;
-  bool inverted = false;
-  for (;;) {
-    const int64_t i = start + len + lane;
-    const bool same = i < n && (uint32_t)(keys[i] >> 32) == upper;
-    if (same && i + 1 < n) {
-      const uint64_t next = keys[i + 1];
-      if ((uint32_t)(next >> 32) == upper && ordered_bits(next, xf) < ordered_bits(keys[i], xf))
-        inverted = true;
-    }
-    const uint64_t lanes = __ballot(same);
-    len += __popcll(lanes);
-    if (lanes != ~0ull) break;
+// Runs of fewer than G keys, one by each G lanes (start: of the lane's run, if there is
+// one for it).  A key's place is the number of keys that go in front of it.
+template <int G, int VALUE_BYTES, typename Val>
+__device__ __forceinline__ void order_runs(uint64_t* keys, Val* vals, uint32_t start, bool any, uint32_t n,
+                                           const KeyXform& xf, int lane) {
+  const int l = lane & (G - 1);
+  const uint32_t at = start + l;
+  const bool have = any && at < n;
+  uint64_t k = 0;
+  Val v{};
+  if (have) {
+    k = keys[at];
+    if constexpr (VALUE_BYTES > 0) v = vals[at];
   }
-  if (__ballot(inverted) == 0ull) return;
+  const uint32_t upper = (uint32_t)__shfl((int)(uint32_t)(k >> 32), 0, G);
+  const bool same = have && (uint32_t)(k >> 32) == upper;
+  const uint64_t lanes = __ballot(same) >> (lane & ~(G - 1));
+  const int len = __builtin_ctzll(~lanes);
+  const uint32_t o = (uint32_t)ordered_bits(k, xf);  // the upper halves agree
+  int rank = 0;
+  if constexpr (G == kWaveSize) {
+    for (int j = 0; j < len; ++j) {
+      const uint32_t q = (uint32_t)__builtin_amdgcn_readlane((int)o, j);
+      if (q < o || (q == o && j < l)) ++rank;
+    }
+  } else {
+#pragma unroll 8
+    for (int j = 0; j < G; ++j) {
+      const uint32_t q = (uint32_t)__shfl((int)o, j, G);
+      if (j < len && (q < o || (q == o && j < l))) ++rank;
+    }
+  }
+  if (l < len && rank != l) {
+    keys[start + rank] = k;
+    if constexpr (VALUE_BYTES > 0) vals[start + rank] = v;
+  }
+}
+
+// A run of 64 to 127 keys, by a wave with two keys per lane.
+template <int VALUE_BYTES, typename Val>
+__device__ __forceinline__ void order_two_rows(uint64_t* keys, Val* vals, uint32_t start, uint32_t n,
+                                               const KeyXform& xf, int lane) {
+  const uint32_t first = start + lane;
+  const uint32_t second = min(first + kWaveSize, n - 1);
+  const uint64_t k0 = keys[first], k1 = keys[second];
+  Val v0{}, v1{};
+  if constexpr (VALUE_BYTES > 0) {
+    v0 = vals[first];
+    v1 = vals[second];
+  }
+  const bool same = first + kWaveSize < n &&
+                    (uint32_t)(k1 >> 32) == (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(k0 >> 32));
+  const int more = __builtin_ctzll(~__ballot(same));  // not all of them
+  const uint32_t o0 = (uint32_t)ordered_bits(k0, xf), o1 = (uint32_t)ordered_bits(k1, xf);
+  int rank0 = 0, rank1 = 0;
+  for (int j = 0; j < kWaveSize; ++j) {
+    const uint32_t q = (uint32_t)__builtin_amdgcn_readlane((int)o0, j);
+    if (q < o0 || (q == o0 && j < lane)) ++rank0;
+    if (q <= o1) ++rank1;
+  }
+  for (int j = 0; j < more; ++j) {
+    const uint32_t q = (uint32_t)__builtin_amdgcn_readlane((int)o1, j);
+    if (q < o0) ++rank0;
+    if (q < o1 || (q == o1 && j < lane)) ++rank1;
+  }
+  keys[start + rank0] = k0;
+  if constexpr (VALUE_BYTES > 0) vals[start + rank0] = v0;
+  if (lane < more) {
+    keys[start + rank1] = k1;
+    if constexpr (VALUE_BYTES > 0) vals[start + rank1] = v1;
+  }
+}
+
+// `count` elements from one buffer to the other, kTieMerges of a thread in flight.
+template <typename E>
+__device__ __forceinline__ void copy_rows(E* to, const E* from, uint32_t count, int t) {
+  for (uint32_t row = t; row < count; row += kTieMerges * kTieBlock) {
+    E e[kTieMerges];
+#pragma unroll
+    for (int u = 0; u < kTieMerges; ++u) e[u] = from[min(row + u * kTieBlock, count - 1)];
+#pragma unroll
+    for (int u = 0; u < kTieMerges; ++u)
+      if (row + u * kTieBlock < count) to[row + u * kTieBlock] = e[u];
+  }
+}
+
+// LDS in which a block orders a piece of a run.
+struct TiePiece {
+  static constexpr int kKeys = kTieBlock * kTieItems;
+  uint32_t o[kKeys];   // ordered lower halves
+  uint16_t from[kKeys];  // places they came from
+  uint32_t counts[kTieWaves][kRadix];
+  uint32_t totals[kTieWaves];
+};
+static_assert(kRadix == kTieBlock, "a thread scans the counts of one digit");
+
+// Exclusive sums of the digit counts of all waves, digits first, in their place.
+__device__ __forceinline__ void scan_counts(TiePiece& p, uint32_t* s_totals, int t) {
+  const int lane = t & (kWaveSize - 1);
+  uint32_t total = 0;
+#pragma unroll
+  for (int w = 0; w < kTieWaves; ++w) total += p.counts[w][t];
+  uint32_t sum = total;
+#pragma unroll
+  for (int step = 1; step < kWaveSize; step <<= 1) {
+    const uint32_t other = shfl_up(sum, step);
+    if (lane >= step) sum += other;
+  }
+  if (lane == kWaveSize - 1) s_totals[t / kWaveSize] = sum;
+  __syncthreads();
+  uint32_t off = sum - total;
+  for (int w = 0; w < t / kWaveSize; ++w) off += s_totals[w];
+#pragma unroll
+  for (int w = 0; w < kTieWaves; ++w) {
+    const uint32_t c = p.counts[w][t];
+    p.counts[w][t] = off;
+    off += c;
+  }
+}
+
+// Puts a piece, whose lower halves are in p.o, into their order, stable: four digits, each as a
+// pass of the sort ranks it (returning LDS adds on counters of the wave, which serve
+// lanes in lane order).  A wave holds kTieItems rows of 64 neighbouring keys.
+__device__ __forceinline__ void sort_piece(TiePiece& p, uint32_t* s_totals, int t) {
+  const int lane = t & (kWaveSize - 1), wave = t / kWaveSize;
+  const int base = wave * (kTieItems * kWaveSize) + lane;
+  uint32_t* counts = p.counts[wave];
+  for (int shift = 0; shift < 32; shift += 8) {
+    uint32_t o[kTieItems], from[kTieItems];  // from: place it came from, and above it the rank
+#pragma unroll
+    for (int q = 0; q < kRadix / kWaveSize; ++q) counts[q * kWaveSize + lane] = 0u;
+#pragma unroll
+    for (int u = 0; u < kTieItems; ++u) {
+      o[u] = p.o[base + u * kWaveSize];
+      from[u] = shift == 0 ? (uint32_t)(base + u * kWaveSize) : p.from[base + u * kWaveSize];
+    }
+    // (The counters are the wave's own, and its LDS instructions run in order.)
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int u = 0; u < kTieItems; ++u) from[u] |= atomicAdd(&counts[(o[u] >> shift) & (kRadix - 1)], 1u) << 16;
+    __syncthreads();
+    scan_counts(p, s_totals, t);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kTieItems; ++u) {
+      const uint32_t at = counts[(o[u] >> shift) & (kRadix - 1)] + (from[u] >> 16);
+      p.o[at] = o[u];
+      p.from[at] = (uint16_t)from[u];
+    }
+    __syncthreads();
+  }
+}
+
+// (Whole sorts of 2^21 u64 keys, us: uniform 115; one cluster of 1000, 2000 and 3000 keys 127,
+// 125 and 153, where a wave that merged it in memory, with an agent-scope fence per
+// level, took 305, 549 and 811; 1 % of the keys in runs of 32 with neighbouring upper
+// halves 160 / 314, of 2^27 keys 2687 / 6656.  By a bitonic sort of 1024 keys at a time
+// 3000 keys took 206, by merges alone in LDS 200.)
+
+// A run of 128 keys or more, by a block.  Pieces of kTieItems keys per thread are
+// ordered in LDS, by their lower halves; a piece that is in order (many copies of
+// one key) is left alone.  Then pieces are merged through memory if they have to
+// be, every key finding its place in the other piece by bisection, first among every
+// 2^k-th key, which LDS holds.  The other buffer's same range is scratch.
+// (Not inlined: its registers made the loop that every input goes through spill,
+// 29.1 us instead of 26.4 at 2^24 uniform keys.)
+template <typename Val, int VALUE_BYTES>
+__device__ __attribute__((noinline)) void order_long_run(
+    uint64_t* keys, uint64_t* other_keys, Val* vals, Val* other_vals, uint32_t start, uint32_t n,
+    uint64_t xor_mask, uint64_t reference_term, uint64_t total_term,
+    __attribute__((address_space(3))) TiePiece* lds_piece) {
+  const KeyXform xf{xor_mask, reference_term, total_term};
+  TiePiece& p = *(TiePiece*)lds_piece;
+  uint32_t* s_totals = p.totals;
+  const int t = threadIdx.x;
+  constexpr int kPiece = TiePiece::kKeys;
   uint64_t* src = keys + start;
   uint64_t* dst = other_keys + start;
   Val* src_vals = VALUE_BYTES > 0 ? vals + start : nullptr;
   Val* dst_vals = VALUE_BYTES > 0 ? other_vals + start : nullptr;
-  for (int64_t width = 1; width < len; width <<= 1) {
-    for (int64_t i = lane; i < len; i += kWaveSize) {
-      const uint64_t k = src[i];
-      const uint64_t o = ordered_bits(k, xf);
-      const int64_t pair = i & ~(2 * width - 1);
-      const int64_t middle = pair + width < len ? pair + width : len;
-      const int64_t end = pair + 2 * width < len ? pair + 2 * width : len;
-      const bool left = i < middle;
-      int64_t lo = left ? middle : pair, hi = left ? end : middle;
-      const int64_t first = lo;
-      while (lo < hi) {  // keys of the other half that go in front of this one
-        const int64_t m = lo + (hi - lo) / 2;
-        const uint64_t q = ordered_bits(src[m], xf);
-        if (left ? q < o : q <= o) lo = m + 1;
-        else hi = m;
-      }
-      const int64_t at = pair + (left ? i - pair : i - middle) + (lo - first);
-      dst[at] = k;
-      if constexpr (VALUE_BYTES > 0) dst_vals[at] = src_vals[i];
+  const uint64_t first_key = src[0];
+  const uint64_t upper_ordered = ordered_bits(first_key, xf) & ~0xFFFFFFFFull;
+  const uint32_t left = n - start;
+  uint32_t total = 0, largest = 0;
+  bool merge = false;
+  for (;;) {
+    int count = 0;
+#pragma unroll
+    for (int u = 0; u < kTieItems; ++u) {
+      const uint32_t i = u * kTieBlock + t;
+      const uint64_t k = src[total + i < left ? total + i : left - 1];
+      const bool same = total + i < left && (k >> 32) == (first_key >> 32);
+      p.o[i] = same ? (uint32_t)ordered_bits(k, xf) : 0xFFFFFFFFu;  // what is behind the run stays there
+      count += __popcll(__ballot(same));
     }
-    __threadfence();  // the next step reads what other lanes wrote
+    if (t % kWaveSize == 0) s_totals[t / kWaveSize] = (uint32_t)count;
+    __syncthreads();
+    count = 0;
+    for (int w = 0; w < kTieWaves; ++w) count += (int)s_totals[w];
+    bool inverted = false;
+    for (int i = t; i + 1 < count; i += kTieBlock) inverted |= p.o[i] > p.o[i + 1];
+    if (__syncthreads_or(inverted)) {
+      sort_piece(p, s_totals, t);
+      for (int i = t; i < count; i += kTieBlock)
+        src[total + i] = raw_bits((uint64_t)(upper_ordered | p.o[i]), xf);
+      if constexpr (VALUE_BYTES > 0) {
+        for (int row = t; row < count; row += kTieMerges * kTieBlock) {
+          Val v[kTieMerges];
+#pragma unroll
+          for (int u = 0; u < kTieMerges; ++u) v[u] = src_vals[total + p.from[min(row + u * kTieBlock, count - 1)]];
+#pragma unroll
+          for (int u = 0; u < kTieMerges; ++u)
+            if (row + u * kTieBlock < count) dst_vals[total + row + u * kTieBlock] = v[u];
+        }
+        __syncthreads();
+        copy_rows(src_vals + total, dst_vals + total, (uint32_t)count, t);
+      }
+    }
+    if (count > 0) {
+      merge |= total > 0 && p.o[0] < largest;
+      largest = p.o[count - 1];
+    }
+    total += (uint32_t)count;
+    __syncthreads();
+    if (count < kPiece) break;
+  }
+  if (!merge) return;
+  uint32_t* s_samples = reinterpret_cast<uint32_t*>(&p);
+  // Every piece begins with a sample, or there are none (beyond 2^23 keys).
+  int shift = 0;
+  while (((total - 1) >> shift) + 1 > (uint32_t)(sizeof(p) / 4)) ++shift;
+  const bool sampled = 1 << shift <= kPiece;
+  for (uint32_t width = kPiece; width < total; width <<= 1) {
+#pragma unroll 4
+    for (uint32_t i = t; sampled && i << shift < total; i += kTieBlock)
+      s_samples[i] = (uint32_t)ordered_bits(src[i << shift], xf);
+    __syncthreads();
+    // kTieMerges keys of a thread at once: a bisection is a chain of loads.
+    for (uint32_t row = t; row < total; row += kTieMerges * kTieBlock) {
+      uint32_t o[kTieMerges], lo[kTieMerges], hi[kTieMerges];
+      auto middle_of = [&](uint32_t i) {
+        const uint32_t pair = i & ~(2 * width - 1);
+        return total - pair > width ? pair + width : total;
+      };
+#pragma unroll
+      for (int u = 0; u < kTieMerges; ++u) {
+        const uint32_t i = min(row + u * kTieBlock, total - 1);
+        o[u] = (uint32_t)ordered_bits(src[i], xf);
+      }
+      // Keys of the other piece that go in front of this one: among the samples, ...
+      auto bounds = [&](uint32_t i, uint32_t& first, uint32_t& end) {
+        const uint32_t pair = i & ~(2 * width - 1), middle = middle_of(i);
+        first = i < middle ? middle : pair;
+        end = i < middle ? (total - pair > 2 * width ? pair + 2 * width : total) : middle;
+      };
+#pragma unroll
+      for (int u = 0; u < kTieMerges; ++u) {
+        uint32_t first, end;
+        bounds(min(row + u * kTieBlock, total - 1), first, end);
+        lo[u] = first >> shift;
+        hi[u] = sampled && first < end ? ((end - 1) >> shift) + 1 : lo[u];
+      }
+      for (uint32_t step = width >> shift; step > 0; step >>= 1) {
+#pragma unroll
+        for (int u = 0; u < kTieMerges; ++u) {
+          if (lo[u] >= hi[u]) continue;
+          const uint32_t i = row + u * kTieBlock, m = (lo[u] + hi[u]) >> 1;
+          const uint32_t q = s_samples[m];
+          if (i < middle_of(i) ? q < o[u] : q <= o[u]) lo[u] = m + 1;
+          else hi[u] = m;
+        }
+      }
+      // ... then among the keys between two of them.
+#pragma unroll
+      for (int u = 0; u < kTieMerges; ++u) {
+        uint32_t first, end;
+        bounds(min(row + u * kTieBlock, total - 1), first, end);
+        const uint32_t sample = lo[u];
+        hi[u] = sampled && sample << shift < end ? sample << shift : end;
+        lo[u] = sampled && sample << shift > first ? ((sample - 1) << shift) + 1 : first;
+      }
+      for (uint32_t step = sampled ? (1u << shift) >> 1 : width; step > 0; step >>= 1) {
+#pragma unroll
+        for (int u = 0; u < kTieMerges; ++u) {
+          if (lo[u] >= hi[u]) continue;
+          const uint32_t i = row + u * kTieBlock, m = (lo[u] + hi[u]) >> 1;
+          const uint32_t q = (uint32_t)ordered_bits(src[m], xf);
+          if (i < middle_of(i) ? q < o[u] : q <= o[u]) lo[u] = m + 1;
+          else hi[u] = m;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kTieMerges; ++u) {
+        const uint32_t i = row + u * kTieBlock;
+        lo[u] += i - middle_of(i);  // its place, from either half
+        if (i < total) dst[lo[u]] = raw_bits((uint64_t)(upper_ordered | o[u]), xf);
+      }
+      if constexpr (VALUE_BYTES > 0) {
+        Val v[kTieMerges];
+#pragma unroll
+        for (int u = 0; u < kTieMerges; ++u) v[u] = src_vals[min(row + u * kTieBlock, total - 1)];
+#pragma unroll
+        for (int u = 0; u < kTieMerges; ++u)
+          if (row + u * kTieBlock < total) dst_vals[lo[u]] = v[u];
+      }
+    }
+    __syncthreads();  // the next step reads what other threads wrote
     uint64_t* k = src; src = dst; dst = k;
     Val* v = src_vals; src_vals = dst_vals; dst_vals = v;
   }
   if (src != keys + start) {
-    for (int64_t i = lane; i < len; i += kWaveSize) {
-      dst[i] = src[i];
-      if constexpr (VALUE_BYTES > 0) dst_vals[i] = src_vals[i];
-    }
+    copy_rows(dst, src, total, t);
+    if constexpr (VALUE_BYTES > 0) copy_rows(dst_vals, src_vals, total, t);
   }
+  __syncthreads();
 }
 
-// (Compiled for 32 waves per CU, as the copy of finish() wants them too.)
+// (Compiled for 32 waves per CU, as the copy of finish() wants them too.)  long_starts:
+// scratch, kTieLongsPerChunk words for every chunk that a block's waves take.
 template <int VALUE_BYTES>
-__global__ __launch_bounds__(256, 8) void ties_kernel(
+__global__ __launch_bounds__(kTieBlock, 8) void ties_kernel(
     uint64_t* keys_a, uint64_t* keys_b, typename ValueOf<VALUE_BYTES>::type* vals_a,
     typename ValueOf<VALUE_BYTES>::type* vals_b, int64_t n, KeyXform xf,
-    const SortPlan* __restrict__ plan, int values_from_index) {
+    const SortPlan* __restrict__ plan, int values_from_index, uint32_t* long_starts) {
   using Val = typename ValueOf<VALUE_BYTES>::type;
+  __shared__ TiePiece s_piece;
+  __shared__ uint32_t s_longs;
   if (plan->ties_left == 0) {  // every digit was sorted
     finish<8, VALUE_BYTES>(keys_a, keys_b, vals_a, vals_b, n, plan, values_from_index);
     return;
@@ -2177,10 +2446,13 @@ __global__ __launch_bounds__(256, 8) void ties_kernel(
   uint64_t* keys = keys_a;  // an even number of passes ran
   Val* vals = vals_a;
   const int lane = threadIdx.x & (kWaveSize - 1);
-  const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWaveSize;
-  const int64_t waves = (int64_t)gridDim.x * blockDim.x / kWaveSize;
-  constexpr int64_t kChunk = kTieRows * kWaveSize;
-  for (int64_t base = wave * kChunk; base < n; base += waves * kChunk) {
+  const int64_t wave = (int64_t)blockIdx.x * kTieWaves + threadIdx.x / kWaveSize;
+  const int64_t waves = (int64_t)gridDim.x * kTieWaves;
+  const int64_t rounds = (n + waves * kTieChunk - 1) / (waves * kTieChunk);
+  long_starts += (int64_t)blockIdx.x * rounds * (kTieWaves * kTieLongsPerChunk);
+  if (threadIdx.x == 0) s_longs = 0u;
+  __syncthreads();
+  for (int64_t base = wave * kTieChunk; base < n; base += waves * kTieChunk) {
     // Upper halves of the rows; what lies outside of the input repeats the
     // nearest key and is masked below.
     uint32_t upper[kTieRows];
@@ -2190,7 +2462,7 @@ __global__ __launch_bounds__(256, 8) void ties_kernel(
       upper[r] = (uint32_t)(keys[i < n ? i : n - 1] >> 32);
     }
     uint32_t before = (uint32_t)(keys[base > 0 ? base - 1 : 0] >> 32);
-    const uint32_t after = (uint32_t)(keys[base + kChunk < n ? base + kChunk : n - 1] >> 32);
+    const uint32_t after = (uint32_t)(keys[base + kTieChunk < n ? base + kTieChunk : n - 1] >> 32);
     uint32_t leads = 0;  // rows in which this lane holds a run's first key
 #pragma unroll
     for (int r = 0; r < kTieRows; ++r) {
@@ -2207,49 +2479,72 @@ __global__ __launch_bounds__(256, 8) void ties_kernel(
       before = last;
     }
     while (__ballot(leads != 0) != 0ull) {
-      int64_t start = 0;
-      bool is_long = false;
+      uint32_t start = 0;  // n is below 2^31
+      int places = 0;      // more than the run has keys: 0 if this lane has ordered it
       if (leads != 0) {
-        start = base + (int64_t)(__builtin_ctz(leads) * kWaveSize + lane);
+        start = (uint32_t)base + (uint32_t)(__builtin_ctz(leads) * kWaveSize + lane);
         leads &= leads - 1;
-        const uint64_t k0 = keys[start];
-        int len = 2;
-        while (start + len < n && (keys[start + len] >> 32) == (k0 >> 32)) {
-          if (++len > kTieRun) break;
-        }
-        is_long = len > kTieRun;
-        if (!is_long) {
-          for (int j = 1; j < len; ++j) {
-            const uint64_t k = keys[start + j];
-            const uint64_t o = ordered_bits(k, xf);
-            int at = j;
-            Val v{};
-            for (; at > 0; --at) {
-              const uint64_t q = keys[start + at - 1];
-              if (ordered_bits(q, xf) <= o) break;
-              if constexpr (VALUE_BYTES > 0) {
-                if (at == j) v = vals[start + j];
-                vals[start + at] = vals[start + at - 1];
-              }
-              keys[start + at] = q;
-            }
-            if (at < j) {
-              keys[start + at] = k;
-              if constexpr (VALUE_BYTES > 0) vals[start + at] = v;
-            }
+        const uint32_t last = (uint32_t)n - 1;
+        const uint64_t k0 = keys[start], k1 = keys[start + 1], k2 = keys[min(start + 2, last)],
+                       k3 = keys[min(start + 3, last)];
+        auto same = [&](uint64_t k, uint32_t j) { return start + j <= last && (k >> 32) == (k0 >> 32); };
+        if (!same(k3, 3)) {
+          // Lower halves with their places, so that equal keys keep their order.
+          uint64_t x[3] = {ordered_bits(k0, xf) << 32, ordered_bits(k1, xf) << 32 | 1u,
+                           same(k2, 2) ? ordered_bits(k2, xf) << 32 | 2u : ~0ull << 32 | 2u};
+          auto order = [&](int i, int j) {
+            const uint64_t lo = x[i] < x[j] ? x[i] : x[j];
+            x[j] = x[i] < x[j] ? x[j] : x[i];
+            x[i] = lo;
+          };
+          order(0, 1); order(1, 2); order(0, 1);
+          const uint64_t upper_ordered = ordered_bits(k0, xf) & ~0xFFFFFFFFull;
+          Val v[3];
+          if constexpr (VALUE_BYTES > 0) {
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+              if ((uint32_t)x[j] != (uint32_t)j) v[j] = vals[start + (uint32_t)x[j]];
           }
+#pragma unroll
+          for (int j = 0; j < 3; ++j) {
+            if ((uint32_t)x[j] == (uint32_t)j) continue;
+            keys[start + j] = raw_bits((uint64_t)(upper_ordered | x[j] >> 32), xf);
+            if constexpr (VALUE_BYTES > 0) vals[start + j] = v[j];
+          }
+        } else {
+          const uint64_t k15 = keys[min(start + 15, last)], k31 = keys[min(start + 31, last)],
+                         k63 = keys[min(start + 63, last)], k127 = keys[min(start + 127, last)];
+          places = same(k127, 127) ? 256 : same(k63, 63) ? 128 : same(k31, 31) ? 64 : same(k15, 15) ? 32 : 16;
+          if (places == 256) long_starts[atomicAdd(&s_longs, 1u)] = start;
         }
       }
-      for (uint64_t longs = __ballot(is_long); longs != 0ull; longs &= longs - 1) {
-        const int owner = __builtin_ctzll(longs);
-        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)start, owner);
-        const uint32_t hi =
-            (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)start >> 32), owner);
-        order_long_run<Val, VALUE_BYTES>(keys, keys_b, vals, vals_b,
-                                         (int64_t)(((uint64_t)hi << 32) | lo), n, xf, lane);
-      }
+      // Runs of G lanes, as many at once as the wave has room for.
+      auto order_all = [&](auto width) {
+        constexpr int G = decltype(width)::value;
+        for (uint64_t owners = __ballot(places == G); owners != 0ull;) {
+          int mine = -1;
+          for (int g = 0; g < kWaveSize / G && owners != 0ull; ++g, owners &= owners - 1)
+            if (lane / G == g) mine = __builtin_ctzll(owners);
+          const uint32_t s = (uint32_t)__shfl((int)start, mine < 0 ? 0 : mine);
+          order_runs<G, VALUE_BYTES>(keys, vals, s, mine >= 0, (uint32_t)n, xf, lane);
+        }
+      };
+      if (__ballot(places != 0) == 0ull) continue;
+      order_all(std::integral_constant<int, 16>{});
+      order_all(std::integral_constant<int, 32>{});
+      order_all(std::integral_constant<int, 64>{});
+      for (uint64_t owners = __ballot(places == 128); owners != 0ull; owners &= owners - 1)
+        order_two_rows<VALUE_BYTES>(
+            keys, vals, (uint32_t)__builtin_amdgcn_readlane((int)start, __builtin_ctzll(owners)), (uint32_t)n, xf,
+            lane);
     }
   }
+  __syncthreads();
+  const uint32_t longs = s_longs;
+  for (uint32_t r = 0; r < longs; ++r)  // the same in every thread
+    order_long_run<Val, VALUE_BYTES>(keys, keys_b, vals, vals_b, long_starts[r], (uint32_t)n, xf.xor_mask,
+                                     xf.reference_term, xf.total_term,
+                                     (__attribute__((address_space(3))) TiePiece*)&s_piece);
 }
 
 // ---- host side -------------------------------------------------------------
@@ -2594,11 +2889,17 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
   if (rc != ILGPU_HIP_SUCCESS) return rc;
   if constexpr (KEY_BYTES == 8) {
     if (ties.table != nullptr) {
-      int64_t blocks = div_up(a.n, 256 * kTieRows);
+      int64_t blocks = div_up(a.n, kTieBlock * kTieRows);
       if (blocks > (int64_t)cus * 8) blocks = (int64_t)cus * 8;
+      // The list of long runs lies in the status words, which the passes are done
+      // with: kTieLongsPerChunk words per chunk, for at most twice as many chunks as
+      // there are (the last round of a grid), against 256 words per tile and digit position.
+      static_assert(2 * kTieLongsPerChunk * 4 * (tile_keys(8, 0, kSortBlockLarge) / kTieChunk + 1) <= 8 * kRadix * 4,
+                    "room for the list of long runs");
       ProfileScope scope(stream, "sort_finish");
-      hipLaunchKernelGGL((ties_kernel<VALUE_BYTES>), dim3((unsigned)blocks), dim3(256), 0, stream,
-                         keys_a, keys_b, vals_a, vals_b, a.n, xf, plan, from_index);
+      hipLaunchKernelGGL((ties_kernel<VALUE_BYTES>), dim3((unsigned)blocks), dim3(kTieBlock), 0, stream,
+                         keys_a, keys_b, vals_a, vals_b, a.n, xf, plan, from_index,
+                         reinterpret_cast<uint32_t*>(base + L.status));
       ILGPU_HIP_CHECK(hipGetLastError());
       return ILGPU_HIP_SUCCESS;
     }

@@ -1968,3 +1968,100 @@ def test_sort_of_long_inputs_chooses_its_digits(kind, passes):
     assert capi.radix_sort_passes(temp, n, np.uint64, 4)[0] == passes
     order = np.argsort(keys, kind="stable")
     assert np.array_equal(d.numpy(), keys[order]) and np.array_equal(v.numpy(), order)
+
+
+def cluster(keys, length, seed, copies=1):
+    """Gives `length` keys at random places one upper half and random lower ones,
+    every lower half `copies` times."""
+    rng = np.random.default_rng(seed)
+    places = rng.permutation(keys.size)[:length]
+    upper = rng.integers(0, 1 << 32, dtype=np.uint64) << np.uint64(32)
+    lower = rng.integers(0, 1 << 32, -(-length // copies), dtype=np.uint64)
+    keys[places] = upper | rng.permutation(np.repeat(lower, copies)[:length])
+    return keys
+
+
+def sort_index_pairs(keys, value_dtype=np.uint32, descending=False):
+    """(keys, values, executed passes) of an argsort on the GPU."""
+    d, v = D.from_numpy(keys), D.zeros(keys.size, value_dtype)
+    size = np.dtype(value_dtype).itemsize
+    temp = capi.temp_buffer(capi.radix_sort_temp_bytes(keys.size, keys.dtype, size))
+    capi.radix_sort_pairs(d, v, temp, descending=descending, values_from_index=True)
+    sync()
+    return d.numpy(), v.numpy(), capi.radix_sort_passes(temp, keys.size, keys.dtype, size)[0]
+
+
+# Runs around what sixteen lanes, a wave, and a block's LDS (2048 keys) take, with one,
+# two and three pieces to merge.
+@pytest.mark.parametrize("n,lengths", [
+    (TIE_LENGTH, [63, 64, 65, 255, 256, 257, 511, 513]), (TIE_LENGTH, [2047, 2048]),
+    (TIE_LENGTH, [2049, 255]), (TIE_LENGTH, [3000]), (1 << 23, [6200]), (1 << 23, [4097])])
+@pytest.mark.parametrize("copies", [1, 3])
+def test_sort_orders_long_runs_of_one_upper_half(n, lengths, copies):
+    note("long runs", n, lengths, copies)
+    keys = upper_half_keys(n, 81)
+    for c, length in enumerate(lengths):
+        cluster(keys, length, 82 + c, copies)
+    got, values, executed = sort_index_pairs(keys, descending=copies == 3)
+    order = np.argsort(~keys if copies == 3 else keys, kind="stable")
+    assert np.array_equal(got, keys[order]) and np.array_equal(values, order)
+    assert executed == 4
+
+
+@pytest.mark.parametrize("value_dtype", [np.uint8, np.uint16, np.uint32, np.float32, np.float64, "V16"])
+def test_sort_orders_neighbouring_runs_with_values_of_every_size(value_dtype):
+    """Runs of 2 to 40 keys side by side, over the ends of rows and chunks."""
+    n = TIE_LENGTH
+    note("neighbouring runs", str(value_dtype))
+    rng = np.random.default_rng(83)
+    keys = upper_half_keys(n, 84)
+    lengths = np.concatenate([np.repeat(np.arange(2, 9), 12), np.repeat(np.arange(9, 41), 1)])
+    rng.shuffle(lengths)
+    upper = np.repeat(np.arange(lengths.size, dtype=np.uint64) + np.uint64(7), lengths) << np.uint64(32)
+    keys[rng.permutation(n)[:upper.size]] = upper | rng.integers(0, 12, upper.size, dtype=np.uint64)
+    order = np.argsort(keys, kind="stable")
+    if value_dtype == "V16":
+        rows = np.stack([np.arange(n, dtype=np.uint64), rng.integers(0, 1 << 62, n, dtype=np.uint64)], axis=1)
+        values = np.ascontiguousarray(rows).view("V16").reshape(-1)
+        d, v = D.from_numpy(keys), D.from_numpy(values)
+        temp = capi.temp_buffer(capi.radix_sort_temp_bytes(n, np.uint64, 16))
+        capi.radix_sort_pairs(d, v, temp)
+        sync()
+        got, got_values = d.numpy(), v.numpy().view(np.uint64).reshape(-1, 2)
+        executed = capi.radix_sort_passes(temp, n, np.uint64, 16)[0]
+        assert np.array_equal(got_values, rows[order])
+    else:
+        got, got_values, executed = sort_index_pairs(keys, value_dtype)
+        assert np.array_equal(got_values, order.astype(value_dtype))
+    assert np.array_equal(got, keys[order]) and executed == 4
+
+
+@pytest.mark.parametrize("dtype", [np.uint64, np.float64])
+@pytest.mark.parametrize("pairs", [False, True])
+def test_large_block_passes_leave_the_ties(dtype, pairs):
+    """The pipelined pass and the 1024-thread block, float conversion in and out
+    around passes that start at the upper half; an odd number of its digits too."""
+    n = TIE_LENGTH
+    for upper_digits in ([4, 3] if dtype is np.uint64 else [4]):
+        note("large block ties", np.dtype(dtype).name, pairs, upper_digits)
+        bits = cluster(upper_half_keys(n, 85, TIE_RUNS[:9]), 300, 86)
+        if upper_digits == 3:
+            bits >>= np.uint64(8)
+        sign = np.uint64(1 << 63)
+        order_bits = bits if dtype is np.uint64 else bits ^ sign ^ (np.uint64(1) - (bits >> np.uint64(63)))
+        order = np.argsort(order_bits, kind="stable")
+        keys, values = D.from_numpy(bits.view(dtype)), D.zeros(n, np.uint32)
+        temp = capi.temp_buffer(capi.radix_sort_temp_bytes(n, dtype, 4 if pairs else 0))
+        capi.sort_set_parameter(capi.SORT_PARAM_LARGE_BLOCK_MIN_TILES_PER_CU, 0)
+        try:
+            if pairs:
+                capi.radix_sort_pairs(keys, values, temp, values_from_index=True)
+            else:
+                capi.radix_sort_keys(keys, temp)
+            sync()
+        finally:
+            capi.sort_set_parameter(capi.SORT_PARAM_LARGE_BLOCK_MIN_TILES_PER_CU, -1)
+        assert capi.radix_sort_passes(temp, n, dtype, 4 if pairs else 0)[0] == 4
+        assert np.array_equal(keys.numpy().view(np.uint64), bits[order])
+        if pairs:
+            assert np.array_equal(values.numpy(), order)
