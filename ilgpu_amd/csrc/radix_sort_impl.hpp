@@ -313,35 +313,57 @@ static_assert(sizeof(SortPlan) <= 256, "the temp view holds 256 bytes for the pl
 // 8-byte keys whose upper halves rarely meet are sorted by that half alone, four
 // passes instead of eight; what is left is to order the few neighbours whose
 // upper halves are the same (ties_kernel), which reads the keys once.  Whether
-// they rarely meet no digit histogram tells, so the histogram kernel
-// also draws up to kTieSamples keys from positions that are independent of each
-// other and counts the draws whose upper half it has met before at another position,
-// in a hash table of kTieSlots entries, upper half and position (in the alternate key
-// buffer, which no pass has written yet).  m draws of which c meet an earlier one: about 2 n c / m^2 ties per
-// key.  The short way is taken up to half a tie per key: uniform keys have n / 2^32
-// of them.
+// they rarely meet no digit histogram tells, so the histogram kernel also draws m
+// keys, one from every m-th part of the input (positions that differ), and counts
+// the upper halves that are drawn twice or more, those that are drawn three times or more,
+// and the pairs of draws that share one, c (c - 1) / 2 where one is drawn c times.
+// A run of L keys gives some L (L - 1) / 2 * m^2 / n^2 of them.
+// The short way is taken
+//   up to m^2 / n upper halves that are drawn twice or more: as many pairs as there are
+//   keys (uniform keys have n^2 / 2^33 pairs);
+//   up to kTieGroups upper halves that are drawn three times or more: short inputs,
+//   of which a key in 64 is drawn, would pass with some thousand runs of a few dozen
+//   keys, and where those lie side by side a few waves would order all of them;
+//   up to 3 m^2 / n pairs, which is what a run of sqrt(6 n) keys gives: the longest that
+//   ties_kernel orders in about the time of the passes that are saved (3500 of
+//   2^21 keys, 28 000 of 2^27).
+// (The draws that met an earlier one, counted once each, bound neither: one run of
+// 16 000 keys, a thousand of 32.)
+// (Whole sorts of u64 keys with a copy in front, us, all eight digits / the count of
+// draws that met an earlier one / this.  2^21 keys: uniform 173 / 120 / 115; one cluster of
+// 1000 keys 174 / 305 / 127, of 3000 173 / 811 / 153, of 16 000, refused, 174 / 5126 / 176; 2^24:
+// uniform 622 / 393 / 390, one cluster of 4000 620 / 1356 / 435; 2^27: uniform 4231 / 2740 / 2722,
+// one cluster of 16 000 4261 / 4243 / 3010, every upper half taken from as many as there are
+// keys 4268 / 4263 / 3540.)
 // From kTieMinKeys keys on: below that a pass takes so little time that the
 // sampling, the ties kernel and four passes that return at once cost the same.
-// (Whole sorts with the copy of the keys in front of them, all digits / upper half, us: 2^27
-// pairs of uniform u64 keys and generated u32 values 5964 / 3642, 2^22 pairs 289 / 183; keys
-// alone 2^27 4187 / 2760, 2^24 616 / 388, 2^21 177 / 122.  Where the draws say no the sampling
-// is lost: values below 10^6 as int64, three passes, 2^24 336 / 337, 2^22 126 / 127; with
-// 2^17 draws, a table of 2^19 entries and fewer waves in the last kernel 340 / 351 and
-// 126 / 132.)
+// Where the draws say no the sampling is lost: Zipf values below 2^15 as int64, two passes,
+// 2^21 keys 79.8 / 83.4 / 81.7, 2^22 95.5 / 97.7 / 98.2, 2^24 239 / 235 / 240; values
+// below 10^6, three passes, 2^21 97.9 / 99.8 / 98.2.
 constexpr int kTiePasses = 4;                // passes over the upper half
-constexpr uint32_t kTieSamples = 1u << 16;
-constexpr uint32_t kTieSlotBits = 18;
-constexpr uint32_t kTieSlots = 1u << kTieSlotBits;
+constexpr uint32_t kTieGroups = 8;
+// Draws: one key of 256 within these limits (2^18 draws of 2^27 keys cost 0.7 % more where they
+// say no).
+constexpr int kTieMinSampleBits = 15, kTieMaxSampleBits = 16;
+constexpr int kTieSlotsPerDrawLog2 = 2;
+// Slots that a draw tries before it goes uncounted: in its block's table, and in the
+// grid's, where the second try lies behind the first vectors (one in 60 upper halves
+// finds both taken).
+constexpr int kTieBlockProbes = 8;
 #ifndef ILGPU_HIP_SORT_TIE_MIN_LOG2
 #define ILGPU_HIP_SORT_TIE_MIN_LOG2 21
 #endif
 constexpr int64_t kTieMinKeys = 1ll << ILGPU_HIP_SORT_TIE_MIN_LOG2;
-static_assert(kTieMinKeys >= (int64_t)kTieSlots, "the table lies in the alternate keys");
+static_assert(kTieMinKeys >= 1ll << (kTieMinSampleBits + kTieSlotsPerDrawLog2) &&
+                  kTieSlotsPerDrawLog2 <= 8,
+              "the table lies in the alternate keys");
 struct TieSampling {
-  unsigned long long* table;  // nullptr: no sampling
-  uint32_t* collisions;       // eight counts, kTicketStride words apart
-  uint32_t samples;       // at most one per thread of the histogram's grid
-  uint32_t max_collisions;
+  // Upper halves met, in open addressing: upper half << 32 | times drawn, 0 where
+  // nothing is.  nullptr: no sampling.
+  unsigned long long* table;
+  uint32_t* counts;         // kTicketGroups times {pairs, doubles, groups}, kTicketStride words apart
+  uint32_t sample_bits;     // log2 of the number of draws
+  uint32_t max_doubles, max_pairs;
 };
 
 // The first active lane's key, as a wave-uniform value.
@@ -367,39 +389,71 @@ __global__ __launch_bounds__(kHistBlock) void sort_histogram_kernel(
     int replica_shift, uint32_t* __restrict__ global_hist, TieSampling ties) {
   using V = typename Vec16<K>::type;
   constexpr int VN = Vec16<K>::N;
-  extern __shared__ uint32_t s_hist[];  // [passes][256][replicas]
+  extern __shared__ __align__(8) uint32_t s_hist[];  // [passes][256][replicas]
   const int words = (passes * kRadix) << replica_shift;
-  // This thread's draw of the tie sampling.  Draws meet within their block first, in LDS: where
-  // many keys share an upper half, all draws of the grid would queue at one slot of the
-  // table (2^17 draws: 1.5 ms).  An empty slot holds 0, a draw its complement, so
-  // that small keys do not look like empty slots.  Of two draws that share a slot the
-  // later one stays, and a third that meets the first goes uncounted: rare at four
-  // slots per draw.
-  unsigned long long draw = 0, met = 0;  // upper half, position
-  bool collided = false, drawn = false;
+  // This thread's draw of the tie sampling.  Draws meet within their block first, in
+  // LDS: where many keys share an upper half, all draws of the grid would queue
+  // at one slot of the table (2^17 draws: 1.5 ms).  The thread that enters an upper
+  // half into the block's table takes it to the grid's, with its count; the answer is
+  // looked at when the keys have been counted.
+  __shared__ uint32_t s_pairs, s_doubles, s_groups;
+  uint32_t upper = 0, drawn = 0, slot = 0;  // drawn: times in this block, 0 for all but one thread
+  unsigned long long met = 0;
+  // The first blocks draw, a key per thread: the others, one of which is next to each of them
+  // on its compute unit in long inputs, have more of the LDS meanwhile (2^24 keys with 128 draws
+  // per block 41 us, with 512 in a quarter of the blocks 37.6).
+  const bool sampling = sizeof(K) == 8 && ties.table != nullptr &&
+                        blockIdx.x * (uint32_t)kHistBlock < (1u << ties.sample_bits);
   if constexpr (sizeof(K) == 8) {
-    if (ties.table != nullptr) {
-      constexpr uint32_t kBlockSlots = 4 * kHistBlock;
-      static_assert(kBlockSlots <= (uint32_t)kRadix * 8, "a slot is a counter of the histogram");
+    if (sampling) {
+      constexpr int kBlockSlotBits = 10;
+      constexpr uint32_t kBlockSlots = 1u << kBlockSlotBits;
+      static_assert(kBlockSlots >= 2 * kHistBlock && kBlockSlots * 2 <= kMaxPasses * kRadix,
+                    "room for every draw in the counters of the histogram");
+      auto* block_table = reinterpret_cast<unsigned long long*>(s_hist);
+      for (uint32_t i = threadIdx.x; i < kBlockSlots; i += kHistBlock) block_table[i] = 0ull;
+      if (threadIdx.x == 0) s_pairs = s_doubles = s_groups = 0u;
+      static_assert(1 << kTieMinSampleBits >= kHistBlock, "a block's threads all draw");
       const uint32_t s = blockIdx.x * (uint32_t)kHistBlock + threadIdx.x;
-      drawn = s < ties.samples;
-      if (drawn) {
+      {
         uint64_t z = ((uint64_t)s + 1ull) * 0x9E3779B97F4A7C15ull;  // splitmix64
         z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
         z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
         z ^= z >> 31;
-        const uint64_t at = __umul64hi(z, (uint64_t)n);
-        draw = (keys[at] & ~0xFFFFFFFFull) | at;
+        // A random place in part s of the input.
+        const uint64_t at = ((uint64_t)s << 32 | (uint32_t)z) << (32 - ties.sample_bits);
+        upper = (uint32_t)(keys[__umul64hi(at, (uint64_t)n)] >> 32);
       }
-      for (uint32_t i = threadIdx.x; i < kBlockSlots; i += kHistBlock) s_hist[i] = 0u;
       __syncthreads();
-      const uint32_t upper = (uint32_t)(draw >> 32);
-      const uint32_t hash = upper * 0x9E3779B1u;
-      if (drawn)
-        collided = atomicExch(&s_hist[hash % kBlockSlots], ~upper) == ~upper;
-      if (drawn && !collided)
-        met = ~atomicExch(&ties.table[hash >> (32 - kTieSlotBits)], ~draw);
+      // (The lanes that agree with the first one go together: keys that all share an upper half
+      // would queue at one word 512 deep, 2 us.)
+      const uint64_t same = __ballot(upper == (uint32_t)__builtin_amdgcn_readfirstlane((int)upper));
+      const int lane = threadIdx.x & (kWaveSize - 1);
+      drawn = lane == 0 ? (uint32_t)__popcll(same) : (same >> lane & 1ull ? 0u : 1u);
+      if (drawn != 0) {
+        slot = (upper * 0x85EBCA6Bu) >> (32 - kBlockSlotBits);
+        int probe = 0;
+        for (; probe < kTieBlockProbes; ++probe) {
+          const unsigned long long old =
+              atomicCAS(&block_table[slot], 0ull, (unsigned long long)upper << 32 | drawn);
+          if (old == 0ull) break;
+          if ((uint32_t)(old >> 32) == upper) {
+            atomicAdd(&block_table[slot], (unsigned long long)drawn);
+            drawn = 0;
+            break;
+          }
+          slot = (slot + 1) & (kBlockSlots - 1);
+        }
+        if (probe == kTieBlockProbes) slot = kBlockSlots;
+      }
       __syncthreads();
+      if (drawn != 0 && slot < kBlockSlots) drawn = (uint32_t)block_table[slot];
+      // (No sum counts more than one too many at a time, so that none overflows.)
+      const uint32_t pairs = min(drawn * (drawn - 1) / 2, ties.max_pairs + 1);
+      if (drawn > 1) atomicAdd(&s_pairs, pairs);
+      if (drawn > 1 && pairs > ties.max_pairs) drawn = 0;  // enough said
+      slot = (upper * 0x9E3779B1u) >> (32 - kTieSlotsPerDrawLog2 - ties.sample_bits);
+      if (drawn != 0) met = atomicCAS(&ties.table[slot], 0ull, (unsigned long long)upper << 32 | drawn);
     }
   }
   for (int i = threadIdx.x; i < words; i += kHistBlock) s_hist[i] = 0u;
@@ -527,6 +581,12 @@ __global__ __launch_bounds__(kHistBlock) void sort_histogram_kernel(
       for (int u = 0; u < kHistUnroll; ++u) count_vector(checked, v0[u]);
       i += kHistUnroll * stride;
     }
+    if constexpr (sizeof(K) == 8) {  // the tie sampling's second slot
+      if (met != 0ull && (uint32_t)(met >> 32) != upper) {
+        slot ^= 1u;
+        met = atomicCAS(&ties.table[slot], 0ull, (unsigned long long)upper << 32 | drawn);
+      }
+    }
     for (; i + (kHistUnroll - 1) * stride < nvec; i += kHistUnroll * stride) {
       V v[kHistUnroll];
 #pragma unroll
@@ -553,11 +613,23 @@ __global__ __launch_bounds__(kHistBlock) void sort_histogram_kernel(
   flush_key_run();
   flush_half_run();
   if constexpr (sizeof(K) == 8) {
-    if (drawn && !collided) collided = (met >> 32) == (draw >> 32) && met != draw;
+    if (drawn != 0) {
+      uint32_t before = 0;
+      if (met != 0ull && (uint32_t)(met >> 32) == upper) {
+        before = (uint32_t)atomicAdd(&ties.table[slot], (unsigned long long)drawn);
+        atomicAdd(&s_pairs, min(drawn * before, ties.max_pairs + 1));
+      }
+      if (before < 2 && before + drawn >= 2) atomicAdd(&s_doubles, 1u);
+      if (before < 3 && before + drawn >= 3) atomicAdd(&s_groups, 1u);
+    }
+    __syncthreads();
     // One add per block, to one of eight lines: 2^11 adds to one word, a wave each, took 20 us.
-    const int collisions = __syncthreads_count(collided);
-    if (threadIdx.x == 0 && collisions != 0)
-      atomicAdd(ties.collisions + (blockIdx.x % kTicketGroups) * kTicketStride, (uint32_t)collisions);
+    if (sampling && threadIdx.x == 0 && s_pairs != 0) {
+      uint32_t* counts = ties.counts + (blockIdx.x % kTicketGroups) * kTicketStride;
+      atomicAdd(&counts[0], s_pairs);
+      atomicAdd(&counts[1], s_doubles);
+      atomicAdd(&counts[2], s_groups);
+    }
   } else {
     __syncthreads();
   }
@@ -587,19 +659,28 @@ __global__ __launch_bounds__(kRadix) void plan_kernel(
   uint32_t counts[kMaxPasses];
 #pragma unroll
   for (int p = 0; p < kMaxPasses; ++p) counts[p] = p < passes ? global_hist[p * kRadix + d] : 0u;
-  // The lower digits [0, left) are left to the ties if the draws rarely met and
+  // The lower digits [0, left) are left to the ties if the draws rarely meet and
   // that saves at least two passes (a digit that all keys share needs none).
   // An even number of passes ends in the caller's buffer, where the ties are ordered: an
   // odd one takes a lower digit along.
   int left = 0;
   if (ties.table != nullptr) {
-    uint32_t collisions = 0;
-    for (int g = 0; g < kTicketGroups; ++g) collisions += ties.collisions[g * kTicketStride];
-    if (collisions <= ties.max_collisions) {
-      uint32_t varies = 0;
+    uint32_t pairs = 0, doubles = 0, groups = 0;
+    for (int g = 0; g < kTicketGroups; ++g) {
+      pairs += ties.counts[g * kTicketStride];
+      doubles += ties.counts[g * kTicketStride + 1];
+      groups += ties.counts[g * kTicketStride + 2];
+    }
+    if (pairs <= ties.max_pairs && doubles <= ties.max_doubles && groups <= kTieGroups) {
+      uint32_t trivial = 0;
 #pragma unroll
-      for (int p = 0; p < kMaxPasses; ++p)
-        varies |= __syncthreads_or(counts[p] == n) ? 0u : 1u << p;
+      for (int p = 0; p < kMaxPasses; ++p) trivial |= counts[p] == n ? 1u << p : 0u;
+      if (d == 0) s_trivial = 0;
+      __syncthreads();
+      if (trivial != 0) atomicOr(&s_trivial, (int)trivial);
+      __syncthreads();
+      const uint32_t varies = ~(uint32_t)s_trivial & ((1u << kMaxPasses) - 1u);
+      __syncthreads();
       left = kMaxPasses - kTiePasses;
       if (__popc(varies >> left) & 1)
         while (left > 0 && !(varies >> --left & 1u)) {}
@@ -2816,47 +2897,50 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
                              ? 1
                              : (a.value_source == ILGPU_HIP_VALUES_FROM_INDEX_AS_FLOAT ? 2 : 0);
 
+  int shift = 0;  // replicas of the histogram: as many as kHistLdsWords of LDS counters hold
+  while ((1 << (shift + 1)) <= 32 &&
+         ((passes * kRadix) << (shift + 1)) <= kHistLdsWords)
+    ++shift;
+  const size_t hist_lds = (size_t)((passes * kRadix) << shift) * 4;
+  // A block's fixed cost is its flush, one global atomic per digit value and
+  // position, which all blocks issue at about the same time.  Up to half a
+  // block per CU as soon as every thread has four vectors to count, more
+  // only when every thread has sixteen (2^20 u32 keys: 7.5 us instead of
+  // 15.5 with one vector per thread; 2^22: 12.3 instead of 17.1).
+  const int64_t vectors = div_up(a.n, Vec16<K>::N);
+  const int64_t few = std::min<int64_t>(div_up(vectors, kHistBlock * 4), std::max(cus / 2, 1));
+  int64_t hist_blocks = std::max(few, div_up(vectors, kHistBlock * 16));
+  // Two blocks of 64 KiB of counters are resident per CU: no second round.
+  if (hist_blocks > (int64_t)cus * ILGPU_HIP_SORT_HIST_BLOCKS_PER_CU)
+    hist_blocks = (int64_t)cus * ILGPU_HIP_SORT_HIST_BLOCKS_PER_CU;
+  if (hist_blocks < 1) hist_blocks = 1;
+
   TieSampling ties{};
+  int64_t table_words = 0;
   if (KEY_BYTES == 8 && a.n >= kTieMinKeys) {
+    uint32_t bits = kTieMinSampleBits;
+    while (bits < kTieMaxSampleBits && a.n >> (bits + 9) != 0) ++bits;
+    while ((1ll << bits) > hist_blocks * kHistBlock) --bits;  // few compute units
     ties.table = reinterpret_cast<unsigned long long*>(keys_b);
-    // A word of the first ticket's line that no group uses, cleared with it.
-    ties.collisions = reinterpret_cast<uint32_t*>(base + L.tickets) + 1;
+    // Words of the first tickets' lines that no group uses, cleared with them.
+    ties.counts = reinterpret_cast<uint32_t*>(base + L.tickets) + 1;
+    ties.sample_bits = bits;
+    ties.max_doubles = (uint32_t)((1ull << (2 * bits)) / (uint64_t)a.n);
+    ties.max_pairs = (uint32_t)((3ull << (2 * bits)) / (uint64_t)a.n);
+    table_words = 2ll << (bits + kTieSlotsPerDrawLog2);
   }
   int32_t rc = launch_zero_words(stream, hist, (L.total - L.zero_begin) / 4,
-                                 reinterpret_cast<uint32_t*>(ties.table),
-                                 ties.table != nullptr ? 2 * (int64_t)kTieSlots : 0);
+                                 reinterpret_cast<uint32_t*>(ties.table), table_words);
   if (rc != ILGPU_HIP_SUCCESS) return rc;
 
   {
-    int shift = 0;  // replicas: as many as kHistLdsWords of LDS counters hold
-    while ((1 << (shift + 1)) <= 32 &&
-           ((passes * kRadix) << (shift + 1)) <= kHistLdsWords)
-      ++shift;
-    const size_t lds = (size_t)((passes * kRadix) << shift) * 4;
-    // A block's fixed cost is its flush, one global atomic per digit value and
-    // position, which all blocks issue at about the same time.  Up to half a
-    // block per CU as soon as every thread has four vectors to count, more
-    // only when every thread has sixteen (2^20 u32 keys: 7.5 us instead of
-    // 15.5 with one vector per thread; 2^22: 12.3 instead of 17.1).
-    const int64_t vectors = div_up(a.n, Vec16<K>::N);
-    const int64_t few = std::min<int64_t>(div_up(vectors, kHistBlock * 4), std::max(cus / 2, 1));
-    int64_t blocks = std::max(few, div_up(vectors, kHistBlock * 16));
-    // Two blocks of 64 KiB of counters are resident per CU: no second round.
-    if (blocks > (int64_t)cus * ILGPU_HIP_SORT_HIST_BLOCKS_PER_CU)
-      blocks = (int64_t)cus * ILGPU_HIP_SORT_HIST_BLOCKS_PER_CU;
-    if (blocks < 1) blocks = 1;
-    if (ties.table != nullptr) {
-      ties.samples = (uint32_t)std::min<int64_t>(kTieSamples, blocks * kHistBlock);
-      ties.max_collisions =
-          (uint32_t)((uint64_t)ties.samples * ties.samples / (4ull * (uint64_t)a.n));
-    }
     ProfileScope scope(stream, "sort_histogram");
     auto* histogram_kernel = sort_histogram_kernel<K, false>;
     if constexpr (KEY_BYTES >= 2) {  // there is no 1-byte floating-point key
       if ((xf.reference_term | xf.total_term) != 0) histogram_kernel = sort_histogram_kernel<K, true>;
     }
-    hipLaunchKernelGGL(histogram_kernel, dim3((unsigned)blocks),
-                       dim3(kHistBlock), lds, stream, keys_a, a.n, xf, passes,
+    hipLaunchKernelGGL(histogram_kernel, dim3((unsigned)hist_blocks),
+                       dim3(kHistBlock), hist_lds, stream, keys_a, a.n, xf, passes,
                        shift, hist, ties);
     ILGPU_HIP_CHECK(hipGetLastError());
   }

@@ -1991,6 +1991,22 @@ def sort_index_pairs(keys, value_dtype=np.uint32, descending=False):
     return d.numpy(), v.numpy(), capi.radix_sort_passes(temp, keys.size, keys.dtype, size)[0]
 
 
+@pytest.mark.parametrize("kind,length,copies", [
+    ("one cluster", 16_000, 1), ("copies of one key", 16_000, 16_000), ("forty clusters", 500, 1)])
+def test_sort_takes_every_digit_where_many_keys_share_an_upper_half(kind, length, copies):
+    """Of 2^21 keys the longest run left to the ties is some 4096 keys (its draws
+    are a sixty-fourth of it), and no more than eight runs are drawn three times."""
+    n = TIE_LENGTH
+    note("clusters", kind)
+    keys = upper_half_keys(n, 79)
+    for c in range(40 if kind == "forty clusters" else 1):
+        cluster(keys, length, 80 + c, copies)
+    got, values, executed = sort_index_pairs(keys)
+    order = np.argsort(keys, kind="stable")
+    assert np.array_equal(got, keys[order]) and np.array_equal(values, order)
+    assert executed == 8
+
+
 # Runs around what sixteen lanes, a wave, and a block's LDS (2048 keys) take, with one,
 # two and three pieces to merge.
 @pytest.mark.parametrize("n,lengths", [
@@ -2065,3 +2081,38 @@ def test_large_block_passes_leave_the_ties(dtype, pairs):
         assert np.array_equal(keys.numpy().view(np.uint64), bits[order])
         if pairs:
             assert np.array_equal(values.numpy(), order)
+
+
+def test_sorts_of_long_inputs_can_be_captured_and_replayed():
+    """The draws' table and counts are cleared by every replay, whichever way the
+    keys of the one before went."""
+    import torch
+    n = TIE_LENGTH
+    static = torch.zeros(n, dtype=torch.int64, device="cuda:0")
+    work = torch.zeros(n, dtype=torch.int64, device="cuda:0")
+    d_work = D(n, np.uint64, _bytes=work.view(torch.uint8))
+    values = D.zeros(n, np.uint32)
+    temp = capi.temp_buffer(capi.radix_sort_temp_bytes(n, np.uint64, 4))
+
+    def calls():
+        work.copy_(static)
+        capi.radix_sort_pairs(d_work, values, temp, values_from_index=True)
+
+    calls()  # the one-time queries
+    sync()
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        with torch.cuda.graph(graph, stream=side):
+            calls()
+    sync()
+    for replay, (length, executed) in enumerate([(700, 4), (16_000, 8), (2100, 4), (20, 4)]):
+        note("replay", replay)
+        keys = cluster(upper_half_keys(n, 90 + replay), length, 91 + replay)
+        static.copy_(torch.from_numpy(keys.view(np.int64)))
+        assert torch.rand(1 << 20, device="cuda:0").sum().item() > 0  # eager work between replays
+        graph.replay()
+        sync()
+        order = np.argsort(keys, kind="stable")
+        assert np.array_equal(d_work.numpy(), keys[order]) and np.array_equal(values.numpy(), order)
+        assert capi.radix_sort_passes(temp, n, np.uint64, 4)[0] == executed
