@@ -2569,7 +2569,17 @@ __global__ __launch_bounds__(kTieBlock, 8) void ties_kernel(
         const uint64_t k0 = keys[start], k1 = keys[start + 1], k2 = keys[min(start + 2, last)],
                        k3 = keys[min(start + 3, last)];
         auto same = [&](uint64_t k, uint32_t j) { return start + j <= last && (k >> 32) == (k0 >> 32); };
-        if (!same(k3, 3)) {
+        if (!same(k2, 2)) {  // by itself: as two of the three below it cost 2^27 uniform pairs 1 %
+          if (ordered_bits(k1, xf) < ordered_bits(k0, xf)) {
+            if constexpr (VALUE_BYTES > 0) {
+              const Val v = vals[start];
+              vals[start] = vals[start + 1];
+              vals[start + 1] = v;
+            }
+            keys[start] = k1;
+            keys[start + 1] = k0;
+          }
+        } else if (!same(k3, 3)) {
           // Lower halves with their places, so that equal keys keep their order.
           uint64_t x[3] = {ordered_bits(k0, xf) << 32, ordered_bits(k1, xf) << 32 | 1u,
                            same(k2, 2) ? ordered_bits(k2, xf) << 32 | 2u : ~0ull << 32 | 2u};
