@@ -320,12 +320,18 @@ def run_extras(args, torch, capi, datagen, timer, wrap):
     if cpu_on:
         from oracle import cpu_oracle as O
 
-    def timed(name, prepare, fn, algo_bytes, kernel, kernel_bytes=None):
+    def timed(name, prepare, fn, algo_bytes, kernel, kernel_bytes=None, passes=None):
+        """passes: for a sort, gives the passes that ran, of as many launches as there are
+        digits; algo_bytes is then a function of them."""
         ms, _ = timer.run(prepare, fn, K, W)
         capi.profile_enable(True)
         timer.run(prepare, fn, K, 0)
         launches, k_ms = kernel_stats(capi, kernel)
         capi.profile_enable(False)
+        if passes is not None:
+            executed = passes()
+            algo_bytes = algo_bytes(executed)
+            k_ms *= launches / K / max(executed, 1)   # the other launches return at once
         t = float(np.median(ms))
         kb = kernel_bytes if kernel_bytes is not None else algo_bytes
         k_gbs = kb / (k_ms * 1e-3) / 1e9 if k_ms else 0.0
@@ -335,6 +341,8 @@ def run_extras(args, torch, capi, datagen, timer, wrap):
                  "frac_of_hbm_peak": round(algo_bytes / (t * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
                  "roofline": dict(roofline(k_gbs, *measured_traffic(name, args.log2n == 28)),
                                   kernel=kernel, avg_launch_ms=round(k_ms, 4))}
+        if passes is not None:
+            entry["passes_executed"] = executed
         out[name] = entry
         log(f"[bench] {name}: {t:.3f} ms/step, {entry['algorithmic_gbs']:.0f} GB/s "
             f"({100 * entry['frac_of_hbm_peak']:.1f}% of peak)")
@@ -422,7 +430,11 @@ def run_extras(args, torch, capi, datagen, timer, wrap):
     temp = capi.temp_buffer(capi.radix_sort_temp_bytes(n27, np.uint64, 4))
     e = timed("radix_sort_pairs_u64_u32_2^27", lambda: wk.copy_(k64),
               lambda: capi.radix_sort_pairs(dk, dv, temp, values_from_index=True),
-              n27 * (8.0 * 17 + 4.0 * 16), "sort_onesweep", n27 * 2.0 * 12)
+              # The histogram's read, the passes, and the read that orders what four
+              # passes over the upper half leave.
+              lambda p: n27 * (8.0 * (2 * p + 1) + 4.0 * 2 * p + (8.0 if p < 8 else 0.0)),
+              "sort_onesweep", n27 * 2.0 * 12,
+              passes=lambda: capi.radix_sort_passes(temp, n27, np.uint64, 4)[0])
     e["gpairs_per_s"] = round(n27 / (e["ms_per_step"] * 1e-3) / 1e9, 3)
     # stability + permutation: keys[values] reproduces the output, keys sorted
     # (unsigned order = signed order after flipping the sign bit), ties by index
