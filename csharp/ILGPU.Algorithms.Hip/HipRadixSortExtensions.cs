@@ -90,7 +90,8 @@ namespace ILGPU.Algorithms.Hip
 
         /// <summary>How many 8-bit passes the last sort that used temp ran and how
         /// many it found unnecessary (a pass whose digit is the same for every key
-        /// is skipped); same length, key type and value size (0 for keys only) as
+        /// is skipped, and so are the lower digits of 2^21 or more 8-byte keys whose upper
+        /// halves rarely meet, which are put in order after the passes); same length, key type and value size (0 for keys only) as
         /// that sort.  Waits for the stream.  The reference runs every pass whatever
         /// the keys and has nothing to report.</summary>
         public static (int Executed, int Skipped) GetRadixSortPasses<T, TRadixSortOperation>(

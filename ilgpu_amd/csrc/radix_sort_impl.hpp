@@ -9,10 +9,12 @@
 //   zero      clears the global digit histograms, tile tickets and look-back
 //             status words (one launch);
 //   histogram one read of the keys builds the 256-bin histogram of every digit
-//             position in LDS (replicated counters) and adds it to global;
+//             position in LDS (replicated counters) and adds it to global; from
+//             8-byte keys it also draws a sample of upper halves;
 //   plan      one block turns the histograms into exclusive digit offsets,
 //             marks passes whose digit is the same for every key (they are
-//             skipped) and records which buffer each pass reads;
+//             skipped), or whose digit is left to the ties since the upper halves
+//             drawn rarely meet, and records which buffer each pass reads;
 //   pass x k  onesweep: a block takes a tile by ticket, ranks its keys (one
 //             returning LDS add per key on per-wave digit counters; the LDS
 //             serves the lanes of an instruction in lane order, so equal digits
@@ -20,7 +22,9 @@
 //             its 256 digit counts, resolves the counts of all earlier tiles by
 //             decoupled look-back, stages the tile in digit order through LDS
 //             and writes each digit's run to its final place;
-//   finish    copies the result back if an odd number of passes ran.
+//   finish    copies the result back if an odd number of passes ran; after
+//             passes over the upper half of 8-byte keys it orders the runs of
+//             keys that share one (ties_kernel).
 //
 // Keys and values stay in separate arrays (structure of arrays); a value
 // travels with its key through the same tile-local permutation.
@@ -32,7 +36,7 @@
 // first pass that runs, and converted back by the last one.
 //
 // Algorithmic HBM traffic for n keys of k bytes, values of v bytes and P
-// executed passes: n * (k * (2P + 1) + v * 2P) bytes.
+// executed passes: n * (k * (2P + 1) + v * 2P) bytes, and n * k where ties are left.
 //
 // This header holds the kernels and their launch code as templates; one
 // translation unit per key size (radix_sort_k1/2/4/8.hip) instantiates them, so
@@ -297,7 +301,7 @@ constexpr uint32_t kNoHotDigit = 0xFFFFFFFFu;
 constexpr int kMaxHot = 4;
 // Device-resident description of the passes, written by plan_kernel.
 struct SortPlan {
-  uint32_t skip[kMaxPasses];        // digit identical for all keys
+  uint32_t skip[kMaxPasses];        // digit identical for all keys, or left to the ties
   uint32_t src_is_alt[kMaxPasses];  // pass reads the alternate buffer
   // Up to kMaxHot digits that each hold an eighth of the keys or more, most
   // frequent first; unused entries are kNoHotDigit.
