@@ -2185,7 +2185,7 @@ __global__ __launch_bounds__(256) void finish_kernel(
 // A read of the keys, then: a lane takes kTieRows keys, a row of a wave 64
 // neighbouring ones, and the runs of all rows are ordered together, since each
 // costs a chain of two or three memory round trips.  Runs of two or three keys, which nearly
-// all of them are, are ordered by the lane that sees the first one, longer ones by 16, 32 or
+// all of them are, are ordered by the lane that sees the first one, longer ones by 8 to
 // 64 lanes with a key per lane, or a wave with two.  Runs of 128 keys and more wait until
 // the block's waves have seen all of their keys, and are then ordered by the block.
 constexpr int kTieRows = 8;
@@ -2197,13 +2197,14 @@ constexpr int kTieMerges = 4;       // memory reads of a thread in flight where 
 // Runs of 128 keys and more that can start in one chunk.
 constexpr int kTieLongsPerChunk = kTieChunk / 128;
 
-// Runs of fewer than G keys, one by each G lanes (start: of the lane's run, if there is
-// one for it).  A key's place is the number of keys that go in front of it.
-template <int G, int VALUE_BYTES, typename Val>
+// Runs of fewer than `width` keys, one by each `width` lanes (start: of the lane's run, if
+// there is one for it; width: 8 to 64).  A key's place is the number of keys that go in
+// front of it.
+template <int VALUE_BYTES, typename Val>
 __device__ __forceinline__ void order_runs(uint64_t* keys, Val* vals, uint32_t start, bool any, uint32_t n,
-                                           const KeyXform& xf, int lane) {
-  const int l = lane & (G - 1);
-  const uint32_t at = start + l;
+                                           const KeyXform& xf, int lane, int width) {
+  const int first = lane & ~(width - 1);
+  const uint32_t at = start + (uint32_t)(lane - first);
   const bool have = any && at < n;
   uint64_t k = 0;
   Val v{};
@@ -2211,27 +2212,27 @@ __device__ __forceinline__ void order_runs(uint64_t* keys, Val* vals, uint32_t s
     k = keys[at];
     if constexpr (VALUE_BYTES > 0) v = vals[at];
   }
-  const uint32_t upper = (uint32_t)__shfl((int)(uint32_t)(k >> 32), 0, G);
-  const bool same = have && (uint32_t)(k >> 32) == upper;
-  const uint64_t lanes = __ballot(same) >> (lane & ~(G - 1));
-  const int len = __builtin_ctzll(~lanes);
+  const bool same = have && (uint32_t)(k >> 32) == (uint32_t)__shfl((int)(uint32_t)(k >> 32), first);
+  const int end = first + __builtin_ctzll(~(__ballot(same) >> first));
   const uint32_t o = (uint32_t)ordered_bits(k, xf);  // the upper halves agree
-  int rank = 0;
-  if constexpr (G == kWaveSize) {
+  int rank = first;
+  if (width == kWaveSize) {  // one run: `end` is the same in every lane
+    const int len = __builtin_amdgcn_readfirstlane(end);
     for (int j = 0; j < len; ++j) {
       const uint32_t q = (uint32_t)__builtin_amdgcn_readlane((int)o, j);
-      if (q < o || (q == o && j < l)) ++rank;
+      if (q < o || (q == o && j < lane)) ++rank;
     }
   } else {
-#pragma unroll 8
-    for (int j = 0; j < G; ++j) {
-      const uint32_t q = (uint32_t)__shfl((int)o, j, G);
-      if (j < len && (q < o || (q == o && j < l))) ++rank;
+#pragma unroll 4
+    for (int j = 0; j < width; ++j) {
+      const int other = first + j;
+      const uint32_t q = (uint32_t)__shfl((int)o, other);
+      if (other < end && (q < o || (q == o && other < lane))) ++rank;
     }
   }
-  if (l < len && rank != l) {
-    keys[start + rank] = k;
-    if constexpr (VALUE_BYTES > 0) vals[start + rank] = v;
+  if (lane < end && rank != lane) {
+    keys[start + (uint32_t)(rank - first)] = k;
+    if constexpr (VALUE_BYTES > 0) vals[start + (uint32_t)(rank - first)] = v;
   }
 }
 
@@ -2607,27 +2608,25 @@ __global__ __launch_bounds__(kTieBlock, 8) void ties_kernel(
             if constexpr (VALUE_BYTES > 0) vals[start + j] = v[j];
           }
         } else {
-          const uint64_t k15 = keys[min(start + 15, last)], k31 = keys[min(start + 31, last)],
-                         k63 = keys[min(start + 63, last)], k127 = keys[min(start + 127, last)];
-          places = same(k127, 127) ? 256 : same(k63, 63) ? 128 : same(k31, 31) ? 64 : same(k15, 15) ? 32 : 16;
+          const uint64_t k7 = keys[min(start + 7, last)], k15 = keys[min(start + 15, last)],
+                         k31 = keys[min(start + 31, last)], k63 = keys[min(start + 63, last)],
+                         k127 = keys[min(start + 127, last)];
+          places = 8 << (int)same(k7, 7) << (int)same(k15, 15) << (int)same(k31, 31) << (int)same(k63, 63)
+                     << (int)same(k127, 127);
           if (places == 256) long_starts[atomicAdd(&s_longs, 1u)] = start;
         }
       }
-      // Runs of G lanes, as many at once as the wave has room for.
-      auto order_all = [&](auto width) {
-        constexpr int G = decltype(width)::value;
-        for (uint64_t owners = __ballot(places == G); owners != 0ull;) {
-          int mine = -1;
-          for (int g = 0; g < kWaveSize / G && owners != 0ull; ++g, owners &= owners - 1)
-            if (lane / G == g) mine = __builtin_ctzll(owners);
-          const uint32_t s = (uint32_t)__shfl((int)start, mine < 0 ? 0 : mine);
-          order_runs<G, VALUE_BYTES>(keys, vals, s, mine >= 0, (uint32_t)n, xf, lane);
-        }
-      };
       if (__ballot(places != 0) == 0ull) continue;
-      order_all(std::integral_constant<int, 16>{});
-      order_all(std::integral_constant<int, 32>{});
-      order_all(std::integral_constant<int, 64>{});
+      // As many runs at once as the wave has room for.
+      for (int width = 8; width <= kWaveSize; width <<= 1) {
+        for (uint64_t owners = __ballot(places == width); owners != 0ull;) {
+          int mine = -1;
+          for (int first = 0; first < kWaveSize && owners != 0ull; first += width, owners &= owners - 1)
+            if ((lane & ~(width - 1)) == first) mine = __builtin_ctzll(owners);
+          const uint32_t s = (uint32_t)__shfl((int)start, mine < 0 ? 0 : mine);
+          order_runs<VALUE_BYTES>(keys, vals, s, mine >= 0, (uint32_t)n, xf, lane, width);
+        }
+      }
       for (uint64_t owners = __ballot(places == 128); owners != 0ull; owners &= owners - 1)
         order_two_rows<VALUE_BYTES>(
             keys, vals, (uint32_t)__builtin_amdgcn_readlane((int)start, __builtin_ctzll(owners)), (uint32_t)n, xf,
