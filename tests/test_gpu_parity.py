@@ -299,6 +299,19 @@ def test_histogram_of_columns_that_crowd_one_bin(bins, stride):
             assert overflow.numpy()[0] == 0
 
 
+@pytest.mark.parametrize("dtype,locator", [
+    (np.float32, capi.LOCATOR_IDENTITY), (np.float64, capi.LOCATOR_MODULO),
+    (np.int64, capi.LOCATOR_MODULO), (np.uint64, capi.LOCATOR_IDENTITY), (np.int16, capi.LOCATOR_IDENTITY)])
+def test_histogram_of_crowded_columns_of_other_types(dtype, locator):
+    rng = np.random.default_rng(3)
+    n, bins = 70_003, 2000
+    note("histogram crowded", np.dtype(dtype).name, locator)
+    low, high = (0, bins) if locator == capi.LOCATOR_IDENTITY else (-50, 2 * bins)  # the oracle's bins
+    column = np.where(rng.random(n) < 0.8, 1999, rng.integers(low, high, n)).astype(dtype)
+    for bin_dtype in (np.int32, np.float32):
+        assert_hist_equal(column, np.zeros(bins, dtype=bin_dtype), locator)
+
+
 def test_histogram_many_bins_uses_global_atomics():
     n, bins = 200000, 100000
     v = random_ints(np.int32, n, seed=4, lo=0, hi=bins - 1)
