@@ -226,12 +226,16 @@ def main():
     hist_launches, hist_ms = kernel_stats(capi, "sort_histogram")
     kernel_ms = {name: round(kernel_stats(capi, name)[1], 4) for name in
                  ("zero_words", "sort_histogram", "sort_plan", "sort_onesweep",
-                  "sort_finish")}
+                  "sort_local", "sort_finish")}
     capi.profile_enable(False)
     passes, _ = capi.radix_sort_passes(temp, n, np.uint32)   # executed, from the sort's plan
+    # The launches of the passes that do not run return at once.
+    pass_ms *= pass_launches / K / max(passes, 1)
+    kernel_ms["sort_onesweep"] = round(pass_ms, 4)
+    local_sort = 2 if passes < 4 else 0  # random keys: the rest in one read and one write
     pass_bytes = 2.0 * n * 4            # read + write of the keys, one pass
     pass_gbs = pass_bytes / (pass_ms * 1e-3) / 1e9 if pass_ms else 0.0
-    sort_bytes = n * 4.0 * (2 * passes + 1)
+    sort_bytes = n * 4.0 * (2 * passes + 1 + local_sort)
     sort_gbs = sort_bytes / (ms_per_step * 1e-3) / 1e9
 
     # Cheap verification on the GPU: sorted, and the same multiset checksum.
@@ -286,7 +290,7 @@ def main():
                                "uniform over the full 32-bit range "
                                "(SplitMix64 seed 0x123456789ABCDEF0)",
                    "n": n, "passes_executed": passes,
-                   "algorithmic_bytes_per_key": 4 * (2 * passes + 1)},
+                   "algorithmic_bytes_per_key": 4 * (2 * passes + 1 + local_sort)},
         "roofline": dict(roofline(pass_gbs, *measured_traffic(
                              "radix_sort_u32_uniform_2^28", args.log2n == 28)),
                          kernel="onesweep_pipelined_kernel<4, false>",
@@ -430,9 +434,8 @@ def run_extras(args, torch, capi, datagen, timer, wrap):
     temp = capi.temp_buffer(capi.radix_sort_temp_bytes(n27, np.uint64, 4))
     e = timed("radix_sort_pairs_u64_u32_2^27", lambda: wk.copy_(k64),
               lambda: capi.radix_sort_pairs(dk, dv, temp, values_from_index=True),
-              # The histogram's read, the passes, and the read that orders what four
-              # passes over the upper half leave.
-              lambda p: n27 * (8.0 * (2 * p + 1) + 4.0 * 2 * p + (8.0 if p < 8 else 0.0)),
+              # The histogram's read, the passes, and the local sort of what they leave.
+              lambda p: n27 * (8.0 * (2 * p + 1) + 4.0 * 2 * p + (2.0 * 12 if p < 8 else 0.0)),
               "sort_onesweep", n27 * 2.0 * 12,
               passes=lambda: capi.radix_sort_passes(temp, n27, np.uint64, 4)[0])
     e["gpairs_per_s"] = round(n27 / (e["ms_per_step"] * 1e-3) / 1e9, 3)
@@ -478,7 +481,7 @@ def run_extras(args, torch, capi, datagen, timer, wrap):
         timer.run(lambda: wk.copy_(part), lambda: capi.radix_sort_keys(kv, tp), 1, 0)
         launches = sum(kernel_stats(capi, k)[0] for k in
                        ("zero_words", "sort_histogram", "sort_plan", "sort_onesweep",
-                        "sort_finish", "sort_small"))
+                        "sort_local", "sort_finish", "sort_small"))
         capi.profile_enable(False)
         t = float(np.median(ms))
         if cpu_on:
@@ -491,7 +494,7 @@ def run_extras(args, torch, capi, datagen, timer, wrap):
             ok = bool(((wk.to(torch.int64) & 0xFFFFFFFF) == ref64).all().item())
             del ref64
         passes, _ = capi.radix_sort_passes(tp, m, np.uint32)
-        algo = m * 4.0 * (2 * passes + 1)
+        algo = m * 4.0 * (2 * passes + 1 + (2 if passes < 4 else 0))  # and the local sort
         out[f"radix_sort_u32_2^{log2m}"] = {
             "ms_per_step": round(t, 4), "gkeys_per_s": round(m / (t * 1e-3) / 1e9, 2),
             "passes_executed": passes, "kernel_launches": launches,

@@ -7,13 +7,16 @@
 // keys is
 //
 //   zero      clears the global digit histograms, tile tickets and look-back
-//             status words (one launch);
+//             status words (one launch), and draws keys where the local sort is
+//             offered;
 //   histogram one read of the keys builds the 256-bin histogram of every digit
 //             position in LDS (replicated counters) and adds it to global; from
-//             8-byte keys it also draws a sample of upper halves;
+//             8-byte keys it also draws a sample of upper halves, and one block
+//             of it looks at the draws for the local sort;
 //   plan      one block turns the histograms into exclusive digit offsets,
 //             marks passes whose digit is the same for every key (they are
-//             skipped), or whose digit is left to the ties since the upper halves
+//             skipped), is left to the local sort since passes over the one or two
+//             topmost digits make short runs, or to the ties since the upper halves
 //             drawn rarely meet, and records which buffer each pass reads;
 //   pass x k  onesweep: a block takes a tile by ticket, ranks its keys (one
 //             returning LDS add per key on per-wave digit counters; the LDS
@@ -23,8 +26,10 @@
 //             decoupled look-back, stages the tile in digit order through LDS
 //             and writes each digit's run to its final place;
 //   finish    copies the result back if an odd number of passes ran; after
-//             passes over the upper half of 8-byte keys it orders the runs of
-//             keys that share one (ties_kernel).
+//             passes over the topmost digits it sorts the runs of keys that agree
+//             in them, a window of whole runs at a time in LDS (local_sort_kernel,
+//             radix_sort_local.hpp); after passes over the upper half of 8-byte keys it
+//             orders the runs of keys that share one (ties_kernel).
 //
 // Keys and values stay in separate arrays (structure of arrays); a value
 // travels with its key through the same tile-local permutation.
@@ -36,7 +41,8 @@
 // first pass that runs, and converted back by the last one.
 //
 // Algorithmic HBM traffic for n keys of k bytes, values of v bytes and P
-// executed passes: n * (k * (2P + 1) + v * 2P) bytes, and n * k where ties are left.
+// executed passes: n * (k * (2P + 1) + v * 2P) bytes, n * k where ties are left, and
+// 2 n (k + v) where the local sort follows.
 //
 // This header holds the kernels and their launch code as templates; one
 // translation unit per key size (radix_sort_k1/2/4/8.hip) instantiates them, so
@@ -47,7 +53,9 @@
 
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <type_traits>
 
 #include "kernels.hpp"
@@ -311,6 +319,7 @@ struct SortPlan {
   uint32_t executed;                // number of passes that run
   uint32_t final_in_alt;            // result sits in the alternate buffer
   uint32_t ties_left;               // the lower digits are left to ties_kernel
+  uint32_t local_from;              // the digits below this one are left to local_sort_kernel
 };
 static_assert(sizeof(SortPlan) <= 256, "the temp view holds 256 bytes for the plan");
 
@@ -370,6 +379,184 @@ struct TieSampling {
   uint32_t max_doubles, max_pairs;
 };
 
+// Whether the local sort (local_sort_kernel) can do what passes over the topmost digits leave is asked
+// of m draws, one from every m-th part of the input, before anything is counted:
+// sort_draw_kernel draws them and one block of the histogram kernel looks at them.
+//   Keys may not crowd: sixteen of them in one of the local sort's bins, of which there are some
+//   four for every key, send a window the slow way.  Of draws that agree down to a bin (in
+//   log2(n) + 1 bits from the topmost one that differs) there are some m^2 / 4n if
+//   the keys spread evenly and k m^2 / 2n if each bin in use holds k of them; up to 1.25 m^2 / n
+//   are taken (k = 2.5; from k = 5 on a window in nine has such a bin).
+//   Two digits make runs that fit a window if few draws share a 16-bit prefix: a run of L keys
+//   is drawn L m / n times and gives half the square of that in pairs of draws.
+//   (Whether one digit does, its counts tell exactly.)
+// (2^26 u32 keys, every value some 30 times, with a copy in front, us: every digit sorted 750, the local
+// sort 1236.)
+constexpr int kLocalMinDrawBits = 12, kLocalMaxDrawBits = 16;
+struct LocalSampling {
+  const void* draws;        // keys in their ordered form.  nullptr: not asked
+  uint32_t* from;           // out: the lowest digit of the prefix whose runs are short (0: they are not),
+                            // and in the next word whether the keys spread
+  uint32_t draw_bits;       // log2 of the number of draws
+  uint32_t bin_bits;        // of a draw, from the topmost bit that differs on
+  uint32_t max_equal;       // draws that meet an earlier one in these bits
+  uint32_t max_pairs;       // pairs of draws that share a 16-bit prefix
+  uint32_t max_draws;       // of one prefix
+};
+// Where the draws lie in the alternate keys: behind the table of TieSampling.
+constexpr int64_t kLocalDrawsOffset = 8ll << (kTieMaxSampleBits + kTieSlotsPerDrawLog2);
+
+// Clears words[0..count) and more[0..more_count) and takes the draws of LocalSampling.
+template <typename K, bool FLOAT_KEYS>
+__global__ __launch_bounds__(256) void sort_draw_kernel(
+    uint32_t* words, int64_t count, uint32_t* more, int64_t more_count, const K* __restrict__ keys,
+    int64_t n, KeyXform xf, K* draws, uint32_t draw_bits) {
+  const int64_t stride = (int64_t)gridDim.x * 256;
+  const int64_t first = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  for (int64_t s = first; s < 1ll << draw_bits; s += stride) {
+    uint64_t z = ((uint64_t)s + 1ull) * 0x9E3779B97F4A7C15ull;  // splitmix64
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+    z ^= z >> 31;
+    const uint64_t at = ((uint64_t)s << 32 | (uint32_t)z) << (32 - draw_bits);  // a random place in part s
+    const K k = keys[__umul64hi(at, (uint64_t)n)];
+    const K o = FLOAT_KEYS ? ordered_bits(k, xf) : (K)(k ^ (K)xf.xor_mask);
+    draws[s] = o;
+  }
+  for (int64_t i = first; i < count; i += stride) words[i] = 0u;
+  for (int64_t i = first; i < more_count; i += stride) more[i] = 0u;
+}
+
+// By one block of the histogram kernel, with its LDS: what the draws say, into local.from[0..1].
+// (The draws are held in registers where one chunk is all of them: short inputs wait for this block.)
+template <typename K>
+__device__ __forceinline__ void choose_local_digits(const LocalSampling& local, uint32_t* s_table) {
+  constexpr int kTableBits = 14;  // words
+  static_assert(kHistLdsWords >= 1 << kTableBits, "a byte for every 16-bit prefix");
+  constexpr int kPerVector = 16 / (int)sizeof(K);
+  constexpr int kVectors = (1 << 14) / kPerVector / kHistBlock;  // of a thread and a chunk of 2^14 draws
+  using V = typename Vec16<K>::type;
+  const int t = threadIdx.x;
+  __shared__ unsigned long long s_diff;
+  __shared__ uint32_t s_equal, s_pairs, s_draws;
+  auto clear_table = [&]() {
+    for (int i = t; i < (1 << kTableBits) / 4; i += kHistBlock)
+      reinterpret_cast<uint4*>(s_table)[i] = make_uint4(0u, 0u, 0u, 0u);
+  };
+  const V* draws = static_cast<const V*>(local.draws);
+  const int vectors = (1 << local.draw_bits) / kPerVector;
+  const int chunks = local.draw_bits > 14 ? 1 << (local.draw_bits - 14) : 1;
+  V d[kVectors];
+  auto load = [&](int chunk) {
+#pragma unroll
+    for (int v = 0; v < kVectors; ++v) {
+      const int i = (chunk * kVectors + v) * kHistBlock + t;
+      d[v] = draws[i < vectors ? i : 0];
+    }
+  };
+  auto in_use = [&](int chunk, int v) { return (chunk * kVectors + v) * kHistBlock + t < vectors; };
+  load(0);
+  const K first = static_cast<const K*>(local.draws)[0];
+  clear_table();
+  if (t == 0) {
+    s_diff = 0ull;
+    s_equal = s_pairs = s_draws = 0u;
+  }
+  K diff = 0;
+#pragma unroll
+  for (int v = 0; v < kVectors; ++v)
+#pragma unroll
+    for (int u = 0; u < kPerVector; ++u) diff |= (K)(d[v][u] ^ first);
+#pragma unroll
+  for (int s = 1; s < kWaveSize; s <<= 1) diff |= shfl(diff, (t & (kWaveSize - 1)) ^ s);
+  __syncthreads();
+  if ((t & (kWaveSize - 1)) == 0) atomicOr(&s_diff, (unsigned long long)diff);
+  __syncthreads();
+  const int top_bit = s_diff != 0ull ? 63 - __builtin_clzll(s_diff) : 0;  // the topmost bit that differs
+  const int top = top_bit / 8;                                            // and its digit
+  if (top < 3) return;  // two digits at least have to be below the passes' for the way to pay
+  // 32 bits from the topmost one that differs on.
+  auto upper = [&](K k) -> uint32_t {
+    return top_bit >= 31 ? (uint32_t)(k >> (top_bit - 31)) : (uint32_t)k << (31 - top_bit);
+  };
+
+  // Draws that meet an earlier one, in a table of open addressing: of many draws those of one part
+  // of the values, which half fill it.
+  const int parts_log2 = (int)local.draw_bits > kTableBits - 1 ? (int)local.draw_bits - (kTableBits - 1) : 0;
+  constexpr uint32_t kSlots = 1u << kTableBits;
+  uint32_t equal = 0;
+  for (int chunk = 0; chunk < chunks; ++chunk) {
+    if (chunks > 1) load(chunk);
+#pragma unroll
+    for (int v = 0; v < kVectors; ++v) {
+      if (!in_use(chunk, v)) continue;
+      uint32_t value[kPerVector], slot[kPerVector], old[kPerVector];
+#pragma unroll
+      for (int u = 0; u < kPerVector; ++u) {
+        value[u] = upper(d[v][u]) >> (32 - local.bin_bits);  // at most 31 bits
+        uint32_t hash = value[u] * 0x9E3779B1u;
+        hash = (hash ^ hash >> 16) * 0x85EBCA6Bu;
+        slot[u] = hash >> (32 - kTableBits);
+        old[u] = 0u;
+        if ((hash & ((1u << parts_log2) - 1u)) == 0u) old[u] = atomicCAS(&s_table[slot[u]], 0u, value[u] + 1u);
+      }
+#pragma unroll
+      for (int u = 0; u < kPerVector; ++u) {
+        for (int probe = 0; probe < 8 && old[u] != 0u && old[u] != value[u] + 1u; ++probe) {
+          slot[u] = (slot[u] + 1u) & (kSlots - 1u);
+          old[u] = atomicCAS(&s_table[slot[u]], 0u, value[u] + 1u);
+        }
+        equal += old[u] == value[u] + 1u;
+      }
+    }
+  }
+#pragma unroll
+  for (int s = 1; s < kWaveSize; s <<= 1) equal += shfl(equal, (t & (kWaveSize - 1)) ^ s);
+  if ((t & (kWaveSize - 1)) == 0) atomicAdd(&s_equal, equal);
+  __syncthreads();
+  if (s_equal > local.max_equal >> parts_log2) return;
+  if (t == 0) local.from[1] = 1u;
+  if (local.max_pairs == 0u) return;  // one digit is enough
+
+  // Draws of every prefix, a byte each (of 2^15 draws at most: with 2^16 the histogram of 2^26 keys
+  // waited 16 us for this block).
+  clear_table();
+  __syncthreads();
+  uint32_t pairs = 0, most = 0;
+  for (int chunk = 0; chunk < chunks && chunk < 2; ++chunk) {
+    if (chunks > 1) load(chunk);
+#pragma unroll
+    for (int v = 0; v < kVectors; ++v) {
+      // (Far too many of one prefix: enough.  A count that runs over says the same.)
+      if (!in_use(chunk, v) || most >= 128u) continue;
+      uint32_t old[kPerVector];
+#pragma unroll
+      for (int u = 0; u < kPerVector; ++u) {
+        const uint32_t prefix = (uint32_t)(d[v][u] >> (8 * (top - 1))) & 0xFFFFu;
+        const uint32_t at = (prefix & 3u) * 8u;
+        old[u] = (atomicAdd(&s_table[prefix >> 2], 1u << at) >> at) & 0xFFu;
+      }
+#pragma unroll
+      for (int u = 0; u < kPerVector; ++u) {
+        pairs += old[u];
+        most = most < old[u] ? old[u] : most;
+      }
+    }
+  }
+#pragma unroll
+  for (int s = 1; s < kWaveSize; s <<= 1) {
+    pairs += shfl(pairs, (t & (kWaveSize - 1)) ^ s);
+    const uint32_t other = shfl(most, (t & (kWaveSize - 1)) ^ s);
+    most = most < other ? other : most;
+  }
+  if ((t & (kWaveSize - 1)) == 0) {
+    atomicAdd(&s_pairs, pairs);
+    atomicMax(&s_draws, most + 1u);
+  }
+  __syncthreads();
+  if (t == 0 && s_pairs <= local.max_pairs && s_draws <= local.max_draws) local.from[0] = (uint32_t)(top - 1);
+}
+
 // The first active lane's key, as a wave-uniform value.
 __device__ __forceinline__ uint64_t readfirstlane_key(uint64_t k) {
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)k);
@@ -390,10 +577,19 @@ __device__ __forceinline__ uint32_t readfirstlane_key(uint8_t k) {
 template <typename K, bool FLOAT_KEYS>
 __global__ __launch_bounds__(kHistBlock) void sort_histogram_kernel(
     const K* __restrict__ keys, int64_t n, KeyXform xf, int passes,
-    int replica_shift, uint32_t* __restrict__ global_hist, TieSampling ties) {
+    int replica_shift, uint32_t* __restrict__ global_hist, TieSampling ties, LocalSampling local) {
   using V = typename Vec16<K>::type;
   constexpr int VN = Vec16<K>::N;
   extern __shared__ __align__(8) uint32_t s_hist[];  // [passes][256][replicas]
+  // Blocks that count, and this one among them: where draws are looked at the last block of the
+  // grid does that.
+  const uint32_t counting = gridDim.x - (sizeof(K) >= 4 && local.draws != nullptr ? 1u : 0u);
+  if constexpr (sizeof(K) >= 4) {
+    if (blockIdx.x == counting) {
+      choose_local_digits<K>(local, s_hist);
+      return;
+    }
+  }
   const int words = (passes * kRadix) << replica_shift;
   // This thread's draw of the tie sampling.  Draws meet within their block first, in
   // LDS: where many keys share an upper half, all draws of the grid would queue
@@ -563,7 +759,7 @@ __global__ __launch_bounds__(kHistBlock) void sort_histogram_kernel(
   const V* body = reinterpret_cast<const V*>(keys + head);
   const int64_t nvec = (n - head) / VN;
   const int64_t tail_start = head + nvec * VN;
-  const int64_t stride = (int64_t)gridDim.x * kHistBlock;
+  const int64_t stride = (int64_t)counting * kHistBlock;
   // The first round's vectors are requested, and by the first of them a wave
   // decides whether it looks for runs at all: the check costs keys that vary
   // 1 to 2 % of a sort when every vector pays it.
@@ -648,99 +844,129 @@ __global__ __launch_bounds__(kHistBlock) void sort_histogram_kernel(
 }
 
 // ---- plan: exclusive digit offsets, skipped passes, buffer parity ---------
-__global__ __launch_bounds__(kRadix) void plan_kernel(
+// One block; every 256 threads take a digit position, four at a time.  (One position after the other,
+// a chain of barriers, took 4.5 us for 4-byte keys and 8.4 for 8-byte keys.)
+constexpr int kPlanGroups = 4;
+constexpr int kPlanBlock = kPlanGroups * kRadix;
+__global__ __launch_bounds__(kPlanBlock) void plan_kernel(
     const uint32_t* __restrict__ global_hist, uint32_t* __restrict__ excl,
-    SortPlan* __restrict__ plan, int passes, uint32_t n, TieSampling ties) {
-  __shared__ uint32_t s_wave[kRadix / kWaveSize];
-  __shared__ int s_trivial;
-  __shared__ unsigned long long s_hot[kMaxHot];  // count << 8 | digit, most frequent first
-  const int d = threadIdx.x;
+    SortPlan* __restrict__ plan, int passes, uint32_t n, TieSampling ties,
+    const uint32_t* __restrict__ local_from, uint32_t local_max_run) {
+  constexpr int kRounds = kMaxPasses / kPlanGroups;
+  constexpr int kGroupWaves = kRadix / kWaveSize;
+  constexpr int kFrequent = 8;  // digits with an eighth of the keys: no more than eight
+  __shared__ uint32_t s_wave[kMaxPasses][kGroupWaves];
+  __shared__ uint32_t s_most[kMaxPasses];  // keys of a position's most frequent digit
+  __shared__ uint32_t s_frequent[kMaxPasses];
+  __shared__ unsigned long long s_hot[kMaxPasses][kFrequent];  // count << 8 | digit
+  const int d = threadIdx.x & (kRadix - 1);
+  const int group = threadIdx.x / kRadix;
   const int lane = d & (kWaveSize - 1);
   const int wave = d / kWaveSize;
-  uint32_t parity = 0, executed = 0, first = passes, last = passes;
-  // The counts of every pass in one round trip (the loop below is a chain of
-  // barriers that a load inside it would wait behind, pass after pass).
-  uint32_t counts[kMaxPasses];
+  uint32_t counts[kRounds], inclusive[kRounds];
 #pragma unroll
-  for (int p = 0; p < kMaxPasses; ++p) counts[p] = p < passes ? global_hist[p * kRadix + d] : 0u;
-  // The lower digits [0, left) are left to the ties if the draws rarely meet and
-  // that saves at least two passes (a digit that all keys share needs none).
-  // An even number of passes ends in the caller's buffer, where the ties are ordered: an
-  // odd one takes a lower digit along.
-  int left = 0;
+  for (int r = 0; r < kRounds; ++r) {
+    const int p = r * kPlanGroups + group;
+    counts[r] = p < passes ? global_hist[p * kRadix + d] : 0u;
+  }
+  uint32_t pairs = 0, doubles = 0, groups = 0;
   if (ties.table != nullptr) {
-    uint32_t pairs = 0, doubles = 0, groups = 0;
     for (int g = 0; g < kTicketGroups; ++g) {
       pairs += ties.counts[g * kTicketStride];
       doubles += ties.counts[g * kTicketStride + 1];
       groups += ties.counts[g * kTicketStride + 2];
     }
-    if (pairs <= ties.max_pairs && doubles <= ties.max_doubles && groups <= kTieGroups) {
-      uint32_t trivial = 0;
-#pragma unroll
-      for (int p = 0; p < kMaxPasses; ++p) trivial |= counts[p] == n ? 1u << p : 0u;
-      if (d == 0) s_trivial = 0;
-      __syncthreads();
-      if (trivial != 0) atomicOr(&s_trivial, (int)trivial);
-      __syncthreads();
-      const uint32_t varies = ~(uint32_t)s_trivial & ((1u << kMaxPasses) - 1u);
-      __syncthreads();
-      left = kMaxPasses - kTiePasses;
-      if (__popc(varies >> left) & 1)
-        while (left > 0 && !(varies >> --left & 1u)) {}
-      if (__popc(varies & ((1u << left) - 1u)) < 2) left = 0;
-    }
   }
+  const bool spread = local_from != nullptr && local_from[1] != 0u;
+  const int two_digits = spread ? (int)local_from[0] : 0;
+  if (threadIdx.x < kMaxPasses) s_most[threadIdx.x] = s_frequent[threadIdx.x] = 0u;
+  if (threadIdx.x < kMaxPasses * kFrequent) s_hot[threadIdx.x / kFrequent][threadIdx.x % kFrequent] = 0ull;
+  __syncthreads();
 #pragma unroll
-  for (int p = 0; p < kMaxPasses; ++p) {
-    if (p >= passes) break;
-    if (d < kMaxHot) s_hot[d] = 0ull;
-    if (d == 0) s_trivial = 0;
-    __syncthreads();
-    const uint32_t c = counts[p];
-    if (c == n) s_trivial = 1;
-    // A digit qualifies with an eighth of the keys (two lanes of a
-    // sub-tile row on average); kMaxHot rounds of "largest below the previous
-    // one" order the most frequent ones.
-    const unsigned long long mine = ((unsigned long long)c << 8) | (unsigned long long)d;
-    const bool frequent = (uint64_t)c * 8 >= (uint64_t)n;
-    for (int h = 0; h < kMaxHot; ++h) {
-      if (frequent && (h == 0 || mine < s_hot[h - 1])) atomicMax(&s_hot[h], mine);
-      __syncthreads();
-    }
-    uint32_t inc = c;
+  for (int r = 0; r < kRounds; ++r) {
+    const int p = r * kPlanGroups + group;
+    const uint32_t c = counts[r];
+    uint32_t inc = c, most = c;
 #pragma unroll
     for (int s = 1; s < kWaveSize; s <<= 1) {
       const uint32_t o = shfl_up(inc, s);
       if (lane >= s) inc += o;
+      const uint32_t q = shfl(most, lane ^ s);
+      most = most < q ? q : most;
     }
-    if (lane == kWaveSize - 1) s_wave[wave] = inc;
-    __syncthreads();
+    inclusive[r] = inc;
+    if (lane == kWaveSize - 1) s_wave[p][wave] = inc;
+    if (lane == 0) atomicMax(&s_most[p], most);
+    // A digit qualifies as dominant with an eighth of the keys (two lanes of a sub-tile row on
+    // average).
+    if (c != 0u && (uint64_t)c * kFrequent >= (uint64_t)n)
+      s_hot[p][atomicAdd(&s_frequent[p], 1u)] = ((unsigned long long)c << 8) | (unsigned long long)d;
+  }
+  __syncthreads();
+  uint32_t varies = 0;  // positions whose digit is not the same for every key
+#pragma unroll
+  for (int p = 0; p < kMaxPasses; ++p) varies |= p < passes && s_most[p] != n ? 1u << p : 0u;
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    const int p = r * kPlanGroups + group;
+    if (p >= passes) break;
     uint32_t off = 0;
-    for (int w = 0; w < wave; ++w) off += s_wave[w];
-    excl[p * kRadix + d] = off + inc - c;
-    const bool trivial = s_trivial != 0 || p < left;
-    if (d == 0) {
-      plan->skip[p] = trivial ? 1u : 0u;
-      plan->src_is_alt[p] = parity;
-      for (int h = 0; h < kMaxHot; ++h)
-        plan->hot[p][h] = s_hot[h] != 0ull ? (uint32_t)(s_hot[h] & 0xFFull) : kNoHotDigit;
+#pragma unroll
+    for (int w = 0; w < kGroupWaves; ++w) off += w < wave ? s_wave[p][w] : 0u;
+    excl[p * kRadix + d] = off + inclusive[r] - counts[r];
+    // The most frequent of the dominant digits, most frequent first.
+    if (d < kFrequent) {
+      const unsigned long long mine = s_hot[p][d];
+      int before = 0;
+#pragma unroll
+      for (int h = 0; h < kFrequent; ++h)
+        before += s_hot[p][h] > mine || (s_hot[p][h] == mine && h < d) ? 1 : 0;
+      if (before < kMaxHot) plan->hot[p][before] = mine != 0ull ? (uint32_t)(mine & 0xFFull) : kNoHotDigit;
     }
-    if (!trivial) {
-      if (executed == 0) first = p;
-      last = p;
+  }
+  if (threadIdx.x != 0) return;
+
+  // The lower digits [0, left) are left to the local sort, if the draws say that the keys
+  // spread and that saves two passes at least (a digit that all keys share needs none): below
+  // the topmost digit that differs where none of its values has more keys than a window
+  // (local_max_run != 0: the input may be short enough for that), or below two digits where the
+  // draws found short runs.
+  int left = 0, local = 0;
+  if (spread && varies != 0u) {
+    const int top = 31 - __builtin_clz(varies);
+    if (local_max_run == 0) local = two_digits;
+    else if (s_most[top] <= local_max_run) local = top;
+    if (__popc(varies & ((1u << local) - 1u)) < 2) local = 0;
+    left = local;
+  }
+  // Or to the ties, if the draws rarely meet and that saves at least two passes.  An
+  // even number of passes ends in the caller's buffer, where the ties are ordered: an
+  // odd one takes a lower digit along.
+  if (ties.table != nullptr && local == 0 && pairs <= ties.max_pairs && doubles <= ties.max_doubles &&
+      groups <= kTieGroups) {
+    left = kMaxPasses - kTiePasses;
+    if (__popc(varies >> left) & 1)
+      while (left > 0 && !(varies >> --left & 1u)) {}
+    if (__popc(varies & ((1u << left) - 1u)) < 2) left = 0;
+  }
+  uint32_t parity = 0, executed = 0, first = (uint32_t)passes, last = (uint32_t)passes;
+  for (int p = 0; p < passes; ++p) {
+    const bool skipped = !(varies >> p & 1u) || p < left;
+    plan->skip[p] = skipped ? 1u : 0u;
+    plan->src_is_alt[p] = parity;
+    if (!skipped) {
+      if (executed == 0) first = (uint32_t)p;
+      last = (uint32_t)p;
       parity ^= 1u;
       ++executed;
     }
-    __syncthreads();
   }
-  if (d == 0) {
-    plan->first_executed = first;
-    plan->last_executed = last;
-    plan->executed = executed;
-    plan->final_in_alt = parity;
-    plan->ties_left = left > 0 ? 1u : 0u;
-  }
+  plan->first_executed = first;
+  plan->last_executed = last;
+  plan->executed = executed;
+  plan->final_in_alt = parity;
+  plan->ties_left = left > 0 && local == 0 ? 1u : 0u;
+  plan->local_from = (uint32_t)local;
 }
 
 // ---- onesweep pass ---------------------------------------------------------
@@ -2525,6 +2751,7 @@ __global__ __launch_bounds__(kTieBlock, 8) void ties_kernel(
   using Val = typename ValueOf<VALUE_BYTES>::type;
   __shared__ TiePiece s_piece;
   __shared__ uint32_t s_longs;
+  if (plan->local_from != 0) return;  // local_sort_kernel has done it
   if (plan->ties_left == 0) {  // every digit was sorted
     finish<8, VALUE_BYTES>(keys_a, keys_b, vals_a, vals_b, n, plan, values_from_index);
     return;
@@ -2641,6 +2868,8 @@ __global__ __launch_bounds__(kTieBlock, 8) void ties_kernel(
                                      (__attribute__((address_space(3))) TiePiece*)&s_piece);
 }
 
+#include "radix_sort_local.hpp"
+
 // ---- host side -------------------------------------------------------------
 
 struct TempLayout {
@@ -2689,6 +2918,15 @@ TempLayout make_layout(int64_t n, int key_bytes, int value_bytes, int block = kS
   off += L.status_stride * key_bytes;  // one status array per pass
   L.total = off;
   return L;
+}
+
+// Lengths at which the local sort is offered.  Below the first its draws would not fit the alternate
+// keys.  8-byte keys between the other two are sorted by their upper half (TieSampling).
+constexpr int64_t kLocalMinKeys = 1ll << 14;
+constexpr int64_t kLocalMinKeysAfterTies = (1ll << 23) + 1;
+static_assert(kLocalMinKeys >= 1ll << kLocalMinDrawBits, "the draws lie in the alternate keys");
+inline bool local_wanted(int64_t n, int key_bytes) {
+  return n >= kLocalMinKeys && (key_bytes != 8 || n < kTieMinKeys || n >= kLocalMinKeysAfterTies);
 }
 
 KeyXform make_xform(int32_t key_type, int32_t flags) {
@@ -2942,9 +3180,52 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
     ties.max_pairs = (uint32_t)((3ull << (2 * bits)) / (uint64_t)a.n);
     table_words = 2ll << (bits + kTieSlotsPerDrawLog2);
   }
-  int32_t rc = launch_zero_words(stream, hist, (L.total - L.zero_begin) / 4,
-                                 reinterpret_cast<uint32_t*>(ties.table), table_words);
-  if (rc != ILGPU_HIP_SUCCESS) return rc;
+  // The local sort: inputs whose topmost digit alone can make runs that fit a window ask the
+  // digit's counts, longer ones the draws.
+  constexpr bool kLocal = local_sorts(KEY_BYTES, VALUE_BYTES);
+  LocalSampling local{};
+  uint32_t local_max_run = 0;
+  if constexpr (kLocal) {
+    constexpr int64_t kWindow = local_window(KEY_BYTES, VALUE_BYTES);
+    if (local_wanted(a.n, KEY_BYTES)) {
+      const int64_t of_one_digit = kWindow * kRadix * 15 / 16;
+      local.draw_bits = a.n <= 1ll << 21 ? kLocalMinDrawBits
+                        : (a.n <= 1ll << 23 ? 13 : (a.n <= 1ll << 25 ? 14 : kLocalMaxDrawBits));
+      const double draws = (double)(1ll << local.draw_bits), n = (double)a.n;
+      while (local.bin_bits < 31 && a.n >> local.bin_bits != 0) ++local.bin_bits;  // log2(n) + 1
+      local.max_equal = (uint32_t)(1.25 * draws * draws / n) + 6u;
+      if (a.n <= of_one_digit) {
+        local_max_run = (uint32_t)kWindow;
+      } else {
+        // Runs of 0.6 windows, as the mean over the keys.
+        const double looked_at = std::min(draws, 32768.0);
+        local.max_pairs = (uint32_t)(looked_at * looked_at * 0.5 * (0.6 * (double)kWindow / n)) + 1u;
+        const double of_window = looked_at * (double)kWindow / n;
+        const double most = of_window + 5.0 * std::sqrt(of_window) + 6.0;
+        local.max_draws = most < 100.0 ? (uint32_t)most : 100u;
+      }
+      local.draws = reinterpret_cast<char*>(keys_b) + (ties.table != nullptr ? kLocalDrawsOffset : 0);
+      // Words of the first ticket's line that no group uses, cleared with it.
+      local.from = reinterpret_cast<uint32_t*>(base + L.tickets) + 4;
+    }
+  }
+  int32_t rc;
+  if (local.draws != nullptr) {
+    auto* draw_kernel = sort_draw_kernel<K, false>;
+    if ((xf.reference_term | xf.total_term) != 0) draw_kernel = sort_draw_kernel<K, true>;
+    const int64_t words = (L.total - L.zero_begin) / 4;
+    const int64_t blocks = std::min<int64_t>(
+        div_up(std::max(std::max(words, table_words), (int64_t)1 << local.draw_bits), 256), (int64_t)cus * 8);
+    ProfileScope scope(stream, "zero_words");
+    hipLaunchKernelGGL(draw_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, hist, words,
+                       reinterpret_cast<uint32_t*>(ties.table), table_words, keys_a, a.n, xf,
+                       static_cast<K*>(const_cast<void*>(local.draws)), local.draw_bits);
+    ILGPU_HIP_CHECK(hipGetLastError());
+  } else {
+    rc = launch_zero_words(stream, hist, (L.total - L.zero_begin) / 4,
+                           reinterpret_cast<uint32_t*>(ties.table), table_words);
+    if (rc != ILGPU_HIP_SUCCESS) return rc;
+  }
 
   {
     ProfileScope scope(stream, "sort_histogram");
@@ -2952,15 +3233,18 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
     if constexpr (KEY_BYTES >= 2) {  // there is no 1-byte floating-point key
       if ((xf.reference_term | xf.total_term) != 0) histogram_kernel = sort_histogram_kernel<K, true>;
     }
+    // (One block more looks at the draws, unless that would start a second round.)
+    if (local.draws != nullptr && (hist_blocks < (int64_t)cus * ILGPU_HIP_SORT_HIST_BLOCKS_PER_CU || hist_blocks < 2))
+      ++hist_blocks;
     hipLaunchKernelGGL(histogram_kernel, dim3((unsigned)hist_blocks),
                        dim3(kHistBlock), hist_lds, stream, keys_a, a.n, xf, passes,
-                       shift, hist, ties);
+                       shift, hist, ties, local);
     ILGPU_HIP_CHECK(hipGetLastError());
   }
   {
     ProfileScope scope(stream, "sort_plan");
-    hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(kRadix), 0, stream, hist, excl,
-                       plan, passes, (uint32_t)a.n, ties);
+    hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(kPlanBlock), 0, stream, hist, excl,
+                       plan, passes, (uint32_t)a.n, ties, local.from, local_max_run);
   }
   ILGPU_HIP_CHECK(hipGetLastError());
 
@@ -2984,6 +3268,20 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
   } else
     rc = launch_passes<KEY_BYTES, VALUE_BYTES, kSortBlock>(stream, a, L, base, xf, cus);
   if (rc != ILGPU_HIP_SUCCESS) return rc;
+  if constexpr (kLocal) {
+    if (local.draws != nullptr) {
+      const int64_t blocks = std::min<int64_t>((int64_t)cus * 4, div_up(a.n, 1024));
+      const int finishes = ties.table == nullptr ? 1 : 0;
+      auto* kernel = local_sort_kernel<KEY_BYTES, VALUE_BYTES, false>;
+      if ((xf.reference_term | xf.total_term) != 0) kernel = local_sort_kernel<KEY_BYTES, VALUE_BYTES, true>;
+      ProfileScope scope(stream, "sort_local");
+      hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(LocalBlock::kBlock), 0, stream, keys_a, keys_b,
+                         vals_a, vals_b, (uint32_t)a.n, xf, plan, from_index, finishes,
+                         reinterpret_cast<uint2*>(base + L.status));
+      ILGPU_HIP_CHECK(hipGetLastError());
+      if (finishes) return ILGPU_HIP_SUCCESS;
+    }
+  }
   if constexpr (KEY_BYTES == 8) {
     if (ties.table != nullptr) {
       int64_t blocks = div_up(a.n, kTieBlock * kTieRows);

@@ -185,9 +185,9 @@ int32_t ilgpu_hip_radix_sort_pairs(ilgpu_hip_stream_t stream, void *keys,
 
 /* How many 8-bit passes the last sort that used `temp` ran and how many it
  * found unnecessary (a pass whose digit is the same for every key is skipped:
- * keys below 2^16 run two passes of four, equal keys none; so are the lower digits of 2^21
- * or more 8-byte keys whose upper halves rarely meet, which are put in order after
- * the passes: random keys run four of eight).  Same n, key_type
+ * keys below 2^16 run two passes of four, equal keys none; so are the lower digits that are
+ * sorted after the passes, where few keys share the topmost ones: random keys of 4 and 8
+ * bytes run one pass or two, and four of eight from 2^21 to 2^23 8-byte keys).  Same n, key_type
  * and value_bytes (0 for keys only) as that sort, dense views; waits for
  * `stream`.  The reference runs all NumBits / 2 passes whatever the keys
  * (RadixSortExtensions.cs:1276-1334) and has nothing to report. */

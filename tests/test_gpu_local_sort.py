@@ -1,0 +1,174 @@
+"""The local sort: passes over the topmost digits, then windows of whole runs in
+LDS.  Against numpy's stable sort, bit for bit, at the lengths of runs and inputs
+where another branch takes over."""
+import numpy as np
+import pytest
+
+from ilgpu_amd import capi
+from tests.test_gpu_parity import D, note, sync
+
+pytestmark = pytest.mark.gpu
+
+
+def order_bits(bits, dtype, descending, total_order):
+    """The unsigned bits whose order the sort gives, for keys of these bits."""
+    width = bits.dtype.itemsize * 8
+    sign = bits.dtype.type(1 << (width - 1))
+    kind = np.dtype(dtype).kind
+    if kind == "u":
+        out = bits
+    elif kind == "i":
+        out = bits ^ sign
+    elif total_order:
+        out = np.where(bits & sign, ~bits, bits ^ sign)
+    else:  # as the reference writes it: the last bit of positive values is flipped
+        out = bits ^ sign ^ (bits.dtype.type(1) - (bits >> bits.dtype.type(width - 1)))
+    return ~out if descending else out
+
+
+def check(bits, dtype, value_dtype=None, descending=False, total_order=False, from_index=True):
+    """Sorts keys of these bits; the number of passes that ran."""
+    n = bits.size
+    expect = np.argsort(order_bits(bits, dtype, descending, total_order), kind="stable")
+    keys = D.from_numpy(bits.view(dtype))
+    size = 0 if value_dtype is None else np.dtype(value_dtype).itemsize
+    temp = capi.temp_buffer(capi.radix_sort_temp_bytes(n, dtype, size))
+    if value_dtype is None:
+        capi.radix_sort_keys(keys, temp, descending=descending, float_total_order=total_order)
+    else:
+        places = np.arange(n).astype(value_dtype)
+        values = D.zeros(n, value_dtype) if from_index else D.from_numpy(places)
+        capi.radix_sort_pairs(keys, values, temp, descending=descending,
+                              float_total_order=total_order, values_from_index=from_index)
+    sync()
+    assert np.array_equal(keys.numpy().view(bits.dtype), bits[expect])
+    if value_dtype is not None:
+        assert np.array_equal(values.numpy(), places[expect])
+    return capi.radix_sort_passes(temp, n, dtype, size)[0]
+
+
+def random_bits(n, width, seed):
+    return np.random.default_rng(seed).integers(0, 1 << width, n, dtype=f"uint{width}", endpoint=False)
+
+
+# A full window: keys of 4 bytes, of 8, and pairs of either with values of up to 8 bytes.
+WINDOWS = {(4, False): 9216, (8, False): 4608, (4, True): 6144, (8, True): 3584}
+
+
+@pytest.mark.parametrize("dtype,descending,total_order", [
+    (np.uint32, False, False), (np.int32, True, False), (np.float32, False, False),
+    (np.float32, True, True), (np.uint64, True, False), (np.int64, False, False),
+    (np.float64, False, False), (np.float64, True, True)])
+@pytest.mark.parametrize("value_dtype", [None, np.uint8, np.uint16, np.uint32, np.uint64])
+def test_random_keys_take_one_or_two_passes(dtype, descending, total_order, value_dtype):
+    """One pass up to 240 windows, two beyond; at both sides of that and at the shortest."""
+    size = np.dtype(dtype).itemsize
+    window = WINDOWS[size, value_dtype is not None]
+    for n, passes in [(18433, 1), (100_003, 1), (240 * window, 1), (240 * window + 1, 2)]:
+        note("local sort", np.dtype(dtype).name, descending, total_order, value_dtype, n)
+        ran = check(random_bits(n, 8 * size, n), dtype, value_dtype, descending, total_order,
+                    from_index=n % 2 == 0)
+        assert ran == passes
+
+
+@pytest.mark.parametrize("size", [4, 8])
+@pytest.mark.parametrize("pairs", [False, True])
+def test_runs_of_every_length_around_a_window(size, pairs):
+    """One digit's runs of exactly a window, and of one key more (which need all digits or
+    two); runs of two digits that are longer than a window, which a block orders through memory."""
+    window = WINDOWS[size, pairs]
+    width = 8 * size
+    kind = np.dtype(f"uint{width}")
+    value = np.uint32 if pairs else None
+    rng = np.random.default_rng(size)
+    for longest in (window, window + 1):
+        note("one digit", size, pairs, longest)
+        top = np.repeat(np.arange(16), [longest, 1, 2, 63, 64, 65, window // 2] + 9 * [window - 1])
+        low = random_bits(top.size, width, 3) >> kind.type(8)
+        bits = rng.permutation(top.astype(kind) << kind.type(width - 8) | low)
+        ran = check(bits, kind, value)
+        assert ran == 1 if longest == window else ran > 1
+    # (8-byte keys from 2^21 to 2^23 take the passes over their upper half.)
+    for length in (window - 1, window, window + 1, 2 * window + 1):
+        note("two digits", size, pairs, length)
+        n = 241 * window
+        bits = random_bits(n, width, length)
+        at = rng.permutation(n)[:length]
+        low = random_bits(length, width, 5) & kind.type((1 << (width - 16)) - 1)
+        bits[at] = kind.type(0x1234 << (width - 16)) | low
+        if length > window:
+            low[: length // 2] = low[0]  # copies of one key within the long run
+            bits[at] = kind.type(0x1234 << (width - 16)) | low
+        check(bits, kind, value, descending=length % 2 == 0)
+
+
+@pytest.mark.parametrize("size", [4, 8])
+@pytest.mark.parametrize("value_dtype", [None, np.uint32, np.uint64])
+def test_windows_whose_keys_crowd_are_sorted_by_digits(size, value_dtype):
+    """A few runs of one digit hold many copies, or keys side by side: bins of sixteen keys
+    and more, and more bins of two than are listed; the other runs are random."""
+    width = 8 * size
+    kind = np.dtype(f"uint{width}")
+    bits = random_bits(200_003, width, 11)
+    top = bits >> kind.type(width - 8)
+    rng = np.random.default_rng(12)
+    low = kind.type((1 << (width - 8)) - 1)
+    for run, values in [(3, 1), (7, 15), (8, 17), (9, 300), (10, 380)]:
+        inside = np.flatnonzero(top == run)
+        few = rng.integers(0, 1 << (width - 8), values, dtype=kind) & low
+        bits[inside] = kind.type(run << (width - 8)) | few[rng.integers(0, values, inside.size)]
+    inside = np.flatnonzero(top == 200)
+    bits[inside] = kind.type(200 << (width - 8)) | rng.permutation(inside.size).astype(kind)
+    note("crowded windows", size, value_dtype)
+    assert check(bits, kind, value_dtype, from_index=False) == 1
+    assert check(bits, kind, value_dtype, descending=True) == 1
+
+
+def test_inputs_that_would_crowd_most_windows_take_every_digit():
+    note("many copies")
+    rng = np.random.default_rng(13)
+    values = random_bits(10_000, 32, 14)
+    assert check(values[rng.integers(0, values.size, 300_000)], np.uint32) == 4
+    bits = random_bits(300_000, 64, 15) & np.uint64(0xFFFF00000000FFFF)
+    assert check(bits, np.uint64, np.uint32) == 4  # the digits that differ
+
+
+def test_digits_that_all_keys_share_do_not_hide_the_topmost():
+    """8-byte keys of 40 bits, and of 24 (no two digits to save)."""
+    note("forty bits")
+    for n, passes in [(100_003, 1), (1_500_001, 2)]:
+        assert check(random_bits(n, 64, n) >> np.uint64(24), np.int64, np.uint32) == passes
+    assert check(random_bits(100_003, 64, 16) >> np.uint64(40), np.uint64) == 3
+
+
+def test_local_sorts_can_be_captured_and_replayed():
+    """Draws, windows and what is put off are told anew by every replay."""
+    import torch
+    n = 240 * 9216 + 77
+    static = torch.zeros(n, dtype=torch.int32, device="cuda:0")
+    work = torch.zeros(n, dtype=torch.int32, device="cuda:0")
+    keys = D(n, np.uint32, _bytes=work.view(torch.uint8))
+    temp = capi.temp_buffer(capi.radix_sort_temp_bytes(n, np.uint32))
+
+    def calls():
+        work.copy_(static)
+        capi.radix_sort_keys(keys, temp)
+
+    calls()  # the one-time queries
+    sync()
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        with torch.cuda.graph(graph, stream=side):
+            calls()
+    sync()
+    few = random_bits(1000, 32, 17)
+    inputs = [random_bits(n, 32, 18), few[np.random.default_rng(19).integers(0, 1000, n)], random_bits(n, 32, 20)]
+    for replay, (bits, passes) in enumerate(zip(inputs, (2, 4, 2))):
+        note("replay", replay)
+        static.copy_(torch.from_numpy(bits.view(np.int32)))
+        assert torch.rand(1 << 20, device="cuda:0").sum().item() > 0  # eager work between replays
+        graph.replay()
+        sync()
+        assert np.array_equal(keys.numpy(), np.sort(bits))
+        assert capi.radix_sort_passes(temp, n, np.uint32)[0] == passes
