@@ -172,3 +172,32 @@ def test_local_sorts_can_be_captured_and_replayed():
         sync()
         assert np.array_equal(keys.numpy(), np.sort(bits))
         assert capi.radix_sort_passes(temp, n, np.uint32)[0] == passes
+
+
+@pytest.mark.parametrize("dtype,descending,total_order", [
+    (np.uint64, False, False), (np.int64, True, False), (np.float64, False, False),
+    (np.float64, True, True)])
+@pytest.mark.parametrize("value_dtype", [None, np.uint32])
+def test_one_tile_sorts_by_the_topmost_digits(dtype, descending, total_order, value_dtype):
+    """8-byte keys of one tile: neighbours of one prefix (some hundred of them, in runs of
+    two to four), a prefix of as many keys as a key looks at and of one more (all digits), prefixes that
+    most keys share (not tried), and keys that are all the same."""
+    rng = np.random.default_rng(21)
+    for n in (2, 2048, 2049, 9216 if value_dtype is None else 7168):
+        for prefix in (0, 2, 24, 25, 26, n):
+            note("one tile by prefix", np.dtype(dtype).name, n, prefix)
+            bits = random_bits(n, 64, n + prefix)
+            shared = rng.permutation(n)[:min(prefix, n)]
+            bits[shared] = (bits[shared[:1]] & np.uint64(0xFFFFFFFF00000000)) | random_bits(shared.size, 32, 22)
+            for first in range(0, min(n, 300) - 4, 4):  # runs of two to four
+                run = slice(first, first + 2 + first // 4 % 3)
+                bits[run] = (bits[first] & np.uint64(0xFFFFFFFFFF000000)) | (bits[run] & np.uint64(0xFFFFFF))
+            check(bits, dtype, value_dtype, descending, total_order)
+    check(np.full(777, 5, np.uint64), np.uint64, np.uint32)
+
+
+def test_one_tile_of_narrow_keys_skips_the_digits_they_share():
+    note("narrow keys")
+    for n in (18_432, 12_289, 777):
+        check(random_bits(n, 32, n) & np.uint32(0x000FF0F0), np.uint32, descending=n % 2 == 0)
+        check(random_bits(min(n, 9216), 64, n) & np.uint64(0x00FF00000000FF00), np.int64, np.uint32)
