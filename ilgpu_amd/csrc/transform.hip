@@ -90,7 +90,8 @@ __global__ __launch_bounds__(kBlock) void transform_kernel(
 
 // Dense views: K consecutive elements per thread, K chosen so that the wider
 // of the two element types moves as one 16-byte vector.  The last n % K
-// elements go through the scalar kernel.
+// elements go one by one through threads of the first block (a launch of their own
+// cost 2.5 us: 3 000 017 uint32 5.5 + 2.6 us in two kernels).
 template <typename E, int K> struct alignas(sizeof(E) * K) Pack { E v[K]; };
 
 // Streaming (non-temporal) access to a pack as one machine vector of its size:
@@ -128,7 +129,10 @@ template <typename P> __device__ __forceinline__ void store_pack(P* p, const P& 
 
 template <typename S, typename T, int K>
 __global__ __launch_bounds__(kBlock) void transform_dense_kernel(
-    const Pack<S, K>* source, Pack<T, K>* target, int64_t packs, int op, int64_t factor) {
+    const Pack<S, K>* source, Pack<T, K>* target, int64_t packs, int rest, int op, int64_t factor) {
+  if (blockIdx.x == 0 && (int)threadIdx.x < rest)
+    reinterpret_cast<T*>(target + packs)[threadIdx.x] =
+        convert<S, T>(apply_transformer<S>(reinterpret_cast<const S*>(source + packs)[threadIdx.x], op, factor));
   const int64_t step = (int64_t)gridDim.x * kBlock;
   for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < packs; i += step) {
     const Pack<S, K> in = load_pack(&source[i]);
@@ -156,15 +160,8 @@ int32_t transform_typed(hipStream_t stream, const TransformArgs& a) {
       hipLaunchKernelGGL((transform_dense_kernel<S, T, K>), dim3((unsigned)grid_for(packs)),
                          dim3(kBlock), 0, stream,
                          static_cast<const Pack<S, K>*>(a.source),
-                         static_cast<Pack<T, K>*>(a.target), packs, a.transformer, a.factor);
-      ILGPU_HIP_CHECK(hipGetLastError());
-      const int64_t done = packs * K;
-      if (done == a.n) return ILGPU_HIP_SUCCESS;
-      hipLaunchKernelGGL((transform_kernel<S, T>), dim3(1), dim3(kBlock), 0, stream,
-                         static_cast<const S*>(a.source) + done, (int64_t)1,
-                         static_cast<T*>(a.target) + done, (int64_t)1,
-                         static_cast<const int32_t*>(nullptr), a.n - done, a.transformer,
-                         a.factor);
+                         static_cast<Pack<T, K>*>(a.target), packs, (int)(a.n - packs * K),
+                         a.transformer, a.factor);
       ILGPU_HIP_CHECK(hipGetLastError());
       return ILGPU_HIP_SUCCESS;
     }
