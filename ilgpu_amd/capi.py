@@ -258,10 +258,26 @@ def temp_buffer(nbytes: int) -> DeviceArray:
     return DeviceArray((nbytes + 3) // 4, np.int32)
 
 
+_current_stream_ptr = None
+
+
+def _find_current_stream():
+    """torch's current stream on the current device as a pointer, without the
+    Stream object around it (2.8 us of a call's 7.4 on the host, 0.3 without)."""
+    global _current_stream_ptr
+    import torch
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    device = torch.cuda.current_device
+    if raw is not None:
+        _current_stream_ptr = lambda: raw(device())  # noqa: E731
+    else:
+        _current_stream_ptr = lambda: torch.cuda.current_stream().cuda_stream  # noqa: E731
+    return _current_stream_ptr
+
+
 def _stream_ptr(stream) -> int:
     if stream is None:
-        import torch
-        return torch.cuda.current_stream().cuda_stream
+        return (_current_stream_ptr or _find_current_stream())()
     return getattr(stream, "cuda_stream", stream)
 
 
