@@ -130,9 +130,6 @@ template <typename P> __device__ __forceinline__ void store_pack(P* p, const P& 
 template <typename S, typename T, int K>
 __global__ __launch_bounds__(kBlock) void transform_dense_kernel(
     const Pack<S, K>* source, Pack<T, K>* target, int64_t packs, int rest, int op, int64_t factor) {
-  if (blockIdx.x == 0 && (int)threadIdx.x < rest)
-    reinterpret_cast<T*>(target + packs)[threadIdx.x] =
-        convert<S, T>(apply_transformer<S>(reinterpret_cast<const S*>(source + packs)[threadIdx.x], op, factor));
   const int64_t step = (int64_t)gridDim.x * kBlock;
   for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < packs; i += step) {
     const Pack<S, K> in = load_pack(&source[i]);
@@ -142,6 +139,9 @@ __global__ __launch_bounds__(kBlock) void transform_dense_kernel(
       out.v[k] = convert<S, T>(apply_transformer<S>(in.v[k], op, factor));
     store_pack(&target[i], out);
   }
+  if (blockIdx.x == 0 && (int)threadIdx.x < rest)
+    reinterpret_cast<T*>(target + packs)[threadIdx.x] =
+        convert<S, T>(apply_transformer<S>(reinterpret_cast<const S*>(source + packs)[threadIdx.x], op, factor));
 }
 
 template <typename S, typename T>
