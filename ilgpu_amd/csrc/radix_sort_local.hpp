@@ -90,27 +90,21 @@ __device__ __forceinline__ uint32_t local_run_start(const K* src, uint32_t x, ui
   }
 }
 
-// `count` elements, by `blocks` blocks (this one: `block`): four neighbouring ones at a time, two
-// such loads of a thread in flight, a block's next to each other.
+// `count` elements, by `blocks` blocks (this one: `block`): four neighbouring ones at a time, the
+// grid's next to each other, past the caches: HBM bounds it.  (Two loads of a thread in flight and plain
+// stores, keys below 10^6 with a copy in front, us, before / now: u32 2^23 135.8 / 132.6, 2^24 217.6 / 211.4, 2^26
+// 632.9 / 617.8, pairs of 2^24 u32 343.9 / 328.5; four loads, each a grid further on: 2^24 225.)
 template <typename E>
 __device__ __forceinline__ void local_copy(const E* from, E* to, uint32_t count, uint32_t block, uint32_t blocks) {
-  struct alignas(sizeof(E)) Four { E e[4]; };
-  constexpr uint32_t kBlock = (uint32_t)LocalBlock::kBlock, kLoads = 2;
+  typedef E Four __attribute__((ext_vector_type(4), aligned(sizeof(E))));
+  constexpr uint32_t kBlock = (uint32_t)LocalBlock::kBlock;
   const uint32_t t = threadIdx.x;
   const uint32_t fours = count / 4;
   const Four* f = reinterpret_cast<const Four*>(from);
   Four* g = reinterpret_cast<Four*>(to);
-  const uint32_t chunks = fours / (kLoads * kBlock);
-  for (uint32_t chunk = block; chunk < chunks; chunk += blocks) {
-    const uint32_t i = chunk * (kLoads * kBlock) + t;
-    Four v[kLoads];
-#pragma unroll
-    for (uint32_t u = 0; u < kLoads; ++u) v[u] = f[i + u * kBlock];
-#pragma unroll
-    for (uint32_t u = 0; u < kLoads; ++u) g[i + u * kBlock] = v[u];
-  }
+  for (uint32_t i = block * kBlock + t; i < fours; i += blocks * kBlock) __builtin_nontemporal_store(f[i], &g[i]);
   if (block == 0)
-    for (uint32_t i = chunks * (kLoads * kBlock) * 4 + t; i < count; i += kBlock) to[i] = from[i];
+    for (uint32_t i = fours * 4 + t; i < count; i += kBlock) to[i] = from[i];
 }
 
 // ---- digit by digit -------------------------------------------------------------
