@@ -59,6 +59,7 @@
 #include <type_traits>
 
 #include "kernels.hpp"
+#include "radix_sort_local_rules.hpp"
 
 namespace ilgpu_hip {
 

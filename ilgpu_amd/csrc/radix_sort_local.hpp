@@ -31,28 +31,6 @@
 // block.  Both are decided from the keys themselves: the answer is right whatever
 // the plan believed of them.
 
-struct LocalBlock {
-  static constexpr int kBlock = 256;
-  static constexpr int kWaves = kBlock / kWaveSize;
-  static constexpr int kStageBytes = 36 * 1024;  // four blocks share a compute unit's LDS
-  static constexpr int kBinsLog2 = 15;
-  static constexpr int kBins = 1 << kBinsLog2;
-  // A thread scans 32 words, four bins each; rows of 36 spread a wave's
-  // 16-byte accesses over all banks.
-  static constexpr int kRowWords = kBins / 4 / kBlock;
-  static constexpr int kRowStride = kRowWords + 4;
-  static constexpr int kList = 1984;  // bins of two keys or more that a window may have (some 1070 in a full one)
-};
-static_assert(LocalBlock::kBlock * LocalBlock::kRowStride * 4 == LocalBlock::kStageBytes, "the counts fill the stage");
-// Pairs keep the place a key came from next to it.
-constexpr int local_items(int key_bytes, int value_bytes) {
-  return LocalBlock::kStageBytes / (key_bytes + (value_bytes > 0 ? 2 : 0)) / LocalBlock::kBlock & ~1;
-}
-constexpr int local_window(int key_bytes, int value_bytes) {
-  return local_items(key_bytes, value_bytes) * LocalBlock::kBlock;
-}
-constexpr bool local_sorts(int key_bytes, int value_bytes) { return key_bytes >= 4 && value_bytes <= 8; }
-
 struct LocalLds {
   __attribute__((aligned(16))) unsigned char stage[LocalBlock::kStageBytes];
   uint16_t list[LocalBlock::kList];
@@ -500,24 +478,19 @@ __global__ __launch_bounds__(LocalBlock::kBlock, 4) void local_sort_kernel(
       count = (uint32_t)__builtin_amdgcn_readfirstlane((int)count);
       span = (K)(upper_last - low - 1);
     }
-    // bin = ((key - low) >> shift) * scale >> 16: the shift leaves 18 bits, the scale spreads
-    // what they hold over all the bins.
-    const int span_bits = sizeof(K) == 8 ? 64 - __builtin_clzll((uint64_t)span | 1ull)
-                                         : 32 - __builtin_clz((uint32_t)span | 1u);
-    const int shift = span_bits > 18 ? span_bits - 18 : 0;
-    uint32_t scale = 0x7FFFFFFFu / ((uint32_t)(span >> shift) + 1u);
-    if (scale > 1u << 16) scale = 1u << 16;
+    const LocalScale bins_of_span = local_scale<K>(span);
+    const int shift = bins_of_span.shift;
+    const uint32_t scale = bins_of_span.scale;
     K minus_low = (K)(0 - low);
     if constexpr (sizeof(K) == 4) asm("" : "+v"(minus_low));  // (xor and sum in one instruction)
     auto scaled = [&](K k) -> uint32_t {  // of a key as it is held: its bin in the upper half, 15 bits
       return (uint32_t)__umul24((uint32_t)((K)(ordered(k) + minus_low) >> shift), scale);  // (it returns an int)
     };
     auto bin_of = [&](K k) -> uint32_t { return scaled(k) >> 16; };
-    // A bin's code, 16 bits: the byte offset of its word, and which of the word's four counts it is.
     auto codes_of = [&](K k0, K k1) -> uint32_t {  // of two keys
       typedef uint16_t Two __attribute__((ext_vector_type(2)));
       const Two bins = __builtin_bit_cast(Two, __builtin_amdgcn_perm(scaled(k1), scaled(k0), 0x07060302u));
-      return __builtin_bit_cast(uint32_t, (Two)((bins >> (uint16_t)7) * (uint16_t)16 + bins));
+      return __builtin_bit_cast(uint32_t, local_bin_codes(bins));
     };
     auto word_at = [&](uint32_t codes, int which) -> uint32_t* {
       return reinterpret_cast<uint32_t*>(s_words + ((which == 0 ? codes & 0xFFFFu : codes >> 16) & ~3u));
@@ -552,6 +525,8 @@ __global__ __launch_bounds__(LocalBlock::kBlock, 4) void local_sort_kernel(
         for (int g = 0; g < kGroup && j0 + g < kItems; ++g) {
           const int j = j0 + g;
           ranks[j / 8] |= __builtin_amdgcn_ubfe(old[g], count_at(place[j / 2], j % 2), 4u) << (4 * (j % 8));
+          if (!decltype(full)::value && (int)t >= (int)count - j * kBlock)
+            place[j / 2] = local_codes_without(place[j / 2], j % 2);
         }
       };
 #pragma unroll
@@ -621,7 +596,7 @@ __global__ __launch_bounds__(LocalBlock::kBlock, 4) void local_sort_kernel(
         for (int g = 0; g < kGroup && j0 + g < kItems; ++g) {
           const int j = j0 + g;
           r[g] = __builtin_amdgcn_ubfe(ranks[j / 8], 4 * (j % 8), 4u);
-          w[g] = *word_at(place[j / 2], j % 2);  // (of some bin where there is no key)
+          w[g] = *word_at(place[j / 2], j % 2);  // (of the first bin where there is no key)
         }
         uint32_t seconds = 0;
 #pragma unroll

@@ -1,0 +1,27 @@
+// The sizes and the arithmetic of the local sort as plain functions, for tests/test_local_sort_rules.py.
+#include "../../ilgpu_amd/csrc/radix_sort_local_rules.hpp"
+
+using namespace ilgpu_hip;
+
+extern "C" {
+
+int32_t rule_window(int32_t key_bytes, int32_t value_bytes) { return local_window(key_bytes, value_bytes); }
+int32_t rule_stage_bytes() { return LocalBlock::kStageBytes; }
+
+// The codes of two keys' bins in a window whose keys are up to `span` behind its lowest, as the kernel
+// packs them; has_key: bit 0 the first, bit 1 the second key is one of the window.
+uint32_t rule_codes(int32_t key_bytes, uint64_t span, uint64_t first, uint64_t second, int32_t has_key) {
+  const LocalScale s = key_bytes == 8 ? local_scale<uint64_t>(span) : local_scale<uint32_t>((uint32_t)span);
+  uint32_t codes = 0;
+  for (int which = 0; which < 2; ++which) {
+    const uint64_t key = which == 0 ? first : second;
+    const uint32_t shifted = key_bytes == 8 ? (uint32_t)(key >> s.shift) : (uint32_t)key >> s.shift;
+    const uint32_t scaled = (shifted & 0xFFFFFFu) * s.scale;  // 24 bits times 17
+    codes |= (uint32_t)local_bin_codes<uint16_t>((uint16_t)(scaled >> 16)) << (16 * which);
+  }
+  for (int which = 0; which < 2; ++which)
+    if (!(has_key >> which & 1)) codes = local_codes_without(codes, which);
+  return codes;
+}
+
+}  // extern "C"
