@@ -3049,6 +3049,8 @@ TempLayout make_layout(int64_t n, int key_bytes, int value_bytes, int block = kS
 constexpr int64_t kLocalMinKeys = 1ll << 14;
 constexpr int64_t kLocalMinKeysAfterTies = (1ll << 23) + 1;
 static_assert(kLocalMinKeys >= 1ll << kLocalMinDrawBits, "the draws lie in the alternate keys");
+static_assert(kLocalMinKeysAfterTies * 8 >= kLocalDrawsOffset + (8ll << kLocalMaxDrawBits),
+              "the draws lie in the alternate keys, behind the table");
 inline bool local_wanted(int64_t n, int key_bytes) {
   return n >= kLocalMinKeys && (key_bytes != 8 || n < kTieMinKeys || n >= kLocalMinKeysAfterTies);
 }
@@ -3311,7 +3313,8 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
   uint32_t local_max_run = 0;
   if constexpr (kLocal) {
     constexpr int64_t kWindow = local_window(KEY_BYTES, VALUE_BYTES);
-    if (local_wanted(a.n, KEY_BYTES)) {
+    if (local_wanted(a.n, KEY_BYTES) &&
+        local_deferred_bytes(a.n, local_blocks(a.n, cus), (uint32_t)kWindow) <= L.total - L.status) {
       const int64_t of_one_digit = kWindow * kRadix * 15 / 16;
       local.draw_bits = a.n <= 1ll << 21 ? kLocalMinDrawBits
                         : (a.n <= 1ll << 23 ? 13 : (a.n <= 1ll << 25 ? 14 : kLocalMaxDrawBits));
@@ -3394,7 +3397,7 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
   if (rc != ILGPU_HIP_SUCCESS) return rc;
   if constexpr (kLocal) {
     if (local.draws != nullptr) {
-      const int64_t blocks = std::min<int64_t>((int64_t)cus * 4, div_up(a.n, 1024));
+      const int64_t blocks = local_blocks(a.n, cus);
       const int finishes = ties.table == nullptr ? 1 : 0;
       auto* kernel = local_sort_kernel<KEY_BYTES, VALUE_BYTES, false>;
       if ((xf.reference_term | xf.total_term) != 0) kernel = local_sort_kernel<KEY_BYTES, VALUE_BYTES, true>;

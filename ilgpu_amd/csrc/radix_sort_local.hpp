@@ -316,12 +316,6 @@ __device__ __attribute__((noinline)) void local_long_run(
   }
 }
 
-// Windows and runs that a block may have to put off.  Two windows in a row hold more than one
-// full window between them, unless the second ends the block's part.
-__host__ __device__ constexpr uint32_t local_deferred(uint32_t part, uint32_t window) {
-  return 2 * (part / window) + 6;
-}
-
 // ---- the kernel -------------------------------------------------------------------
 // Rows of a window as a buffer: what lies behind its `count` elements is read as zero and not
 // written.  (No scalar offset: it would not be part of what the hardware holds against the

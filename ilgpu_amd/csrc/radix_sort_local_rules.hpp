@@ -35,6 +35,20 @@ constexpr int local_window(int key_bytes, int value_bytes) {
 }
 constexpr bool local_sorts(int key_bytes, int value_bytes) { return key_bytes >= 4 && value_bytes <= 8; }
 
+// Blocks of the local sort: a compute unit holds four.
+inline int64_t local_blocks(int64_t n, int64_t cus) {
+  const int64_t of_keys = (n + 1023) / 1024;
+  return of_keys < cus * 4 ? of_keys : cus * 4;
+}
+// Windows and runs that a block may have to put off, at most all of them.  Two windows in a row hold more than one
+// full window between them, unless the second ends the block's part.
+ILGPU_HIP_RULE constexpr uint32_t local_deferred(uint32_t part, uint32_t window) { return 2 * (part / window) + 6; }
+// What the lists of all blocks take, two words an entry.  They lie in the status words of the passes, some 0.11
+// bytes per key and more against 0.05; where they would not fit the local sort is not offered.
+inline int64_t local_deferred_bytes(int64_t n, int64_t blocks, uint32_t window) {
+  return blocks * (int64_t)local_deferred((uint32_t)((n + blocks - 1) / blocks), window) * 8;
+}
+
 // ---- bins -------------------------------------------------------------------
 // bin = ((key - low) >> shift) * scale >> 16: the shift leaves 18 bits, the scale spreads
 // what they hold over all the bins.  Keys of the window, up to low + span, have bins below kBins; others

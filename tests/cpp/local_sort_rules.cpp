@@ -8,6 +8,12 @@ extern "C" {
 int32_t rule_window(int32_t key_bytes, int32_t value_bytes) { return local_window(key_bytes, value_bytes); }
 int32_t rule_stage_bytes() { return LocalBlock::kStageBytes; }
 
+int64_t rule_blocks(int64_t n, int64_t cus) { return local_blocks(n, cus); }
+uint32_t rule_deferred(uint32_t part, uint32_t window) { return local_deferred(part, window); }
+int64_t rule_deferred_bytes(int64_t n, int64_t blocks, uint32_t window) {
+  return local_deferred_bytes(n, blocks, window);
+}
+
 // The codes of two keys' bins in a window whose keys are up to `span` behind its lowest, as the kernel
 // packs them; has_key: bit 0 the first, bit 1 the second key is one of the window.
 uint32_t rule_codes(int32_t key_bytes, uint64_t span, uint64_t first, uint64_t second, int32_t has_key) {
