@@ -55,7 +55,6 @@
 
 #include <algorithm>
 #include <atomic>
-#include <cmath>
 #include <type_traits>
 
 #include "kernels.hpp"
@@ -393,16 +392,11 @@ struct TieSampling {
 //   (Whether one digit does, its counts tell exactly.)
 // (2^26 u32 keys, every value some 30 times, with a copy in front, us: every digit sorted 750, the local
 // sort 1236.)
-constexpr int kLocalMinDrawBits = 12, kLocalMaxDrawBits = 16;
 struct LocalSampling {
   const void* draws;        // keys in their ordered form.  nullptr: not asked
   uint32_t* from;           // out: the lowest digit of the prefix whose runs are short (0: they are not),
                             // and in the next word whether the keys spread
-  uint32_t draw_bits;       // log2 of the number of draws
-  uint32_t bin_bits;        // of a draw, from the topmost bit that differs on
-  uint32_t max_equal;       // draws that meet an earlier one in these bits
-  uint32_t max_pairs;       // pairs of draws that share a 16-bit prefix
-  uint32_t max_draws;       // of one prefix
+  LocalLimits limits;
 };
 // Where the draws lie in the alternate keys: behind the table of TieSampling.
 constexpr int64_t kLocalDrawsOffset = 8ll << (kTieMaxSampleBits + kTieSlotsPerDrawLog2);
@@ -415,14 +409,9 @@ __global__ __launch_bounds__(256) void sort_draw_kernel(
   const int64_t stride = (int64_t)gridDim.x * 256;
   const int64_t first = (int64_t)blockIdx.x * 256 + threadIdx.x;
   for (int64_t s = first; s < 1ll << draw_bits; s += stride) {
-    uint64_t z = ((uint64_t)s + 1ull) * 0x9E3779B97F4A7C15ull;  // splitmix64
-    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-    z ^= z >> 31;
-    const uint64_t at = ((uint64_t)s << 32 | (uint32_t)z) << (32 - draw_bits);  // a random place in part s
-    const K k = keys[__umul64hi(at, (uint64_t)n)];
+    const K k = keys[local_draw_place((uint64_t)s, (int)draw_bits, (uint64_t)n)];
     const K o = FLOAT_KEYS ? ordered_bits(k, xf) : (K)(k ^ (K)xf.xor_mask);
-    draws[s] = o;
+    draws[local_draw_slot((uint32_t)s, (int)draw_bits)] = o;
   }
   for (int64_t i = first; i < count; i += stride) words[i] = 0u;
   for (int64_t i = first; i < more_count; i += stride) more[i] = 0u;
@@ -435,7 +424,7 @@ __device__ __forceinline__ void choose_local_digits(const LocalSampling& local, 
   constexpr int kTableBits = 14;  // words
   static_assert(kHistLdsWords >= 1 << kTableBits, "a byte for every 16-bit prefix");
   constexpr int kPerVector = 16 / (int)sizeof(K);
-  constexpr int kVectors = (1 << 14) / kPerVector / kHistBlock;  // of a thread and a chunk of 2^14 draws
+  constexpr int kVectors = (1 << kLocalChunkBits) / kPerVector / kHistBlock;  // of a thread and a chunk of draws
   using V = typename Vec16<K>::type;
   const int t = threadIdx.x;
   __shared__ unsigned long long s_diff;
@@ -445,8 +434,9 @@ __device__ __forceinline__ void choose_local_digits(const LocalSampling& local, 
       reinterpret_cast<uint4*>(s_table)[i] = make_uint4(0u, 0u, 0u, 0u);
   };
   const V* draws = static_cast<const V*>(local.draws);
-  const int vectors = (1 << local.draw_bits) / kPerVector;
-  const int chunks = local.draw_bits > 14 ? 1 << (local.draw_bits - 14) : 1;
+  const LocalLimits& limits = local.limits;
+  const int vectors = (1 << limits.draw_bits) / kPerVector;
+  const int chunks = (int)limits.draw_bits > kLocalChunkBits ? 1 << (limits.draw_bits - kLocalChunkBits) : 1;
   V d[kVectors];
   auto load = [&](int chunk) {
 #pragma unroll
@@ -473,8 +463,10 @@ __device__ __forceinline__ void choose_local_digits(const LocalSampling& local, 
   __syncthreads();
   if ((t & (kWaveSize - 1)) == 0) atomicOr(&s_diff, (unsigned long long)diff);
   __syncthreads();
-  const int top_bit = s_diff != 0ull ? 63 - __builtin_clzll(s_diff) : 0;  // the topmost bit that differs
-  const int top = top_bit / 8;                                            // and its digit
+  // The topmost bit that differs in a chunk, and its digit.  (One that fewer than some thousandth of the keys have may be
+  // missed: their runs are shorter than is thought, and no others longer.)
+  const int top_bit = s_diff != 0ull ? 63 - __builtin_clzll(s_diff) : 0;
+  const int top = top_bit / 8;
   if (top < 3) return;  // two digits at least have to be below the passes' for the way to pay
   // 32 bits from the topmost one that differs on.
   auto upper = [&](K k) -> uint32_t {
@@ -482,8 +474,9 @@ __device__ __forceinline__ void choose_local_digits(const LocalSampling& local, 
   };
 
   // Draws that meet an earlier one, in a table of open addressing: of many draws those of one part
-  // of the values, which half fill it.
-  const int parts_log2 = (int)local.draw_bits > kTableBits - 1 ? (int)local.draw_bits - (kTableBits - 1) : 0;
+  // of the values, which half fill it.  (Single frequent values are mostly in another part: those the draws of one
+  // prefix tell.)
+  const int parts_log2 = (int)limits.draw_bits > kTableBits - 1 ? (int)limits.draw_bits - (kTableBits - 1) : 0;
   constexpr uint32_t kSlots = 1u << kTableBits;
   uint32_t equal = 0;
   for (int chunk = 0; chunk < chunks; ++chunk) {
@@ -494,7 +487,7 @@ __device__ __forceinline__ void choose_local_digits(const LocalSampling& local, 
       uint32_t value[kPerVector], slot[kPerVector], old[kPerVector];
 #pragma unroll
       for (int u = 0; u < kPerVector; ++u) {
-        value[u] = upper(d[v][u]) >> (32 - local.bin_bits);  // at most 31 bits
+        value[u] = upper(d[v][u]) >> (32 - limits.bin_bits);  // at most 31 bits
         uint32_t hash = value[u] * 0x9E3779B1u;
         hash = (hash ^ hash >> 16) * 0x85EBCA6Bu;
         slot[u] = hash >> (32 - kTableBits);
@@ -515,16 +508,16 @@ __device__ __forceinline__ void choose_local_digits(const LocalSampling& local, 
   for (int s = 1; s < kWaveSize; s <<= 1) equal += shfl(equal, (t & (kWaveSize - 1)) ^ s);
   if ((t & (kWaveSize - 1)) == 0) atomicAdd(&s_equal, equal);
   __syncthreads();
-  if (s_equal > local.max_equal >> parts_log2) return;
+  if (s_equal > limits.max_equal >> parts_log2) return;
   if (t == 0) local.from[1] = 1u;
-  if (local.max_pairs == 0u) return;  // one digit is enough
+  if (limits.max_pairs == 0u) return;  // one digit is enough
 
-  // Draws of every prefix, a byte each (of 2^15 draws at most: with 2^16 the histogram of 2^26 keys
-  // waited 16 us for this block).
+  // Draws of every prefix, a byte each (of 2^15 draws from all over the input at most: with 2^16 the histogram of 2^26
+  // keys waited 16 us for this block).
   clear_table();
   __syncthreads();
   uint32_t pairs = 0, most = 0;
-  for (int chunk = 0; chunk < chunks && chunk < 2; ++chunk) {
+  for (int chunk = 0; chunk < chunks && chunk < 1 << (kLocalPrefixBits - kLocalChunkBits); ++chunk) {
     if (chunks > 1) load(chunk);
 #pragma unroll
     for (int v = 0; v < kVectors; ++v) {
@@ -555,7 +548,7 @@ __device__ __forceinline__ void choose_local_digits(const LocalSampling& local, 
     atomicMax(&s_draws, most + 1u);
   }
   __syncthreads();
-  if (t == 0 && s_pairs <= local.max_pairs && s_draws <= local.max_draws) local.from[0] = (uint32_t)(top - 1);
+  if (t == 0 && s_pairs <= limits.max_pairs && s_draws <= limits.max_draws) local.from[0] = (uint32_t)(top - 1);
 }
 
 // The first active lane's key, as a wave-uniform value.
@@ -3310,27 +3303,11 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
   // digit's counts, longer ones the draws.
   constexpr bool kLocal = local_sorts(KEY_BYTES, VALUE_BYTES);
   LocalSampling local{};
-  uint32_t local_max_run = 0;
   if constexpr (kLocal) {
     constexpr int64_t kWindow = local_window(KEY_BYTES, VALUE_BYTES);
     if (local_wanted(a.n, KEY_BYTES) &&
         local_deferred_bytes(a.n, local_blocks(a.n, cus), (uint32_t)kWindow) <= L.total - L.status) {
-      const int64_t of_one_digit = kWindow * kRadix * 15 / 16;
-      local.draw_bits = a.n <= 1ll << 21 ? kLocalMinDrawBits
-                        : (a.n <= 1ll << 23 ? 13 : (a.n <= 1ll << 25 ? 14 : kLocalMaxDrawBits));
-      const double draws = (double)(1ll << local.draw_bits), n = (double)a.n;
-      while (local.bin_bits < 31 && a.n >> local.bin_bits != 0) ++local.bin_bits;  // log2(n) + 1
-      local.max_equal = (uint32_t)(1.25 * draws * draws / n) + 6u;
-      if (a.n <= of_one_digit) {
-        local_max_run = (uint32_t)kWindow;
-      } else {
-        // Runs of 0.6 windows, as the mean over the keys.
-        const double looked_at = std::min(draws, 32768.0);
-        local.max_pairs = (uint32_t)(looked_at * looked_at * 0.5 * (0.6 * (double)kWindow / n)) + 1u;
-        const double of_window = looked_at * (double)kWindow / n;
-        const double most = of_window + 5.0 * std::sqrt(of_window) + 6.0;
-        local.max_draws = most < 100.0 ? (uint32_t)most : 100u;
-      }
+      local.limits = local_limits(a.n, KEY_BYTES, VALUE_BYTES);
       local.draws = reinterpret_cast<char*>(keys_b) + (ties.table != nullptr ? kLocalDrawsOffset : 0);
       // Words of the first ticket's line that no group uses, cleared with it.
       local.from = reinterpret_cast<uint32_t*>(base + L.tickets) + 4;
@@ -3342,11 +3319,11 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
     if ((xf.reference_term | xf.total_term) != 0) draw_kernel = sort_draw_kernel<K, true>;
     const int64_t words = (L.total - L.zero_begin) / 4;
     const int64_t blocks = std::min<int64_t>(
-        div_up(std::max(std::max(words, table_words), (int64_t)1 << local.draw_bits), 256), (int64_t)cus * 8);
+        div_up(std::max(std::max(words, table_words), (int64_t)1 << local.limits.draw_bits), 256), (int64_t)cus * 8);
     ProfileScope scope(stream, "zero_words");
     hipLaunchKernelGGL(draw_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, hist, words,
                        reinterpret_cast<uint32_t*>(ties.table), table_words, keys_a, a.n, xf,
-                       static_cast<K*>(const_cast<void*>(local.draws)), local.draw_bits);
+                       static_cast<K*>(const_cast<void*>(local.draws)), local.limits.draw_bits);
     ILGPU_HIP_CHECK(hipGetLastError());
   } else {
     rc = launch_zero_words(stream, hist, (L.total - L.zero_begin) / 4,
@@ -3371,7 +3348,7 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
   {
     ProfileScope scope(stream, "sort_plan");
     hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(kPlanBlock), 0, stream, hist, excl,
-                       plan, passes, (uint32_t)a.n, ties, local.from, local_max_run);
+                       plan, passes, (uint32_t)a.n, ties, local.from, local.limits.max_run);
   }
   ILGPU_HIP_CHECK(hipGetLastError());
 

@@ -5,6 +5,8 @@
 
 #include <stdint.h>
 
+#include <cmath>
+
 #ifdef __HIPCC__
 #define ILGPU_HIP_RULE __host__ __device__
 #else
@@ -47,6 +49,63 @@ ILGPU_HIP_RULE constexpr uint32_t local_deferred(uint32_t part, uint32_t window)
 // bytes per key and more against 0.05; where they would not fit the local sort is not offered.
 inline int64_t local_deferred_bytes(int64_t n, int64_t blocks, uint32_t window) {
   return blocks * (int64_t)local_deferred((uint32_t)((n + blocks - 1) / blocks), window) * 8;
+}
+
+// ---- draws ---------------------------------------------------------------------
+// Whether the local sort can do what passes over the topmost digits leave is asked of m draws,
+// one from every m-th part of the input, before anything is counted (radix_sort_impl.hpp:
+// sort_draw_kernel, choose_local_digits).
+constexpr int kLocalMinDrawBits = 12, kLocalMaxDrawBits = 16;
+constexpr int kLocalChunkBits = 14;   // draws that the block that looks at them holds at a time
+constexpr int kLocalPrefixBits = 15;  // draws whose prefixes are counted
+constexpr int local_draw_bits(int64_t n) {
+  return n <= 1ll << 21 ? kLocalMinDrawBits : (n <= 1ll << 23 ? 13 : (n <= 1ll << 25 ? 14 : kLocalMaxDrawBits));
+}
+// A random place in part s of 2^bits.
+ILGPU_HIP_RULE inline uint64_t local_draw_place(uint64_t s, int bits, uint64_t n) {
+  uint64_t z = (s + 1ull) * 0x9E3779B97F4A7C15ull;  // splitmix64
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+  z ^= z >> 31;
+  const uint64_t at = (s << 32 | (uint32_t)z) << (32 - bits);
+  return (uint64_t)(((unsigned __int128)at * n) >> 64);
+}
+// Where it is kept: every chunk holds draws from all over the input.  (Not all the questions look at all
+// chunks.  With the parts in a row, columns filled in front and padded behind passed: 2^28 u32 keys of which the
+// second half was the same, a second on one compute unit instead of 2.3 ms.)
+ILGPU_HIP_RULE constexpr uint32_t local_draw_slot(uint32_t s, int bits) {
+  return bits <= kLocalChunkBits ? s : (s & ((1u << (bits - kLocalChunkBits)) - 1u)) << kLocalChunkBits |
+                                           s >> (bits - kLocalChunkBits);
+}
+
+// What the draws may show.
+struct LocalLimits {
+  uint32_t draw_bits;  // log2 of the number of draws
+  uint32_t bin_bits;   // of a draw, from the topmost bit that differs on
+  uint32_t max_equal;  // draws that meet an earlier one in these bits
+  uint32_t max_pairs;  // pairs of draws that share a 16-bit prefix (0: one digit makes runs that may fit a window,
+                       // which its counts tell)
+  uint32_t max_draws;  // of one prefix
+  uint32_t max_run;    // keys of a run of one digit (0: two digits)
+};
+inline LocalLimits local_limits(int64_t keys, int key_bytes, int value_bytes) {
+  const int64_t window = local_window(key_bytes, value_bytes);
+  LocalLimits limits{};
+  limits.draw_bits = (uint32_t)local_draw_bits(keys);
+  const double draws = (double)(1ll << limits.draw_bits), n = (double)keys;
+  while (limits.bin_bits < 31 && keys >> limits.bin_bits != 0) ++limits.bin_bits;  // log2(n) + 1
+  limits.max_equal = (uint32_t)(1.25 * draws * draws / n) + 6u;
+  if (keys <= window * 256 * 15 / 16) {
+    limits.max_run = (uint32_t)window;
+  } else {
+    // Runs of 0.6 windows, as the mean over the keys.
+    const double looked_at = std::fmin(draws, (double)(1ll << kLocalPrefixBits));
+    limits.max_pairs = (uint32_t)(looked_at * looked_at * 0.5 * (0.6 * (double)window / n)) + 1u;
+    const double of_window = looked_at * (double)window / n;
+    const double most = of_window + 5.0 * std::sqrt(of_window) + 6.0;
+    limits.max_draws = most < 100.0 ? (uint32_t)most : 100u;
+  }
+  return limits;
 }
 
 // ---- bins -------------------------------------------------------------------

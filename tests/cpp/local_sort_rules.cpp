@@ -14,6 +14,24 @@ int64_t rule_deferred_bytes(int64_t n, int64_t blocks, uint32_t window) {
   return local_deferred_bytes(n, blocks, window);
 }
 
+// The draws of n keys: their places in the input and where they are kept; the number of them.
+int32_t rule_draws(int64_t n, uint64_t* places, uint32_t* slots) {
+  const int bits = local_draw_bits(n);
+  for (uint32_t s = 0; s < 1u << bits; ++s) {
+    places[s] = local_draw_place(s, bits, (uint64_t)n);
+    slots[s] = local_draw_slot(s, bits);
+  }
+  return 1 << bits;
+}
+int32_t rule_chunk_draws() { return 1 << kLocalChunkBits; }
+int32_t rule_prefix_draws() { return 1 << kLocalPrefixBits; }
+void rule_limits(int64_t n, int32_t key_bytes, int32_t value_bytes, uint32_t* out) {
+  const LocalLimits limits = local_limits(n, key_bytes, value_bytes);
+  const uint32_t all[] = {limits.draw_bits, limits.bin_bits,  limits.max_equal,
+                          limits.max_pairs, limits.max_draws, limits.max_run};
+  for (int i = 0; i < 6; ++i) out[i] = all[i];
+}
+
 // The codes of two keys' bins in a window whose keys are up to `span` behind its lowest, as the kernel
 // packs them; has_key: bit 0 the first, bit 1 the second key is one of the window.
 uint32_t rule_codes(int32_t key_bytes, uint64_t span, uint64_t first, uint64_t second, int32_t has_key) {

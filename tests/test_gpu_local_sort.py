@@ -133,6 +133,48 @@ def test_inputs_that_would_crowd_most_windows_take_every_digit():
     assert check(bits, np.uint64, np.uint32) == 4  # the digits that differ
 
 
+def check_on_device(bits, dtype, value_dtype=None):
+    """`check` for long columns: an int64 or int32 tensor of the keys' bits; ascending integers."""
+    import torch
+    n, width = bits.numel(), bits.element_size()
+    low = torch.iinfo(bits.dtype).min if np.dtype(dtype).kind == "u" else 0
+    expect = torch.sort(bits ^ low, stable=True)
+    work = bits.clone()
+    keys = D(n, dtype, _bytes=work.view(torch.uint8))
+    size = 0 if value_dtype is None else np.dtype(value_dtype).itemsize
+    temp = capi.temp_buffer(capi.radix_sort_temp_bytes(n, dtype, size))
+    if value_dtype is None:
+        capi.radix_sort_keys(keys, temp)
+    else:
+        values = D.zeros(n, value_dtype)
+        capi.radix_sort_pairs(keys, values, temp, values_from_index=True)
+    sync()
+    assert torch.equal(work, expect.values ^ low)
+    if value_dtype is not None:
+        held = values.bytes.view({4: torch.int32, 8: torch.int64}[size]).to(torch.int64)
+        assert torch.equal(held, expect.indices)
+    return capi.radix_sort_passes(temp, n, dtype, size)[0]
+
+
+@pytest.mark.parametrize("dtype,value_dtype", [(np.uint32, None), (np.int32, np.uint32), (np.uint64, None)])
+def test_long_columns_whose_parts_differ_take_every_digit(dtype, value_dtype):
+    """More draws than are looked at, from a column that is filled in front and padded behind (or the
+    other way round): a single run of the padding would be one block's."""
+    import torch
+    n = (1 << 25) + 3
+    width = 8 * np.dtype(dtype).itemsize
+    kind = {32: torch.int32, 64: torch.int64}[width]
+    uniform = torch.from_numpy(random_bits(n, width, 31).view(f"int{width}")).to("cuda:0")
+    note("uniform", np.dtype(dtype).name, n)
+    assert check_on_device(uniform, dtype, value_dtype) == 2
+    for value in (-1, (1 << (width - 1)) - 1, 0x3F800000):
+        for first, last in [(0.5, 1), (0, 0.5), (0.75, 1), (0.99, 1)]:
+            note("padded", np.dtype(dtype).name, value, first, last)
+            bits = uniform.clone()
+            bits[int(first * n):int(last * n)] = torch.tensor(value, dtype=kind)
+            assert check_on_device(bits, dtype, value_dtype) == width // 8
+
+
 def test_digits_that_all_keys_share_do_not_hide_the_topmost():
     """8-byte keys of 40 bits, and of 24 (no two digits to save)."""
     note("forty bits")

@@ -27,7 +27,39 @@ def rules(tmp_path_factory):
     lib.rule_deferred.restype = ctypes.c_uint32
     lib.rule_deferred_bytes.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_uint32]
     lib.rule_deferred_bytes.restype = ctypes.c_int64
+    lib.rule_draws.argtypes = [ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p]
+    lib.rule_limits.argtypes = [ctypes.c_int64, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p]
     return lib
+
+
+class Limits(ctypes.Structure):
+    _fields_ = [(name, ctypes.c_uint32) for name in
+                ("draw_bits", "bin_bits", "max_equal", "max_pairs", "max_draws", "max_run")]
+
+
+def draws_of(rules, n):
+    """The places of n keys that are drawn, in the order in which the draws are kept."""
+    places, slots = np.zeros(1 << 16, np.uint64), np.zeros(1 << 16, np.uint32)
+    m = rules.rule_draws(n, places.ctypes.data, slots.ctypes.data)
+    assert sorted(slots[:m]) == list(range(m))
+    kept = np.zeros(m, np.uint64)
+    kept[slots[:m]] = places[:m]
+    return kept
+
+
+def two_digits_are_enough(rules, n, key_bytes, value_bytes, keys_at):
+    """What the draws say of keys in their ordered form: the same questions with numpy."""
+    limits = Limits()
+    rules.rule_limits(n, key_bytes, value_bytes, ctypes.addressof(limits))
+    assert limits.max_run == 0 and limits.max_pairs > 0
+    keys = keys_at(draws_of(rules, n))
+    differ = int(np.bitwise_or.reduce(keys[: rules.rule_chunk_draws()] ^ keys[0]))
+    top = (differ.bit_length() - 1) // 8
+    if top < 3:
+        return False
+    prefixes = (keys[: rules.rule_prefix_draws()] >> keys.dtype.type(8 * (top - 1))) & keys.dtype.type(0xFFFF)
+    counts = np.bincount(prefixes.astype(np.int64), minlength=1 << 16)
+    return counts.max() <= limits.max_draws and (counts * (counts - 1) // 2).sum() <= limits.max_pairs
 
 
 @pytest.mark.parametrize("size", [4, 8])
@@ -93,3 +125,33 @@ def test_what_is_put_off_fits_the_status_words(rules, key_bytes, value_bytes):
         for cus in (1, 32, 64, 256, 304, 1024):
             blocks = rules.rule_blocks(n, cus)
             assert rules.rule_deferred_bytes(n, blocks, window) <= key_bytes * 1024 * -(-n // tile)
+
+
+def test_every_chunk_of_draws_is_from_all_over_the_input(rules):
+    for n in (1 << 14, (1 << 21) + 1, (1 << 23) + 1, (1 << 25) + 1, 1 << 28, (1 << 31) - 1):
+        places = draws_of(rules, n)
+        assert places.max() < n and places.size <= n
+        assert np.unique(places).size == places.size
+        for chunk in places.reshape(-1, min(places.size, rules.rule_chunk_draws())):
+            in_64_parts = np.bincount((chunk * np.uint64(64) // np.uint64(n)).astype(np.int64), minlength=64)
+            # (A part of the input that is no whole number of elements may give its draw to the next 64th.)
+            assert np.abs(in_64_parts - chunk.size // 64).max() <= 2
+
+
+@pytest.mark.parametrize("n,key_bytes,value_bytes", [
+    (1 << 23, 4, 0), ((1 << 25) + 1, 4, 0), (1 << 28, 4, 0), (1 << 26, 4, 4), ((1 << 25) + 1, 8, 0), (1 << 27, 8, 4)])
+def test_columns_whose_parts_differ_are_refused_by_the_draws(rules, n, key_bytes, value_bytes):
+    """Uniform keys are taken; with a part of the input that is all one value, wherever it
+    lies and whatever the value, they are not (a hundredth is ten windows and more here)."""
+    kind = np.dtype(f"uint{8 * key_bytes}").type
+    largest = (1 << 8 * key_bytes) - 1
+
+    def uniform(places):
+        return np.random.default_rng(7).integers(0, largest, places.size, dtype=kind, endpoint=True)
+
+    assert two_digits_are_enough(rules, n, key_bytes, value_bytes, uniform)
+    for value in [largest, largest >> 1, largest // 3, 0, 1, 0x3F800000]:
+        for first, last in [(0.5, 1), (0, 0.5), (0.75, 1), (0.3, 0.4), (0.9, 1), (0.99, 1), (0, 0.01)]:
+            def padded(places):
+                return np.where((places >= int(first * n)) & (places < int(last * n)), kind(value), uniform(places))
+            assert not two_digits_are_enough(rules, n, key_bytes, value_bytes, padded), (value, first, last)
