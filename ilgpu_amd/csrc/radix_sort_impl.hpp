@@ -845,7 +845,7 @@ constexpr int kPlanBlock = kPlanGroups * kRadix;
 __global__ __launch_bounds__(kPlanBlock) void plan_kernel(
     const uint32_t* __restrict__ global_hist, uint32_t* __restrict__ excl,
     SortPlan* __restrict__ plan, int passes, uint32_t n, TieSampling ties,
-    const uint32_t* __restrict__ local_from, uint32_t local_max_run) {
+    const uint32_t* __restrict__ local_from, uint32_t local_max_run, uint32_t local_window_keys) {
   constexpr int kRounds = kMaxPasses / kPlanGroups;
   constexpr int kGroupWaves = kRadix / kWaveSize;
   constexpr int kFrequent = 8;  // digits with an eighth of the keys: no more than eight
@@ -924,12 +924,14 @@ __global__ __launch_bounds__(kPlanBlock) void plan_kernel(
   // spread and that saves two passes at least (a digit that all keys share needs none): below
   // the topmost digit that differs where none of its values has more keys than a window
   // (local_max_run != 0: the input may be short enough for that), or below two digits where the
-  // draws found short runs.
+  // draws found short runs and no count speaks for a long one.
   int left = 0, local = 0;
   if (spread && varies != 0u) {
     const int top = 31 - __builtin_clz(varies);
-    if (local_max_run == 0) local = two_digits;
-    else if (s_most[top] <= local_max_run) local = top;
+    if (local_max_run == 0) {
+      if (two_digits != 0 && local_counts_allow(n, s_most[two_digits + 1], s_most[two_digits], local_window_keys))
+        local = two_digits;
+    } else if (s_most[top] <= local_max_run) local = top;
     if (__popc(varies & ((1u << local) - 1u)) < 2) local = 0;
     left = local;
   }
@@ -3348,7 +3350,8 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
   {
     ProfileScope scope(stream, "sort_plan");
     hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(kPlanBlock), 0, stream, hist, excl,
-                       plan, passes, (uint32_t)a.n, ties, local.from, local.limits.max_run);
+                       plan, passes, (uint32_t)a.n, ties, local.from, local.limits.max_run,
+                       (uint32_t)local_window(KEY_BYTES, VALUE_BYTES));
   }
   ILGPU_HIP_CHECK(hipGetLastError());
 

@@ -218,7 +218,9 @@ __device__ __attribute__((noinline)) void local_window_by_digits(
 }
 
 // A run longer than a window: by the block, through memory, one pass for each of its lower
-// digits that differ between its keys.  `other` is scratch at the run's own place; the
+// digits that differ between its keys.  (Of one digit there are none, of two the counts allow n / 256 keys and a
+// window, or n / 4096 keys: local_counts_allow.  A run of 9300 keys takes 27 to 45 us more than short ones, of 50 000 u32 110 to
+// 190, of 25 000 u64 250 to 330, copies of a key the most.)  `other` is scratch at the run's own place; the
 // result ends in `result`, which is one of the two.
 template <int KEY_BYTES, int VALUE_BYTES>
 __device__ __attribute__((noinline)) void local_long_run(

@@ -108,6 +108,17 @@ inline LocalLimits local_limits(int64_t keys, int key_bytes, int value_bytes) {
   return limits;
 }
 
+// Two digits are refused by their exact counts where the draws may have missed a long run, which is one
+// block's: one of L keys adds L to the count of its lower digit, and other keys spread over that digit
+// evenly where their runs are short.  `most_upper` and `most_lower`: keys of the most frequent upper and lower digit.
+// A block takes 3 ns for a key of 4 bytes and 11 for one of 8, once a run is longer than a window; n / 4096
+// keys are half of what the local sort gains.  Whatever the keys are, no run is longer than n / 256 and that.
+// The 256 runs of an upper digit are longer than a window if it has 256 windows.
+ILGPU_HIP_RULE constexpr bool local_counts_allow(uint32_t n, uint32_t most_upper, uint32_t most_lower,
+                                                 uint32_t window) {
+  return most_upper <= (uint64_t)window * 256 && most_lower <= n / 256 + (window > n / 4096 ? window : n / 4096);
+}
+
 // ---- bins -------------------------------------------------------------------
 // bin = ((key - low) >> shift) * scale >> 16: the shift leaves 18 bits, the scale spreads
 // what they hold over all the bins.  Keys of the window, up to low + span, have bins below kBins; others

@@ -32,6 +32,10 @@ void rule_limits(int64_t n, int32_t key_bytes, int32_t value_bytes, uint32_t* ou
   for (int i = 0; i < 6; ++i) out[i] = all[i];
 }
 
+int32_t rule_counts_allow(uint32_t n, uint32_t most_upper, uint32_t most_lower, uint32_t window) {
+  return local_counts_allow(n, most_upper, most_lower, window);
+}
+
 // The codes of two keys' bins in a window whose keys are up to `span` behind its lowest, as the kernel
 // packs them; has_key: bit 0 the first, bit 1 the second key is one of the window.
 uint32_t rule_codes(int32_t key_bytes, uint64_t span, uint64_t first, uint64_t second, int32_t has_key) {

@@ -175,6 +175,57 @@ def test_long_columns_whose_parts_differ_take_every_digit(dtype, value_dtype):
             assert check_on_device(bits, dtype, value_dtype) == width // 8
 
 
+@pytest.mark.parametrize("dtype,value_dtype", [
+    (np.uint32, None), (np.uint32, np.uint32), (np.uint64, None), (np.uint64, np.uint64)])
+def test_a_run_that_the_draws_let_pass_is_told_by_the_counts(dtype, value_dtype):
+    """Two windows of keys of one prefix among uniform ones: copies, and different ones, which of 8-byte keys
+    the passes over the upper half and the ties order (and of copies, where these are as many as those order)."""
+    size = np.dtype(dtype).itemsize
+    width = 8 * size
+    kind = np.dtype(dtype).type
+    window = WINDOWS[size, value_dtype is not None]
+    n = (1 << 23) + 1
+    uniform = random_bits(n, width, 41)
+    at = np.random.default_rng(42).permutation(n)[:2 * window]
+    low = random_bits(at.size, width, 43) & kind((1 << (width - 16)) - 1)
+    for name, keys, passes in [("copies", low[:1], (4, size)), ("different", low, (4,))]:
+        note("two windows", np.dtype(dtype).name, value_dtype, name)
+        bits = uniform.copy()
+        bits[at] = kind(0x3456 << (width - 16)) | keys
+        assert check(bits, dtype, value_dtype) in passes
+    note("one window", np.dtype(dtype).name, value_dtype)
+    bits[at[window // 2:]] = uniform[at[window // 2:]]
+    assert check(bits, dtype, value_dtype) == 2
+
+
+@pytest.mark.parametrize("size", [4, 8])
+@pytest.mark.parametrize("value_dtype", [None, np.uint16, np.uint64])
+def test_runs_longer_than_a_window_that_no_count_tells(size, value_dtype):
+    """A block orders them through memory: no other key has the run's lower digit.  Different keys, copies,
+    and both, of keys whose last digits are the same or not."""
+    window = WINDOWS[size, value_dtype is not None]
+    width = 8 * size
+    kind = np.dtype(f"uint{width}").type
+    n = (600 if size == 4 else 450) * window
+    assert size == 4 or n < 1 << 21  # where the passes over the upper half come first
+    rng = np.random.default_rng(size)
+    bits = random_bits(n, width, 51)
+    bare = np.flatnonzero((bits >> kind(width - 16) & kind(0xFF)) == 0x34)
+    bits[bare] += rng.integers(1, 0x100 - 0x34, bare.size, dtype=kind) << kind(width - 16)
+    for length in (window + 1, 3 * window // 2, 7 * window // 4):
+        # (Nothing but copies crowd the draws of 4-byte keys alone, and those of longer runs.)
+        only_copies = length == window + 1 and (size == 8 or value_dtype is not None)
+        for copies, mask in [(0, 0), (4, 0), (0, 0xFF)] + [(1, 0)] * only_copies:
+            note("long run", size, value_dtype, length, copies, mask)
+            at = rng.permutation(n)[:length]
+            low = random_bits(length, width, 52) & kind((1 << (width - 16)) - 1 - mask)
+            if copies:
+                low[::copies] = low[0]
+            keys = bits.copy()
+            keys[at] = kind(0x1234 << (width - 16)) | low
+            assert check(keys, np.dtype(kind), value_dtype, descending=length % 2 == 0) == 2
+
+
 def test_digits_that_all_keys_share_do_not_hide_the_topmost():
     """8-byte keys of 40 bits, and of 24 (no two digits to save)."""
     note("forty bits")

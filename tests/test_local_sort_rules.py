@@ -155,3 +155,19 @@ def test_columns_whose_parts_differ_are_refused_by_the_draws(rules, n, key_bytes
             def padded(places):
                 return np.where((places >= int(first * n)) & (places < int(last * n)), kind(value), uniform(places))
             assert not two_digits_are_enough(rules, n, key_bytes, value_bytes, padded), (value, first, last)
+
+
+@pytest.mark.parametrize("key_bytes,value_bytes", KINDS)
+def test_counts_of_two_digits_bound_a_run(rules, key_bytes, value_bytes):
+    """The digits' counts of uniform keys pass, with the scatter of 256 of them, as far as the draws let uniform
+    keys pass (runs of 0.6 windows); a run of two windows and of n / 2000 keys more does not, nor does
+    a digit whose runs are all longer than a window."""
+    window = rules.rule_window(key_bytes, value_bytes)
+    rng = np.random.default_rng(5)
+    for n in (window * 240 + 1, 1 << 23, 1 << 25, int(0.6 * window * 65536)):
+        for _ in range(20):
+            upper, lower = rng.multinomial(n, [1 / 256] * 256, 2)
+            assert rules.rule_counts_allow(n, int(upper.max()), int(lower.max()), window)
+            run = 2 * window + n // 2000
+            assert not rules.rule_counts_allow(n, int(upper[0]) + run, int(lower[0]) + run, window)
+    assert not rules.rule_counts_allow(1 << 30, 256 * window + 1, (1 << 30) // 256, window)
