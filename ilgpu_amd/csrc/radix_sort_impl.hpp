@@ -2226,29 +2226,58 @@ void onesweep_pipelined_kernel(
 // a tile has so few keys that of 8-byte keys the three topmost digits that differ (up to 2048
 // integers) or the four topmost tell all but a few pairs apart: only those run, and where
 // neighbours are then in the wrong order every key looks for the ones of its prefix that go the
-// other way round.  A row of keys per wave is asked beforehand how often they share a prefix, and
-// where one has more than kSmallSortReach keys all the digits follow.
-// (Kernel, us, every digit / this: 2000 int64 uniform 13.6 / 7.5, with u32 index values 14.9 / 8.3, below 10^6
-// 13.2 / 7.0, normal doubles 14.6 / 10.6; 9000 uint64 uniform 32.3 / 22.4; 18 000 u32 below 10^6 31.2 / 22.1.)
+// other way round.  Which pays while few different keys share a prefix, so 512 keys from all over the input
+// are asked: each takes its prefix's slot in LDS and looks at the one before, and those that meet another key of
+// their prefix are counted.  (Copies of a key need no order.)  Where a prefix has more than kSmallSortReach keys all the
+// same, and they are in the wrong order, all the digits follow.
+// (Kernel, us, every digit / this: 2000 int64 uniform 13.6 / 7.4, with u32 index values 14.9 / 8.3, below 10^6
+// 13.2 / 6.5, time stamps within 17 s 13.7 / 11.7, normal doubles 14.6 / 10.6; 9000 uniform 32.3 / 21.1, 18 000 u32 below
+// 10^6 31.2 / 22.1.  A prefix of 30 of 2000 keys 13.6 / 13.3, of 9000 32.3 / 30.2; of a tenth, all digits, 13.5 / 14.3 and
+// 32.2 / 33.6, signed numbers of 40 bits 13.3 / 13.8 and 31.3 / 32.5: the question.  With 8 keys of a row and wave asked, and
+// runs of up to 24 taken: a tenth 36.7 and 116, 40 bits 14.8 and 165, where many runs of some 20 were looked through,
+// or the prefix's passes were for nothing.)
 // (Two digits and the same of 4-byte keys: a key in four has a neighbour to look at, 18 000 keys 68 us
 // instead of 34.6.)
-constexpr int kSmallSortReach = 24;
-constexpr int kSmallSortAlike = 16;  // of the 512 keys asked
+constexpr int kSmallSortReach = 256;
+constexpr int kSmallSortAlike = 12;  // of a wave's keys asked
+constexpr int kAskedSlotsLog2 = 11;
+// `clashes`: keys asked that meet another of their prefix.  Half a key beside every key is too many: all
+// waves would look at neighbours (7000 keys in 20 bursts, 1.4 others per key, 35.2 us all digits, 40.7 by prefix; 2000 in
+// 20 bursts, 0.4 per key, 17.5 and 15.3).
+__device__ __forceinline__ bool small_sort_few_meet(int clashes, int n) {
+  return (int64_t)clashes * (n > kSortBlock ? n : kSortBlock) <= kSortBlock * kSortBlock / 4;
+}
+// `pairs`: of the keys asked that differ from another of their prefix.  Of a run of L keys some k = 512 L / n are asked, which
+// makes k^2 / 2 and fewer of them; the runs that cost as much to look through as the passes that are saved have some
+// 35 keys of 2000, 80 of 9000.
+__device__ __forceinline__ bool small_sort_spreads(int pairs, int n) {
+  const int64_t m = n > kSortBlock ? n : kSortBlock;
+  const int64_t run = kSortBlock * (30 + m / 256);
+  return 2 * pairs * m * m <= run * run;
+}
 
-// OR over the lanes of a wave, in every lane.
-__device__ __forceinline__ uint32_t wave_or(uint32_t v) {
-  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);  // row_shr:1
-  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);
-  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);
-  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);
-  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);  // row_bcast:15
-  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+// OR over the lanes of a wave, and the sum, in every lane.
+template <typename Join>
+__device__ __forceinline__ uint32_t wave_join(uint32_t v, Join join) {
+  v = join(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false));  // row_shr:1
+  v = join(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false));
+  v = join(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false));
+  v = join(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false));
+  v = join(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));  // row_bcast:15
+  v = join(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));  // row_bcast:31
   return (uint32_t)__builtin_amdgcn_readlane((int)v, kWaveSize - 1);
+}
+__device__ __forceinline__ uint32_t wave_or(uint32_t v) {
+  return wave_join(v, [](uint32_t a, uint32_t b) { return a | b; });
+}
+__device__ __forceinline__ int wave_sum(int v) {
+  return (int)wave_join((uint32_t)v, [](uint32_t a, uint32_t b) { return a + b; });
 }
 
 constexpr int kSmallSortItemsA = 4, kSmallSortItemsB = 12, kSmallSortItemsC = 24;
+// (One block runs: registers and LDS are not shared with others.)
 template <int KEY_BYTES, int VALUE_BYTES, bool FLOAT_KEYS, int ITEMS>
-__global__ __launch_bounds__(kSortBlock, ILGPU_HIP_SORT_WAVES_PER_EU)
+__global__ __launch_bounds__(kSortBlock, KEY_BYTES == 8 ? 2 : ILGPU_HIP_SORT_WAVES_PER_EU)
 void small_sort_kernel(typename KeyOf<KEY_BYTES>::type* keys,
                        typename ValueOf<VALUE_BYTES>::type* vals, int n, KeyXform xf,
                        int values_from_index) {
@@ -2269,8 +2298,10 @@ void small_sort_kernel(typename KeyOf<KEY_BYTES>::type* keys,
   __shared__ __attribute__((aligned(16))) unsigned char s_stage[kStageBytes];
   __shared__ uint32_t s_scan[kRadix / kWaveSize];
   __shared__ uint64_t s_diff[kSubTiles];
-  __shared__ uint32_t s_alike[kSubTiles];
   __shared__ uint32_t s_inverted, s_far;
+  __shared__ int s_clashes[kSubTiles], s_pairs[kSubTiles];
+  __shared__ uint64_t s_asked[KEY_BYTES == 8 ? kSortBlock : 1];
+  __shared__ uint16_t s_to[KEY_BYTES == 8 ? kSortBlock * kItems : 1];  // where a staged key belongs
   uint32_t* s_counter = reinterpret_cast<uint32_t*>(s_stage);
   K* s_keys = reinterpret_cast<K*>(s_stage);
   Val* s_vals = reinterpret_cast<Val*>(s_stage);
@@ -2281,8 +2312,16 @@ void small_sort_kernel(typename KeyOf<KEY_BYTES>::type* keys,
   const int first_local = wave * kSubTileKeys + lane;
   uint32_t* my_counters = s_counter + wave * kRadix;
 
-  K key[kItems];
+  K key[kItems], asked = 0;
   Val val[kPairs ? kItems : 1];
+  uint32_t* s_words = reinterpret_cast<uint32_t*>(s_stage);  // two tables of kAskedSlotsLog2
+  if constexpr (KEY_BYTES == 8) {
+    static_assert(8 << kAskedSlotsLog2 <= kStageBytes && (8 << kAskedSlotsLog2) % (16 * kSortBlock) == 0, "");
+    asked = keys[(uint32_t)tid * (uint32_t)n / kSortBlock];
+#pragma unroll
+    for (int i = 0; i < (8 << kAskedSlotsLog2) / (16 * kSortBlock); ++i)
+      reinterpret_cast<uint4*>(s_stage)[i * kSortBlock + tid] = make_uint4(0u, 0u, 0u, 0u);
+  }
 #pragma unroll
   for (int j = 0; j < kItems; ++j) {
     const int local = first_local + j * kSubLanes;
@@ -2322,6 +2361,11 @@ void small_sort_kernel(typename KeyOf<KEY_BYTES>::type* keys,
     if constexpr (KEY_BYTES == 8) diff |= (uint64_t)wave_or((uint32_t)((uint64_t)mine >> 32)) << 32;
     if (lane == 0) s_diff[wave] = diff;
     if (tid == 0) s_inverted = s_far = 0u;
+    if constexpr (KEY_BYTES == 8) {
+      if constexpr (FLOAT_KEYS) asked = ordered_bits(asked, xf);
+      else asked = ordered(asked);
+      s_asked[tid] = asked;
+    }
     __syncthreads();
 #pragma unroll
     for (int w = 0; w < kSubTiles; ++w) diff |= s_diff[w];
@@ -2335,14 +2379,41 @@ void small_sort_kernel(typename KeyOf<KEY_BYTES>::type* keys,
     prefix_shift = top_bits > 8 * kPrefixDigits ? top_bits - 8 * kPrefixDigits : 0;
     by_prefix = digits > kPrefixDigits;
     if (by_prefix) {
-      const uint64_t prefix = (uint64_t)ordered(key[0]) >> prefix_shift;
-      const uint64_t same = __ballot(first_local < n && prefix == readfirstlane_key(prefix));
-      if (lane == 0) s_alike[wave] = same != 0ull ? (uint32_t)__popcll(same) - 1u : 0u;
+      const uint64_t prefix = (uint64_t)asked >> prefix_shift;
+      const uint32_t slot = ((uint32_t)prefix * 0x9E3779B1u) >> (32 - kAskedSlotsLog2);
+      // (A wave that sees many of one prefix asks no more: all would wait for one word.)
+      const int alike = __popcll(__ballot(prefix == readfirstlane_key(prefix) &&
+                                          (uint64_t)asked != readfirstlane_key((uint64_t)asked)));
+      bool clash = false;
+      if (alike <= kSmallSortAlike) {
+        const uint32_t before = __hip_atomic_exchange(&s_words[slot], (uint32_t)tid + 1u, __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (before != 0u) {
+          const uint64_t other = s_asked[before - 1u];
+          clash = other >> prefix_shift == prefix && other != (uint64_t)asked;
+        }
+      }
+      int clashes = __popcll(__ballot(clash));
+      if (lane == 0) s_clashes[wave] = alike <= kSmallSortAlike ? clashes : 1 << 20;
       __syncthreads();
-      uint32_t alike = 0;
+      clashes = 0;
 #pragma unroll
-      for (int w = 0; w < kSubTiles; ++w) alike += s_alike[w];
-      by_prefix = __builtin_amdgcn_readfirstlane((int)alike) <= kSmallSortAlike;
+      for (int w = 0; w < kSubTiles; ++w) clashes += s_clashes[w];
+      clashes = __builtin_amdgcn_readfirstlane(clashes);
+      by_prefix = small_sort_few_meet(clashes, n);
+      if (by_prefix && clashes != 0) {  // how many of them share a prefix
+        int pairs = 0;
+        if (clash)
+          pairs = (int)__hip_atomic_fetch_add(&s_words[(1 << kAskedSlotsLog2) + slot], 1u, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_WORKGROUP);
+        pairs = wave_sum(pairs);
+        if (lane == 0) s_pairs[wave] = pairs;
+        __syncthreads();
+        pairs = 0;
+#pragma unroll
+        for (int w = 0; w < kSubTiles; ++w) pairs += s_pairs[w];
+        by_prefix = small_sort_spreads(__builtin_amdgcn_readfirstlane(pairs), n);
+      }
     }
   }
   int shift = by_prefix ? prefix_shift : 0;
@@ -2351,14 +2422,19 @@ void small_sort_kernel(typename KeyOf<KEY_BYTES>::type* keys,
     const bool last_of_prefix = by_prefix && shift + 8 >= top_bits;
     if (!by_prefix && (diff >> shift & 0xFFull) == 0) continue;
     // Positions past the end take digit 255 and come last in memory order, so
-    // they stay behind every key through every pass.
+    // they stay behind every key through every pass.  (The length is made opaque: held from one pass to the
+    // next the rows' masks spill.)
+    int length = n;
+    asm volatile("" : "+s"(length));
     auto item_digit = [&](int j) -> uint32_t {
-      if (first_local + j * kSubLanes >= n) return (uint32_t)(kRadix - 1);
+      if (first_local + j * kSubLanes >= length) return (uint32_t)(kRadix - 1);
       return (uint32_t)(ordered(key[j]) >> shift) & (kRadix - 1);
     };
     __syncthreads();  // the stage of the previous pass has been read
-    for (int i = tid; i < TileCfg::kCounterWords; i += kSortBlock) s_counter[i] = 0u;
-    __syncthreads();
+    // (A wave clears its own counters, and needs no barrier for that.)
+    static_assert(kRadix == 4 * kSubLanes, "four counters per lane");
+    reinterpret_cast<uint4*>(my_counters)[lane] = make_uint4(0u, 0u, 0u, 0u);
+    __builtin_amdgcn_wave_barrier();
 
     uint32_t packed[kItems / 2];  // rank in the sub-tile, then position in the tile
 #pragma unroll
@@ -2420,40 +2496,56 @@ void small_sort_kernel(typename KeyOf<KEY_BYTES>::type* keys,
 #pragma unroll
         for (int j = 0; j < kItems; ++j) {
           const int at = j * kSortBlock + tid;
-          if (at + 1 < n) inverted = inverted || ordered(s_keys[at]) > ordered(s_keys[at + 1]);
+          if (at + 1 < length) inverted = inverted || ordered(s_keys[at]) > ordered(s_keys[at + 1]);
         }
         if (inverted) s_inverted = 1u;
         __syncthreads();
         if (s_inverted != 0u) {
           // Keys of the same prefix are next to each other, equal keys in their order: a key moves
           // by the smaller ones behind it and the larger ones in front of it.
-#pragma unroll
-          for (int j = 0; j < kItems; ++j) {
-            if (first_local + j * kSubLanes >= n) continue;
-            const int at = (int)(j % 2 == 0 ? packed[j / 2] & 0xFFFFu : packed[j / 2] >> 16);
-            const K o = ordered(key[j]);
+          for (int at = tid; at < length; at += kSortBlock) {
+            const K o = ordered(s_keys[at]);
             const K prefix = (K)(o >> prefix_shift);
             int to = at;
-            for (int q = at + 1; q < n; ++q) {
-              const K other = ordered(s_keys[q]);
-              if ((K)(other >> prefix_shift) != prefix) break;
-              to += other < o ? 1 : 0;
-              if (q - at >= kSmallSortReach) { s_far = 1u; break; }
-            }
-            for (int q = at - 1; q >= 0; --q) {
-              const K other = ordered(s_keys[q]);
-              if ((K)(other >> prefix_shift) != prefix) break;
-              to -= other > o ? 1 : 0;
-              if (at - q >= kSmallSortReach) { s_far = 1u; break; }
-            }
-            if (j % 2 == 0) packed[j / 2] = (packed[j / 2] & 0xFFFF0000u) | (uint32_t)to;
-            else packed[j / 2] = (packed[j / 2] & 0xFFFFu) | (uint32_t)to << 16;
+            auto look = [&](int step) {
+              const int next = at + step;
+              if (next < 0 || next >= length || (K)(ordered(s_keys[next]) >> prefix_shift) != prefix) return;
+              for (int q = next;; q += 4 * step) {  // four keys at a time
+                K other[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                  const int from = q + e * step;
+                  other[e] = ordered(s_keys[from < 0 ? 0 : (from < length ? from : length - 1)]);
+                }
+                bool same = true;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                  const int from = q + e * step;
+                  same = same && from >= 0 && from < length && (K)(other[e] >> prefix_shift) == prefix;
+                  if (same) to += step > 0 ? (other[e] < o ? 1 : 0) : (other[e] > o ? -1 : 0);
+                }
+                if (!same) break;
+                if ((q - at) * step > kSmallSortReach) {
+                  s_far = 1u;
+                  break;
+                }
+              }
+            };
+            look(1);
+            look(-1);
+            s_to[at] = (uint16_t)to;
           }
           __syncthreads();
           if (s_far != 0u) {  // from the order before this pass, which the registers still hold
             by_prefix = false;
             shift = -8;
             continue;
+          }
+#pragma unroll
+          for (int j = 0; j < kItems; j += 2) {
+            // (Positions behind the keys keep their places.)
+            const uint32_t p0 = packed[j / 2] & 0xFFFFu, p1 = packed[j / 2] >> 16;
+            packed[j / 2] = ((int)p0 < length ? s_to[p0] : p0) | ((int)p1 < length ? s_to[p1] : p1) << 16;
           }
 #pragma unroll
           for (int j = 0; j < kItems; ++j)

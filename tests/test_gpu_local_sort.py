@@ -289,6 +289,63 @@ def test_one_tile_sorts_by_the_topmost_digits(dtype, descending, total_order, va
     check(np.full(777, 5, np.uint64), np.uint64, np.uint32)
 
 
+def with_a_cluster(n, length, seed, unasked=False):
+    """Random 8-byte keys, `length` of which share their upper half: anywhere, or where the block
+    asks no key (it asks the 512 at t * n / 512)."""
+    bits = random_bits(n, 64, seed)
+    places = np.arange(n)
+    if unasked:
+        places = np.setdiff1d(places, np.arange(512) * n // 512)
+    at = np.random.default_rng(seed).permutation(places)[:length]
+    bits[at] = np.uint64(0x12345678 << 32) | random_bits(at.size, 32, seed + 1).astype(np.uint64)
+    return bits
+
+
+@pytest.mark.parametrize("dtype", [np.int64, np.uint64, np.float64])
+@pytest.mark.parametrize("value_dtype", [None, np.uint32, np.uint64])
+def test_one_tile_whose_keys_cluster(dtype, value_dtype):
+    """Prefixes of as many keys as are taken and looked through, of more than a key looks at where none of
+    them is asked, of all but the first keys, many prefixes of some 20 keys each, and copies."""
+    for n in (500, 2048, 5000, 9216 if value_dtype is None else 5120 if value_dtype is np.uint64 else 7168):
+        for length, unasked in [(20, False), (35, False), (90, False), (n // 10, False), (n - 3, False),
+                                (257, True), (262, True), (300, True), (n // 3, True)]:
+            note("cluster", np.dtype(dtype).name, value_dtype, n, length, unasked)
+            check(with_a_cluster(n, length, n + length, unasked), dtype, value_dtype, from_index=False,
+                  descending=length % 2 == 0, total_order=True)
+        note("forty signed bits", np.dtype(dtype).name, value_dtype, n)
+        check((random_bits(n, 64, n).view(np.int64) >> 24).view(np.uint64), dtype, value_dtype, total_order=True)
+        few = random_bits(n // 10, 64, n)
+        check(few[np.random.default_rng(n).integers(0, few.size, n)], dtype, value_dtype, from_index=False)
+
+
+def test_one_tile_whose_keys_cluster_takes_no_longer_than_every_digit():
+    """9000 keys: a third of the passes more where a prefix says nothing, not passes for nothing and keys that
+    look through hundreds of others (five times as long)."""
+    import torch
+    temp = capi.temp_buffer(capi.radix_sort_temp_bytes(9000, np.uint64))
+
+    def us(bits):
+        source, keys = D.from_numpy(bits), D(9000, np.uint64)
+        times = []
+        for _ in range(15):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            for _ in range(20):
+                capi.transform(source, keys)
+                capi.radix_sort_keys(keys, temp)
+            end.record()
+            sync()
+            times.append(start.elapsed_time(end) * 50)
+        return sorted(times)[7]
+
+    uniform = us(random_bits(9000, 64, 61))
+    for name, bits in [("a tenth", with_a_cluster(9000, 900, 62)), ("80", with_a_cluster(9000, 80, 63)),
+                       ("forty signed bits", (random_bits(9000, 64, 64).view(np.int64) >> 24).view(np.uint64))]:
+        clustered = us(bits)
+        note(name, uniform, clustered)
+        assert clustered < 2.5 * uniform
+
+
 def test_one_tile_of_narrow_keys_skips_the_digits_they_share():
     note("narrow keys")
     for n in (18_432, 12_289, 777):
