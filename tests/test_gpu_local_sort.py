@@ -226,6 +226,57 @@ def test_runs_longer_than_a_window_that_no_count_tells(size, value_dtype):
             assert check(keys, np.dtype(kind), value_dtype, descending=length % 2 == 0) == 2
 
 
+def crowded_bits(n, width, seed):
+    """Values of every width some 30 times each: neither the local sort nor the ties take them."""
+    values = random_bits(n // 30, width, seed)
+    return values[np.random.default_rng(seed).integers(0, values.size, n)]
+
+
+@pytest.mark.parametrize("dtype,descending", [
+    (np.uint32, True), (np.int32, False), (np.float32, True), (np.uint64, False), (np.float64, True)])
+@pytest.mark.parametrize("value_dtype", [None, np.uint16, np.uint32, np.uint64])
+def test_refused_inputs_take_every_pass(dtype, descending, value_dtype):
+    """The chains of four and eight passes, at the edges of the short tiles and with every choice of tile."""
+    size = np.dtype(dtype).itemsize
+    edges = [512 * 6144, 512 * 9216 + 1, 512 * 12288] if size == 4 else [128 * 3072, 128 * 4096 + 1, 128 * 6144 + 1]
+    edges = [18_433, 100_003] + (edges if value_dtype is None else [221_261])
+    for n in edges:
+        for large_block, short_tiles in [(-1, -1), (0, -1), (2**31 - 1, 0)]:
+            if n > 400_000 and large_block >= 0:
+                continue
+            capi.sort_set_parameter(capi.SORT_PARAM_LARGE_BLOCK_MIN_TILES_PER_CU, large_block)
+            capi.sort_set_parameter(capi.SORT_PARAM_SHORT_TILE_MAX_TILES, short_tiles)
+            note("every pass", np.dtype(dtype).name, value_dtype, n, large_block, short_tiles)
+            assert check(crowded_bits(n, 8 * size, n), dtype, value_dtype, descending, total_order=True,
+                         from_index=n % 2 == 0) == size
+
+
+def test_two_refused_sorts_on_two_streams():
+    """Chains of four pipelined passes and of eight passes of pairs share the GPU."""
+    import torch
+    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    a, b = crowded_bits((1 << 24) + 11, 32, 71), crowded_bits((1 << 23) + 5, 64, 72)
+    d_a = [D.from_numpy(a) for _ in range(3)]
+    d_b = [D.from_numpy(b) for _ in range(3)]
+    d_v = [D.zeros(b.size, np.uint32) for _ in range(3)]
+    t_a = [capi.temp_buffer(capi.radix_sort_temp_bytes(a.size, np.uint32)) for _ in range(3)]
+    t_b = [capi.temp_buffer(capi.radix_sort_temp_bytes(b.size, np.uint64, 4)) for _ in range(3)]
+    sync()
+    note("two refused sorts on two streams")
+    for i in range(3):
+        with torch.cuda.stream(s1):
+            capi.radix_sort_keys(d_a[i], t_a[i])
+        with torch.cuda.stream(s2):
+            capi.radix_sort_pairs(d_b[i], d_v[i], t_b[i], values_from_index=True)
+    sync()
+    e_a, order = np.sort(a), np.argsort(b, kind="stable")
+    for i in range(3):
+        assert capi.radix_sort_passes(t_a[i], a.size, np.uint32)[0] == 4
+        assert capi.radix_sort_passes(t_b[i], b.size, np.uint64, 4)[0] == 8
+        assert np.array_equal(d_a[i].numpy(), e_a)
+        assert np.array_equal(d_b[i].numpy(), b[order]) and np.array_equal(d_v[i].numpy(), order)
+
+
 def test_digits_that_all_keys_share_do_not_hide_the_topmost():
     """8-byte keys of 40 bits, and of 24 (no two digits to save)."""
     note("forty bits")
