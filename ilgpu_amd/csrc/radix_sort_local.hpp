@@ -374,6 +374,7 @@ __global__ __launch_bounds__(LocalBlock::kBlock, 4) void local_sort_kernel(
   constexpr uint32_t kWindow = (uint32_t)local_window(KEY_BYTES, VALUE_BYTES);
   static_assert(kWindow <= 65536, "places are packed two to a register");
   static_assert(kItems % kPack == 0 && kItems % 2 == 0, "a thread's keys are whole vectors");
+  static_assert(kItems <= 64, "a bit for every place of a thread");
   __shared__ LocalLds lds;
 
   const int below = 8 * (int)plan->local_from;
@@ -629,8 +630,7 @@ __global__ __launch_bounds__(LocalBlock::kBlock, 4) void local_sort_kernel(
       }
       __syncthreads();
       listed = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds.listed);
-      crowded = listed > (uint32_t)LocalBlock::kList;
-      if (!crowded) {
+      {
         const uint32_t t = opaque();
         auto stage_group = [&](auto full, int j0) {
 #pragma unroll
@@ -671,33 +671,96 @@ __global__ __launch_bounds__(LocalBlock::kBlock, 4) void local_sort_kernel(
     {
       {
         __syncthreads();
-        // Bins of two keys or more.
-        for (uint32_t e = tid; e < listed; e += kBlock) {
-          const uint32_t at = lds.list[e];
-          const K k0 = s_keys[at], k1 = s_keys[at + 1];
-          uint32_t f0 = 0, f1 = 0;
-          if constexpr (kPairs) {
-            f0 = s_from[at];
-            f1 = s_from[at + 1];
+        // Bins of two keys or more.  Where the list has run over (from some half a copy of every key on) those with a
+        // key in front of a smaller one (equal keys: of an earlier one): at the first such place of a bin, and
+        // all of them are found before any key moves.
+        const bool all_listed = listed <= (uint32_t)LocalBlock::kList;
+        uint32_t next = tid;
+        uint64_t found = 0;  // bit j: place_of(j)
+        auto place_of = [&](uint32_t j) -> uint32_t {  // a thread looks at packs of neighbours, as it writes them
+          return j / kPack * (kBlock * kPack) + (uint32_t)tid * kPack + j % kPack;
+        };
+        if (!all_listed) {
+          auto inverted = [&](K k0, K k1, uint32_t f0, uint32_t f1) -> bool {  // neighbours
+            return ordered(k1) < ordered(k0) || (kPairs && k1 == k0 && f1 < f0);
+          };
+          next = listed;
+#pragma unroll 1
+          for (int j = 0; j < kItems && j * kBlock < (int)count; j += kPack) {
+            const uint32_t at = place_of(j);
+            K k[kPack + 1];
+            uint32_t f[kPack + 1];
+#pragma unroll
+            for (int e = 0; e <= kPack; ++e) {
+              const uint32_t from = e < kPack || at + kPack < kWindow ? at + e : at;
+              k[e] = s_keys[from];
+              f[e] = 0;
+              if constexpr (kPairs) f[e] = s_from[from];
+            }
+#pragma unroll
+            for (int e = 0; e < kPack; ++e)
+              if (at + e + 1 < count && inverted(k[e], k[e + 1], f[e], f[e + 1])) found |= 1ull << (j + e);
           }
-          const uint32_t bin = bin_of(k0);
-          bool swap = ordered(k1) < ordered(k0);
-          if constexpr (kPairs) swap = swap || (k1 == k0 && f1 < f0);
-          if (swap) {
-            s_keys[at] = k1;
-            s_keys[at + 1] = k0;
-            if constexpr (kPairs) {
-              s_from[at] = (uint16_t)f1;
-              s_from[at + 1] = (uint16_t)f0;
+          for (uint64_t left = found; left != 0; left &= left - 1) {
+            const uint32_t j = (uint32_t)__builtin_ctzll(left);
+            const uint32_t at = place_of(j);
+            K k = s_keys[at];
+            const uint32_t bin = bin_of(k);
+            for (uint32_t p = at; p > 0; --p) {
+              const K in_front = s_keys[p - 1];
+              if (bin_of(in_front) != bin) break;
+              uint32_t f0 = 0, f1 = 0;
+              if constexpr (kPairs) {
+                f0 = s_from[p - 1];
+                f1 = s_from[p];
+              }
+              if (inverted(in_front, k, f0, f1)) {
+                found &= ~(1ull << j);
+                break;
+              }
+              k = in_front;
             }
           }
-          for (uint32_t i = at + 2; i < count; ++i) {  // insertion, for the few that hold three or more
+          __syncthreads();
+        }
+        while (next < listed || found != 0) {
+          uint32_t at;
+          if (all_listed) {
+            at = lds.list[next];
+            next += kBlock;
+          } else {
+            at = place_of((uint32_t)__builtin_ctzll(found));
+            found &= found - 1;
+          }
+          const K k0 = s_keys[at], k1 = s_keys[at + 1];
+          const uint32_t bin = bin_of(k0);
+          uint32_t behind_at = 1;
+          if (all_listed) {
+            uint32_t f0 = 0, f1 = 0;
+            if constexpr (kPairs) {
+              f0 = s_from[at];
+              f1 = s_from[at + 1];
+            }
+            bool swap = ordered(k1) < ordered(k0);
+            if constexpr (kPairs) swap = swap || (k1 == k0 && f1 < f0);
+            if (swap) {
+              s_keys[at] = k1;
+              s_keys[at + 1] = k0;
+              if constexpr (kPairs) {
+                s_from[at] = (uint16_t)f1;
+                s_from[at + 1] = (uint16_t)f0;
+              }
+            }
+            behind_at = 2;
+          }
+          // Insertion, for the few that hold three or more.  (It ends at the keys of the bin before, which are smaller.)
+          for (uint32_t i = at + behind_at; i < count; ++i) {
             const K k = s_keys[i];
             if (bin_of(k) != bin) break;
             uint32_t f = 0;
             if constexpr (kPairs) f = s_from[i];
             uint32_t to = i;
-            while (to > at) {
+            while (to > 0) {
               const K p = s_keys[to - 1];
               bool behind = ordered(p) > ordered(k);
               if constexpr (kPairs) behind = behind || (p == k && s_from[to - 1] > f);

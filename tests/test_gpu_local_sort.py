@@ -277,6 +277,56 @@ def test_two_refused_sorts_on_two_streams():
         assert np.array_equal(d_b[i].numpy(), b[order]) and np.array_equal(d_v[i].numpy(), order)
 
 
+@pytest.mark.parametrize("dtype,value_dtype,share", [
+    (np.uint32, None, 0.6), (np.int32, None, 0.4), (np.float32, None, 0.6), (np.uint32, np.uint32, 0.6),
+    (np.int32, np.uint64, 0.65), (np.float32, np.uint16, 0.65), (np.uint64, None, 0.9), (np.float64, None, 0.95)])
+def test_windows_with_more_shared_bins_than_the_list_holds(dtype, value_dtype, share):
+    """Full windows, in which a share of the keys comes twice: copies, and neighbours that differ in the last bit."""
+    size = np.dtype(dtype).itemsize
+    n = 240 * WINDOWS[size, value_dtype is not None]
+    rng = np.random.default_rng(size)
+    for descending in (False, True):
+        for twin in (0, 1):
+            note("shared bins", np.dtype(dtype).name, value_dtype, descending, twin)
+            bits = random_bits(n, 8 * size, 81)
+            twice = int(share * n) // 2
+            bits[twice:2 * twice] = bits[:twice] ^ bits.dtype.type(twin)
+            bits = bits[rng.permutation(n)]
+            assert check(bits, dtype, value_dtype, descending, total_order=True, from_index=twin == 0) == 1
+
+
+def test_few_copies_of_every_value_take_little_longer_than_none():
+    """2^26 keys, each value one time and a half on average: all windows were sorted by digits, in twice the time."""
+    import torch
+    n = 1 << 26
+    generator = torch.Generator(device="cuda:0")
+    generator.manual_seed(91)
+    few = torch.randint(-(1 << 31), 1 << 31, (2 * n // 3,), generator=generator, device="cuda:0").to(torch.int32)
+    copies = few[torch.randint(0, few.numel(), (n,), generator=generator, device="cuda:0")]
+    uniform = torch.randint(-(1 << 31), 1 << 31, (n,), generator=generator, device="cuda:0").to(torch.int32)
+    temp = capi.temp_buffer(capi.radix_sort_temp_bytes(n, np.int32))
+    keys = D(n, np.int32)
+
+    def us(column):
+        source = D(n, np.int32, _bytes=column.view(torch.uint8))
+        times = []
+        for _ in range(9):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            capi.transform(source, keys)
+            capi.radix_sort_keys(keys, temp)
+            end.record()
+            sync()
+            times.append(start.elapsed_time(end) * 1000)
+        return sorted(times)[4]
+
+    us(uniform)
+    base, some = us(uniform), us(copies)
+    note("copies", base, some)
+    assert torch.equal(keys.bytes.view(torch.int32), torch.sort(copies).values)
+    assert some < 1.5 * base
+
+
 def test_digits_that_all_keys_share_do_not_hide_the_topmost():
     """8-byte keys of 40 bits, and of 24 (no two digits to save)."""
     note("forty bits")
