@@ -386,7 +386,9 @@ struct TieSampling {
 //   four for every key, send a window the slow way.  Of draws that agree down to a bin (in
 //   log2(n) + 1 bits from the topmost one that differs) there are some m^2 / 4n if
 //   the keys spread evenly and k m^2 / 2n if each bin in use holds k of them; up to 1.25 m^2 / n
-//   are taken (k = 2.5; from k = 5 on a window in nine has such a bin).
+//   are taken (k = 2.5; from k = 5 on a window in nine has such a bin).  Of 4-byte keys after two digits
+//   0.9 m^2 / n: there, bins that have to be put into order cost as much as is saved from k = 1 on (with a copy in front, us,
+//   every digit / the local sort, k = 1, 2, 3: 2^26 keys 656 / 665 / 775 / 840, pairs 1112 / 1083 / 1253 / 1383).
 //   Two digits make runs that fit a window if few draws share a 16-bit prefix: a run of L keys
 //   is drawn L m / n times and gives half the square of that in pairs of draws.
 //   (Whether one digit does, its counts tell exactly.)
@@ -474,13 +476,21 @@ __device__ __forceinline__ void choose_local_digits(const LocalSampling& local, 
   };
 
   // Draws that meet an earlier one, in a table of open addressing: of many draws those of one part
-  // of the values, which half fill it.  (Single frequent values are mostly in another part: those the draws of one
+  // of the values at a time, which half fill it, and of some parts.  (Single frequent values are mostly in another part: those the draws of one
   // prefix tell.)
-  const int parts_log2 = (int)limits.draw_bits > kTableBits - 1 ? (int)limits.draw_bits - (kTableBits - 1) : 0;
+  static_assert(kTableBits == kLocalPartBits + 1, "draws of a part half fill the table");
   constexpr uint32_t kSlots = 1u << kTableBits;
+  const uint32_t part_mask = (uint32_t)local_parts((int)limits.draw_bits) - 1u;
   uint32_t equal = 0;
-  for (int chunk = 0; chunk < chunks; ++chunk) {
+  for (int turn = 0; turn < chunks * (int)limits.parts; ++turn) {
+    const int chunk = turn & (chunks - 1);
+    const uint32_t part = (uint32_t)(turn / chunks);
     if (chunks > 1) load(chunk);
+    if (chunk == 0 && part != 0u) {
+      __syncthreads();
+      clear_table();
+      __syncthreads();
+    }
 #pragma unroll
     for (int v = 0; v < kVectors; ++v) {
       if (!in_use(chunk, v)) continue;
@@ -492,7 +502,7 @@ __device__ __forceinline__ void choose_local_digits(const LocalSampling& local, 
         hash = (hash ^ hash >> 16) * 0x85EBCA6Bu;
         slot[u] = hash >> (32 - kTableBits);
         old[u] = 0u;
-        if ((hash & ((1u << parts_log2) - 1u)) == 0u) old[u] = atomicCAS(&s_table[slot[u]], 0u, value[u] + 1u);
+        if ((hash & part_mask) == part) old[u] = atomicCAS(&s_table[slot[u]], 0u, value[u] + 1u);
       }
 #pragma unroll
       for (int u = 0; u < kPerVector; ++u) {
@@ -508,7 +518,7 @@ __device__ __forceinline__ void choose_local_digits(const LocalSampling& local, 
   for (int s = 1; s < kWaveSize; s <<= 1) equal += shfl(equal, (t & (kWaveSize - 1)) ^ s);
   if ((t & (kWaveSize - 1)) == 0) atomicAdd(&s_equal, equal);
   __syncthreads();
-  if (s_equal > limits.max_equal >> parts_log2) return;
+  if (s_equal > limits.max_equal) return;
   if (t == 0) local.from[1] = 1u;
   if (limits.max_pairs == 0u) return;  // one digit is enough
 

@@ -57,9 +57,18 @@ inline int64_t local_deferred_bytes(int64_t n, int64_t blocks, uint32_t window) 
 // sort_draw_kernel, choose_local_digits).
 constexpr int kLocalMinDrawBits = 12, kLocalMaxDrawBits = 16;
 constexpr int kLocalChunkBits = 14;   // draws that the block that looks at them holds at a time
+constexpr int kLocalPartBits = 13;    // draws of one part of the values
 constexpr int kLocalPrefixBits = 15;  // draws whose prefixes are counted
 constexpr int local_draw_bits(int64_t n) {
   return n <= 1ll << 21 ? kLocalMinDrawBits : (n <= 1ll << 23 ? 13 : (n <= 1ll << 25 ? 14 : kLocalMaxDrawBits));
+}
+// Parts of the values, and those whose draws are asked whether they meet: as many as the block has time for while
+// others count the keys, some 37 us each with 2^16 draws.  (All four of 2^27 + 1 u32 keys 1063 -> 1129 us, both
+// of 10^7 150 -> 162, one of 2^28 takes a column of six copies of every value one time in nine.)
+constexpr int local_parts(int draw_bits) { return draw_bits > kLocalPartBits ? 1 << (draw_bits - kLocalPartBits) : 1; }
+constexpr int local_parts_asked(int64_t n, int draw_bits) {
+  const int64_t parts = n >> 26 < 1 ? 1 : n >> 26;
+  return parts < local_parts(draw_bits) ? (int)parts : local_parts(draw_bits);
 }
 // A random place in part s of 2^bits.
 ILGPU_HIP_RULE inline uint64_t local_draw_place(uint64_t s, int bits, uint64_t n) {
@@ -82,7 +91,8 @@ ILGPU_HIP_RULE constexpr uint32_t local_draw_slot(uint32_t s, int bits) {
 struct LocalLimits {
   uint32_t draw_bits;  // log2 of the number of draws
   uint32_t bin_bits;   // of a draw, from the topmost bit that differs on
-  uint32_t max_equal;  // draws that meet an earlier one in these bits
+  uint32_t parts;      // of the values, that are asked
+  uint32_t max_equal;  // draws of these that meet an earlier one in these bits
   uint32_t max_pairs;  // pairs of draws that share a 16-bit prefix (0: one digit makes runs that may fit a window,
                        // which its counts tell)
   uint32_t max_draws;  // of one prefix
@@ -94,8 +104,12 @@ inline LocalLimits local_limits(int64_t keys, int key_bytes, int value_bytes) {
   limits.draw_bits = (uint32_t)local_draw_bits(keys);
   const double draws = (double)(1ll << limits.draw_bits), n = (double)keys;
   while (limits.bin_bits < 31 && keys >> limits.bin_bits != 0) ++limits.bin_bits;  // log2(n) + 1
-  limits.max_equal = (uint32_t)(1.25 * draws * draws / n) + 6u;
-  if (keys <= window * 256 * 15 / 16) {
+  const int parts = local_parts((int)limits.draw_bits);
+  limits.parts = (uint32_t)local_parts_asked(keys, (int)limits.draw_bits);
+  const bool one_digit = keys <= window * 256 * 15 / 16;
+  const double most_equal = (key_bytes == 4 && !one_digit ? 0.9 : 1.25) * draws * draws / n;
+  limits.max_equal = ((uint32_t)most_equal + 6u) * limits.parts / (uint32_t)parts;
+  if (one_digit) {
     limits.max_run = (uint32_t)window;
   } else {
     // Runs of 0.6 windows, as the mean over the keys.

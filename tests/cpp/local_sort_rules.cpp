@@ -25,11 +25,12 @@ int32_t rule_draws(int64_t n, uint64_t* places, uint32_t* slots) {
 }
 int32_t rule_chunk_draws() { return 1 << kLocalChunkBits; }
 int32_t rule_prefix_draws() { return 1 << kLocalPrefixBits; }
+int32_t rule_parts(int32_t draw_bits) { return local_parts(draw_bits); }
 void rule_limits(int64_t n, int32_t key_bytes, int32_t value_bytes, uint32_t* out) {
   const LocalLimits limits = local_limits(n, key_bytes, value_bytes);
-  const uint32_t all[] = {limits.draw_bits, limits.bin_bits,  limits.max_equal,
+  const uint32_t all[] = {limits.draw_bits, limits.bin_bits,  limits.parts,  limits.max_equal,
                           limits.max_pairs, limits.max_draws, limits.max_run};
-  for (int i = 0; i < 6; ++i) out[i] = all[i];
+  for (int i = 0; i < 7; ++i) out[i] = all[i];
 }
 
 int32_t rule_counts_allow(uint32_t n, uint32_t most_upper, uint32_t most_lower, uint32_t window) {

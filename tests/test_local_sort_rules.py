@@ -34,7 +34,7 @@ def rules(tmp_path_factory):
 
 class Limits(ctypes.Structure):
     _fields_ = [(name, ctypes.c_uint32) for name in
-                ("draw_bits", "bin_bits", "max_equal", "max_pairs", "max_draws", "max_run")]
+                ("draw_bits", "bin_bits", "parts", "max_equal", "max_pairs", "max_draws", "max_run")]
 
 
 def draws_of(rules, n):
@@ -155,6 +155,36 @@ def test_columns_whose_parts_differ_are_refused_by_the_draws(rules, n, key_bytes
             def padded(places):
                 return np.where((places >= int(first * n)) & (places < int(last * n)), kind(value), uniform(places))
             assert not two_digits_are_enough(rules, n, key_bytes, value_bytes, padded), (value, first, last)
+
+
+@pytest.mark.parametrize("n", [18_433, 300_000, 2_000_000, 3_000_000, 10_000_019, 1 << 25, 1 << 26, 1 << 28])
+@pytest.mark.parametrize("key_bytes", [4, 8])
+def test_columns_of_many_copies_are_refused_by_the_draws(rules, n, key_bytes):
+    """Of the draws of the parts of the values that are asked, those that meet an earlier one in
+    their bin, for 20 columns of each kind: different keys are taken, and from eight copies of every value on, when
+    most windows have a bin of sixteen keys, they are not."""
+    limits = Limits()
+    rules.rule_limits(n, key_bytes, 0, ctypes.addressof(limits))
+    kind = np.dtype(f"uint{8 * key_bytes}").type
+    bins = kind(8 * key_bytes - limits.bin_bits)
+    share = limits.parts / rules.rule_parts(limits.draw_bits)
+    rng = np.random.default_rng(n)
+
+    def mixed(x):  # a random number for each
+        x = (x + np.uint64(1)) * np.uint64(0x9E3779B97F4A7C15)
+        x = (x ^ x >> np.uint64(30)) * np.uint64(0xBF58476D1CE4E5B9)
+        return x ^ x >> np.uint64(29)
+
+    taken = {0: 0, 8: 0}
+    for copies in taken:
+        for _ in range(20):
+            m = 1 << limits.draw_bits
+            values = n // copies if copies else 1 << 63
+            keys = mixed(rng.integers(0, values, m, dtype=np.uint64)) >> np.uint64(64 - 8 * key_bytes)
+            in_bins = keys.astype(kind) >> bins
+            asked = in_bins[(mixed(in_bins.astype(np.uint64)) >> np.uint64(40)) < share * (1 << 24)]
+            taken[copies] += asked.size - np.unique(asked).size <= limits.max_equal
+    assert taken[0] >= 19 and taken[8] <= 1
 
 
 @pytest.mark.parametrize("key_bytes,value_bytes", KINDS)
