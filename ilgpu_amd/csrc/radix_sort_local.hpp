@@ -25,6 +25,10 @@
 // 238 / 193, 2^20 71.5 / 52.0; u64 keys with index values 2^27 3572 / 2723, where four passes and the ties
 // came before; 300 000 u64 keys with values 120 / 54.)
 //
+// Values that come half a time or more each on average share more bins than the list of them holds in a full window: there
+// every thread looks at its places for keys in the wrong order instead.  (u32 keys with a copy in front, us, every digit / such
+// windows by digits / this: 2^28 keys, each value once on average, 2365 / 4525 / 2385, 2^26 656 / 1129 / 665, 2 000 000 92 / 116 / 86.)
+//
 // Windows whose keys crowd a bin with sixteen or more (many copies of a key,
 // keys clustered within a run) are sorted digit by digit in LDS, like a tile of
 // the sort; a run longer than a window digit by digit through memory, by its

@@ -25,7 +25,7 @@ struct LocalBlock {
   // 16-byte accesses over all banks.
   static constexpr int kRowWords = kBins / 4 / kBlock;
   static constexpr int kRowStride = kRowWords + 4;
-  static constexpr int kList = 1984;  // bins of two keys or more that a window may have (some 1070 in a full one)
+  static constexpr int kList = 1984;  // bins of two keys or more that a window lists (some 1070 in a full one of random keys)
 };
 static_assert(LocalBlock::kBlock * LocalBlock::kRowStride * 4 == LocalBlock::kStageBytes, "the counts fill the stage");
 // Pairs keep the place a key came from next to it.
@@ -112,7 +112,10 @@ inline LocalLimits local_limits(int64_t keys, int key_bytes, int value_bytes) {
   if (one_digit) {
     limits.max_run = (uint32_t)window;
   } else {
-    // Runs of 0.6 windows, as the mean over the keys.
+    // Runs of 0.6 windows, as the mean over the keys.  (With 0.95, with a copy in front, us, every digit / the local sort: 2^29
+    // u32 keys 4556 / 3968, but two copies of every value, which 2^16 draws hardly show at that length, 4560 / 8571; 450 * 2^20
+    // 4011 / 3531 and 4008 / 7755; u32 pairs of 300 * 2^20 5043 / 4076, two copies of 260 * 2^20 4367 / 4419.  Those were
+    // windows whose list ran over going the slow way.)
     const double looked_at = std::fmin(draws, (double)(1ll << kLocalPrefixBits));
     limits.max_pairs = (uint32_t)(looked_at * looked_at * 0.5 * (0.6 * (double)window / n)) + 1u;
     const double of_window = looked_at * (double)window / n;
