@@ -679,16 +679,14 @@ __global__ __launch_bounds__(LocalBlock::kBlock, 4) void local_sort_kernel(
         // key in front of a smaller one (equal keys: of an earlier one): at the first such place of a bin, and
         // all of them are found before any key moves.
         const bool all_listed = listed <= (uint32_t)LocalBlock::kList;
-        uint32_t next = tid;
         uint64_t found = 0;  // bit j: place_of(j)
         auto place_of = [&](uint32_t j) -> uint32_t {  // a thread looks at packs of neighbours, as it writes them
           return j / kPack * (kBlock * kPack) + (uint32_t)tid * kPack + j % kPack;
         };
-        if (!all_listed) {
+        if (__builtin_expect(!all_listed, 0)) {
           auto inverted = [&](K k0, K k1, uint32_t f0, uint32_t f1) -> bool {  // neighbours
             return ordered(k1) < ordered(k0) || (kPairs && k1 == k0 && f1 < f0);
           };
-          next = listed;
 #pragma unroll 1
           for (int j = 0; j < kItems && j * kBlock < (int)count; j += kPack) {
             const uint32_t at = place_of(j);
@@ -727,38 +725,10 @@ __global__ __launch_bounds__(LocalBlock::kBlock, 4) void local_sort_kernel(
           }
           __syncthreads();
         }
-        while (next < listed || found != 0) {
-          uint32_t at;
-          if (all_listed) {
-            at = lds.list[next];
-            next += kBlock;
-          } else {
-            at = place_of((uint32_t)__builtin_ctzll(found));
-            found &= found - 1;
-          }
-          const K k0 = s_keys[at], k1 = s_keys[at + 1];
-          const uint32_t bin = bin_of(k0);
-          uint32_t behind_at = 1;
-          if (all_listed) {
-            uint32_t f0 = 0, f1 = 0;
-            if constexpr (kPairs) {
-              f0 = s_from[at];
-              f1 = s_from[at + 1];
-            }
-            bool swap = ordered(k1) < ordered(k0);
-            if constexpr (kPairs) swap = swap || (k1 == k0 && f1 < f0);
-            if (swap) {
-              s_keys[at] = k1;
-              s_keys[at + 1] = k0;
-              if constexpr (kPairs) {
-                s_from[at] = (uint16_t)f1;
-                s_from[at + 1] = (uint16_t)f0;
-              }
-            }
-            behind_at = 2;
-          }
-          // Insertion, for the few that hold three or more.  (It ends at the keys of the bin before, which are smaller.)
-          for (uint32_t i = at + behind_at; i < count; ++i) {
+        // Insertion from place i on, for the few that hold three or more.  (It ends at the keys of the bin before, which
+        // are smaller.)
+        auto insert_from = [&](uint32_t i, uint32_t bin) {
+          for (; i < count; ++i) {
             const K k = s_keys[i];
             if (bin_of(k) != bin) break;
             uint32_t f = 0;
@@ -777,6 +747,35 @@ __global__ __launch_bounds__(LocalBlock::kBlock, 4) void local_sort_kernel(
               s_keys[to] = k;
               if constexpr (kPairs) s_from[to] = (uint16_t)f;
             }
+          }
+        };
+        if (__builtin_expect(!all_listed, 0)) {
+          while (found != 0) {
+            const uint32_t at = place_of((uint32_t)__builtin_ctzll(found));
+            found &= found - 1;
+            insert_from(at + 1, bin_of(s_keys[at]));
+          }
+        } else {
+          for (uint32_t e = tid; e < listed; e += kBlock) {
+            const uint32_t at = lds.list[e];
+            const K k0 = s_keys[at], k1 = s_keys[at + 1];
+            uint32_t f0 = 0, f1 = 0;
+            if constexpr (kPairs) {
+              f0 = s_from[at];
+              f1 = s_from[at + 1];
+            }
+            const uint32_t bin = bin_of(k0);
+            bool swap = ordered(k1) < ordered(k0);
+            if constexpr (kPairs) swap = swap || (k1 == k0 && f1 < f0);
+            if (swap) {
+              s_keys[at] = k1;
+              s_keys[at + 1] = k0;
+              if constexpr (kPairs) {
+                s_from[at] = (uint16_t)f1;
+                s_from[at + 1] = (uint16_t)f0;
+              }
+            }
+            insert_from(at + 2, bin);
           }
         }
         __syncthreads();
