@@ -296,35 +296,36 @@ def test_windows_with_more_shared_bins_than_the_list_holds(dtype, value_dtype, s
 
 
 def test_few_copies_of_every_value_take_little_longer_than_none():
-    """2^26 keys, each value one time and a half on average: all windows were sorted by digits, in twice the time."""
+    """2 000 000 keys, each value once on average: all windows were sorted by digits, in 1.6 times the time."""
     import torch
-    n = 1 << 26
+    n = 2_000_000
     generator = torch.Generator(device="cuda:0")
     generator.manual_seed(91)
-    few = torch.randint(-(1 << 31), 1 << 31, (2 * n // 3,), generator=generator, device="cuda:0").to(torch.int32)
-    copies = few[torch.randint(0, few.numel(), (n,), generator=generator, device="cuda:0")]
     uniform = torch.randint(-(1 << 31), 1 << 31, (n,), generator=generator, device="cuda:0").to(torch.int32)
+    copies = uniform[torch.randint(0, n, (n,), generator=generator, device="cuda:0")]
     temp = capi.temp_buffer(capi.radix_sort_temp_bytes(n, np.int32))
     keys = D(n, np.int32)
 
     def us(column):
         source = D(n, np.int32, _bytes=column.view(torch.uint8))
         times = []
-        for _ in range(9):
+        for _ in range(15):
             start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
             start.record()
-            capi.transform(source, keys)
-            capi.radix_sort_keys(keys, temp)
+            for _ in range(20):
+                capi.transform(source, keys)
+                capi.radix_sort_keys(keys, temp)
             end.record()
             sync()
-            times.append(start.elapsed_time(end) * 1000)
-        return sorted(times)[4]
+            times.append(start.elapsed_time(end) * 50)
+        assert capi.radix_sort_passes(temp, n, np.int32)[0] == 1
+        return sorted(times)[7]
 
     us(uniform)
     base, some = us(uniform), us(copies)
     note("copies", base, some)
     assert torch.equal(keys.bytes.view(torch.int32), torch.sort(copies).values)
-    assert some < 1.5 * base
+    assert some < 1.4 * base
 
 
 def test_digits_that_all_keys_share_do_not_hide_the_topmost():
