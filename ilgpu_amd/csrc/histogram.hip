@@ -32,6 +32,9 @@ constexpr int kUnroll = 2;
 #ifndef ILGPU_HIP_HISTOGRAM_FEW_UNROLL
 #define ILGPU_HIP_HISTOGRAM_FEW_UNROLL 4
 #endif
+#ifndef ILGPU_HIP_HISTOGRAM_FEW_BLOCK
+#define ILGPU_HIP_HISTOGRAM_FEW_BLOCK 1024
+#endif
 constexpr int kFewUnroll = ILGPU_HIP_HISTOGRAM_FEW_UNROLL;  // at most one block per CU
 #ifndef ILGPU_HIP_HISTOGRAM_STRIDED_UNROLL
 #define ILGPU_HIP_HISTOGRAM_STRIDED_UNROLL 4
@@ -190,6 +193,35 @@ __device__ __forceinline__ F add_ones(F x, uint32_t c) {
   return x;
 }
 
+// Whether c ones can be added to a bin that holds x as one c: from a whole number up to
+// 2^24 (2^53) on every step of one is exact until it reaches that, where the bin stays.
+template <typename F>
+__device__ __forceinline__ bool ones_are_exact(F x, uint32_t c) {
+  constexpr F kLimit = (F)(1ull << (sizeof(F) == 4 ? 24 : 53));
+  const F whole = sizeof(F) == 4 ? (F)truncf((float)x) : (F)trunc((double)x);
+  return x == whole && x >= -kLimit && x <= kLimit && (sizeof(F) == 8 || c <= 1u << 24);
+}
+// What follows an addition of c in one to a bin of which ones_are_exact: `before` is what it held. A bin that
+// was taken beyond 2^24 (2^53) is put back to it, the value that the ones would have stopped at.  Whoever
+// adds to such a bin in between finds it beyond as well, or puts it back afterwards, so the last to do so leaves
+// it there.
+template <typename F, typename U>
+__device__ __forceinline__ void settle_fp_bin(F* bin, F before, uint32_t c) {
+  constexpr F kLimit = (F)(1ull << (sizeof(F) == 4 ? 24 : 53));
+  if (before <= kLimit - (F)c) return;
+  U* p = reinterpret_cast<U*>(bin);
+  U limit_bits, old = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __builtin_memcpy(&limit_bits, &kLimit, sizeof(F));
+  while (true) {
+    F x;
+    __builtin_memcpy(&x, &old, sizeof(F));
+    if (x <= kLimit) break;
+    if (__hip_atomic_compare_exchange_strong(p, &old, limit_bits, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT))
+      break;
+  }
+}
+
 // Adds c ones to the floating-point bin b; returns whether an increment found
 // the bin at MaxValue (only a bin that holds MaxValue already: it is not
 // reachable by steps of one).
@@ -236,6 +268,63 @@ __device__ __forceinline__ bool add_to_bin_dyn(int bin_type, void* bins,
   }
 }
 
+// A block's counts, a bin per thread and step, into the bins, which are of type B or, for the unsigned
+// types, of the signed one of that size if `is_signed`; returns whether one of the adds passed MaxValue.  Their answers are asked for kFlushSteps adds
+// at a time: one add after the other, each a round trip to the memory side, the flush of
+// 4096 bins was half of the time of 8 M ints.  Floating-point bins are looked at first: most can
+// take a block's count at once (a compare-and-swap loop per bin, which all blocks try at
+// about the same time: 8 M ints into 4096 float bins 125 us, now 17.6; 2^26 bytes into 256 4238 / 54.6.)
+template <typename B, int BLOCK, int kFlushSteps, typename CountOf>
+__device__ __forceinline__ bool flush_bins(void* bins, int num_bins, int first_bin, bool checked, bool is_signed,
+                                           const CountOf& count_of) {
+  using U = std::conditional_t<sizeof(B) == 4, uint32_t, uint64_t>;
+  U* target = static_cast<U*>(bins);
+  bool passed = false;
+  for (int base = threadIdx.x; base < num_bins; base += kFlushSteps * BLOCK) {
+    uint32_t c[kFlushSteps];
+    U old[kFlushSteps];
+    auto bin_of_step = [&](int s) -> int {
+      const int i = base + s * BLOCK;
+      return i + first_bin < num_bins ? i + first_bin : i + first_bin - num_bins;
+    };
+#pragma unroll
+    for (int s = 0; s < kFlushSteps; ++s) {
+      const int b = bin_of_step(s);
+      c[s] = base + s * BLOCK < num_bins ? count_of(b) : 0u;
+      old[s] = 0;
+      if (c[s] == 0u) continue;
+      if constexpr (is_fp<B>::value)
+        old[s] = __hip_atomic_load(&target[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      else if (checked)
+        old[s] = __hip_atomic_fetch_add(&target[b], (U)c[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      else
+        __hip_atomic_fetch_add(&target[b], (U)c[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if constexpr (is_fp<B>::value) {
+      B before[kFlushSteps];
+#pragma unroll
+      for (int s = 0; s < kFlushSteps; ++s) {
+        if (c[s] == 0u) continue;
+        __builtin_memcpy(&before[s], &old[s], sizeof(B));
+        if (ones_are_exact<B>(before[s], c[s]))
+          before[s] = unsafeAtomicAdd(static_cast<B*>(bins) + bin_of_step(s), (B)c[s]);
+        else
+          passed |= add_to_fp_bin<B, U>(bins, bin_of_step(s), c[s], checked), c[s] = 0u;
+      }
+#pragma unroll
+      for (int s = 0; s < kFlushSteps; ++s)
+        if (c[s] != 0u) settle_fp_bin<B, U>(static_cast<B*>(bins) + bin_of_step(s), before[s], c[s]);
+    } else {
+#pragma unroll
+      for (int s = 0; s < kFlushSteps; ++s)
+        passed |= checked && c[s] != 0u &&
+                  (is_signed ? BinTraits<std::make_signed_t<B>>::passes_max((std::make_signed_t<B>)old[s], c[s])
+                             : BinTraits<B>::passes_max(old[s], c[s]));
+    }
+  }
+  return passed;
+}
+
 // RANGE_CHECK = false when every value of T is a valid bin (e.g. u8 into
 // >= 256 bins with the identity locator).  FORM: the plain loop stands by itself, so that
 // what the others need costs it no registers (2^30 bytes into 256 bins: 3 %).
@@ -245,12 +334,16 @@ enum {
   kFormCrowdedFew,  // the same with at most one block per CU: more loads per thread
   kFormStrided,
 };
+// Threads of a block: where there is at most one per CU, all that it holds (4096 bins, us with 512 / 1024 threads: 2^24
+// ints 18.7 / 17.2, 8 M into int64 bins 17.6 / 15.6).
+constexpr int form_block(int form) { return form == kFormCrowdedFew ? ILGPU_HIP_HISTOGRAM_FEW_BLOCK : kBlock; }
 template <typename T, int LOC, bool RANGE_CHECK, int FORM>
-__global__ __launch_bounds__(kBlock) void histogram_lds_kernel(
+__global__ __launch_bounds__(form_block(FORM)) void histogram_lds_kernel(
     const T* __restrict__ in, int64_t n, int64_t in_stride, void* bins,
     int num_bins, int bin_type, int32_t* overflow, int replica_shift) {
   using V = typename Vec16<T>::type;
   constexpr int VN = Vec16<T>::N;
+  constexpr int kBlock = form_block(FORM);
   extern __shared__ uint32_t s_counts[];
   __shared__ int s_overflow;
 
@@ -369,13 +462,32 @@ __global__ __launch_bounds__(kBlock) void histogram_lds_kernel(
   const int first_bin =
       FORM == kFormPlain ? 0
                          : (int)((uint64_t)blockIdx.x * (uint32_t)num_bins / gridDim.x) & ~(kWaveSize - 1);
-  for (int i = threadIdx.x; i < num_bins; i += kBlock) {
-    const int b = i + first_bin < num_bins ? i + first_bin : i + first_bin - num_bins;
+  auto count_of = [&](int b) -> uint32_t {
     uint32_t c = 0;
     // Rotate the start so that neighbouring bins read different banks.
     for (int r = 0; r < replicas; ++r)
       c += s_counts[(b << replica_shift) + ((r + b) & (replicas - 1))];
-    if (c != 0) passed |= add_to_bin_dyn(bin_type, bins, b, c, checked);
+    return c;
+  };
+  constexpr int kFlushSteps = FORM == kFormPlain ? 1 : 8;
+  auto flush = [&](auto one) {
+    passed = flush_bins<decltype(one), kBlock, kFlushSteps>(
+        bins, num_bins, first_bin, checked, bin_type == ILGPU_HIP_I32 || bin_type == ILGPU_HIP_I64, count_of);
+  };
+  if (FORM == kFormPlain && bin_type != ILGPU_HIP_F32 && bin_type != ILGPU_HIP_F64) {
+    // (Few bins, of which a thread has one to three: steps cost 2 % of 16 MiB of bytes, and their registers a
+    // block per CU of 2^30, 181 -> 250 us.)
+    for (int b = threadIdx.x; b < num_bins; b += kBlock) {
+      const uint32_t c = count_of(b);
+      if (c != 0) passed |= add_to_bin_dyn(bin_type, bins, b, c, checked);
+    }
+  } else {
+    switch (bin_type) {
+      case ILGPU_HIP_I32: case ILGPU_HIP_U32: flush(uint32_t{}); break;
+      case ILGPU_HIP_F32: flush(float{}); break;
+      case ILGPU_HIP_F64: flush(double{}); break;
+      default: flush(uint64_t{}); break;
+    }
   }
   if (checked) {
     if (passed) s_overflow = 1;
@@ -470,7 +582,7 @@ int32_t launch_typed(hipStream_t stream, const void* in, int64_t n,
   auto launch = [&](auto range_check, auto f) {
     hipLaunchKernelGGL(
         (histogram_lds_kernel<T, LOC, decltype(range_check)::value, decltype(f)::value>),
-        dim3((unsigned)blocks), dim3(kBlock), lds_bytes, stream, src, n, in_stride, bins,
+        dim3((unsigned)blocks), dim3(form_block(decltype(f)::value)), lds_bytes, stream, src, n, in_stride, bins,
         (int)num_bins, bin_type, overflow, shift);
   };
   auto launch_form = [&](auto range_check) {

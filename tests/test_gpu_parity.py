@@ -399,6 +399,26 @@ def test_histogram_floating_point_bins_take_their_ones_in_bin_precision(bin_dtyp
     assert bits_equal(got, want) and ov == want_ov == 0
 
 
+@pytest.mark.parametrize("bin_dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("bins", [256, 4096, 5000])
+def test_histogram_floating_point_bins_that_many_blocks_add_to(bin_dtype, bins):
+    # A block adds its count to a bin in one where the bin holds a whole number up to 2^24 (2^53), and a
+    # bin that is taken beyond is put back; others are added to one by one.  Every bin gets some 30 to 600 ones
+    # of many blocks: from below, at and above the bound, from fractions and from what is not finite.
+    limit = 2.0 ** (24 if bin_dtype == np.float32 else 53)
+    starts = np.array([0.0, 7.0, limit - 700, limit - 20, limit - 1, limit, limit + 2, limit + 4, -5.0, -limit,
+                       -limit - 2, 0.5, -2.25, limit / 2 - 3, 1e20, np.inf, -np.inf, np.finfo(bin_dtype).max,
+                       -0.0], dtype=bin_dtype)
+    before = np.resize(starts, bins)
+    values = np.random.default_rng(bins).integers(0, bins, 150_000).astype(np.int32)
+    for checked in (True, False):
+        note("histogram fp bins", np.dtype(bin_dtype).name, bins, checked)
+        got, overflow = gpu_histogram(values, before.copy(), capi.LOCATOR_IDENTITY, checked=checked)
+        want, want_overflow = O.histogram(values, before.copy())
+        assert bits_equal(got, want)
+        assert overflow == (want_overflow if checked else 0)
+
+
 # --------------------------------------------------------------- radix sort
 def gpu_sort(keys, **kw):
     d = D.from_numpy(keys)
