@@ -52,6 +52,9 @@ int64_t radix_sort_max_length();
 int32_t launch_radix_sort(hipStream_t stream, const SortArgs& args);
 // ILGPU_HIP_SORT_PARAM_* (validated by the caller); negative = default.
 void set_sort_parameter(int32_t parameter, int32_t value);
+// Polls of an empty status word before a look-back (of a pass, of a scan without tickets) counts or
+// folds the tile itself.
+uint32_t lookback_spin_limit();
 // Device check of the LDS behaviour the sort's ranking relies on: lanes of one
 // returning LDS atomic that share an address are served in lane order.
 // mismatches[0] (device) receives the number of lanes found out of order.

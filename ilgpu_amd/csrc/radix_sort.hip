@@ -144,6 +144,8 @@ void set_sort_parameter(int32_t parameter, int32_t value) {
     g_sort_small_kernel.store(value == 0 ? 0 : 1, std::memory_order_relaxed);
 }
 
+uint32_t lookback_spin_limit() { return g_sort_spin_limit.load(std::memory_order_relaxed); }
+
 int32_t launch_lds_atomic_order_selftest(hipStream_t stream, int rows, int64_t* mismatches) {
   int32_t rc = launch_zero_words(stream, reinterpret_cast<uint32_t*>(mismatches), 2);
   if (rc != ILGPU_HIP_SUCCESS) return rc;

@@ -17,8 +17,13 @@
 //   (j, lane, element): each lane scans its vector, the wave scans the vector
 //   totals once per j, and the running totals of earlier j are folded in.
 //
-// Tile ids come from a global ticket, so a tile's predecessors have always
-// started.  Status words are read and written with agent-scope atomics: the
+// Block b takes tile b.  Blocks start in index order in practice, but nothing promises that a tile's
+// predecessors run, so nobody waits without bound: after as many polls as a pass of the sort makes a
+// missing tile is folded from the input (resolve_prefix).  Where the output overlaps the input, which may be
+// overwritten by then, tile ids come from a global ticket instead, and a tile's predecessors have always
+// started; a ticket costs a tile a round trip before its loads and 12 to 18 ns behind the ticket before
+// (calls, us, with tickets / without: 2^23 int64 31.5 / 23.5, 2^22 17.6 / 14.8, 2^23 int32 17.5 / 14.6,
+// 10^6 double Max 14.0 / 11.2, 2^28 int32 361 / 357.5).  Status words are read and written with agent-scope atomics: the
 // eight XCDs of the device have separate L2s.
 //   4-byte T: one 64-bit word {flag, value} per tile;
 //   8-byte T: two such words per tile, one per half of the value.
@@ -81,6 +86,7 @@ constexpr int kVecs = ILGPU_HIP_SCAN_VECS;
 template <typename T> constexpr int scan_vecs() {
   return sizeof(T) == 8 ? ILGPU_HIP_SCAN_VECS8 : kVecs;
 }
+constexpr uint32_t kNoLimit = ~0u;  // of polls
 constexpr uint32_t kFlagInvalid = 0, kFlagAggregate = 1, kFlagPrefix = 2;
 constexpr int64_t kHeaderBytes = 256;  // ticket counter, padded
 
@@ -89,21 +95,23 @@ template <typename T> constexpr int tile_elems() {
 }
 // Short tiles, a quarter as long: an input of a few dozen full tiles leaves most
 // compute units idle, and the scan lasts as long as one tile takes from its
-// loads to its stores.  Inputs of two to kShortMaxTiles full tiles take them.
+// loads to its stores.  Inputs of two to kShortMaxTiles full tiles take them, or to
+// kShortMaxTilesTicketed where the tiles are handed out by tickets, one after the other (12 to 18 ns each).
 // Their status words stand a quarter of a line apart, so that they fit the
 // temp view of the full tiles; that few words are not what such an input waits for.
-// (Kernel time in us, full / short tiles: 130 000 int32 18.0 / 6.8, 500 000 12.2 / 5.4, 10^6
-// 13.2 / 6.4, 1.9 * 10^6 float 18.2 / 9.9; 130 000 int64 9.8 / 5.5, 500 000 10.0 / 7.0, 10^6 the same.
-// From 128 full tiles on the longer chain costs more than the shorter tiles
-// save: a call on 2^21 int64 takes 14.3 / 17.5, on 2^22 18.0 / 30.0.)
+// (Calls, us, tickets and a walk / no tickets and full tiles / short ones: 2.5 * 10^6 double Max 27.6 / 27.3 / 17.7,
+// 3.5 * 10^6 29.6 / 28.4 / 23.8, 2.5 * 10^6 int32 14.4 / 9.6 / 9.6, 6.3 * 10^6 14.6 / 13.8 / 11.7, 2^21 int64 13.0 / 12.4 /
+// 10.5, 3 * 10^6 14.7 / 13.7 / 12.6, but 3.5 * 10^6, 214 full tiles, 15.5 / 14.0 / 15.1 and 2^22 17.7 / 14.8 / 18.0.
+// Tiles an eighth as long: 10^6 double Max 12.3 against 11.1, 2^21 int64 16.1 against 10.6.)
 #ifndef ILGPU_HIP_SCAN_SHORT_DIVISOR
 #define ILGPU_HIP_SCAN_SHORT_DIVISOR 4
 #endif
 #ifndef ILGPU_HIP_SCAN_SHORT_MAX_TILES
-#define ILGPU_HIP_SCAN_SHORT_MAX_TILES 64
+#define ILGPU_HIP_SCAN_SHORT_MAX_TILES 192
 #endif
 constexpr int kShortDivisor = ILGPU_HIP_SCAN_SHORT_DIVISOR;
 constexpr int64_t kShortMaxTiles = ILGPU_HIP_SCAN_SHORT_MAX_TILES;
+constexpr int64_t kShortMaxTilesTicketed = 64;
 static_assert(kStatusStride / kShortDivisor >= 2, "two status words per tile of 8-byte elements");
 // Status words per tile of VECS vectors per thread.
 template <typename T, int VECS> constexpr int status_stride() {
@@ -143,13 +151,16 @@ template <typename T, int STRIDE> struct TileState<T, STRIDE, 4> {
     __hip_atomic_store(&words[(int64_t)tile * STRIDE], w, __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
   }
-  // Spins until the tile has published something; returns its flag.
-  __device__ __forceinline__ uint32_t wait(int tile, T* v) const {
+  // Spins until the tile has published something; returns its flag, or kFlagInvalid
+  // after `limit` polls.
+  __device__ __forceinline__ uint32_t wait(int tile, T* v, uint32_t limit = kNoLimit) const {
     uint64_t w;
+    uint32_t polls = 0;
     while (true) {
       w = __hip_atomic_load(&words[(int64_t)tile * STRIDE], __ATOMIC_RELAXED,
                             __HIP_MEMORY_SCOPE_AGENT);
       if ((uint32_t)(w >> 32) != kFlagInvalid) break;
+      if (limit != kNoLimit && polls++ >= limit) return kFlagInvalid;
       __builtin_amdgcn_s_sleep(1);
     }
     *v = from_bits<T>((uint32_t)w);
@@ -173,13 +184,15 @@ template <typename T, int STRIDE> struct TileState<T, STRIDE, 8> {
     __hip_atomic_store(&w[1], ((uint64_t)flag << 32) | (bits >> 32),
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  __device__ __forceinline__ uint32_t wait(int tile, T* v) const {
+  __device__ __forceinline__ uint32_t wait(int tile, T* v, uint32_t limit = kNoLimit) const {
     uint64_t lo, hi;
+    uint32_t polls = 0;
     const uint64_t* w = &words[(int64_t)tile * STRIDE];
     while (true) {
       lo = __hip_atomic_load(&w[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       hi = __hip_atomic_load(&w[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if ((uint32_t)(lo >> 32) != kFlagInvalid && (lo >> 32) == (hi >> 32)) break;
+      if (limit != kNoLimit && polls++ >= limit) return kFlagInvalid;
       __builtin_amdgcn_s_sleep(1);
     }
     *v = from_bits<T>((uint64_t)(uint32_t)lo | (hi << 32));
@@ -275,9 +288,11 @@ __device__ __forceinline__ T wave_reduce(T v) {
 
 // Executed by the first wave of the block.  Publishes the tile's aggregate,
 // resolves the exclusive prefix of the tile and publishes the inclusive one.
-template <typename T, int OP, int STRIDE>
+// `fold(t)` is the aggregate of tile t from the input, for a tile that has not published it within
+// `limit` polls.
+template <typename T, int OP, int STRIDE, typename Fold>
 __device__ __forceinline__ T resolve_prefix(const TileState<T, STRIDE>& st, int tile,
-                                            T aggregate, int lane) {
+                                            T aggregate, int lane, uint32_t limit, const Fold& fold) {
   using F = Functor<T, OP>;
   if (tile == 0) {
     if (lane == 0) st.publish(0, kFlagPrefix, aggregate);
@@ -290,7 +305,10 @@ __device__ __forceinline__ T resolve_prefix(const TileState<T, STRIDE>& st, int 
     const int idx = base - lane;
     T val = F::identity();
     uint32_t flag = kFlagPrefix;  // virtual prefix in front of tile 0
-    if (idx >= 0) flag = st.wait(idx, &val);
+    if (idx >= 0) {
+      flag = st.wait(idx, &val, limit);
+      if (flag == kFlagInvalid) val = fold(idx);
+    }
     const uint64_t has_prefix = __ballot(flag == kFlagPrefix);
     // Lanes run from the nearest predecessor (lane 0) to the farthest; the
     // first lane holding an inclusive prefix ends the walk.
@@ -306,6 +324,34 @@ __device__ __forceinline__ T resolve_prefix(const TileState<T, STRIDE>& st, int 
   return exclusive;
 }
 
+// Of a short tile, by the whole block: thread t waits for two neighbouring tiles, so the prefix is one round trip
+// behind the slowest aggregate in front of it (a walk by one wave takes one per 64 tiles: 10^6 double Max 12.4
+// against 11.4 us a call, 500 000 11.9 against 10.8).  Only aggregates are published.  Called by every thread; ends with a
+// barrier.  (Not behind tickets, which come one after the other: 10^6 int64 11.2 against 10.5 by a walk.)
+template <typename T, int OP, int STRIDE, typename Fold>
+__device__ __forceinline__ T resolve_prefix_at_once(const TileState<T, STRIDE>& st, int tile, T aggregate,
+                                                    int wave, int lane, T* s_front, uint32_t limit,
+                                                    const Fold& fold) {
+  using F = Functor<T, OP>;
+  if (threadIdx.x == 0) st.publish(tile, kFlagAggregate, aggregate);
+  constexpr int kPer = (int)(kShortMaxTiles * kShortDivisor + kBlock - 1) / kBlock;
+  T val = F::identity();
+#pragma unroll
+  for (int p = 0; p < kPer; ++p) {
+    const int front = (int)threadIdx.x * kPer + p;
+    T one = F::identity();
+    if (front < tile && st.wait(front, &one, limit) == kFlagInvalid) one = fold(front);
+    val = F::apply(val, one);
+  }
+  const T front = read_lane<T>(wave_inclusive_scan<T, OP>(val, lane), kWaveSize - 1);
+  if (lane == 0) s_front[wave] = front;
+  __syncthreads();
+  T exclusive = s_front[0];
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w) exclusive = F::apply(exclusive, s_front[w]);
+  return exclusive;
+}
+
 // Four waves per SIMD, i.e. 128 registers and two blocks per CU: left to itself
 // the compiler takes 180 to 256 registers for the floating-point Max and Min
 // kernels, which halves their residency (measured 0.56 -> 0.44 ms at 2^28 float).
@@ -313,7 +359,7 @@ template <typename T, int OP, bool VECTOR, int VECS>
 __global__ __launch_bounds__(kBlock, ILGPU_HIP_SCAN_WAVES_PER_EU) void scan_kernel(
     const T* __restrict__ in, T* __restrict__ out, int64_t n,
     int64_t in_stride, int64_t out_stride, int inclusive,
-    uint32_t* __restrict__ ticket, TileState<T, status_stride<T, VECS>()> st) {
+    uint32_t* __restrict__ ticket, TileState<T, status_stride<T, VECS>()> st, uint32_t limit) {
   using F = Functor<T, OP>;
   using V = typename Vec16<T>::type;
   constexpr int VN = Vec16<T>::N;
@@ -323,16 +369,18 @@ __global__ __launch_bounds__(kBlock, ILGPU_HIP_SCAN_WAVES_PER_EU) void scan_kern
 
   __shared__ int s_tile;
   __shared__ T s_wave_total[kWaves];
+  __shared__ T s_front[kWaves];  // of a short tile: what lies in front, in parts of 64 tiles
   __shared__ T s_prefix;
+  constexpr bool kShort = VECS != scan_vecs<T>();
 
-  // An input of one tile comes without ticket and status words (and without
+  // An input of one tile comes without status words (and without
   // the launch that clears them): there is nobody to wait for or to tell.
-  const bool alone = ticket == nullptr;
-  if (!alone) {
+  const bool alone = gridDim.x == 1;
+  if (ticket != nullptr) {
     if (threadIdx.x == 0) s_tile = (int)atomicAdd(ticket, 1u);
     __syncthreads();
   }
-  const int tile = alone ? 0 : s_tile;
+  const int tile = ticket != nullptr ? s_tile : (int)blockIdx.x;
   const int lane = threadIdx.x & (kWaveSize - 1);
   // The wave index and everything derived from it are wave-uniform: kept in
   // scalar registers, so a lane addresses its vectors by one 32-bit offset.
@@ -369,6 +417,31 @@ __global__ __launch_bounds__(kBlock, ILGPU_HIP_SCAN_WAVES_PER_EU) void scan_kern
       }
   }
 
+  // A full tile's elements, in parts, so that a floating-point sum is as exact as a tile's own.
+  auto fold_tile = [&](int t) -> T {
+    constexpr int kPart = 64;
+    static_assert(kTile % kPart == 0, "whole parts");
+    T sum = F::identity();
+    for (int e0 = 0; e0 < kTile; e0 += kPart) {
+      T part = F::identity();
+      for (int e = e0; e < e0 + kPart; ++e) part = F::apply(part, in[((int64_t)t * kTile + e) * in_stride]);
+      sum = F::apply(sum, part);
+    }
+    return sum;
+  };
+  auto prefix_of_tile = [&](T block_total) -> T {
+    if (kShort && ticket == nullptr && !ILGPU_HIP_SCAN_PROBE_NO_LOOKBACK)
+      return resolve_prefix_at_once<T, OP>(st, tile, block_total, wave, lane, s_front, limit, fold_tile);
+    if (wave == 0) {
+      const T exclusive = ILGPU_HIP_SCAN_PROBE_NO_LOOKBACK || alone
+                              ? F::identity()
+                              : resolve_prefix<T, OP>(st, tile, block_total, lane, limit, fold_tile);
+      if (lane == 0) s_prefix = exclusive;
+    }
+    __syncthreads();
+    return s_prefix;
+  };
+
   if constexpr (sizeof(T) == 8) {
     // Register-lean form for 8-byte elements, whose per-row prefixes would
     // take two registers each: the prefix of the lower lanes is folded into
@@ -402,14 +475,7 @@ __global__ __launch_bounds__(kBlock, ILGPU_HIP_SCAN_WAVES_PER_EU) void scan_kern
       if (w == wave) wave_prefix = block_total;
       block_total = F::apply(block_total, s_wave_total[w]);
     }
-    if (wave == 0) {
-      const T exclusive = ILGPU_HIP_SCAN_PROBE_NO_LOOKBACK || alone
-                              ? F::identity()
-                              : resolve_prefix<T, OP>(st, tile, block_total, lane);
-      if (lane == 0) s_prefix = exclusive;
-    }
-    __syncthreads();
-    T running = F::apply(s_prefix, wave_prefix);
+    T running = F::apply(prefix_of_tile(block_total), wave_prefix);
     V* dst = reinterpret_cast<V*>(out + wave_base);
 #pragma unroll
     for (int j = 0; j < kTileVecs; ++j) {
@@ -474,15 +540,7 @@ __global__ __launch_bounds__(kBlock, ILGPU_HIP_SCAN_WAVES_PER_EU) void scan_kern
     block_total = F::apply(block_total, s_wave_total[w]);
   }
 
-  if (wave == 0) {
-    const T exclusive = ILGPU_HIP_SCAN_PROBE_NO_LOOKBACK || alone
-                            ? F::identity()
-                            : resolve_prefix<T, OP>(st, tile, block_total, lane);
-    if (lane == 0) s_prefix = exclusive;
-  }
-  __syncthreads();
-
-  T running = F::apply(s_prefix, wave_prefix);  // prefix of row 0 of this wave
+  T running = F::apply(prefix_of_tile(block_total), wave_prefix);  // prefix of row 0 of this wave
   V* dst = reinterpret_cast<V*>(out + wave_base);
 #pragma unroll
   for (int j = 0; j < kTileVecs; ++j) {
@@ -642,7 +700,8 @@ __global__ __launch_bounds__(kBlock) void unique_kernel(
   }
   if (wave == 0) {
     const uint32_t exclusive =
-        alone ? 0u : resolve_prefix<uint32_t, ILGPU_HIP_OP_ADD>(st, tile, block_total, lane);
+        alone ? 0u : resolve_prefix<uint32_t, ILGPU_HIP_OP_ADD>(st, tile, block_total, lane, kNoLimit,
+                                                                [](int) { return 0u; });
     if (lane == 0) s_prefix = exclusive;
   }
   __syncthreads();
@@ -685,7 +744,7 @@ template <typename T> int64_t num_tiles(int64_t n) {
 template <typename T, int OP, int VECS>
 int32_t launch_tiles(hipStream_t stream, const void* in, int64_t in_stride,
                      void* out, int64_t out_stride, int64_t n, int32_t kind,
-                     void* temp) {
+                     void* temp, bool apart) {
   const int64_t tiles = div_up(n, (int64_t)kBlock * VECS * Vec16<T>::N);
   char* base = reinterpret_cast<char*>(align_up((int64_t)(uintptr_t)temp, 256));
   uint32_t* ticket = reinterpret_cast<uint32_t*>(base);
@@ -695,9 +754,10 @@ int32_t launch_tiles(hipStream_t stream, const void* in, int64_t in_stride,
     const int64_t zero_words = (kHeaderBytes + tiles * status_stride<T, VECS>() * 8) / 4;
     const int32_t rc = launch_zero_words(stream, reinterpret_cast<uint32_t*>(base), zero_words);
     if (rc != ILGPU_HIP_SUCCESS) return rc;
-  } else {
-    ticket = nullptr;  // one tile: one launch
   }
+  // (One tile: one launch.)
+  if (tiles == 1 || apart) ticket = nullptr;
+  const uint32_t limit = ticket != nullptr ? kNoLimit : lookback_spin_limit();
   // Element strides above one (Stride1D.General) take the scalar path.
   const bool vector = in_stride == 1 && out_stride == 1 &&
                       (reinterpret_cast<uintptr_t>(in) & 15) == 0 &&
@@ -708,12 +768,12 @@ int32_t launch_tiles(hipStream_t stream, const void* in, int64_t in_stride,
     hipLaunchKernelGGL((scan_kernel<T, OP, true, VECS>), dim3((unsigned)tiles),
                        dim3(kBlock), 0, stream, static_cast<const T*>(in),
                        static_cast<T*>(out), n, in_stride, out_stride,
-                       inclusive, ticket, st);
+                       inclusive, ticket, st, limit);
   } else {
     hipLaunchKernelGGL((scan_kernel<T, OP, false, VECS>), dim3((unsigned)tiles),
                        dim3(kBlock), 0, stream, static_cast<const T*>(in),
                        static_cast<T*>(out), n, in_stride, out_stride,
-                       inclusive, ticket, st);
+                       inclusive, ticket, st, limit);
   }
   ILGPU_HIP_CHECK(hipGetLastError());
   return ILGPU_HIP_SUCCESS;
@@ -724,10 +784,16 @@ int32_t launch_typed(hipStream_t stream, const void* in, int64_t in_stride,
                      void* out, int64_t out_stride, int64_t n, int32_t kind,
                      void* temp) {
   const int64_t tiles = num_tiles<T>(n);
-  if (tiles > 1 && tiles <= kShortMaxTiles)
+  // Whether the views, from their first byte to their last, do not meet.
+  const auto end = [&](const void* p, int64_t stride) {
+    return reinterpret_cast<uintptr_t>(p) + (uintptr_t)((n - 1) * stride + 1) * sizeof(T);
+  };
+  const bool apart = end(in, in_stride) <= reinterpret_cast<uintptr_t>(out) ||
+                     end(out, out_stride) <= reinterpret_cast<uintptr_t>(in);
+  if (tiles > 1 && tiles <= (apart ? kShortMaxTiles : kShortMaxTilesTicketed))
     return launch_tiles<T, OP, scan_vecs<T>() / kShortDivisor>(
-        stream, in, in_stride, out, out_stride, n, kind, temp);
-  return launch_tiles<T, OP, scan_vecs<T>()>(stream, in, in_stride, out, out_stride, n, kind, temp);
+        stream, in, in_stride, out, out_stride, n, kind, temp, apart);
+  return launch_tiles<T, OP, scan_vecs<T>()>(stream, in, in_stride, out, out_stride, n, kind, temp, apart);
 }
 
 template <typename T>

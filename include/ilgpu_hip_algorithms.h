@@ -234,9 +234,10 @@ int32_t ilgpu_hip_sort_check_device(ilgpu_hip_stream_t stream);
  *     waiting and counts that tile's digit itself from the source keys (tiles
  *     are handed to fixed groups of blocks, so a tile may wait for one whose
  *     group has no resident block; with this bound every block finishes
- *     whatever the others do).  Default 4096; 0 makes every look-back that
- *     meets an empty word take the slow path at once, which is how the tests
- *     exercise it.
+ *     whatever the others do).  A scan into another view takes the same bound
+ *     and folds the tile from the input.  Default 4096; 0 makes every look-back
+ *     that meets an empty word take the slow path at once, which is how the
+ *     tests exercise it.
  *   LARGE_BLOCK_MIN_TILES_PER_CU  inputs of at least this many 1024-thread
  *     tiles per compute unit are sorted with 1024-thread blocks (longer runs
  *     per digit), smaller ones with 512-thread blocks (more blocks for fewer
