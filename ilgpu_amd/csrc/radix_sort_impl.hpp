@@ -186,6 +186,13 @@ __device__ __forceinline__ bool status_is_aggregate(uint32_t w) {
 __device__ __forceinline__ uint32_t status_value(uint32_t w) {
   return status_is_aggregate(w) ? w & kStatusCountMask : w - 1u;
 }
+// Where all tiles of a pass run at once (a grid of as many blocks as there are tiles) nothing is published
+// but counts: a tile's own, as above, and by the last tile of kLookGroup tiles, in place of its own, theirs
+// together, with the top bits 10.
+constexpr int kLookGroup = 16;
+constexpr uint32_t kStatusGroup = 2u << 30;
+__device__ __forceinline__ uint32_t status_group(uint32_t count) { return kStatusGroup | count; }
+__device__ __forceinline__ bool status_is_group(uint32_t w) { return (w & kStatusAggregate) == kStatusGroup; }
 constexpr int64_t kMaxSortLength = 0x7fffffffll;  // like the reference: int.MaxValue
 
 template <int KEY_BYTES> struct KeyOf;
@@ -1070,7 +1077,7 @@ __device__ __forceinline__ int ticket_tile(uint32_t k, uint32_t g, uint32_t grou
 }
 
 // Sorts one tile by the digit of `pass` and scatters it.
-template <int KEY_BYTES, int VALUE_BYTES, bool FLOAT_KEYS, bool FULL, bool HOT, int BLOCK, int ITEMS>
+template <int KEY_BYTES, int VALUE_BYTES, bool FLOAT_KEYS, bool FULL, bool HOT, int BLOCK, int ITEMS, bool AT_ONCE>
 __device__ __forceinline__ void sort_tile(
     typename KeyOf<KEY_BYTES>::type (&key)[ITEMS],
     const typename KeyOf<KEY_BYTES>::type* __restrict__ src_keys,
@@ -1238,7 +1245,7 @@ __device__ __forceinline__ void sort_tile(
 #pragma unroll
     for (int s = 0; s < kSubTiles; ++s) count += s_counter[s * kRadix + tid];
     __hip_atomic_store(&tile_status[tid],
-                       tile == 0 ? status_prefix(count) : status_aggregate(count),
+                       tile == 0 && !AT_ONCE ? status_prefix(count) : status_aggregate(count),
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     inc = count;
 #pragma unroll
@@ -1267,11 +1274,13 @@ __device__ __forceinline__ void sort_tile(
         run += t;
       }
     }
+    if constexpr (!AT_ONCE) {
 #pragma unroll
-    for (int u = 0; u < kLookback; ++u) {
-      const int idx = tile - 1 - u < 0 ? 0 : tile - 1 - u;
-      first_step[u] = __hip_atomic_load(&status[(int64_t)idx * kRadix + tid],
-                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (int u = 0; u < kLookback; ++u) {
+        const int idx = tile - 1 - u < 0 ? 0 : tile - 1 - u;
+        first_step[u] = __hip_atomic_load(&status[(int64_t)idx * kRadix + tid],
+                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
     }
   }
   __syncthreads();
@@ -1290,7 +1299,83 @@ __device__ __forceinline__ void sort_tile(
   for (int j = 0; j < kItems; ++j)
     s_keys[j % 2 == 0 ? packed[j / 2] & 0xFFFFu : packed[j / 2] >> 16] = key[j];
 
-  if (tid < kRadix) {
+  // Keys of digit d in tile t, a full one, from the source.
+  auto count_tile = [&](int t, uint32_t d) -> uint32_t {
+    const K* other = src_keys + (int64_t)t * TileCfg::kTile;
+    uint32_t c = 0;
+#pragma unroll 4
+    for (int i = 0; i < TileCfg::kTile; ++i) {
+      K k = other[i];
+      if constexpr (FLOAT_KEYS) k = ordered_bits(k, xf_in);
+      c += digit(k) == d;
+    }
+    return c;
+  };
+  if constexpr (AT_ONCE) {
+    static_assert(BLOCK == 2 * kRadix, "two halves of a thread per digit");
+    // Every tile publishes its counts at about the same time, so a walk would meet nothing but counts and take as
+    // many round trips as its tile has predecessors in fours.  Instead one half of the block sums
+    // the counts of the tiles in front within the group, the other those of the groups in front: two round
+    // trips behind each other, since the group's last tile sums its group before the others see it.
+    // (Inside a pass of 2^21 u32 keys, 342 tiles, the slowest tile waits 4 us for it instead of 7.6.  Sorts with a copy
+    // in front, us, a walk / this: u32 keys 2^20 55.0 / 48.9, 2^21 69.4 / 63.2, below 10^6 2^20 63.1 / 53.6; normal floats
+    // 2^20 74.1 / 64.7; pairs of 2^21 u32 85.2 / 77.4, 2^20 Zipf 60.5 / 53.4, of 2^20 u64 with u32 85.7 / 79.2.)
+    const uint32_t d = (uint32_t)tid & (kRadix - 1);
+    const bool groups = __builtin_amdgcn_readfirstlane(tid) >= kRadix;
+    const int group = tile / kLookGroup;
+    const int span = groups ? kLookGroup : 1;                       // tiles that a word stands for
+    const int words = groups ? group : tile % kLookGroup;           // to be summed
+    const int first = groups ? kLookGroup - 1 : group * kLookGroup;  // row of the first one
+    // A count has the top bits 11, a group's 10: with this added it is at least kStatusAggregate, and
+    // anything else is not.
+    const uint32_t to_aggregate = groups ? kStatusAggregate - kStatusGroup : 0u;
+    auto word = [&](int row) -> uint32_t {
+      return __hip_atomic_load(&status[(int64_t)row * kRadix + d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    uint32_t before = groups ? excl[pass * kRadix + d] : 0u;
+    for (int at = 0; at < words; at += kLookGroup) {
+      uint32_t sum;
+      for (uint32_t polls = 0;; ++polls) {
+        uint32_t w[kLookGroup], least = ~0u;
+#pragma unroll
+        for (int u = 0; u < kLookGroup; ++u) w[u] = word(first + (at + u < words ? at + u : at) * span);
+        sum = 0;
+#pragma unroll
+        for (int u = 0; u < kLookGroup; ++u) {
+          least = min(least, w[u] + to_aggregate);
+          sum += w[u] & (at + u < words ? kStatusCountMask : 0u);
+        }
+        if (least >= kStatusAggregate) break;
+        if (polls >= spin_limit) {
+          // A tile may not be running (see below): what has not been published is counted.
+          sum = 0;
+          for (int u = at; u < words && u < at + kLookGroup; ++u) {
+            const int row = first + u * span;
+            const uint32_t whole = word(row);
+            if (whole + to_aggregate >= kStatusAggregate) {
+              sum += whole & kStatusCountMask;
+              continue;
+            }
+            uint32_t of_row = 0;
+            for (int t = row - (span - 1); t <= row; ++t) {
+              const uint32_t one = word(t);
+              if (one != 0u && !status_is_aggregate(one)) of_row = 0;  // the group's last tile has summed it by now
+              of_row += one != 0u ? one & kStatusCountMask : count_tile(t, d);
+            }
+            sum += of_row;
+          }
+          break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+      }
+      before += sum;
+    }
+    if (groups) s_global_off[d] = before;
+    else if (tile % kLookGroup == kLookGroup - 1)
+      __hip_atomic_store(&tile_status[d], status_group(before + count), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (!groups) s_global_off[d] += before - digit_start;
+  } else if (tid < kRadix) {
     // Keys with this digit in earlier tiles: walk back over the status words,
     // kLookback tiles per step.  The loads of a step are unconditional (index
     // clamped) so that they are in flight together; positions in front of
@@ -1325,15 +1410,7 @@ __device__ __forceinline__ void sort_tile(
             // full tile: it precedes this one) and go on as if the tile had
             // published its own count.  Slow, and never needed while every
             // group of blocks is resident.
-            const K* other = src_keys + (int64_t)(t - u) * TileCfg::kTile;
-            uint32_t c = 0;
-#pragma unroll 4
-            for (int i = 0; i < TileCfg::kTile; ++i) {
-              K k = other[i];
-              if constexpr (FLOAT_KEYS) k = ordered_bits(k, xf_in);
-              c += digit(k) == (uint32_t)tid;
-            }
-            s[u] = status_aggregate(c);
+            s[u] = status_aggregate(count_tile(t - u, (uint32_t)tid));
             break;
           }
           __builtin_amdgcn_s_sleep(1);
@@ -1388,7 +1465,9 @@ __device__ __forceinline__ void sort_tile(
   }
 }
 
-template <int KEY_BYTES, int VALUE_BYTES, bool FLOAT_KEYS, int BLOCK, int ITEMS>
+// AT_ONCE: one tile per block, which is not handed out (see below), and a look-back for tiles that all run at the same
+// time.
+template <int KEY_BYTES, int VALUE_BYTES, bool FLOAT_KEYS, int BLOCK, int ITEMS, bool AT_ONCE>
 __global__ __launch_bounds__(BLOCK, ILGPU_HIP_SORT_WAVES_PER_EU)
 void onesweep_kernel(
     typename KeyOf<KEY_BYTES>::type* keys_a,
@@ -1453,7 +1532,7 @@ void onesweep_kernel(
   // covers that as it does with tickets.
   for (int round = 0;; ++round) {
     int tile;
-    if (ticket == nullptr) {
+    if (AT_ONCE || ticket == nullptr) {
       if (round > 0) break;
       tile = (int)blockIdx.x;
     } else {
@@ -1490,7 +1569,7 @@ void onesweep_kernel(
           z[i] = make_uint4(0u, 0u, 0u, 0u);
       }
       __syncthreads();
-      sort_tile<KEY_BYTES, VALUE_BYTES, FLOAT_KEYS, kFull, kHot, BLOCK, ITEMS>(
+      sort_tile<KEY_BYTES, VALUE_BYTES, FLOAT_KEYS, kFull, kHot, BLOCK, ITEMS, AT_ONCE>(
           key, src_keys, dst_keys, src_vals, dst_vals, tile_base, valid, tile, pass, xf, excl,
           status, make_index, s_stage, s_global_off, s_scan, hot, spin_limit, in_raw, out_raw);
     };
@@ -3189,7 +3268,8 @@ KeyXform make_xform(int32_t key_type, int32_t flags) {
 }
 
 // The passes of one sort with tiles of BLOCK threads and ITEMS keys per thread.
-template <int KEY_BYTES, int VALUE_BYTES, int BLOCK,
+// AT_ONCE: a block for every tile.
+template <int KEY_BYTES, int VALUE_BYTES, int BLOCK, bool AT_ONCE = false,
           int ITEMS = items_per_thread(KEY_BYTES, VALUE_BYTES)>
 int32_t launch_passes(hipStream_t stream, const SortArgs& a, const TempLayout& L, char* base,
                       const KeyXform& xf, int cus) {
@@ -3207,26 +3287,28 @@ int32_t launch_passes(hipStream_t stream, const SortArgs& a, const TempLayout& L
                              ? 1
                              : (a.value_source == ILGPU_HIP_VALUES_FROM_INDEX_AS_FLOAT ? 2 : 0);
   const bool float_keys = (xf.reference_term | xf.total_term) != 0;
-  auto* pass_kernel = onesweep_kernel<KEY_BYTES, VALUE_BYTES, false, BLOCK, ITEMS>;
+  auto* pass_kernel = onesweep_kernel<KEY_BYTES, VALUE_BYTES, false, BLOCK, ITEMS, AT_ONCE>;
   if constexpr (KEY_BYTES >= 2) {  // there is no 1-byte floating-point key
-    if (float_keys) pass_kernel = onesweep_kernel<KEY_BYTES, VALUE_BYTES, true, BLOCK, ITEMS>;
+    if (float_keys) pass_kernel = onesweep_kernel<KEY_BYTES, VALUE_BYTES, true, BLOCK, ITEMS, AT_ONCE>;
   }
-  // Resident blocks per CU of this instantiation: asked once per device and
-  // kernel (the query costs microseconds, which small sorts would feel).
-  static std::atomic<int> cached_per_cu[kMaxCachedDevices][2];  // per instantiation
-  const int device = current_device();
-  std::atomic<int>* cached =
-      device >= 0 && device < kMaxCachedDevices ? &cached_per_cu[device][float_keys ? 1 : 0]
-                                                : nullptr;
-  int per_cu = cached ? cached->load(std::memory_order_relaxed) : 0;
-  if (per_cu == 0) {
-    ILGPU_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &per_cu, pass_kernel, BLOCK, 0));
-    if (per_cu < 1) per_cu = 1;
-    if (cached) cached->store(per_cu, std::memory_order_relaxed);
+  int64_t grid = L.tiles;
+  if constexpr (!AT_ONCE) {
+    // Resident blocks per CU of this instantiation: asked once per device and
+    // kernel (the query costs microseconds, which small sorts would feel).
+    static std::atomic<int> cached_per_cu[kMaxCachedDevices][2];  // per instantiation
+    const int device = current_device();
+    std::atomic<int>* cached =
+        device >= 0 && device < kMaxCachedDevices ? &cached_per_cu[device][float_keys ? 1 : 0]
+                                                  : nullptr;
+    int per_cu = cached ? cached->load(std::memory_order_relaxed) : 0;
+    if (per_cu == 0) {
+      ILGPU_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+          &per_cu, pass_kernel, BLOCK, 0));
+      if (per_cu < 1) per_cu = 1;
+      if (cached) cached->store(per_cu, std::memory_order_relaxed);
+    }
+    grid = std::min((int64_t)cus * per_cu, L.tiles);
   }
-  int64_t grid = (int64_t)cus * per_cu;
-  if (grid > L.tiles) grid = L.tiles;
   // Every group of blocks needs a block: a grid below eight blocks (few tiles, or
   // a device with very few compute units) forms as many groups as it has blocks.
   const int groups = grid < kTicketGroups ? (int)grid : kTicketGroups;
@@ -3466,6 +3548,9 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
   }
   ILGPU_HIP_CHECK(hipGetLastError());
 
+  // Full tiles, no more of them than run at the same time, two per compute unit, look back as short ones do.
+  // (Not every value size is worth two more kernels.)
+  constexpr bool kAtOnce = KEY_BYTES >= 4 && (VALUE_BYTES == 0 || VALUE_BYTES == 4 || VALUE_BYTES == 8);
   if (use_pipelined) {
     if constexpr (VALUE_BYTES == 0)
       rc = launch_passes_pipelined<KEY_BYTES>(stream, a, L, base, xf, cus);
@@ -3477,14 +3562,18 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
       constexpr int kB = short_items_per_thread(KEY_BYTES, 1);
       constexpr int kC = short_items_per_thread(KEY_BYTES, 2);
       if (short_items == kA)
-        rc = launch_passes<KEY_BYTES, 0, kSortBlock, kA>(stream, a, L, base, xf, cus);
+        rc = launch_passes<KEY_BYTES, 0, kSortBlock, true, kA>(stream, a, L, base, xf, cus);
       else if (short_items == kB)
-        rc = launch_passes<KEY_BYTES, 0, kSortBlock, kB>(stream, a, L, base, xf, cus);
+        rc = launch_passes<KEY_BYTES, 0, kSortBlock, true, kB>(stream, a, L, base, xf, cus);
       else
-        rc = launch_passes<KEY_BYTES, 0, kSortBlock, kC>(stream, a, L, base, xf, cus);
+        rc = launch_passes<KEY_BYTES, 0, kSortBlock, true, kC>(stream, a, L, base, xf, cus);
     }
-  } else
+  } else if (kAtOnce && L.tiles <= 2 * (int64_t)cus) {
+    if constexpr (kAtOnce)
+      rc = launch_passes<KEY_BYTES, VALUE_BYTES, kSortBlock, true>(stream, a, L, base, xf, cus);
+  } else {
     rc = launch_passes<KEY_BYTES, VALUE_BYTES, kSortBlock>(stream, a, L, base, xf, cus);
+  }
   if (rc != ILGPU_HIP_SUCCESS) return rc;
   if constexpr (kLocal) {
     if (local.draws != nullptr) {
