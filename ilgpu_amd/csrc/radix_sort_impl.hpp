@@ -3583,7 +3583,7 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
       if ((xf.reference_term | xf.total_term) != 0) kernel = local_sort_kernel<KEY_BYTES, VALUE_BYTES, true>;
       ProfileScope scope(stream, "sort_local");
       hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(LocalBlock::kBlock), 0, stream, keys_a, keys_b,
-                         vals_a, vals_b, (uint32_t)a.n, xf, plan, from_index, finishes,
+                         vals_a, vals_b, (uint32_t)a.n, xf, plan, excl, from_index, finishes,
                          reinterpret_cast<uint2*>(base + L.status));
       ILGPU_HIP_CHECK(hipGetLastError());
       if (finishes) return ILGPU_HIP_SUCCESS;
