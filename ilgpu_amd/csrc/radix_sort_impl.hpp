@@ -251,6 +251,11 @@ constexpr int items_per_thread(int key_bytes, int value_bytes) {
   if (registers == 2) return value_bytes <= 2 ? 20 : ILGPU_HIP_SORT_PAIR_ITEMS2;
   return registers == 3 ? ILGPU_HIP_SORT_PAIR_ITEMS3 : ILGPU_HIP_SORT_PAIR_ITEMS4;
 }
+// 4-byte floating-point keys without values, whose order takes registers of its own, in full tiles of 512 threads: with 36
+// keys 33 registers spill, with 32 a third fewer, and none where all tiles run at once.  (Normal keys with a copy in front, us,
+// 36 / 32: 8 * 10^6 165 / 135, 9.6 * 10^6 187 / 181, 14 * 10^6 229 / 224, 20 000 003 305 / 279, 25 * 10^6 348 / 330; 28 and 24 keys for
+// 20 000 003: 303 and 310.  Integer keys lose by it: whole numbers below 10^6, 14 * 10^6 176 / 182, 9.6 * 10^6 140 / 145.)
+constexpr int kFloatItems = 32;
 constexpr int tile_keys(int key_bytes, int value_bytes, int block) {
   return block * items_per_thread(key_bytes, value_bytes);
 }
@@ -329,6 +334,22 @@ struct SortPlan {
   uint32_t local_from;              // the digits below this one are left to local_sort_kernel
 };
 static_assert(sizeof(SortPlan) <= 256, "the temp view holds 256 bytes for the plan");
+
+// Passes that take turns with two status arrays: each clears the words of the next one that runs, which the pass before it is
+// done with, and only the first array is cleared beforehand.  In tiles of all lengths but full ones of 512 threads, which lose
+// half a percent by it (14 * 10^6 u32 keys 175 -> 176 us): 2^27 u64 keys clear 9 MB of 75 (2004 -> 1995 us a sort), 2^28 u32 8
+// of 32 (2062 -> 2054), and tiles shorter than what the temp view is sized for find room.
+constexpr bool sort_status_turns(int key_bytes, int block, bool at_once, bool float_tile) {
+  return key_bytes > 1 && (block > ILGPU_HIP_SORT_BLOCK || at_once || float_tile);
+}
+// Clears the words of the pass that runs after this one, if there is one.
+__device__ __forceinline__ void clear_next_status(uint32_t* status, int64_t region_words, const SortPlan* plan, int pass,
+                                                  int threads) {
+  if (plan->last_executed == (uint32_t)pass) return;
+  uint4* words = reinterpret_cast<uint4*>(status + (plan->src_is_alt[pass] != 0 ? 0 : region_words));
+  for (int64_t i = (int64_t)blockIdx.x * threads + threadIdx.x; i < region_words / 4; i += (int64_t)gridDim.x * threads)
+    words[i] = make_uint4(0u, 0u, 0u, 0u);
+}
 
 // 8-byte keys whose upper halves rarely meet are sorted by that half alone, four
 // passes instead of eight; what is left is to order the few neighbours whose
@@ -1474,7 +1495,7 @@ void onesweep_kernel(
     typename KeyOf<KEY_BYTES>::type* keys_b,
     typename ValueOf<VALUE_BYTES>::type* vals_a,
     typename ValueOf<VALUE_BYTES>::type* vals_b, int64_t n, int pass,
-    KeyXform xf, const uint32_t* __restrict__ excl, uint32_t* status,
+    KeyXform xf, const uint32_t* __restrict__ excl, uint32_t* all_status,
     uint32_t* ticket, const SortPlan* __restrict__ plan, int num_tiles,
     int values_from_index, int groups, int chunk_shift, uint32_t spin_limit) {
   using K = typename KeyOf<KEY_BYTES>::type;
@@ -1490,6 +1511,12 @@ void onesweep_kernel(
 
   if (plan->skip[pass]) return;
   const bool src_alt = plan->src_is_alt[pass] != 0;
+  constexpr bool kTurns = sort_status_turns(KEY_BYTES, BLOCK, AT_ONCE,
+                                            FLOAT_KEYS && KEY_BYTES == 4 && VALUE_BYTES == 0 && ITEMS == kFloatItems);
+  const int64_t region_words = (int64_t)num_tiles * kRadix;
+  uint32_t* status = all_status + (kTurns ? (src_alt ? region_words : 0) : pass * region_words);
+  // (A block of one tile does it when the tile is done: the others wait for its counts.)
+  if constexpr (kTurns && !AT_ONCE) clear_next_status(all_status, region_words, plan, pass, BLOCK);
   uint32_t hot[kMaxHot];
 #pragma unroll
   for (int h = 0; h < kMaxHot; ++h) hot[h] = plan->hot[pass][h];
@@ -1577,6 +1604,7 @@ void onesweep_kernel(
     else if (hot[0] == kNoHotDigit) run(std::true_type{}, std::false_type{});
     else run(std::true_type{}, std::true_type{});
   }
+  if constexpr (kTurns && AT_ONCE) clear_next_status(all_status, region_words, plan, pass, BLOCK);
 }
 
 // ---- onesweep pass, pipelined form (keys without values, large inputs) --------
@@ -2011,7 +2039,7 @@ template <int KEY_BYTES, bool FLOAT_KEYS>
 __global__ __launch_bounds__(1024, ILGPU_HIP_SORT_WAVES_PER_EU)
 void onesweep_pipelined_kernel(
     typename KeyOf<KEY_BYTES>::type* keys_a, typename KeyOf<KEY_BYTES>::type* keys_b, int64_t n,
-    int pass, KeyXform xf, const uint32_t* __restrict__ excl, uint32_t* status, uint32_t* ticket,
+    int pass, KeyXform xf, const uint32_t* __restrict__ excl, uint32_t* all_status, uint32_t* ticket,
     const SortPlan* __restrict__ plan, int num_tiles, int groups, int chunk_shift,
     uint32_t spin_limit, int with_scanner) {
   using K = typename KeyOf<KEY_BYTES>::type;
@@ -2037,6 +2065,9 @@ void onesweep_pipelined_kernel(
 
   if (plan->skip[pass]) return;
   const bool src_alt = plan->src_is_alt[pass] != 0;
+  const int64_t region_words = (int64_t)num_tiles * kRadix;
+  uint32_t* status = all_status + (src_alt ? region_words : 0);
+  clear_next_status(all_status, region_words, plan, pass, 1024);
   const K* src_keys = src_alt ? keys_b : keys_a;
   K* dst_keys = src_alt ? keys_a : keys_b;
   const int shift = pass * 8;
@@ -3219,7 +3250,8 @@ TempLayout make_layout(int64_t n, int key_bytes, int value_bytes, int block = kS
   L.tickets = off; off += kMaxPasses * kTicketGroups * kTicketStride * 4;
   L.status = off;
   L.status_stride = L.tiles * kRadix * 4;
-  off += L.status_stride * key_bytes;  // one status array per pass
+  // One status array per pass, or two by turns (sort_status_turns).
+  off += L.status_stride * key_bytes;
   L.total = off;
   return L;
 }
@@ -3287,8 +3319,10 @@ int32_t launch_passes(hipStream_t stream, const SortArgs& a, const TempLayout& L
                              ? 1
                              : (a.value_source == ILGPU_HIP_VALUES_FROM_INDEX_AS_FLOAT ? 2 : 0);
   const bool float_keys = (xf.reference_term | xf.total_term) != 0;
-  auto* pass_kernel = onesweep_kernel<KEY_BYTES, VALUE_BYTES, false, BLOCK, ITEMS, AT_ONCE>;
-  if constexpr (KEY_BYTES >= 2) {  // there is no 1-byte floating-point key
+  constexpr bool kOfKeys = KEY_BYTES == 4 && VALUE_BYTES == 0 && BLOCK == kSortBlock;
+  constexpr bool kOnlyFloats = kOfKeys && ITEMS == kFloatItems, kNoFloats = kOfKeys && ITEMS == ILGPU_HIP_SORT_ITEMS;
+  auto* pass_kernel = onesweep_kernel<KEY_BYTES, VALUE_BYTES, kOnlyFloats, BLOCK, ITEMS, AT_ONCE>;
+  if constexpr (KEY_BYTES >= 2 && !kNoFloats) {  // there is no 1-byte floating-point key
     if (float_keys) pass_kernel = onesweep_kernel<KEY_BYTES, VALUE_BYTES, true, BLOCK, ITEMS, AT_ONCE>;
   }
   int64_t grid = L.tiles;
@@ -3317,9 +3351,8 @@ int32_t launch_passes(hipStream_t stream, const SortArgs& a, const TempLayout& L
   int chunk_shift = 0;
   while (chunk_shift < kMaxChunkShift && (grid << (chunk_shift + 1)) <= L.tiles) ++chunk_shift;
   const uint32_t spin_limit = g_sort_spin_limit.load(std::memory_order_relaxed);
+  uint32_t* status = reinterpret_cast<uint32_t*>(base + L.status);
   for (int p = 0; p < passes; ++p) {
-    uint32_t* status =
-        reinterpret_cast<uint32_t*>(base + L.status + (int64_t)p * L.status_stride);
     {
       ProfileScope scope(stream, "sort_onesweep");
       hipLaunchKernelGGL(pass_kernel,
@@ -3362,9 +3395,8 @@ int32_t launch_passes_pipelined(hipStream_t stream, const SortArgs& a, const Tem
 #endif
   // One block scans instead of sorting when the grid can spare it.
   const int with_scanner = ILGPU_HIP_SORT_SCANNER && grid >= 64 ? 1 : 0;
+  uint32_t* status = reinterpret_cast<uint32_t*>(base + L.status);
   for (int p = 0; p < KEY_BYTES; ++p) {
-    uint32_t* status =
-        reinterpret_cast<uint32_t*>(base + L.status + (int64_t)p * L.status_stride);
     {
       ProfileScope scope(stream, "sort_onesweep");
       hipLaunchKernelGGL(pass_kernel, dim3((unsigned)grid), dim3(1024), 0, stream, keys_a, keys_b,
@@ -3443,12 +3475,19 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
   if (short_max_tiles > 2 * (int64_t)cus) short_max_tiles = 2 * (int64_t)cus;
   const int short_items =
       use_large ? 0 : pick_short_items(a.n, KEY_BYTES, VALUE_BYTES, short_max_tiles);
-  const TempLayout L =
+  const bool float_tiles = KEY_BYTES == 4 && VALUE_BYTES == 0 && (xf.reference_term | xf.total_term) != 0 &&
+                           !use_large && short_items == 0;
+  TempLayout L =
       make_layout(a.n, KEY_BYTES, VALUE_BYTES, use_large ? kSortBlockLarge : kSortBlock,
                   use_pipelined ? pipelined_tile_keys(KEY_BYTES)
                                 : (short_items > 0 ? kSortBlock * short_items
-                                             : tile_keys(KEY_BYTES, VALUE_BYTES,
-                                                         use_large ? kSortBlockLarge : kSortBlock)));
+                                   : float_tiles   ? kSortBlock * kFloatItems
+                                                   : tile_keys(KEY_BYTES, VALUE_BYTES,
+                                                               use_large ? kSortBlockLarge : kSortBlock)));
+  // (What the temp view is sized for: the layout's own, or somewhat less where its tiles are shorter than full ones, which two
+  // status arrays fit all the same.)
+  static_assert(2 * ILGPU_HIP_SORT_ITEMS < 4 * kFloatItems, "two arrays for these tiles in four for full ones");
+  L.total = std::min(L.total, make_layout(a.n, KEY_BYTES, VALUE_BYTES).total);
   char* base = reinterpret_cast<char*>(align_up((int64_t)(uintptr_t)a.temp, 256));
   K* keys_a = static_cast<K*>(a.keys);
   K* keys_b = reinterpret_cast<K*>(base + L.alt_keys);
@@ -3509,10 +3548,17 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
     }
   }
   int32_t rc;
+  // Full tiles, no more of them than run at the same time, two per compute unit, look back as short ones do.
+  // (Not every value size is worth two more kernels.
+  // Full tiles of 4-byte keys would spill: 2^23 u32 keys 125 -> 132 us.)
+  constexpr bool kAtOnce = VALUE_BYTES == 0 ? KEY_BYTES == 8 : KEY_BYTES >= 4 && (VALUE_BYTES == 4 || VALUE_BYTES == 8);
+  const bool full_at_once = kAtOnce && !use_large && short_items == 0 && !float_tiles && L.tiles <= 2 * (int64_t)cus;
+  const bool turns = sort_status_turns(KEY_BYTES, use_large ? kSortBlockLarge : kSortBlock,
+                                       short_items > 0 || full_at_once, float_tiles);
+  const int64_t words = ((turns ? L.status + L.status_stride : L.total) - L.zero_begin) / 4;
   if (local.draws != nullptr) {
     auto* draw_kernel = sort_draw_kernel<K, false>;
     if ((xf.reference_term | xf.total_term) != 0) draw_kernel = sort_draw_kernel<K, true>;
-    const int64_t words = (L.total - L.zero_begin) / 4;
     const int64_t blocks = std::min<int64_t>(
         div_up(std::max(std::max(words, table_words), (int64_t)1 << local.limits.draw_bits), 256), (int64_t)cus * 8);
     ProfileScope scope(stream, "zero_words");
@@ -3521,7 +3567,7 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
                        static_cast<K*>(const_cast<void*>(local.draws)), local.limits.draw_bits);
     ILGPU_HIP_CHECK(hipGetLastError());
   } else {
-    rc = launch_zero_words(stream, hist, (L.total - L.zero_begin) / 4,
+    rc = launch_zero_words(stream, hist, words,
                            reinterpret_cast<uint32_t*>(ties.table), table_words);
     if (rc != ILGPU_HIP_SUCCESS) return rc;
   }
@@ -3548,9 +3594,6 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
   }
   ILGPU_HIP_CHECK(hipGetLastError());
 
-  // Full tiles, no more of them than run at the same time, two per compute unit, look back as short ones do.
-  // (Not every value size is worth two more kernels.)
-  constexpr bool kAtOnce = KEY_BYTES >= 4 && (VALUE_BYTES == 0 || VALUE_BYTES == 4 || VALUE_BYTES == 8);
   if (use_pipelined) {
     if constexpr (VALUE_BYTES == 0)
       rc = launch_passes_pipelined<KEY_BYTES>(stream, a, L, base, xf, cus);
@@ -3568,7 +3611,12 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
       else
         rc = launch_passes<KEY_BYTES, 0, kSortBlock, true, kC>(stream, a, L, base, xf, cus);
     }
-  } else if (kAtOnce && L.tiles <= 2 * (int64_t)cus) {
+  } else if (float_tiles) {
+    if constexpr (KEY_BYTES == 4 && VALUE_BYTES == 0)
+      rc = L.tiles <= 2 * (int64_t)cus
+               ? launch_passes<4, 0, kSortBlock, true, kFloatItems>(stream, a, L, base, xf, cus)
+               : launch_passes<4, 0, kSortBlock, false, kFloatItems>(stream, a, L, base, xf, cus);
+  } else if (full_at_once) {
     if constexpr (kAtOnce)
       rc = launch_passes<KEY_BYTES, VALUE_BYTES, kSortBlock, true>(stream, a, L, base, xf, cus);
   } else {

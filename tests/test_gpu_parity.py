@@ -1076,6 +1076,36 @@ def test_sorts_of_random_shapes_under_random_test_hooks_match_oracle():
                               O.radix_sort(keys, descending=descending)), case
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.uint32, np.uint64])
+def test_passes_that_take_turns_with_two_status_arrays(dtype):
+    # Passes that run and passes that do not in every order (digits that all keys share), three and more of them in a row, in
+    # tiles that take turns: short ones, floating-point ones (512 * 32 keys; all at once up to 512 tiles), large ones, twice over
+    # the same temp memory.
+    size = np.dtype(dtype).itemsize
+    rng = np.random.default_rng(size)
+    lengths = [100_003] + ([512 * 32 * 40 - 1, 512 * 32 * 512, 512 * 32 * 512 + 1] if dtype == np.float32 else [400_000])
+    for large in (-1, 0):
+        capi.sort_set_parameter(capi.SORT_PARAM_LARGE_BLOCK_MIN_TILES_PER_CU, large)
+        try:
+            for n in lengths if large < 0 else lengths[:1]:
+                temp = capi.temp_buffer(capi.radix_sort_temp_bytes(n, dtype))
+                temp.bytes.fill_(0xA5)
+                for mask in (0xFFFFFFFFFFFFFFFF, 0x00FFFF00FF00FFFF, 0xFF00FF7FFF00FF7F, 0x0000FF00FFFFFF00):
+                    bits = (rng.integers(0, 1 << 63, n, dtype=np.uint64) * 2 + 1) & np.uint64(mask)
+                    keys = bits.astype(f"u{size}").view(dtype)
+                    keys[: n // 3] = keys[0]  # (many copies: every digit is sorted)
+                    note("status by turns", np.dtype(dtype).name, large, n, hex(mask))
+                    d = D.from_numpy(keys)
+                    capi.radix_sort_keys(d, temp, float_total_order=True)
+                    sync()
+                    order = keys.view(f"u{size}")
+                    if dtype == np.float32:  # IEEE totalOrder
+                        order = np.where(order >> 31, ~order, order | np.uint32(1 << 31))
+                    assert np.array_equal(d.numpy().view(f"u{size}"), keys.view(f"u{size}")[np.argsort(order, kind="stable")])
+        finally:
+            capi.sort_set_parameter(capi.SORT_PARAM_LARGE_BLOCK_MIN_TILES_PER_CU, -1)
+
+
 @pytest.fixture
 def no_short_tiles():
     """Short inputs of keys take full tiles like pairs and longer inputs do."""
