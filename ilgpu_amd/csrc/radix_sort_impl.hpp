@@ -2336,7 +2336,7 @@ void onesweep_pipelined_kernel(
 // A sort of at most one 512-thread tile runs as one block and one launch: the
 // keys (and values) stay in registers, every pass ranks them like a pass above,
 // moves them through LDS into digit order and takes them back in memory order
-// (lane l of wave w holds positions w*64*I + j*64 + l again), and the last pass
+// (lane l of wave w holds positions w*64*I + j*64 + l again; small_sort_block says how many threads), and the last pass
 // is followed by one coalesced write.  No histogram, plan, tickets, look-back
 // or temp memory.  ITEMS keys per thread: every row costs its rank, its
 // staging and its share of five barriers per pass whether it holds keys or
@@ -2399,15 +2399,26 @@ __device__ __forceinline__ int wave_sum(int v) {
 }
 
 constexpr int kSmallSortItemsA = 4, kSmallSortItemsB = 12, kSmallSortItemsC = 24;
+// Threads of the block for tiles of `rows` keys per 512 threads: twice that many with half of the rows, which wait for the
+// LDS together, where there are more rows than four; of 8-byte keys, which sort few digits and look at their neighbours, the
+// floating-point ones, which sort all digits; of shorter keys, which have one or two digits, only the longest tiles.  (Sorts with a copy in front, us, 512 / 1024 threads: u32 keys 4000 12.6 / 11.8,
+// 9000 20.1 / 18.1, 18 000 30.1 / 24.8, below 10^6 24.3 / 20.5; normal floats 6000 19.0 / 16.4, 18 000 49.2 / 36.5; normal doubles 9000
+// 32.4 / 30.2; but u64 keys below 10^6 9000 17.7 / 18.2, Zipf 17.2 / 18.1, pairs of 5000 u64 21.6 / 23.7, u16 keys 6000 11.4 / 12.9, 18 000 16.8 / 14.3.)
+constexpr int small_sort_block(int key_bytes, int value_bytes, bool floats, int rows) {
+  const bool wide = key_bytes == 8 ? floats && value_bytes == 0 && rows > kSmallSortItemsA
+                                   : rows > (key_bytes == 4 ? kSmallSortItemsA : kSmallSortItemsC);
+  return wide ? 2 * kSortBlock : kSortBlock;
+}
+constexpr int small_sort_items(int block, int rows) { return block == kSortBlock ? rows : (rows / 2 + 1) / 2 * 2; }
 // (One block runs: registers and LDS are not shared with others.)
-template <int KEY_BYTES, int VALUE_BYTES, bool FLOAT_KEYS, int ITEMS>
-__global__ __launch_bounds__(kSortBlock, KEY_BYTES == 8 ? 2 : ILGPU_HIP_SORT_WAVES_PER_EU)
+template <int KEY_BYTES, int VALUE_BYTES, bool FLOAT_KEYS, int BLOCK, int ITEMS>
+__global__ __launch_bounds__(BLOCK, BLOCK == kSortBlock && KEY_BYTES == 8 ? 2 : ILGPU_HIP_SORT_WAVES_PER_EU)
 void small_sort_kernel(typename KeyOf<KEY_BYTES>::type* keys,
                        typename ValueOf<VALUE_BYTES>::type* vals, int n, KeyXform xf,
                        int values_from_index) {
   using K = typename KeyOf<KEY_BYTES>::type;
   using Val = typename ValueOf<VALUE_BYTES>::type;
-  using TileCfg = SortTile<KEY_BYTES, VALUE_BYTES, kSortBlock>;
+  using TileCfg = SortTile<KEY_BYTES, VALUE_BYTES, BLOCK>;
   constexpr int kItems = ITEMS;
   constexpr int kSubTiles = TileCfg::kSubTiles;
   constexpr int kSubTileKeys = kSubLanes * kItems;
@@ -2415,8 +2426,8 @@ void small_sort_kernel(typename KeyOf<KEY_BYTES>::type* keys,
   static_assert(kItems % 2 == 0 && kItems <= TileCfg::kItems, "ranks are packed in pairs");
   // Counters, then the keys, then the values of the tile share these bytes.
   constexpr int kEntryBytes = KEY_BYTES > VALUE_BYTES ? KEY_BYTES : VALUE_BYTES;
-  constexpr int kStageBytes = kSortBlock * kItems * kEntryBytes > TileCfg::kCounterBytes
-                                  ? kSortBlock * kItems * kEntryBytes
+  constexpr int kStageBytes = BLOCK * kItems * kEntryBytes > TileCfg::kCounterBytes
+                                  ? BLOCK * kItems * kEntryBytes
                                   : TileCfg::kCounterBytes;
 
   __shared__ __attribute__((aligned(16))) unsigned char s_stage[kStageBytes];
@@ -2425,7 +2436,7 @@ void small_sort_kernel(typename KeyOf<KEY_BYTES>::type* keys,
   __shared__ uint32_t s_inverted, s_far;
   __shared__ int s_clashes[kSubTiles], s_pairs[kSubTiles];
   __shared__ uint64_t s_asked[KEY_BYTES == 8 ? kSortBlock : 1];
-  __shared__ uint16_t s_to[KEY_BYTES == 8 ? kSortBlock * kItems : 1];  // where a staged key belongs
+  __shared__ uint16_t s_to[KEY_BYTES == 8 ? BLOCK * kItems : 1];  // where a staged key belongs
   uint32_t* s_counter = reinterpret_cast<uint32_t*>(s_stage);
   K* s_keys = reinterpret_cast<K*>(s_stage);
   Val* s_vals = reinterpret_cast<Val*>(s_stage);
@@ -2440,11 +2451,12 @@ void small_sort_kernel(typename KeyOf<KEY_BYTES>::type* keys,
   Val val[kPairs ? kItems : 1];
   uint32_t* s_words = reinterpret_cast<uint32_t*>(s_stage);  // two tables of kAskedSlotsLog2
   if constexpr (KEY_BYTES == 8) {
-    static_assert(8 << kAskedSlotsLog2 <= kStageBytes && (8 << kAskedSlotsLog2) % (16 * kSortBlock) == 0, "");
-    asked = keys[(uint32_t)tid * (uint32_t)n / kSortBlock];
+    static_assert(8 << kAskedSlotsLog2 <= kStageBytes && (8 << kAskedSlotsLog2) % (16 * BLOCK) == 0, "");
+    // (The first kSortBlock threads ask.)
+    if (tid < kSortBlock) asked = keys[(uint32_t)tid * (uint32_t)n / kSortBlock];
 #pragma unroll
-    for (int i = 0; i < (8 << kAskedSlotsLog2) / (16 * kSortBlock); ++i)
-      reinterpret_cast<uint4*>(s_stage)[i * kSortBlock + tid] = make_uint4(0u, 0u, 0u, 0u);
+    for (int i = 0; i < (8 << kAskedSlotsLog2) / (16 * BLOCK); ++i)
+      reinterpret_cast<uint4*>(s_stage)[i * BLOCK + tid] = make_uint4(0u, 0u, 0u, 0u);
   }
 #pragma unroll
   for (int j = 0; j < kItems; ++j) {
@@ -2470,8 +2482,8 @@ void small_sort_kernel(typename KeyOf<KEY_BYTES>::type* keys,
   // The bits in which keys differ, and the prefix that is sorted first.
   // (4-byte keys with fewer rows: half a microsecond for the question, which a digit less gives back
   // where there is one: 2000 uniform u32 keys 6.8 -> 7.4 us, below 10^6 6.8 -> 6.0.)
-  constexpr bool kAsks = KEY_BYTES == 8 || (KEY_BYTES == 4 && !FLOAT_KEYS && kItems > kSmallSortItemsC);
-  constexpr int kPrefixDigits = kItems <= kSmallSortItemsA && !FLOAT_KEYS ? 3 : 4;
+  constexpr bool kAsks = KEY_BYTES == 8 || (KEY_BYTES == 4 && !FLOAT_KEYS && BLOCK * kItems > kSortBlock * kSmallSortItemsC);
+  constexpr int kPrefixDigits = BLOCK * kItems <= kSortBlock * kSmallSortItemsA && !FLOAT_KEYS ? 3 : 4;
   uint64_t diff = ~0ull;
   int top_bits = 8 * KEY_BYTES, prefix_shift = 0;
   bool by_prefix = false;
@@ -2488,7 +2500,7 @@ void small_sort_kernel(typename KeyOf<KEY_BYTES>::type* keys,
     if constexpr (KEY_BYTES == 8) {
       if constexpr (FLOAT_KEYS) asked = ordered_bits(asked, xf);
       else asked = ordered(asked);
-      s_asked[tid] = asked;
+      if (tid < kSortBlock) s_asked[tid] = asked;
     }
     __syncthreads();
 #pragma unroll
@@ -2509,7 +2521,7 @@ void small_sort_kernel(typename KeyOf<KEY_BYTES>::type* keys,
       const int alike = __popcll(__ballot(prefix == readfirstlane_key(prefix) &&
                                           (uint64_t)asked != readfirstlane_key((uint64_t)asked)));
       bool clash = false;
-      if (alike <= kSmallSortAlike) {
+      if (tid < kSortBlock && alike <= kSmallSortAlike) {
         const uint32_t before = __hip_atomic_exchange(&s_words[slot], (uint32_t)tid + 1u, __ATOMIC_RELAXED,
                                                       __HIP_MEMORY_SCOPE_WORKGROUP);
         if (before != 0u) {
@@ -2518,7 +2530,7 @@ void small_sort_kernel(typename KeyOf<KEY_BYTES>::type* keys,
         }
       }
       int clashes = __popcll(__ballot(clash));
-      if (lane == 0) s_clashes[wave] = alike <= kSmallSortAlike ? clashes : 1 << 20;
+      if (lane == 0) s_clashes[wave] = tid >= kSortBlock ? 0 : (alike <= kSmallSortAlike ? clashes : 1 << 20);
       __syncthreads();
       clashes = 0;
 #pragma unroll
@@ -2619,7 +2631,7 @@ void small_sort_kernel(typename KeyOf<KEY_BYTES>::type* keys,
         bool inverted = false;
 #pragma unroll
         for (int j = 0; j < kItems; ++j) {
-          const int at = j * kSortBlock + tid;
+          const int at = j * BLOCK + tid;
           if (at + 1 < length) inverted = inverted || ordered(s_keys[at]) > ordered(s_keys[at + 1]);
         }
         if (inverted) s_inverted = 1u;
@@ -2627,7 +2639,7 @@ void small_sort_kernel(typename KeyOf<KEY_BYTES>::type* keys,
         if (s_inverted != 0u) {
           // Keys of the same prefix are next to each other, equal keys in their order: a key moves
           // by the smaller ones behind it and the larger ones in front of it.
-          for (int at = tid; at < length; at += kSortBlock) {
+          for (int at = tid; at < length; at += BLOCK) {
             const K o = ordered(s_keys[at]);
             const K prefix = (K)(o >> prefix_shift);
             int to = at;
@@ -3418,14 +3430,19 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
     const KeyXform xf = make_xform(a.key_type, a.flags);
     constexpr int kFullItems = items_per_thread(KEY_BYTES, VALUE_BYTES);
     auto launch_small = [&](auto items) -> int32_t {
-      constexpr int kItems = decltype(items)::value;
-      auto* kernel = small_sort_kernel<KEY_BYTES, VALUE_BYTES, false, kItems>;
+      constexpr int kRows = decltype(items)::value;
+      constexpr int kBlock = small_sort_block(KEY_BYTES, VALUE_BYTES, false, kRows);
+      constexpr int kFloatBlock = small_sort_block(KEY_BYTES, VALUE_BYTES, true, kRows);
+      auto* kernel = small_sort_kernel<KEY_BYTES, VALUE_BYTES, false, kBlock, small_sort_items(kBlock, kRows)>;
+      unsigned block = kBlock;
       if constexpr (KEY_BYTES >= 2) {  // there is no 1-byte floating-point key
-        if ((xf.reference_term | xf.total_term) != 0)
-          kernel = small_sort_kernel<KEY_BYTES, VALUE_BYTES, true, kItems>;
+        if ((xf.reference_term | xf.total_term) != 0) {
+          kernel = small_sort_kernel<KEY_BYTES, VALUE_BYTES, true, kFloatBlock, small_sort_items(kFloatBlock, kRows)>;
+          block = kFloatBlock;
+        }
       }
       ProfileScope scope(stream, "sort_small");
-      hipLaunchKernelGGL(kernel, dim3(1), dim3(kSortBlock), 0, stream, static_cast<K*>(a.keys),
+      hipLaunchKernelGGL(kernel, dim3(1), dim3(block), 0, stream, static_cast<K*>(a.keys),
                          static_cast<Val*>(a.values), (int)a.n, xf,
                          a.value_source == ILGPU_HIP_VALUES_FROM_INDEX
                                ? 1

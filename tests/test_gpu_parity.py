@@ -1106,6 +1106,28 @@ def test_passes_that_take_turns_with_two_status_arrays(dtype):
             capi.sort_set_parameter(capi.SORT_PARAM_LARGE_BLOCK_MIN_TILES_PER_CU, -1)
 
 
+@pytest.mark.parametrize("dtype", [np.uint16, np.uint32, np.float32, np.uint64, np.float64])
+def test_one_tile_of_512_or_1024_threads(dtype):
+    # Where another instantiation takes over, and the rows of 1024 threads that hold more than the tile's keys.
+    size = np.dtype(dtype).itemsize
+    full = 18432 if size <= 4 else 9216
+    for n in [m for m in (2048, 2049, 6144, 6145, 12288, 12289, full - 1, full) if m <= full]:
+        for kind in ("bits", "few", "copies"):
+            rng = np.random.default_rng(n)
+            unsigned = rng.integers(0, 1 << 63, n, dtype=np.uint64) if kind == "bits" else \
+                rng.integers(0, 40 if kind == "few" else n // 3, n, dtype=np.uint64) * np.uint64(0x0101)
+            keys = unsigned.astype(f"u{size}").view(dtype)
+            note("one tile", np.dtype(dtype).name, n, kind)
+            for descending in (False, True):
+                assert bits_equal(gpu_sort(keys, descending=descending), O.radix_sort(keys, descending=descending))
+                values = np.arange(n, dtype=np.uint32)
+                pair_limit = 8192 if size <= 4 else 7168
+                if n <= pair_limit:
+                    k, v = gpu_sort_pairs(keys, values, descending=descending)
+                    ek, ev = O.radix_sort_pairs(keys, values, descending=descending)
+                    assert bits_equal(k, ek) and np.array_equal(v, ev)
+
+
 @pytest.fixture
 def no_short_tiles():
     """Short inputs of keys take full tiles like pairs and longer inputs do."""
