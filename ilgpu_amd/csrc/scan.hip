@@ -9,8 +9,8 @@
 //
 // Tile layout (kBlock = 512 threads, 8 waves, kVecs = 16 16-byte vectors per
 // lane, i.e. 128 KiB per tile: time per launch falls with the number of tiles
-// until about this size, then register pressure takes over; inputs of two to 64 such
-// tiles take short ones of 32 KiB):
+// until about this size, then register pressure takes over; inputs of two to 192 such
+// tiles, or of a quarter of one, take short ones of 32 KiB):
 //   wave w owns a contiguous chunk of kVecs*64 vectors; vector j of lane l is
 //   chunk[j*64 + l], so every load/store instruction of a wave covers 1 KiB of
 //   consecutive addresses (dwordx4 per lane).  Scan order inside a wave is
@@ -99,6 +99,9 @@ template <typename T> constexpr int tile_elems() {
 // kShortMaxTilesTicketed where the tiles are handed out by tickets, one after the other (12 to 18 ns each).
 // Their status words stand a quarter of a line apart, so that they fit the
 // temp view of the full tiles; that few words are not what such an input waits for.
+// So does an input of one short tile, which is one launch like one full tile, with a quarter of its rows (calls, us,
+// full / short: 1000 and 4000 double Max 18.5 and 18.9 / 7.1 and 7.4); between one short tile and one full one the launch that
+// clears the status words costs more than the short tiles save (16384 int64 7.4 / 10.0).
 // (Calls, us, tickets and a walk / no tickets and full tiles / short ones: 2.5 * 10^6 double Max 27.6 / 27.3 / 17.7,
 // 3.5 * 10^6 29.6 / 28.4 / 23.8, 2.5 * 10^6 int32 14.4 / 9.6 / 9.6, 6.3 * 10^6 14.6 / 13.8 / 11.7, 2^21 int64 13.0 / 12.4 /
 // 10.5, 3 * 10^6 14.7 / 13.7 / 12.6, but 3.5 * 10^6, 214 full tiles, 15.5 / 14.0 / 15.1 and 2^22 17.7 / 14.8 / 18.0.
@@ -408,13 +411,25 @@ __global__ __launch_bounds__(kBlock, ILGPU_HIP_SCAN_WAVES_PER_EU) void scan_kern
   if (VECTOR && full) {
     load_rows(0, kHalves ? kTileVecs / 2 : kTileVecs);
   } else {
+    // The last tile, or views that are not aligned or not dense.  Whole vectors of the last tile move as such, and only the
+    // lane that holds the view's end goes by elements: by elements everywhere one tile is up to 128 loads and stores
+    // of 1 KiB lines each that one compute unit's address unit takes, and the rest of the chip waits for its end
+    // (calls, us, before / now: 20000 int32 11.8 / 7.4, 2^23 - 1 int32 20.7 / 14.1, 30000001 49.3 / 43.8).
 #pragma unroll
-    for (int j = 0; j < kTileVecs; ++j)
+    for (int j = 0; j < kTileVecs; ++j) {
+      const int e0 = (j * kWaveSize + lane) * VN;
 #pragma unroll
-      for (int k = 0; k < VN; ++k) {
-        const int e = (j * kWaveSize + lane) * VN + k;
-        x[j][k] = e < wave_valid ? in[(wave_base + e) * in_stride] : F::identity();
+      for (int k = 0; k < VN; ++k) x[j][k] = F::identity();
+      if (VECTOR && e0 + VN <= wave_valid) {
+        const V v = *reinterpret_cast<const V*>(in + wave_base + e0);
+#pragma unroll
+        for (int k = 0; k < VN; ++k) x[j][k] = v[k];
+      } else if (e0 < wave_valid) {
+#pragma unroll
+        for (int k = 0; k < VN; ++k)
+          if (e0 + k < wave_valid) x[j][k] = in[(wave_base + e0 + k) * in_stride];
       }
+    }
   }
 
   // A full tile's elements, in parts, so that a floating-point sum is as exact as a tile's own.
@@ -430,10 +445,11 @@ __global__ __launch_bounds__(kBlock, ILGPU_HIP_SCAN_WAVES_PER_EU) void scan_kern
     return sum;
   };
   auto prefix_of_tile = [&](T block_total) -> T {
+    if (alone) return F::identity();
     if (kShort && ticket == nullptr && !ILGPU_HIP_SCAN_PROBE_NO_LOOKBACK)
       return resolve_prefix_at_once<T, OP>(st, tile, block_total, wave, lane, s_front, limit, fold_tile);
     if (wave == 0) {
-      const T exclusive = ILGPU_HIP_SCAN_PROBE_NO_LOOKBACK || alone
+      const T exclusive = ILGPU_HIP_SCAN_PROBE_NO_LOOKBACK
                               ? F::identity()
                               : resolve_prefix<T, OP>(st, tile, block_total, lane, limit, fold_tile);
       if (lane == 0) s_prefix = exclusive;
@@ -488,18 +504,17 @@ __global__ __launch_bounds__(kBlock, ILGPU_HIP_SCAN_WAVES_PER_EU) void scan_kern
 #pragma unroll
         for (int k = 1; k < VN; ++k) r[k] = F::apply(running, x[j][k - 1]);
       }
-      if (VECTOR && full) {
+      const int e0 = (j * kWaveSize + lane) * VN;
+      if (VECTOR && (full || e0 + VN <= wave_valid)) {
         V v;
 #pragma unroll
         for (int k = 0; k < VN; ++k) v[k] = r[k];
         if (ILGPU_HIP_SCAN_NT_STORE) __builtin_nontemporal_store(v, &dst[j * kWaveSize + lane]);
         else dst[j * kWaveSize + lane] = v;
-      } else {
+      } else if (e0 < wave_valid) {
 #pragma unroll
-        for (int k = 0; k < VN; ++k) {
-          const int e = (j * kWaveSize + lane) * VN + k;
-          if (e < wave_valid) out[(wave_base + e) * out_stride] = r[k];
-        }
+        for (int k = 0; k < VN; ++k)
+          if (e0 + k < wave_valid) out[(wave_base + e0 + k) * out_stride] = r[k];
       }
       running = F::apply(running, seg_total[j]);
     }
@@ -551,18 +566,17 @@ __global__ __launch_bounds__(kBlock, ILGPU_HIP_SCAN_WAVES_PER_EU) void scan_kern
       if (inclusive) r[k] = F::apply(before, x[j][k]);
       else r[k] = k == 0 ? before : F::apply(before, x[j][k - 1]);
     }
-    if (VECTOR && full) {
+    const int e0 = (j * kWaveSize + lane) * VN;
+    if (VECTOR && (full || e0 + VN <= wave_valid)) {
       V v;
 #pragma unroll
       for (int k = 0; k < VN; ++k) v[k] = r[k];
       if (ILGPU_HIP_SCAN_NT_STORE) __builtin_nontemporal_store(v, &dst[j * kWaveSize + lane]);
       else dst[j * kWaveSize + lane] = v;
-    } else {
+    } else if (e0 < wave_valid) {
 #pragma unroll
-      for (int k = 0; k < VN; ++k) {
-        const int e = (j * kWaveSize + lane) * VN + k;
-        if (e < wave_valid) out[(wave_base + e) * out_stride] = r[k];
-      }
+      for (int k = 0; k < VN; ++k)
+        if (e0 + k < wave_valid) out[(wave_base + e0 + k) * out_stride] = r[k];
     }
     running = F::apply(running, seg_total[j]);
   }
@@ -790,8 +804,10 @@ int32_t launch_typed(hipStream_t stream, const void* in, int64_t in_stride,
   };
   const bool apart = end(in, in_stride) <= reinterpret_cast<uintptr_t>(out) ||
                      end(out, out_stride) <= reinterpret_cast<uintptr_t>(in);
-  if (tiles > 1 && tiles <= (apart ? kShortMaxTiles : kShortMaxTilesTicketed))
-    return launch_tiles<T, OP, scan_vecs<T>() / kShortDivisor>(
+  constexpr int kShortVecs = scan_vecs<T>() / kShortDivisor;
+  const bool one_short = n <= (int64_t)kBlock * kShortVecs * Vec16<T>::N;
+  if (one_short || (tiles > 1 && tiles <= (apart ? kShortMaxTiles : kShortMaxTilesTicketed)))
+    return launch_tiles<T, OP, kShortVecs>(
         stream, in, in_stride, out, out_stride, n, kind, temp, apart);
   return launch_tiles<T, OP, scan_vecs<T>()>(stream, in, in_stride, out, out_stride, n, kind, temp, apart);
 }

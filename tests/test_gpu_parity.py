@@ -1748,6 +1748,31 @@ def test_scan_into_another_view_and_over_its_input(dtype, op, polls):
         capi.sort_set_parameter(capi.SORT_PARAM_LOOKBACK_SPIN_LIMIT, -1)
 
 
+@pytest.mark.parametrize("dtype", [np.int32, np.int64, np.float32, np.float64])
+@pytest.mark.parametrize("first", [0, 1])
+def test_scan_of_a_last_tile_that_ends_inside_a_vector(dtype, first):
+    # Whole vectors and the one in which the view ends, of one short tile, one full tile and the last of
+    # many; from the first element on, where views are aligned, and from the second, where they are not.  What
+    # lies behind either view stays as it is.
+    full = 512 * 16 * 16 // np.dtype(dtype).itemsize
+    short = full // 4
+    for n in (1, 2, 3, 5, 63, 257, short - 1, short, short + 1, full - 3, full + 2, 193 * full + 7):
+        values = random_ints(np.int32, n, seed=n, lo=-3, hi=4).astype(dtype)
+        for inclusive in (True, False):
+            note("scan tail", np.dtype(dtype).name, n, first, inclusive)
+            want = O.scan(values, op=capi.OP_ADD, inclusive=inclusive)
+            for apart in (True, False):
+                room = D.from_numpy(np.full(first + n + 9, 77, dtype))
+                other = D.from_numpy(np.full(first + n + 9, 77, dtype)) if apart else room
+                room.subview(first, n).bytes.copy_(D.from_numpy(values).bytes)
+                capi.scan(room.subview(first, n), other.subview(first, n), op=capi.OP_ADD,
+                          kind=capi.SCAN_INCLUSIVE if inclusive else capi.SCAN_EXCLUSIVE)
+                sync()
+                got = other.numpy()
+                assert np.array_equal(got[first:first + n], want), (n, apart)
+                assert (got[:first] == 77).all() and (got[first + n:] == 77).all(), (n, apart)
+
+
 # ------------------------------------------------------------- dominant digits
 # A digit that holds an eighth of the keys or more is ranked by ballots instead
 # of LDS slots (up to four such digits per pass).
