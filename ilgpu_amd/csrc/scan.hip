@@ -505,12 +505,14 @@ __global__ __launch_bounds__(kBlock, ILGPU_HIP_SCAN_WAVES_PER_EU) void scan_kern
         for (int k = 1; k < VN; ++k) r[k] = F::apply(running, x[j][k - 1]);
       }
       const int e0 = (j * kWaveSize + lane) * VN;
-      if (VECTOR && (full || e0 + VN <= wave_valid)) {
-        V v;
+      V v;
 #pragma unroll
-        for (int k = 0; k < VN; ++k) v[k] = r[k];
+      for (int k = 0; k < VN; ++k) v[k] = r[k];
+      if (VECTOR && full) {
         if (ILGPU_HIP_SCAN_NT_STORE) __builtin_nontemporal_store(v, &dst[j * kWaveSize + lane]);
         else dst[j * kWaveSize + lane] = v;
+      } else if (VECTOR && e0 + VN <= wave_valid) {
+        dst[j * kWaveSize + lane] = v;
       } else if (e0 < wave_valid) {
 #pragma unroll
         for (int k = 0; k < VN; ++k)
@@ -567,12 +569,14 @@ __global__ __launch_bounds__(kBlock, ILGPU_HIP_SCAN_WAVES_PER_EU) void scan_kern
       else r[k] = k == 0 ? before : F::apply(before, x[j][k - 1]);
     }
     const int e0 = (j * kWaveSize + lane) * VN;
-    if (VECTOR && (full || e0 + VN <= wave_valid)) {
-      V v;
+    V v;
 #pragma unroll
-      for (int k = 0; k < VN; ++k) v[k] = r[k];
+    for (int k = 0; k < VN; ++k) v[k] = r[k];
+    if (VECTOR && full) {
       if (ILGPU_HIP_SCAN_NT_STORE) __builtin_nontemporal_store(v, &dst[j * kWaveSize + lane]);
       else dst[j * kWaveSize + lane] = v;
+    } else if (VECTOR && e0 + VN <= wave_valid) {
+      dst[j * kWaveSize + lane] = v;
     } else if (e0 < wave_valid) {
 #pragma unroll
       for (int k = 0; k < VN; ++k)
