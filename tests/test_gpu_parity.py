@@ -1773,6 +1773,37 @@ def test_scan_of_a_last_tile_that_ends_inside_a_vector(dtype, first):
                 assert (got[:first] == 77).all() and (got[first + n:] == 77).all(), (n, apart)
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("op", [capi.OP_MAX, capi.OP_MIN])
+def test_scan_max_min_bit_for_bit(dtype, op):
+    # Of NaNs of either sign and any payload the first wins; the zeros are ordered; subnormal numbers are
+    # kept.  Every result is one of the inputs, bit for bit.
+    bits = np.dtype(f"uint{8 * np.dtype(dtype).itemsize}").type
+    sign = bits(1) << bits(8 * np.dtype(dtype).itemsize - 1)
+    tiny = np.array([0, 1, 2], bits)
+    outward = 1 if op == capi.OP_MAX else -1
+    nans = np.array([np.nan], dtype).view(bits) | np.array([0, 5, 9], bits)
+    for seed, n in enumerate((40, 700, 5000, 70001)):
+        r = np.random.default_rng(seed)
+        values = -outward * np.sort(r.random(n)).astype(dtype)[::-1]  # new extremes all along
+        values[r.integers(0, n, n // 5)] = dtype(-outward * 3)
+        for at, few in ((n // 2, tiny | sign), (n // 2 + n // 10, tiny)):
+            where = np.arange(at, at + n // 12)
+            values.view(bits)[where] = r.choice(few, where.size)
+        values[n - n // 5] = outward * np.inf
+        values.view(bits)[n - n // 10:] = r.choice(np.concatenate([nans, nans | sign]), n // 10)
+        want, best = np.zeros(n, bits), 0
+        for i in range(n):
+            a, b = values[best], values[i]
+            if not np.isnan(a) and (np.isnan(b) or (b - a) * outward > 0 or
+                                    (a == b == 0 and np.signbit(a) != np.signbit(b) and
+                                     np.signbit(a) == (outward > 0))):
+                best = i
+            want[i] = values.view(bits)[best]
+        note("scan max min bits", np.dtype(dtype).name, op, n)
+        assert np.array_equal(gpu_scan(values, op, True).view(bits), want), n
+
+
 # ------------------------------------------------------------- dominant digits
 # A digit that holds an eighth of the keys or more is ranked by ballots instead
 # of LDS slots (up to four such digits per pass).
