@@ -879,6 +879,33 @@ __global__ __launch_bounds__(kHistBlock) void sort_histogram_kernel(
   }
 }
 
+// `join` over the lanes up to each one, for values that zero leaves as they are: six moves between lanes in place of trips to
+// the LDS.
+template <typename Join>
+__device__ __forceinline__ uint32_t wave_inclusive(uint32_t v, Join join) {
+  v = join(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false));  // row_shr:1
+  v = join(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false));
+  v = join(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false));
+  v = join(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false));
+  v = join(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));  // row_bcast:15
+  v = join(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));  // row_bcast:31
+  return v;
+}
+// Over all of them, in every lane: OR, the sum and the largest.
+template <typename Join>
+__device__ __forceinline__ uint32_t wave_join(uint32_t v, Join join) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)wave_inclusive(v, join), kWaveSize - 1);
+}
+__device__ __forceinline__ uint32_t wave_or(uint32_t v) {
+  return wave_join(v, [](uint32_t a, uint32_t b) { return a | b; });
+}
+__device__ __forceinline__ int wave_sum(int v) {
+  return (int)wave_join((uint32_t)v, [](uint32_t a, uint32_t b) { return a + b; });
+}
+__device__ __forceinline__ uint32_t wave_most(uint32_t v) {
+  return wave_join(v, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
+}
+
 // ---- plan: exclusive digit offsets, skipped passes, buffer parity ---------
 // One block; every 256 threads take a digit position, four at a time.  (One position after the other,
 // a chain of barriers, took 4.5 us for 4-byte keys and 8.4 for 8-byte keys.)
@@ -921,15 +948,11 @@ __global__ __launch_bounds__(kPlanBlock) void plan_kernel(
 #pragma unroll
   for (int r = 0; r < kRounds; ++r) {
     const int p = r * kPlanGroups + group;
+    inclusive[r] = 0u;
+    if (r * kPlanGroups >= passes) break;
     const uint32_t c = counts[r];
-    uint32_t inc = c, most = c;
-#pragma unroll
-    for (int s = 1; s < kWaveSize; s <<= 1) {
-      const uint32_t o = shfl_up(inc, s);
-      if (lane >= s) inc += o;
-      const uint32_t q = shfl(most, lane ^ s);
-      most = most < q ? q : most;
-    }
+    const uint32_t inc = wave_inclusive(c, [](uint32_t a, uint32_t b) { return a + b; });
+    const uint32_t most = wave_most(c);
     inclusive[r] = inc;
     if (lane == kWaveSize - 1) s_wave[p][wave] = inc;
     if (lane == 0) atomicMax(&s_most[p], most);
@@ -2378,24 +2401,6 @@ __device__ __forceinline__ bool small_sort_spreads(int pairs, int n) {
   const int64_t m = n > kSortBlock ? n : kSortBlock;
   const int64_t run = kSortBlock * (30 + m / 256);
   return 2 * pairs * m * m <= run * run;
-}
-
-// OR over the lanes of a wave, and the sum, in every lane.
-template <typename Join>
-__device__ __forceinline__ uint32_t wave_join(uint32_t v, Join join) {
-  v = join(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false));  // row_shr:1
-  v = join(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false));
-  v = join(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false));
-  v = join(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false));
-  v = join(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));  // row_bcast:15
-  v = join(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));  // row_bcast:31
-  return (uint32_t)__builtin_amdgcn_readlane((int)v, kWaveSize - 1);
-}
-__device__ __forceinline__ uint32_t wave_or(uint32_t v) {
-  return wave_join(v, [](uint32_t a, uint32_t b) { return a | b; });
-}
-__device__ __forceinline__ int wave_sum(int v) {
-  return (int)wave_join((uint32_t)v, [](uint32_t a, uint32_t b) { return a + b; });
 }
 
 constexpr int kSmallSortItemsA = 4, kSmallSortItemsB = 12, kSmallSortItemsC = 24;
