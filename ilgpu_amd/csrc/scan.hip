@@ -100,11 +100,11 @@ template <typename T> constexpr int tile_elems() {
 // Their status words stand a quarter of a line apart, so that they fit the
 // temp view of the full tiles; that few words are not what such an input waits for.
 // So does an input of one short tile, which is one launch like one full tile, with a quarter of its rows (calls, us,
-// full / short: 1000 and 4000 double Max 18.5 and 18.9 / 7.1 and 7.4); between one short tile and one full one the launch that
+// full / short: 1000 and 4000 double Max 12.3 and 12.3 / 7.1 and 7.1); between one short tile and one full one the launch that
 // clears the status words costs more than the short tiles save (16384 int64 7.4 / 10.0).
-// (Calls, us, tickets and a walk / no tickets and full tiles / short ones: 2.5 * 10^6 double Max 27.6 / 27.3 / 17.7,
-// 3.5 * 10^6 29.6 / 28.4 / 23.8, 2.5 * 10^6 int32 14.4 / 9.6 / 9.6, 6.3 * 10^6 14.6 / 13.8 / 11.7, 2^21 int64 13.0 / 12.4 /
-// 10.5, 3 * 10^6 14.7 / 13.7 / 12.6, but 3.5 * 10^6, 214 full tiles, 15.5 / 14.0 / 15.1 and 2^22 17.7 / 14.8 / 18.0.
+// (Calls, us, full tiles / short ones: 2^21 double Max 18.4 / 12.8, 3 * 10^6 18.6 / 14.9, 2.5 * 10^6 int32 10.9 / 9.4,
+// 6.3 * 10^6 12.0 / 11.9, 2^21 int64 12.3 / 10.3, 3 * 10^6 12.6 / 12.1, but 3.5 * 10^6, 214 full tiles, 13.3 / 18.4, double Max
+// 18.7 / 22.3, and 2^22 int64 14.6 / 21.1.  With tickets, which come one after the other, 2^21 int64 13.0.
 // Tiles an eighth as long: 10^6 double Max 12.3 against 11.1, 2^21 int64 16.1 against 10.6.)
 #ifndef ILGPU_HIP_SCAN_SHORT_DIVISOR
 #define ILGPU_HIP_SCAN_SHORT_DIVISOR 4
@@ -665,16 +665,32 @@ __global__ __launch_bounds__(kBlock) void unique_kernel(
   // The element in front of the wave's chunk; every other predecessor is in a
   // register of this wave.
   const T chunk_before = wave_base > 0 && wave_base < n ? data[wave_base - 1] : T();
+  // Elements of this wave's chunk that lie inside the view.
+  const int64_t inside = n - wave_base;
+  const int wave_valid = (int)(inside < kWaveElems ? (inside < 0 ? 0 : inside) : kWaveElems);
+  if (VECTOR && full) {
+    const V* src = reinterpret_cast<const V*>(data + wave_base);
 #pragma unroll
-  for (int j = 0; j < kUniqueVecs; ++j) {
-    const int64_t first = wave_base + (int64_t)(j * kWaveSize + lane) * VN;
-    if (VECTOR && full) {
-      const V v = __builtin_nontemporal_load(reinterpret_cast<const V*>(data + first));
+    for (int j = 0; j < kUniqueVecs; ++j) {
+      const V v = __builtin_nontemporal_load(&src[j * kWaveSize + lane]);
 #pragma unroll
       for (int k = 0; k < VN; ++k) x[j][k] = v[k];
-    } else {
+    }
+  } else {
 #pragma unroll
-      for (int k = 0; k < VN; ++k) x[j][k] = first + k < n ? data[first + k] : T();
+    for (int j = 0; j < kUniqueVecs; ++j) {
+      const int e0 = (j * kWaveSize + lane) * VN;
+#pragma unroll
+      for (int k = 0; k < VN; ++k) x[j][k] = T();
+      if (VECTOR && e0 + VN <= wave_valid) {
+        const V v = *reinterpret_cast<const V*>(data + wave_base + e0);
+#pragma unroll
+        for (int k = 0; k < VN; ++k) x[j][k] = v[k];
+      } else if (e0 < wave_valid) {
+#pragma unroll
+        for (int k = 0; k < VN; ++k)
+          if (e0 + k < wave_valid) x[j][k] = data[wave_base + e0 + k];
+      }
     }
   }
   T before[kUniqueVecs];  // the element in front of each vector
@@ -686,23 +702,39 @@ __global__ __launch_bounds__(kBlock) void unique_kernel(
   }
 
   // keep bit k of vector j; kept elements per vector; wave scan per row.
+  // The counts of a few rows, up to 64 * VN each, go through one scan.  (With a scan for each row, element after element
+  // asked whether it lies inside the view, and whole rows without a kept element stored lane by lane, 123
+  // registers instead of 93: sorted Zipf keys, 2^26 u32, 82 -> 72 us, 2^27 of them 302 -> 287 with their copy.)
+  constexpr int kRowsAScan = VN <= 8 ? 3 : 2, kRowBits = 32 / kRowsAScan;
+  static_assert(kWaveSize * VN < 1 << kRowBits, "a row's total has its bits");
   uint32_t keep[kUniqueVecs], lane_excl[kUniqueVecs], seg_total[kUniqueVecs];
 #pragma unroll
   for (int j = 0; j < kUniqueVecs; ++j) {
-    const int64_t first = wave_base + (int64_t)(j * kWaveSize + lane) * VN;
     uint32_t bits = 0;
 #pragma unroll
-    for (int k = 0; k < VN; ++k) {
-      const bool valid = first + k < n;
-      const bool is_first = first + k == 0;
-      const bool d = differs<T>(x[j][k], k == 0 ? before[j] : x[j][k - 1]);
-      if (valid && (is_first || d)) bits |= 1u << k;
+    for (int k = 0; k < VN; ++k)
+      bits |= (differs<T>(x[j][k], k == 0 ? before[j] : x[j][k - 1]) ? 1u : 0u) << k;
+    if (j == 0 && wave_base == 0 && lane == 0) bits |= 1u;  // the first element of all
+    if (!full) {
+      const int left = wave_valid - (j * kWaveSize + lane) * VN;
+      bits &= left >= VN ? (1u << VN) - 1u : (left <= 0 ? 0u : (1u << left) - 1u);
     }
     keep[j] = bits;
-    const uint32_t cnt = (uint32_t)__popc(bits);
+  }
+#pragma unroll
+  for (int j0 = 0; j0 < kUniqueVecs; j0 += kRowsAScan) {
+    uint32_t cnt = 0;
+#pragma unroll
+    for (int r = 0; r < kRowsAScan; ++r)
+      if (j0 + r < kUniqueVecs) cnt |= (uint32_t)__popc(keep[j0 + r]) << (r * kRowBits);
     const uint32_t inc = wave_inclusive_scan<uint32_t, ILGPU_HIP_OP_ADD>(cnt, lane);
-    seg_total[j] = shfl(inc, kWaveSize - 1);
-    lane_excl[j] = inc - cnt;
+    const uint32_t all = read_lane<uint32_t>(inc, kWaveSize - 1), front = inc - cnt;
+#pragma unroll
+    for (int r = 0; r < kRowsAScan; ++r)
+      if (j0 + r < kUniqueVecs) {
+        seg_total[j0 + r] = all >> (r * kRowBits) & ((1u << kRowBits) - 1u);
+        lane_excl[j0 + r] = front >> (r * kRowBits) & ((1u << kRowBits) - 1u);
+      }
   }
   uint32_t wave_total = 0;
 #pragma unroll
@@ -727,6 +759,7 @@ __global__ __launch_bounds__(kBlock) void unique_kernel(
   uint32_t running = s_prefix + wave_prefix;
 #pragma unroll
   for (int j = 0; j < kUniqueVecs; ++j) {
+    if (seg_total[j] == 0u) continue;  // (wave-uniform)
     uint32_t pos = running + lane_excl[j];
     if (keep[j] == (1u << VN) - 1u) {
       // the whole vector survives: one 16-byte store, aligned like an element
