@@ -631,18 +631,24 @@ template <typename T> __device__ __forceinline__ bool differs(T a, T b) {
   else return a != b;
 }
 
-template <typename T> constexpr int unique_tile_elems() {
-  return kBlock * unique_vecs(sizeof(T)) * Vec16<T>::N;
+template <typename T, int VECS> constexpr int unique_tile_elems() {
+  return kBlock * VECS * Vec16<T>::N;
 }
+// Of 4-byte elements that fill the chip with such tiles once (two blocks a compute unit): longer ones, as many as fit 128
+// registers, for fewer tickets and trips between tiles.  (us with a copy of the keys, 12 vectors / 16: sorted Zipf
+// u32 2^27 287 / 273, 2^26 153 / 145, distinct int32 2^27 363 / 354, 3 * 10^7 80.2 / 77.8, but 3 * 10^6, 92 tiles, 18.5 / 21.6.
+// 8-byte elements: 2^27 distinct 707 / 714, 14 vectors 702; 3 * 10^7 171.6 / 174.2, 172.5.)
+constexpr int unique_long_vecs(int elem_bytes) { return elem_bytes == 4 ? 16 : unique_vecs(elem_bytes); }
+constexpr int64_t kUniqueLongTiles = 512;
 
-template <typename T, bool VECTOR>
+template <typename T, bool VECTOR, int VECS>
 __global__ __launch_bounds__(kBlock) void unique_kernel(
     T* data, int64_t n, int64_t* __restrict__ out_length,
     uint32_t* __restrict__ ticket, TileState<uint32_t> st, int num_tiles) {
   using V = typename Vec16<T>::type;
   constexpr int VN = Vec16<T>::N;
-  constexpr int kUniqueVecs = unique_vecs(sizeof(T));
-  constexpr int kTile = unique_tile_elems<T>();
+  constexpr int kUniqueVecs = VECS;
+  constexpr int kTile = unique_tile_elems<T, VECS>();
   constexpr int kWaveElems = kTile / kWaves;
 
   __shared__ int s_tile;
@@ -704,7 +710,7 @@ __global__ __launch_bounds__(kBlock) void unique_kernel(
   // keep bit k of vector j; kept elements per vector; wave scan per row.
   // The counts of a few rows, up to 64 * VN each, go through one scan.  (With a scan for each row, element after element
   // asked whether it lies inside the view, and whole rows without a kept element stored lane by lane, 123
-  // registers instead of 93: sorted Zipf keys, 2^26 u32, 82 -> 72 us, 2^27 of them 302 -> 287 with their copy.)
+  // registers instead of 93 for 12 vectors: sorted Zipf keys, 2^26 u32, 82 -> 72 us, 2^27 of them 302 -> 287 with their copy.)
   constexpr int kRowsAScan = VN <= 8 ? 3 : 2, kRowBits = 32 / kRowsAScan;
   static_assert(kWaveSize * VN < 1 << kRowBits, "a row's total has its bits");
   uint32_t keep[kUniqueVecs], lane_excl[kUniqueVecs], seg_total[kUniqueVecs];
@@ -955,10 +961,10 @@ int64_t unique_temp_bytes(int64_t n, int elem_bytes) {
 }
 
 namespace {
-template <typename T>
-int32_t launch_unique_typed(hipStream_t stream, void* data, int64_t n,
+template <typename T, int VECS>
+int32_t launch_unique_tiles(hipStream_t stream, void* data, int64_t n,
                             int64_t* out_length, void* temp) {
-  const int64_t tiles = div_up(n, (int64_t)unique_tile_elems<T>());
+  const int64_t tiles = div_up(n, (int64_t)unique_tile_elems<T, VECS>());
   char* base = reinterpret_cast<char*>(align_up((int64_t)(uintptr_t)temp, 256));
   uint32_t* ticket = reinterpret_cast<uint32_t*>(base);
   TileState<uint32_t> st;
@@ -973,15 +979,25 @@ int32_t launch_unique_typed(hipStream_t stream, void* data, int64_t n,
   const bool vector = (reinterpret_cast<uintptr_t>(data) & 15) == 0;
   ProfileScope scope(stream, "unique");
   if (vector)
-    hipLaunchKernelGGL((unique_kernel<T, true>), dim3((unsigned)tiles), dim3(kBlock), 0,
+    hipLaunchKernelGGL((unique_kernel<T, true, VECS>), dim3((unsigned)tiles), dim3(kBlock), 0,
                        stream, static_cast<T*>(data), n, out_length, ticket, st,
                        (int)tiles);
   else
-    hipLaunchKernelGGL((unique_kernel<T, false>), dim3((unsigned)tiles), dim3(kBlock), 0,
+    hipLaunchKernelGGL((unique_kernel<T, false, VECS>), dim3((unsigned)tiles), dim3(kBlock), 0,
                        stream, static_cast<T*>(data), n, out_length, ticket, st,
                        (int)tiles);
   ILGPU_HIP_CHECK(hipGetLastError());
   return ILGPU_HIP_SUCCESS;
+}
+
+template <typename T>
+int32_t launch_unique_typed(hipStream_t stream, void* data, int64_t n,
+                            int64_t* out_length, void* temp) {
+  constexpr int kVecs = unique_vecs(sizeof(T)), kLongVecs = unique_long_vecs(sizeof(T));
+  static_assert(kLongVecs >= kVecs, "the temp view is sized for the shorter tiles");
+  if (kLongVecs != kVecs && n >= kUniqueLongTiles * unique_tile_elems<T, kLongVecs>())
+    return launch_unique_tiles<T, kLongVecs>(stream, data, n, out_length, temp);
+  return launch_unique_tiles<T, kVecs>(stream, data, n, out_length, temp);
 }
 }  // namespace
 

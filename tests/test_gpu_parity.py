@@ -1357,6 +1357,20 @@ def test_unique_all_equal_and_all_distinct_large():
     assert count == n and np.array_equal(kept, seq)
 
 
+@pytest.mark.parametrize("dtype", [np.int32, np.float32])
+def test_unique_of_long_tiles(dtype):
+    # From 512 tiles of 32768 4-byte elements on; the last one whole, with an end inside a vector, and of one
+    # element; few runs, so that whole rows keep nothing, and one to two elements each.
+    most = 512 * 32768
+    for n in (most - 1, most, most + 1, most + 2 * 32768 - 3):
+        for runs in (70_000, n * 2 // 3):
+            note("unique long tiles", np.dtype(dtype).name, n, runs)
+            values = np.sort(np.random.default_rng(n).integers(0, runs, n, dtype=np.int32)).astype(dtype)
+            want = values[np.concatenate([[True], values[1:] != values[:-1]])]
+            kept, _, count = gpu_unique(values)
+            assert count == want.size and np.array_equal(kept, want), (n, runs)
+
+
 def test_unique_unaligned_view():
     vals = np.repeat(np.arange(5000, dtype=np.int32), 3)
     base = D.from_numpy(np.concatenate([np.array([99], np.int32), vals]))
