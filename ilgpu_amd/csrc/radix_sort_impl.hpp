@@ -1109,6 +1109,10 @@ __device__ __forceinline__ void load_tile_keys(
 // registers (36 keys and 18 registers of packed ranks in a keys-only sort;
 // fewer items when values ride along) and the blocks of a CU at 160 KiB of
 // LDS together (a 36-key tile stages 72 KiB per 512 threads).
+// Where the code of the large kernels begins.  A tile runs through 40 to 64 KiB of code, which the instruction caches
+// barely hold, and where it lies moved the same instructions by up to 8 us a pass whenever a kernel in front of it
+// grew.  (2^28 u32, us, two boxes, wherever the linker puts it / here: 2059 / 2053 and 2053 / 2048; the others within 0.2 %.)
+#define ILGPU_HIP_SORT_CODE_ALIGNED __attribute__((aligned(4096)))
 #ifndef ILGPU_HIP_SORT_WAVES_PER_EU
 #define ILGPU_HIP_SORT_WAVES_PER_EU 4
 #endif
@@ -1512,7 +1516,7 @@ __device__ __forceinline__ void sort_tile(
 // AT_ONCE: one tile per block, which is not handed out (see below), and a look-back for tiles that all run at the same
 // time.
 template <int KEY_BYTES, int VALUE_BYTES, bool FLOAT_KEYS, int BLOCK, int ITEMS, bool AT_ONCE>
-__global__ __launch_bounds__(BLOCK, ILGPU_HIP_SORT_WAVES_PER_EU)
+__global__ __launch_bounds__(BLOCK, ILGPU_HIP_SORT_WAVES_PER_EU) ILGPU_HIP_SORT_CODE_ALIGNED
 void onesweep_kernel(
     typename KeyOf<KEY_BYTES>::type* keys_a,
     typename KeyOf<KEY_BYTES>::type* keys_b,
@@ -2059,7 +2063,7 @@ __device__ __forceinline__ void pipelined_scan(
 }
 
 template <int KEY_BYTES, bool FLOAT_KEYS>
-__global__ __launch_bounds__(1024, ILGPU_HIP_SORT_WAVES_PER_EU)
+__global__ __launch_bounds__(1024, ILGPU_HIP_SORT_WAVES_PER_EU) ILGPU_HIP_SORT_CODE_ALIGNED
 void onesweep_pipelined_kernel(
     typename KeyOf<KEY_BYTES>::type* keys_a, typename KeyOf<KEY_BYTES>::type* keys_b, int64_t n,
     int pass, KeyXform xf, const uint32_t* __restrict__ excl, uint32_t* all_status, uint32_t* ticket,

@@ -380,7 +380,7 @@ struct LocalRows {
 };
 
 template <int KEY_BYTES, int VALUE_BYTES, bool FLOAT_KEYS>
-__global__ __launch_bounds__(LocalBlock::kBlock, 4) void local_sort_kernel(
+__global__ __launch_bounds__(LocalBlock::kBlock, 4) ILGPU_HIP_SORT_CODE_ALIGNED void local_sort_kernel(
     typename KeyOf<KEY_BYTES>::type* keys_a, typename KeyOf<KEY_BYTES>::type* keys_b,
     typename ValueOf<VALUE_BYTES>::type* vals_a, typename ValueOf<VALUE_BYTES>::type* vals_b, uint32_t n,
     KeyXform xf, const SortPlan* __restrict__ plan, const uint32_t* __restrict__ excl, int values_from_index,
