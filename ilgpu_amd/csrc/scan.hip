@@ -22,8 +22,8 @@
 // missing tile is folded from the input (resolve_prefix).  Where the output overlaps the input, which may be
 // overwritten by then, tile ids come from a global ticket instead, and a tile's predecessors have always
 // started; a ticket costs a tile a round trip before its loads and 12 to 18 ns behind the ticket before
-// (calls, us, with tickets / without: 2^23 int64 31.5 / 23.5, 2^22 17.6 / 14.8, 2^23 int32 17.5 / 14.6,
-// 10^6 double Max 14.0 / 11.2, 2^28 int32 361 / 357.5).  Status words are read and written with agent-scope atomics: the
+// (calls, us, over the input, with tickets / into another view: 2^23 int64 32.2 / 23.1, 2^22 18.8 / 15.0, 2^23 int32
+// 17.4 / 14.1, 10^6 double Max 13.2 / 11.2, 2^28 int32 354.6 / 347.4).  Status words are read and written with agent-scope atomics: the
 // eight XCDs of the device have separate L2s.
 //   4-byte T: one 64-bit word {flag, value} per tile;
 //   8-byte T: two such words per tile, one per half of the value.
@@ -357,7 +357,8 @@ __device__ __forceinline__ T resolve_prefix_at_once(const TileState<T, STRIDE>& 
 
 // Four waves per SIMD, i.e. 128 registers and two blocks per CU: left to itself
 // the compiler takes 180 to 256 registers for the floating-point Max and Min
-// kernels, which halves their residency (measured 0.56 -> 0.44 ms at 2^28 float).
+// kernels, which halves their residency (0.56 -> 0.44 ms at 2^28 float, 0.36 since those
+// take three compares: fp_extreme).
 template <typename T, int OP, bool VECTOR, int VECS>
 __global__ __launch_bounds__(kBlock, ILGPU_HIP_SCAN_WAVES_PER_EU) void scan_kernel(
     const T* __restrict__ in, T* __restrict__ out, int64_t n,
