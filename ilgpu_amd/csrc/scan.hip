@@ -280,13 +280,10 @@ __device__ __forceinline__ T lane_shift_up(T fill, T v) {
   return dpp_move<T, 0x138, 0xf>(fill, v);
 }
 
+// Fold over the lanes of a wave, from lane 0 to lane 63 in this order, in every lane.
 template <typename T, int OP>
-__device__ __forceinline__ T wave_reduce(T v) {
-  using F = Functor<T, OP>;
-#pragma unroll
-  for (int off = kWaveSize / 2; off > 0; off >>= 1)
-    v = F::apply(v, shfl_down(v, off));
-  return shfl(v, 0);
+__device__ __forceinline__ T wave_fold(T v, int lane) {
+  return read_lane<T>(wave_inclusive_scan<T, OP>(v, lane), kWaveSize - 1);
 }
 
 // Executed by the first wave of the block.  Publishes the tile's aggregate,
@@ -305,7 +302,7 @@ __device__ __forceinline__ T resolve_prefix(const TileState<T, STRIDE>& st, int 
   T exclusive = F::identity();
   int base = tile - 1;
   while (true) {
-    const int idx = base - lane;
+    const int idx = base - (kWaveSize - 1 - lane);  // in the input's order: of two NaNs the first wins
     T val = F::identity();
     uint32_t flag = kFlagPrefix;  // virtual prefix in front of tile 0
     if (idx >= 0) {
@@ -313,13 +310,10 @@ __device__ __forceinline__ T resolve_prefix(const TileState<T, STRIDE>& st, int 
       if (flag == kFlagInvalid) val = fold(idx);
     }
     const uint64_t has_prefix = __ballot(flag == kFlagPrefix);
-    // Lanes run from the nearest predecessor (lane 0) to the farthest; the
-    // first lane holding an inclusive prefix ends the walk.
-    const int first = has_prefix != 0
-                          ? __ffsll((unsigned long long)has_prefix) - 1
-                          : kWaveSize - 1;
-    const T contrib = lane <= first ? val : F::identity();
-    exclusive = F::apply(wave_reduce<T, OP>(contrib), exclusive);
+    // The nearest inclusive prefix ends the walk.
+    const int nearest = has_prefix != 0 ? kWaveSize - 1 - __builtin_clzll(has_prefix) : 0;
+    const T contrib = lane >= nearest ? val : F::identity();
+    exclusive = F::apply(wave_fold<T, OP>(contrib, lane), exclusive);
     if (has_prefix != 0) break;  // wave-uniform
     base -= kWaveSize;
   }
@@ -346,7 +340,7 @@ __device__ __forceinline__ T resolve_prefix_at_once(const TileState<T, STRIDE>& 
     if (front < tile && st.wait(front, &one, limit) == kFlagInvalid) one = fold(front);
     val = F::apply(val, one);
   }
-  const T front = read_lane<T>(wave_inclusive_scan<T, OP>(val, lane), kWaveSize - 1);
+  const T front = wave_fold<T, OP>(val, lane);
   if (lane == 0) s_front[wave] = front;
   __syncthreads();
   T exclusive = s_front[0];

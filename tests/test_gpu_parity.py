@@ -1818,6 +1818,32 @@ def test_scan_max_min_bit_for_bit(dtype, op):
         assert np.array_equal(gpu_scan(values, op, True).view(bits), want), n
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("op", [capi.OP_MAX, capi.OP_MIN])
+@pytest.mark.parametrize("over_the_input", [True, False])
+def test_scan_the_first_of_the_nans_of_many_tiles_wins(dtype, op, over_the_input):
+    # Every tile from the fourth on has a NaN of its own payload, so what a tile finds in front of it are NaNs: prefixes, and
+    # up to 64 tiles' own.  In short tiles and in full ones, those by tickets over the input and without beside it.
+    size = np.dtype(dtype).itemsize
+    full = 512 * 16 * 16 // size
+    bits = np.dtype(f"uint{8 * size}").type
+    outward = 1 if op == capi.OP_MAX else -1
+    for tile, n in ((full // 4, 50 * full), (full, 260 * full - 5)):
+        values = (-outward * np.random.default_rng(n).random(n)).astype(dtype)
+        values[::1009] += dtype(outward) * np.arange(values[::1009].size, dtype=dtype)
+        where = np.arange(3 * tile + 77, n, tile)
+        values.view(bits)[where] = np.array([np.nan], dtype).view(bits) | (np.arange(where.size).astype(bits) + bits(1))
+        reference = np.maximum if op == capi.OP_MAX else np.minimum
+        want = reference.accumulate(values[:where[0]]).view(bits)
+        want = np.concatenate([want, np.full(n - where[0], values.view(bits)[where[0]])])
+        note("scan nans of tiles", np.dtype(dtype).name, op, over_the_input, n)
+        source = D.from_numpy(values)
+        target = source if over_the_input else D.zeros(n, dtype)
+        capi.scan(source, target, op=op)
+        sync()
+        assert np.array_equal(target.numpy().view(bits), want), n
+
+
 # ------------------------------------------------------------- dominant digits
 # A digit that holds an eighth of the keys or more is ranked by ballots instead
 # of LDS slots (up to four such digits per pass).
