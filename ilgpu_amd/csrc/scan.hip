@@ -154,28 +154,21 @@ template <typename T, int STRIDE> struct TileState<T, STRIDE, 4> {
     __hip_atomic_store(&words[(int64_t)tile * STRIDE], w, __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
   }
-  // Spins until the tile has published something; returns its flag, or kFlagInvalid
-  // after `limit` polls.
-  __device__ __forceinline__ uint32_t wait(int tile, T* v, uint32_t limit = kNoLimit) const {
-    uint64_t w;
-    uint32_t polls = 0;
-    while (true) {
-      w = __hip_atomic_load(&words[(int64_t)tile * STRIDE], __ATOMIC_RELAXED,
-                            __HIP_MEMORY_SCOPE_AGENT);
-      if ((uint32_t)(w >> 32) != kFlagInvalid) break;
-      if (limit != kNoLimit && polls++ >= limit) return kFlagInvalid;
-      __builtin_amdgcn_s_sleep(1);
-    }
-    *v = from_bits<T>((uint32_t)w);
-    return (uint32_t)(w >> 32);
+  // What the tile has published: its flag, and the value unless that is kFlagInvalid.
+  __device__ __forceinline__ uint32_t read(int tile, T* v) const {
+    const uint64_t w = __hip_atomic_load(&words[(int64_t)tile * STRIDE], __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t flag = (uint32_t)(w >> 32);
+    if (flag != kFlagInvalid) *v = from_bits<T>((uint32_t)w);
+    return flag;
   }
 };
 
 // 8-byte values: two 64-bit words in the tile's line, {flag, low half} and
 // {flag, high half}, each written and read with one relaxed atomic.  A tile writes each
 // state (aggregate, then prefix) once, so two words with the same flag hold
-// the halves of the same value; a reader that catches the words in different
-// states reads again.  No fences: an agent-scope release would write back the
+// the halves of the same value; to a reader that catches the words in different
+// states nothing has been published yet.  No fences: an agent-scope release would write back the
 // whole L2 of the XCD for every tile.
 template <typename T, int STRIDE> struct TileState<T, STRIDE, 8> {
   uint64_t* words;
@@ -187,17 +180,11 @@ template <typename T, int STRIDE> struct TileState<T, STRIDE, 8> {
     __hip_atomic_store(&w[1], ((uint64_t)flag << 32) | (bits >> 32),
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  __device__ __forceinline__ uint32_t wait(int tile, T* v, uint32_t limit = kNoLimit) const {
-    uint64_t lo, hi;
-    uint32_t polls = 0;
+  __device__ __forceinline__ uint32_t read(int tile, T* v) const {
     const uint64_t* w = &words[(int64_t)tile * STRIDE];
-    while (true) {
-      lo = __hip_atomic_load(&w[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      hi = __hip_atomic_load(&w[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if ((uint32_t)(lo >> 32) != kFlagInvalid && (lo >> 32) == (hi >> 32)) break;
-      if (limit != kNoLimit && polls++ >= limit) return kFlagInvalid;
-      __builtin_amdgcn_s_sleep(1);
-    }
+    const uint64_t lo = __hip_atomic_load(&w[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint64_t hi = __hip_atomic_load(&w[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if ((uint32_t)(lo >> 32) == kFlagInvalid || (lo >> 32) != (hi >> 32)) return kFlagInvalid;
     *v = from_bits<T>((uint64_t)(uint32_t)lo | (hi << 32));
     return (uint32_t)(lo >> 32);
   }
@@ -286,10 +273,43 @@ __device__ __forceinline__ T wave_fold(T v, int lane) {
   return read_lane<T>(wave_inclusive_scan<T, OP>(v, lane), kWaveSize - 1);
 }
 
+// The aggregate of tile t, a full one, from the input, by one wave.  In the order in which the tile itself
+// adds up (the vectors of a row, the rows of a wave, the waves), so that it is the same value bit for bit and a sum of
+// floating-point numbers is no less exact for it.  Row after row: it runs where a tile is late, while the tile of
+// its own block is held in registers, which more loads in flight would spill.
+template <typename T, int OP, bool VECTOR, int VECS>
+__device__ __forceinline__ T fold_tile(const T* __restrict__ in, int64_t in_stride, int t, int lane) {
+  using F = Functor<T, OP>;
+  using V = typename Vec16<T>::type;
+  constexpr int VN = Vec16<T>::N;
+  const T* row = in + (int64_t)t * (kBlock * VECS * VN) * (VECTOR ? 1 : in_stride);  // (wave-uniform)
+  T total = F::identity(), wave_total = F::identity();
+#pragma unroll 1
+  for (int j = 0; j < kWaves * VECS; ++j) {
+    T sum;
+    if constexpr (VECTOR) {
+      const V v = reinterpret_cast<const V*>(row)[lane];
+      sum = v[0];
+#pragma unroll
+      for (int k = 1; k < VN; ++k) sum = F::apply(sum, v[k]);
+    } else {
+      const T* p = row + (int64_t)(lane * VN) * in_stride;
+      sum = *p;
+#pragma unroll 1
+      for (int k = 1; k < VN; ++k) sum = F::apply(sum, *(p += in_stride));
+    }
+    row += kWaveSize * VN * (VECTOR ? 1 : in_stride);
+    sum = wave_fold<T, OP>(sum, lane);
+    wave_total = j % VECS == 0 ? sum : F::apply(wave_total, sum);
+    if (j % VECS == VECS - 1) total = j == VECS - 1 ? wave_total : F::apply(total, wave_total);
+  }
+  return total;
+}
+
 // Executed by the first wave of the block.  Publishes the tile's aggregate,
 // resolves the exclusive prefix of the tile and publishes the inclusive one.
-// `fold(t)` is the aggregate of tile t from the input, for a tile that has not published it within
-// `limit` polls.
+// `fold(t)` is the aggregate of tile t from the input, by the whole wave, for a tile that has not published it
+// within `limit` polls.
 template <typename T, int OP, int STRIDE, typename Fold>
 __device__ __forceinline__ T resolve_prefix(const TileState<T, STRIDE>& st, int tile,
                                             T aggregate, int lane, uint32_t limit, const Fold& fold) {
@@ -304,10 +324,21 @@ __device__ __forceinline__ T resolve_prefix(const TileState<T, STRIDE>& st, int 
   while (true) {
     const int idx = base - (kWaveSize - 1 - lane);  // in the input's order: of two NaNs the first wins
     T val = F::identity();
-    uint32_t flag = kFlagPrefix;  // virtual prefix in front of tile 0
-    if (idx >= 0) {
-      flag = st.wait(idx, &val, limit);
-      if (flag == kFlagInvalid) val = fold(idx);
+    uint32_t flag = idx >= 0 ? kFlagInvalid : kFlagPrefix;  // virtual prefix in front of tile 0
+    for (uint32_t polls = 0;; ++polls) {
+      if (flag == kFlagInvalid) flag = st.read(idx, &val);
+      const uint64_t missing = __ballot(flag == kFlagInvalid);
+      if (missing == 0) break;
+      if (limit == kNoLimit || polls < limit) {
+        __builtin_amdgcn_s_sleep(1);
+        continue;
+      }
+      const int late = kWaveSize - 1 - __builtin_clzll(missing);
+      const T folded = fold(base - (kWaveSize - 1 - late));
+      if (lane == late) {
+        val = folded;
+        flag = kFlagAggregate;
+      }
     }
     const uint64_t has_prefix = __ballot(flag == kFlagPrefix);
     // The nearest inclusive prefix ends the walk.
@@ -332,14 +363,40 @@ __device__ __forceinline__ T resolve_prefix_at_once(const TileState<T, STRIDE>& 
   using F = Functor<T, OP>;
   if (threadIdx.x == 0) st.publish(tile, kFlagAggregate, aggregate);
   constexpr int kPer = (int)(kShortMaxTiles * kShortDivisor + kBlock - 1) / kBlock;
-  T val = F::identity();
+  T of_tile[kPer];
+  uint32_t waits = 0;  // a bit per tile
 #pragma unroll
   for (int p = 0; p < kPer; ++p) {
-    const int front = (int)threadIdx.x * kPer + p;
-    T one = F::identity();
-    if (front < tile && st.wait(front, &one, limit) == kFlagInvalid) one = fold(front);
-    val = F::apply(val, one);
+    of_tile[p] = F::identity();
+    if ((int)threadIdx.x * kPer + p < tile) waits |= 1u << p;
   }
+  for (uint32_t polls = 0;; ++polls) {
+#pragma unroll
+    for (int p = 0; p < kPer; ++p)
+      if ((waits >> p & 1u) != 0u && st.read((int)threadIdx.x * kPer + p, &of_tile[p]) != kFlagInvalid)
+        waits &= ~(1u << p);
+    const uint64_t missing = __ballot(waits != 0u);
+    if (missing == 0) break;
+    if (polls < limit) {
+      __builtin_amdgcn_s_sleep(1);
+      continue;
+    }
+    const int late = __builtin_ctzll(missing);
+    const int of_late = __builtin_ctz((uint32_t)__builtin_amdgcn_readlane((int)waits, late));
+    const int front = (wave * kWaveSize + late) * kPer + of_late;
+    const T folded = fold(front);
+    // (For the tiles behind, which wait for it as well; the tile itself publishes the same bits.)
+    if (lane == 0) st.publish(front, kFlagAggregate, folded);
+#pragma unroll
+    for (int p = 0; p < kPer; ++p) {
+      if (lane != late || p != of_late) continue;
+      of_tile[p] = folded;
+      waits &= ~(1u << p);
+    }
+  }
+  T val = of_tile[0];
+#pragma unroll
+  for (int p = 1; p < kPer; ++p) val = F::apply(val, of_tile[p]);
   const T front = wave_fold<T, OP>(val, lane);
   if (lane == 0) s_front[wave] = front;
   __syncthreads();
@@ -367,7 +424,7 @@ __global__ __launch_bounds__(kBlock, ILGPU_HIP_SCAN_WAVES_PER_EU) void scan_kern
 
   __shared__ int s_tile;
   __shared__ T s_wave_total[kWaves];
-  __shared__ T s_front[kWaves];  // of a short tile: what lies in front, in parts of 64 tiles
+  __shared__ T s_front[kWaves];  // of a short tile: what lies in front, a part per wave
   __shared__ T s_prefix;
   constexpr bool kShort = VECS != scan_vecs<T>();
 
@@ -427,26 +484,15 @@ __global__ __launch_bounds__(kBlock, ILGPU_HIP_SCAN_WAVES_PER_EU) void scan_kern
     }
   }
 
-  // A full tile's elements, in parts, so that a floating-point sum is as exact as a tile's own.
-  auto fold_tile = [&](int t) -> T {
-    constexpr int kPart = 64;
-    static_assert(kTile % kPart == 0, "whole parts");
-    T sum = F::identity();
-    for (int e0 = 0; e0 < kTile; e0 += kPart) {
-      T part = F::identity();
-      for (int e = e0; e < e0 + kPart; ++e) part = F::apply(part, in[((int64_t)t * kTile + e) * in_stride]);
-      sum = F::apply(sum, part);
-    }
-    return sum;
-  };
+  auto fold = [&](int t) -> T { return fold_tile<T, OP, VECTOR, VECS>(in, in_stride, t, lane); };
   auto prefix_of_tile = [&](T block_total) -> T {
     if (alone) return F::identity();
     if (kShort && ticket == nullptr && !ILGPU_HIP_SCAN_PROBE_NO_LOOKBACK)
-      return resolve_prefix_at_once<T, OP>(st, tile, block_total, wave, lane, s_front, limit, fold_tile);
+      return resolve_prefix_at_once<T, OP>(st, tile, block_total, wave, lane, s_front, limit, fold);
     if (wave == 0) {
       const T exclusive = ILGPU_HIP_SCAN_PROBE_NO_LOOKBACK
                               ? F::identity()
-                              : resolve_prefix<T, OP>(st, tile, block_total, lane, limit, fold_tile);
+                              : resolve_prefix<T, OP>(st, tile, block_total, lane, limit, fold);
       if (lane == 0) s_prefix = exclusive;
     }
     __syncthreads();

@@ -1762,6 +1762,69 @@ def test_scan_into_another_view_and_over_its_input(dtype, op, polls):
         capi.sort_set_parameter(capi.SORT_PARAM_LOOKBACK_SPIN_LIMIT, -1)
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("form", ["aligned", "from the second element", "every third element"])
+@pytest.mark.parametrize("polls", [-1, 0])
+def test_scan_sums_of_folded_tiles_are_as_exact_as_the_tiles_own(dtype, form, polls):
+    # A tile of a one and then numbers so small that a chain of additions, 64 of them at a time, would lose them all, and
+    # a tile that takes it all away again, in turns: every prefix of whole tiles is 0 or a tile's sum, exactly, if
+    # a tile that is folded (with 0 polls every one that is late) comes out bit for bit as the tile itself would have it.
+    # Then a result has the roundings of its own tile alone, none of anything larger than the tile's sum: of a tile of 16 (4)
+    # rows 3 in a vector of four (1 of two), 6 between lanes, 15 (3) rows and 7 waves in front, 1 for the tiles
+    # in front, 15 (3) rows to the wave's own, 2 to the lane's.
+    real = np.dtype(dtype)
+    full = 512 * 16 * 16 // real.itemsize
+    capi.sort_set_parameter(capi.SORT_PARAM_LOOKBACK_SPIN_LIMIT, polls)
+    try:
+        for tile, n in ((full // 4, 44 * (full // 4) - 3), (full, 195 * full + 1)):
+            roundings = 16 // real.itemsize - 1 + 6 + 2 * (tile * real.itemsize // 8192 - 1) + 7 + 1 + 2
+            small = np.longdouble(dtype(0.9 * 2.0 ** (-25 if real.itemsize == 4 else -54) / 64))
+            at = np.arange(n, dtype=np.int64) % tile
+            falls = np.arange(n, dtype=np.int64) // tile % 2 == 1
+            values = np.where(at == 0, 1, small).astype(dtype)
+            values[falls] = -values[falls]
+            rest = np.where(falls, tile - 1 - at, at).astype(np.longdouble)
+            want = np.where(falls, 0, 1) + rest * small
+            step, first = (3, 0) if form == "every third element" else (1, 1 if form != "aligned" else 0)
+            room = D.zeros(first + n * step, dtype)
+            spread = np.zeros(first + n * step, dtype)
+            spread[first::step] = values
+            room.bytes.copy_(D.from_numpy(spread).bytes)
+            source = room.strided(step) if step > 1 else room.subview(first, n)
+            target = D.zeros(n, dtype)
+            note("scan folds", real.name, form, polls, n)
+            capi.scan(source, target, op=capi.OP_ADD)
+            sync()
+            worst = np.abs(target.numpy().astype(np.longdouble) - want).max()
+            assert worst <= roundings * np.finfo(dtype).eps / 2 * (1 + tile * small), (n, float(worst))
+    finally:
+        capi.sort_set_parameter(capi.SORT_PARAM_LOOKBACK_SPIN_LIMIT, -1)
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.float64])
+def test_scan_that_folds_its_late_tiles_is_not_slow(dtype):
+    # With 0 polls most tiles of the first blocks are folded by those behind them: by whole waves, three to four times
+    # the ordinary scan; by single lanes, element after element, 16 to 80 times.
+    import torch
+    for n in (1 << 20, 1 << 26):
+        source, target = D.zeros(n, dtype), D.zeros(n, dtype)
+        temp = capi.temp_buffer(capi.scan_temp_bytes(n, dtype))
+        took = []
+        for polls in (-1, 0):
+            capi.sort_set_parameter(capi.SORT_PARAM_LOOKBACK_SPIN_LIMIT, polls)
+            note("scan folds in time", np.dtype(dtype).name, n, polls)
+            best = float("inf")
+            for _ in range(6):
+                begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                begin.record()
+                capi.scan(source, target, temp, op=capi.OP_ADD)
+                end.record()
+                sync()
+                best = min(best, begin.elapsed_time(end))
+            took.append(best)
+        assert took[1] <= 10 * took[0], (n, took)
+
+
 @pytest.mark.parametrize("dtype", [np.int32, np.int64, np.float32, np.float64])
 @pytest.mark.parametrize("first", [0, 1])
 def test_scan_of_a_last_tile_that_ends_inside_a_vector(dtype, first):
