@@ -1734,29 +1734,30 @@ def test_scan_edges_of_the_short_tiles(dtype):
 
 @pytest.mark.parametrize("dtype,op", [(np.int32, capi.OP_ADD), (np.int64, capi.OP_ADD), (np.float64, capi.OP_MAX)])
 @pytest.mark.parametrize("polls", [-1, 0])
-def test_scan_into_another_view_and_over_its_input(dtype, op, polls):
+@pytest.mark.parametrize("first", [1, 4])
+def test_scan_into_another_view_and_over_its_input(dtype, op, polls, first):
     # Output apart from the input: no tickets, short tiles up to 192 full ones, and a tile that has not
     # published is folded from the input after `polls` (0: every one that is late).  Output over the input, or
-    # one element in front of it: tickets, and nothing is folded.
+    # one element in front of it: tickets, and nothing is folded.  Of views that begin at a multiple of 16 bytes, which
+    # go by vectors, and of others.
     size = np.dtype(dtype).itemsize
     full = 512 * 16 * 16 // size
     reference = {capi.OP_ADD: np.cumsum, capi.OP_MAX: np.maximum.accumulate}[op]
     capi.sort_set_parameter(capi.SORT_PARAM_LOOKBACK_SPIN_LIMIT, polls)
     try:
         for n in (full + 1, 63 * full + 5, 64 * full + 1, 192 * full, 192 * full + 1):
-            if polls == 0 and n > 64 * full + 1 and size == 8:
-                continue  # some seconds of folding
             values = random_ints(np.int32, n, seed=n, lo=-3, hi=4).astype(dtype)
             want = reference(values, dtype=dtype)
-            for shift in (n, 0, -1):  # elements from the input to the output
-                note("scan", np.dtype(dtype).name, n, polls, shift)
-                room = D.zeros(2 * n + 2, dtype)
-                source, target = room.subview(1, n), room.subview(1 + shift, n)
+            apart = -(-n // 4) * 4
+            for shift in (apart, 0, -1):  # elements from the input to the output
+                note("scan", np.dtype(dtype).name, n, polls, first, shift)
+                room = D.zeros(2 * n + 8, dtype)
+                source, target = room.subview(first, n), room.subview(first + shift, n)
                 source.bytes.copy_(D.from_numpy(values).bytes)
                 capi.scan(source, target, op=op)
                 sync()
                 assert np.array_equal(target.numpy(), want), shift
-                if shift == n:
+                if shift == apart:
                     assert np.array_equal(source.numpy(), values)
     finally:
         capi.sort_set_parameter(capi.SORT_PARAM_LOOKBACK_SPIN_LIMIT, -1)
