@@ -1371,6 +1371,22 @@ def test_unique_of_long_tiles(dtype):
             assert count == want.size and np.array_equal(kept, want), (n, runs)
 
 
+@pytest.mark.parametrize("dtype", [np.uint32, np.float32])
+def test_unique_of_long_tiles_unaligned(dtype):
+    # The same tiles where no vector of the view is aligned: element by element, ending in the last tile and with it.
+    for n in (512 * 32768, 512 * 32768 + 2 * 32768 - 3):
+        note("unique long tiles unaligned", np.dtype(dtype).name, n)
+        values = np.sort(np.random.default_rng(n).integers(0, n // 2, n, dtype=np.int32)).astype(dtype)
+        want = values[np.concatenate([[True], values[1:] != values[:-1]])]
+        room = D.from_numpy(np.concatenate([np.array([7], dtype), values, np.array([9], dtype)]))
+        length = D.zeros(1, np.int64)
+        capi.unique(room.subview(1, n), length)
+        sync()
+        got = room.numpy()
+        assert length.numpy()[0] == want.size and np.array_equal(got[1:1 + want.size], want), n
+        assert got[0] == 7 and got[-1] == 9
+
+
 def test_unique_unaligned_view():
     vals = np.repeat(np.arange(5000, dtype=np.int32), 3)
     base = D.from_numpy(np.concatenate([np.array([99], np.int32), vals]))
