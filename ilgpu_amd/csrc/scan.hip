@@ -419,7 +419,10 @@ __device__ __forceinline__ T resolve_prefix_at_once(const TileState<T, STRIDE>& 
 // the compiler takes 180 to 256 registers for the floating-point Max and Min
 // kernels, which halves their residency (0.56 -> 0.44 ms at 2^28 float, 0.36 since those
 // take three compares: fp_extreme).
-template <typename T, int OP, bool VECTOR, int VECS>
+// TICKETS: with tiles by tickets; a kernel apart, since with both look-backs in it one over its input took longer
+// than before there were two (us, one kernel / two: 10^6 int64 11.65 / 11.15, 2 * 10^6 int32 10.7 / 10.4, 2^22 int64 18.6 / 18.2,
+// 10^7 float 21.75 / 20.7; into another view the same).
+template <typename T, int OP, bool VECTOR, int VECS, bool TICKETS>
 __global__ __launch_bounds__(kBlock, ILGPU_HIP_SCAN_WAVES_PER_EU) void scan_kernel(
     const T* __restrict__ in, T* __restrict__ out, int64_t n,
     int64_t in_stride, int64_t out_stride, int inclusive,
@@ -439,12 +442,12 @@ __global__ __launch_bounds__(kBlock, ILGPU_HIP_SCAN_WAVES_PER_EU) void scan_kern
 
   // An input of one tile comes without status words (and without
   // the launch that clears them): there is nobody to wait for or to tell.
-  const bool alone = gridDim.x == 1;
-  if (ticket != nullptr) {
+  const bool alone = !TICKETS && gridDim.x == 1;
+  if constexpr (TICKETS) {
     if (threadIdx.x == 0) s_tile = (int)atomicAdd(ticket, 1u);
     __syncthreads();
   }
-  const int tile = ticket != nullptr ? s_tile : (int)blockIdx.x;
+  const int tile = TICKETS ? s_tile : (int)blockIdx.x;
   const int lane = threadIdx.x & (kWaveSize - 1);
   // The wave index and everything derived from it are wave-uniform: kept in
   // scalar registers, so a lane addresses its vectors by one 32-bit offset.
@@ -496,12 +499,12 @@ __global__ __launch_bounds__(kBlock, ILGPU_HIP_SCAN_WAVES_PER_EU) void scan_kern
   auto fold = [&](int t) -> T { return fold_tile<T, OP, VECTOR, VECS>(in, in_stride, t, lane); };
   auto prefix_of_tile = [&](T block_total) -> T {
     if (alone) return F::identity();
-    if (kShort && ticket == nullptr && !ILGPU_HIP_SCAN_PROBE_NO_LOOKBACK)
+    if constexpr (kShort && !TICKETS && !ILGPU_HIP_SCAN_PROBE_NO_LOOKBACK)
       return resolve_prefix_at_once<T, OP>(st, tile, block_total, wave, lane, s_front, limit, fold);
     if (wave == 0) {
       const T exclusive = ILGPU_HIP_SCAN_PROBE_NO_LOOKBACK
                               ? F::identity()
-                              : resolve_prefix<T, OP>(st, tile, block_total, lane, limit, fold);
+                              : resolve_prefix<T, OP>(st, tile, block_total, lane, TICKETS ? kNoLimit : limit, fold);
       if (lane == 0) s_prefix = exclusive;
     }
     __syncthreads();
@@ -871,17 +874,10 @@ int32_t launch_tiles(hipStream_t stream, const void* in, int64_t in_stride,
                       (reinterpret_cast<uintptr_t>(out) & 15) == 0;
   const int inclusive = kind == ILGPU_HIP_SCAN_INCLUSIVE ? 1 : 0;
   ProfileScope scope(stream, "scan");
-  if (vector) {
-    hipLaunchKernelGGL((scan_kernel<T, OP, true, VECS>), dim3((unsigned)tiles),
-                       dim3(kBlock), 0, stream, static_cast<const T*>(in),
-                       static_cast<T*>(out), n, in_stride, out_stride,
-                       inclusive, ticket, st, limit);
-  } else {
-    hipLaunchKernelGGL((scan_kernel<T, OP, false, VECS>), dim3((unsigned)tiles),
-                       dim3(kBlock), 0, stream, static_cast<const T*>(in),
-                       static_cast<T*>(out), n, in_stride, out_stride,
-                       inclusive, ticket, st, limit);
-  }
+  auto* kernel = ticket != nullptr ? (vector ? scan_kernel<T, OP, true, VECS, true> : scan_kernel<T, OP, false, VECS, true>)
+                                   : (vector ? scan_kernel<T, OP, true, VECS, false> : scan_kernel<T, OP, false, VECS, false>);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(kBlock), 0, stream, static_cast<const T*>(in),
+                     static_cast<T*>(out), n, in_stride, out_stride, inclusive, ticket, st, limit);
   ILGPU_HIP_CHECK(hipGetLastError());
   return ILGPU_HIP_SUCCESS;
 }
