@@ -1427,16 +1427,35 @@ __device__ __forceinline__ void sort_tile(
     // Keys with this digit in earlier tiles: walk back over the status words,
     // kLookback tiles per step.  The loads of a step are unconditional (index
     // clamped) so that they are in flight together; positions in front of
-    // tile 0 read as an empty inclusive prefix.  A step's loads stand at the end of the one in front of it: where a step
-    // chose between them and first_step at its begin, the compiler waited for one before it issued the next.
-    // (Sorts with a copy in front, us, so / now: 10^7 normal doubles 331 / 321, 20 000 003 normal floats 277 / 265.5, 14 * 10^6 u32 below
-    // 10^6 175 / 171, pairs of 8 * 10^6 u32 174 / 169, of 2^26 below 10^6 with their index 1052 / 1035.)
+    // tile 0 read as an empty inclusive prefix.  Where a step chose for every word between the load and first_step, the
+    // compiler waited for one before it issued the next.  So keys alone have a step's loads at the end of the one in front
+    // of it, and pairs, whose registers that spills, one choice for all the words of a step.
+    // (Sorts with a copy in front, us, word by word / at the end / one choice: 10^7 normal doubles 331 / 321 / 321, 20 000 003 normal
+    // floats 277 / 265 / 272, 14 * 10^6 u32 below 10^6 175 / 171 / 172; pairs of 8 * 10^6 u32 173 / 169 / 169, of 2^26 u32 below 10^6 with
+    // their index 1051 / 1034 / 1035, of 12 * 10^6 normal doubles with bytes 451 / 461 / 450.)
     uint32_t before = 0;
     bool done = tile == 0;
     uint32_t s[kLookback];
+    if constexpr (!kPairs) {
 #pragma unroll
-    for (int u = 0; u < kLookback; ++u) s[u] = first_step[u];
+      for (int u = 0; u < kLookback; ++u) s[u] = first_step[u];
+    }
+    bool preloaded = true;
     for (int t = tile - 1; !done; t -= kLookback) {
+      if constexpr (kPairs) {
+        if (preloaded) {
+#pragma unroll
+          for (int u = 0; u < kLookback; ++u) s[u] = first_step[u];
+        } else {
+#pragma unroll
+          for (int u = 0; u < kLookback; ++u) {
+            const int idx = t - u < 0 ? 0 : t - u;
+            s[u] = __hip_atomic_load(&status[(int64_t)idx * kRadix + tid], __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_AGENT);
+          }
+        }
+        preloaded = false;
+      }
 #pragma unroll
       for (int u = 0; u < kLookback; ++u)
         if (t - u < 0) s[u] = status_prefix(0u);
@@ -1461,12 +1480,14 @@ __device__ __forceinline__ void sort_tile(
         before += status_value(s[u]);
         done = !status_is_aggregate(s[u]);
       }
-      if (done) break;
+      if constexpr (!kPairs) {
+        if (done) break;
 #pragma unroll
-      for (int u = 0; u < kLookback; ++u) {
-        const int next = t - kLookback - u;
-        s[u] = __hip_atomic_load(&status[(int64_t)(next < 0 ? 0 : next) * kRadix + tid],
-                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int u = 0; u < kLookback; ++u) {
+          const int next = t - kLookback - u;
+          s[u] = __hip_atomic_load(&status[(int64_t)(next < 0 ? 0 : next) * kRadix + tid],
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
       }
     }
     if (tile > 0)
