@@ -3597,9 +3597,12 @@ int32_t launch_sized(hipStream_t stream, const SortArgs& a) {
   int32_t rc;
   // Full tiles, no more of them than run at the same time, two per compute unit, look back as short ones do.
   // (Not every value size is worth two more kernels.
-  // Full tiles of 4-byte keys would spill: 2^23 u32 keys 125 -> 132 us.)
+  // Full tiles of 4-byte keys would spill: 2^23 u32 keys 125 -> 132 us.)  Two tiles walk: the second one needs one word, for which
+  // the other look-back has a barrier more (pairs with a copy in front, us, at once / a walk: 13 619 u32 with u64 53.6 / 52.3, 15 564 floats
+  // with u32 56.0 / 54.3, 9728 doubles with u64 83.7 / 82.2; but 9318 doubles with u32, whose walk spills, 101.4 / 104).
   constexpr bool kAtOnce = VALUE_BYTES == 0 ? KEY_BYTES == 8 : KEY_BYTES >= 4 && (VALUE_BYTES == 4 || VALUE_BYTES == 8);
-  const bool full_at_once = kAtOnce && !use_large && short_items == 0 && !float_tiles && L.tiles <= 2 * (int64_t)cus;
+  const bool full_at_once = kAtOnce && !use_large && short_items == 0 && !float_tiles &&
+                            L.tiles > (KEY_BYTES == 8 && VALUE_BYTES == 4 ? 0 : 2) && L.tiles <= 2 * (int64_t)cus;
   const bool turns = sort_status_turns(KEY_BYTES, use_large ? kSortBlockLarge : kSortBlock,
                                        short_items > 0 || full_at_once, float_tiles);
   const int64_t words = ((turns ? L.status + L.status_stride : L.total) - L.zero_begin) / 4;

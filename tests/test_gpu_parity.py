@@ -1128,6 +1128,22 @@ def test_one_tile_of_512_or_1024_threads(dtype):
                     assert bits_equal(k, ek) and np.array_equal(v, ev)
 
 
+@pytest.mark.parametrize("key,value,full", [
+    (np.uint32, np.uint32, 8192), (np.float32, np.uint32, 8192), (np.uint32, np.uint64, 7168), (np.float32, np.uint64, 7168),
+    (np.uint64, np.uint32, 7168), (np.float64, np.uint32, 7168), (np.uint64, np.uint64, 5120), (np.float64, np.uint64, 5120)])
+def test_pairs_of_one_to_three_tiles(key, value, full):
+    # One tile in one launch, by 512 or 1024 threads; two that walk, or look back at once as three do.
+    for n in (full - 1, full, full + 1, 2 * full, 2 * full + 1, 3 * full):
+        keys = np.random.default_rng(n).integers(0, 1 << 62, n).astype(np.uint64)
+        keys = (keys if np.dtype(key).kind == "u" else keys % (n // 2)).astype(key)
+        values = np.arange(n, dtype=value)
+        for descending in (False, True):
+            note("pairs of few tiles", np.dtype(key).name, np.dtype(value).name, n, descending)
+            k, v = gpu_sort_pairs(keys, values, descending=descending)
+            ek, ev = O.radix_sort_pairs(keys, values, descending=descending)
+            assert bits_equal(k, ek) and np.array_equal(v, ev), n
+
+
 @pytest.fixture
 def no_short_tiles():
     """Short inputs of keys take full tiles like pairs and longer inputs do."""
