@@ -2433,10 +2433,12 @@ constexpr int kSmallSortItemsA = 4, kSmallSortItemsB = 12, kSmallSortItemsC = 24
 // LDS together, where there are more rows than four; of 8-byte keys, which sort few digits and look at their neighbours, the
 // floating-point ones, which sort all digits; of shorter keys, which have one or two digits, only the longest tiles.  (Sorts with a copy in front, us, 512 / 1024 threads: u32 keys 4000 12.6 / 11.8,
 // 9000 20.1 / 18.1, 18 000 30.1 / 24.8, below 10^6 24.3 / 20.5; normal floats 6000 19.0 / 16.4, 18 000 49.2 / 36.5; normal doubles 9000
-// 32.4 / 30.2; but u64 keys below 10^6 9000 17.7 / 18.2, Zipf 17.2 / 18.1, pairs of 5000 u64 21.6 / 23.7, u16 keys 6000 11.4 / 12.9, 18 000 16.8 / 14.3.)
+// 32.4 / 30.2; but u64 keys below 10^6 9000 17.7 / 18.2, Zipf 17.2 / 18.1, pairs of 5000 u64 21.6 / 23.7, u16 keys 6000 11.4 / 12.9, 18 000 16.8 / 14.3.
+// Pairs of integers whose rows do not halve into an even number keep 512: 7000 u32 with u64 15.9 / 17.1 in the kernel.)
 constexpr int small_sort_block(int key_bytes, int value_bytes, bool floats, int rows) {
   const bool wide = key_bytes == 8 ? floats && value_bytes == 0 && rows > kSmallSortItemsA
-                                   : rows > (key_bytes == 4 ? kSmallSortItemsA : kSmallSortItemsC);
+                                   : rows > (key_bytes == 4 ? kSmallSortItemsA : kSmallSortItemsC) &&
+                                         (value_bytes == 0 || rows % 4 == 0 || floats);
   return wide ? 2 * kSortBlock : kSortBlock;
 }
 constexpr int small_sort_items(int block, int rows) { return block == kSortBlock ? rows : (rows / 2 + 1) / 2 * 2; }
