@@ -419,6 +419,25 @@ def test_histogram_floating_point_bins_that_many_blocks_add_to(bin_dtype, bins):
         assert overflow == (want_overflow if checked else 0)
 
 
+@pytest.mark.parametrize("bin_dtype", [np.int32, np.float32])
+@pytest.mark.parametrize("bins", [4096, 12000])
+def test_histogram_crowds_in_what_a_round_leaves(bin_dtype, bins):
+    # Up to three vectors of a thread that are no whole round: of lanes that mostly meet in one bin, that do not, that end
+    # inside the wave, and of values that are no bin.  128 to 256 blocks of 1024 threads take four vectors of four ints a round.
+    round_ = 128 * 1024 * 16
+    for n in (4, 255, 4 * 1024 + 3, round_ // 4 - 1, round_ // 2 + 9, round_ - 64, round_ + round_ // 3):
+        values = np.random.default_rng(n).integers(0, bins, n).astype(np.int32)
+        crowd = np.arange(n) // 1024 % 3 != 0
+        values[crowd] = 77
+        values[::97] = -1
+        values[5::193] = bins
+        note("histogram crowds left", np.dtype(bin_dtype).name, bins, n)
+        got, overflow = gpu_histogram(values, np.zeros(bins, bin_dtype), capi.LOCATOR_IDENTITY)
+        inside = values[(values >= 0) & (values < bins)]
+        assert np.array_equal(got, np.bincount(inside, minlength=bins).astype(bin_dtype)), n
+        assert overflow == 0
+
+
 # --------------------------------------------------------------- radix sort
 def gpu_sort(keys, **kw):
     d = D.from_numpy(keys)
