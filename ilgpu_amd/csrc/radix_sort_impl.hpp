@@ -336,9 +336,11 @@ struct SortPlan {
 static_assert(sizeof(SortPlan) <= 256, "the temp view holds 256 bytes for the plan");
 
 // Passes that take turns with two status arrays: each clears the words of the next one that runs, which the pass before it is
-// done with, and only the first array is cleared beforehand.  In tiles of all lengths but full ones of 512 threads, which lose
-// half a percent by it (14 * 10^6 u32 keys 175 -> 176 us): 2^27 u64 keys clear 9 MB of 75 (2004 -> 1995 us a sort), 2^28 u32 8
-// of 32 (2062 -> 2054), and tiles shorter than what the temp view is sized for find room.
+// done with, and only the first array is cleared beforehand.  Tiles shorter than what the temp view is sized for find room that
+// way (tiles that all run at once, floating-point ones), and 2^27 u64 keys clear 9 MB in place of 75 (us, an array for every pass / turns:
+// 2005 / 1994, with index values 2708 / 2699).  Long 4-byte keys, of which two of four passes run, take as long either way
+// (2^26 to 2^28 u32 keys within 0.5 %, which is what two builds of the same code differ by); full tiles of 512 threads lose half a
+// percent (14 * 10^6 u32 keys 175 / 176) and have an array for every pass.
 constexpr bool sort_status_turns(int key_bytes, int block, bool at_once, bool float_tile) {
   return key_bytes > 1 && (block > ILGPU_HIP_SORT_BLOCK || at_once || float_tile);
 }
@@ -1109,13 +1111,16 @@ __device__ __forceinline__ void load_tile_keys(
 // registers (36 keys and 18 registers of packed ranks in a keys-only sort;
 // fewer items when values ride along) and the blocks of a CU at 160 KiB of
 // LDS together (a 36-key tile stages 72 KiB per 512 threads).
-// Where the code of the large kernels begins.  A tile runs through 40 to 64 KiB of code, which the instruction caches
-// barely hold, and where it lies moved the same instructions by up to 8 us a pass whenever a kernel in front of it
-// grew.  (2^28 u32, us, two boxes, wherever the linker puts it / here: 2059 / 2053 and 2053 / 2048; the others within 0.2 %.)
-#define ILGPU_HIP_SORT_CODE_ALIGNED __attribute__((aligned(4096)))
 #ifndef ILGPU_HIP_SORT_WAVES_PER_EU
 #define ILGPU_HIP_SORT_WAVES_PER_EU 4
 #endif
+
+// Where the code of the large kernels begins: at a fixed place, so that what is added to one kernel does not move the others.  A tile
+// runs through 40 to 64 KiB of code, about what the instruction caches hold, and the same instructions take up to 1 % longer at
+// another address.  This one is no better than any other by rule: it measured well, and what grows inside a kernel still moves its
+// own loops.  (us, wherever the linker puts it / here, in one process: u32 2^25 314.5 / 310.5, 50 * 10^6 458.5 / 456.5, 2^26 below
+// 10^6 636 / 631, 2^28 2063 / 2059; u64 2^24 to 2^27, pairs and floats within 0.3 % either way.)
+#define ILGPU_HIP_SORT_CODE_ALIGNED __attribute__((aligned(4096)))
 
 // Tile of a group's k-th draw: its chunks are g, g + 8, g + 16, ... of
 // 2^chunk_shift consecutive tiles.
@@ -1367,7 +1372,8 @@ __device__ __forceinline__ void sort_tile(
     // trips behind each other, since the group's last tile sums its group before the others see it.
     // (Inside a pass of 2^21 u32 keys, 342 tiles, the slowest tile waits 4 us for it instead of 7.6.  Sorts with a copy
     // in front, us, a walk / this: u32 keys 2^20 55.0 / 48.9, 2^21 69.4 / 63.2, below 10^6 2^20 63.1 / 53.6; normal floats
-    // 2^20 74.1 / 64.7; pairs of 2^21 u32 85.2 / 77.4, 2^20 Zipf 60.5 / 53.4, of 2^20 u64 with u32 85.7 / 79.2.)
+    // 2^20 74.1 / 64.7; pairs of 2^21 u32 85.2 / 77.4, 2^20 Zipf 60.5 / 53.4, of 2^20 u64 with u32 85.7 / 79.2; u16 keys 600 000 35.2 / 30.4, 2^20
+    // 39.1 / 32.6, 3 * 10^6 54.2 / 45.0; u8 keys 600 000 28.1 / 26.0, 2^20 30.6 / 27.7, 3 * 10^6 38.0 / 33.5; but 130 000 u16 32.4 / 33.0 and u8 26.7 / 27.2.)
     const uint32_t d = (uint32_t)tid & (kRadix - 1);
     const bool groups = __builtin_amdgcn_readfirstlane(tid) >= kRadix;
     const int group = tile / kLookGroup;
