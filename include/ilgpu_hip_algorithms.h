@@ -335,10 +335,11 @@ int32_t ilgpu_hip_reduce(ilgpu_hip_stream_t stream, const void *in,
  * HistogramOperations.tt:36-40); NULL selects the unchecked variant.
  * in_type: any ilgpu_hip_type except F16.
  * Floating-point bins must live in ordinary device memory (hipMalloc: coarse
- * grained).  With more bins than LDS holds their single increments go through
- * the hardware's floating-point atomic add in L2, which is exact there; for
- * fine-grained, host-mapped or managed memory the hardware does not promise
- * that, and no reference fixture covers floating-point bins at all.
+ * grained).  The counts of a block, and with more bins than LDS holds single
+ * increments, go through the hardware's floating-point atomic add in L2, which
+ * is exact there; for fine-grained, host-mapped or managed memory the hardware
+ * does not promise that, and no reference fixture covers floating-point bins
+ * at all.
  */
 int32_t ilgpu_hip_histogram(ilgpu_hip_stream_t stream, const void *in,
                             int64_t n, int64_t stride, int32_t in_type,
