@@ -495,12 +495,20 @@ __global__ __launch_bounds__(form_block(FORM)) void histogram_lds_kernel(
     return c;
   };
   // (Integer bins one step at a time where there are more blocks than compute units, which hide each other's trips: eight at once
-  // cost 2000 int64 bins of 12 * 10^6 ints 24.55 us in place of 23.9, 2^24 into 3000 27.0 in place of 26.6.)
+  // cost 2000 int64 bins of 12 * 10^6 ints 24.55 us in place of 23.9, 2^24 into 3000 27.0 in place of 26.6.  And where a thread of the
+  // strided form has fewer than eight: every second of 16 * 10^6 ints into 256 bins 27.4 in place of 26.7, into 2000 19.7 in place of
+  // 19.1, but into 4096 26.35 in place of 26.6 and into 12000 33.8 in place of 34.7.)
   auto flush = [&](auto one) {
     using B = decltype(one);
     constexpr int kFlushSteps = FORM == kFormPlain || (FORM == kFormCrowded && !is_fp<B>::value) ? 1 : 8;
-    passed = flush_bins<B, kBlock, kFlushSteps>(
-        bins, num_bins, first_bin, checked, bin_type == ILGPU_HIP_I32 || bin_type == ILGPU_HIP_I64, count_of);
+    auto by = [&](auto steps) {
+      passed = flush_bins<B, kBlock, decltype(steps)::value>(
+          bins, num_bins, first_bin, checked, bin_type == ILGPU_HIP_I32 || bin_type == ILGPU_HIP_I64, count_of);
+    };
+    if constexpr (FORM == kFormStrided && !is_fp<B>::value) {
+      if (num_bins < kFlushSteps * kBlock) return by(std::integral_constant<int, 1>{});
+    }
+    by(std::integral_constant<int, kFlushSteps>{});
   };
   if (FORM == kFormPlain && bin_type != ILGPU_HIP_F32 && bin_type != ILGPU_HIP_F64) {
     // (Few bins, of which a thread has one to three: steps cost 2 % of 16 MiB of bytes, and their registers a

@@ -438,6 +438,31 @@ def test_histogram_crowds_in_what_a_round_leaves(bin_dtype, bins):
         assert overflow == 0
 
 
+@pytest.mark.parametrize("bin_dtype", [np.int32, np.uint32, np.int64, np.uint64, np.float64])
+@pytest.mark.parametrize("bins", [2049, 4095, 4096, 4097])
+def test_histogram_flush_of_strided_views_and_of_many_blocks(bin_dtype, bins):
+    # Integer bins one step at a time below eight for a thread of 512, from there on eight at once; and one step in dense views
+    # with more blocks than compute units (a block per 16 elements of every bin).  Some bins one count from their MaxValue.
+    largest = np.finfo(bin_dtype).max if np.dtype(bin_dtype).kind == "f" else np.iinfo(bin_dtype).max
+    for n, stride in ((90001, 2), (257 * 16 * bins + 77, 1)):
+        values = random_ints(np.int32, n, seed=n, lo=0, hi=bins - 1)
+        full = np.zeros(bins, bin_dtype)
+        if np.dtype(bin_dtype).kind != "f":
+            full[[0, 511, bins - 1]] = largest - np.array([2 * n, 1, 2 * n]).astype(bin_dtype)
+        for before in (np.zeros(bins, bin_dtype), full):
+            note("histogram flush", np.dtype(bin_dtype).name, bins, n, stride, int(before is full))
+            source = D.from_numpy(np.repeat(values, stride))
+            source = source.strided(stride) if stride > 1 else source
+            target, overflow = D.from_numpy(before), D.zeros(1, np.int32)
+            capi.histogram(source, target, overflow)
+            sync()
+            count = np.bincount(values, minlength=bins)
+            with np.errstate(over="ignore"):
+                want = before + count.astype(bin_dtype)
+            assert np.array_equal(target.numpy(), want)
+            assert int(overflow.numpy()[0]) == int(bool(before[511]) and count[511] > 1)
+
+
 # --------------------------------------------------------------- radix sort
 def gpu_sort(keys, **kw):
     d = D.from_numpy(keys)
